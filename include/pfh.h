@@ -326,14 +326,13 @@ typedef struct pfh_schedule {
     int32_t column_block;     /* threads per workgroup of the per-column propagate kernel */
     int32_t xcd_order;        /* bit 0 fill, bit 1 composite: workgroups regrouped so that each of the
                                  8 XCDs (own L2) works on one contiguous range of tiles */
-    int32_t flatten_segs;     /* segments each flatten wave works through (multiple of 64; 0: from the
-                                 segment count) */
-    int32_t flatten_take;     /* idle lanes a flatten wave waits for before handing them new segments
-                                 (1..64; 0: 8) */
+    int32_t flatten_segs;     /* a multiple of 64 up to 65536, or 0; flatten_take: 1..64 (0: 8);
+                                 flatten_deep: 0..12.  Accepted and kept, without effect: a flatten
+                                 wave's lanes share the pieces of all its curves */
+    int32_t flatten_take;
     int32_t column_rows;      /* path columns of more tiles than this are propagated by 16 or 64 lanes
                                  each instead of one (1..64; 0: every column by one lane) */
-    int32_t flatten_deep;     /* curves whose subdivision depth is estimated at this or more are
-                                 flattened by 16 lanes each instead of one (0..12; 0: none) */
+    int32_t flatten_deep;
 } pfh_schedule;
 int pfh_get_schedule(pfh_ctx *ctx, pfh_schedule *out);
 int pfh_set_schedule(pfh_ctx *ctx, const pfh_schedule *in);

@@ -84,12 +84,13 @@ struct Schedule {
     uint32_t composite_block = 256;   // threads per k_composite workgroup (a wave per fb tile)
     uint32_t column_block = 256;      // threads per workgroup of k_propagate / k_entries
     uint32_t xcd_order = 0;           // bit 0 fill, bit 1 composite: workgroups grouped per XCD
-    uint32_t flatten_segs = 0;        // segments per k_flatten wave (multiple of 64), 0: from the count
-    uint32_t flatten_take = 8;        // idle k_flatten lanes a wave waits for before a hand-over (1..64)
+    // flatten_*: kept for callers that set them; a flattener wave takes at most one segment per lane
+    // and its lanes share every curve's pieces, so there is nothing left to choose
+    uint32_t flatten_segs = 0;
+    uint32_t flatten_take = 8;
     uint32_t column_rows = 0;         // path columns of more tiles are walked by 16 or 64 lanes (1..64;
                                       // 0: every column by one lane)
-    uint32_t flatten_deep = 0;        // curves whose estimated subdivision depth is at least this are
-                                      // flattened by 16 lanes each (k_flatten_deep; 0: none)
+    uint32_t flatten_deep = 0;
 };
 
 // Inclusive prefix sum within each 16-lane row of the wave (DPP row shifts: no LDS).
@@ -161,23 +162,8 @@ enum Counter {
                            // TALL_ROWS tiles (and Schedule::column_rows) listed for a wave each
     C_MID = 8 + 64 + 1 + 6,  // [C_MID, C_MID + 6): per phase, columns of more than
                              // Schedule::column_rows tiles and at most TALL_ROWS (k_propagate_rows<16>)
-    C_DEEP = 8 + 64 + 1 + 12,  // [C_DEEP, C_DEEP + DEEP_SLOTS): curves listed for k_flatten_deep, per
-                               // list region
-    C_COUNT = 8 + 64 + 1 + 12 + 256
+    C_COUNT = 8 + 64 + 1 + 12
 };
-// The deep-curve list is split into DEEP_SLOTS regions of deep_slot_cap entries, a listing wave
-// taking region (its index mod DEEP_SLOTS) with that region's counter: no single address takes
-// every wave's add.
-constexpr uint32_t DEEP_SLOTS = 256;
-
-// A curve listed for k_flatten_deep, with what the listing pass loaded of it: its batch segment,
-// its scene | DEEP_QUAD | DEEP_BREAK, and its points (a quad as p0, c, c, p1).
-constexpr uint32_t DEEP_QUAD = 0x40000000u, DEEP_BREAK = 0x80000000u;
-struct __align__(8) DeepCurve {
-    uint32_t seg, scene;
-    float2 p0, c0, c1, p1;
-};
-
 // Arrays zeroed by one launch: p[k] has end[k] - end[k - 1] words (end[-1] = 0), k < n.
 constexpr int ZERO_SPANS = 6;
 struct ZeroSpans {
@@ -283,17 +269,13 @@ struct BatchDev {
     uint32_t *tall_cols;          // [W] columns of the current propagate phase walked by several lanes:
                                   // the C_MID list from the front, the C_TALL list from the back
     uint32_t *seg_cnt;            // [S + 1] chords per segment, then exclusive scan
-    uint64_t *curve_mask;         // [S / 64 + 1] bit i of word j: segment 64 j + i is a curve (to be
-                                  // subdivided), written by the flatten count pass
-    DeepCurve *deep_list;         // [DEEP_SLOTS * deep_slot_cap] with deep_pred: the curves left to
-                                  // k_flatten_deep, per region in no particular order
-    uint32_t deep_slot_cap;       // entries per region: 64 per wave of k_flatten_lines mapped to it
-    uint32_t deep_pred;           // Schedule::flatten_deep (0: every curve through k_flatten)
+    unsigned long long *seg_mask; // [S] a curve's leaves by their start in 64ths (0: flattened by a whole wave),
+                                  // written by the flatten count pass for the emit pass; null: no room for it
     // [L] flattened chords as a point stream, in emission order: per chain of chords a NaN
     // separator and the start point, then each chord's end point; chord i of a path's range
     // [c0, c1) runs from point i to point i + 1 (a pair with a NaN end emits nothing)
     float2 *lines;
-    uint32_t *line_cnt;           // [L + 1] fills per chord, then exclusive scan (emission order)
+    uint32_t *line_cnt;           // [L + 1] with dumps only: fills per chord, then exclusive scan (emission order)
     uint2 *fills;                 // [F] grouped by tile: (x0 | y0 << 16, x1 | y1 << 16)
     uint4 *dump_fills;            // [F] emission order: (x0|y0<<16, x1|y1<<16, global tile, 0)
     uint4 *alpha_rec;             // [A] (fill begin, fill end, backdrop | rule << 8, tile)

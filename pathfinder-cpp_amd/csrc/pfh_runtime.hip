@@ -27,7 +27,7 @@ size_t scan_temp_elems(uint64_t n);
 hipError_t scan_u32(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *tmp, hipStream_t s);
 hipError_t scan_entries(uint2 *inout, uint32_t n, uint32_t *counters, void *tmp, hipStream_t s);
 hipError_t scan_paths(const BatchDev &b, void *tmp, hipStream_t s);
-hipError_t launch_flatten(const BatchDev &b, bool emit, uint32_t segs_per_wave, uint32_t take, hipStream_t s);
+hipError_t launch_flatten(const BatchDev &b, bool emit, uint32_t chunk, hipStream_t s);
 hipError_t launch_bin(const BatchDev &b, bool emit, hipStream_t s);
 hipError_t scan_counted(uint32_t *inout, const uint32_t *n_ptr, uint32_t cap, uint32_t *counters, int counter,
                         uint32_t *tmp, hipStream_t s);
@@ -237,8 +237,8 @@ struct Workspace {
     // around the fill and composite kernels of a batched launch; recorded as event nodes
     // inside captured graphs, so replays time those kernels too
     hipEvent_t kev[3] = {nullptr, nullptr, nullptr};
-    DevBuf scene_table, bases, tile_delta, tile_cnt, tile_fill_off, tile_alpha_idx, tile_bd, tile_st, path_ent, ent_quarter, path_tot, bin_items, col_item, col_bd, tall_cols, curve_mask,
-        deep_list, seg_cnt, lines, line_cnt, fills, dump_fills, alpha_rec, alpha_vis, masks, zbuf, fb_range, keys, vals, keys_alt,
+    DevBuf scene_table, bases, tile_delta, tile_cnt, tile_fill_off, tile_alpha_idx, tile_bd, tile_st, path_ent, ent_quarter, path_tot, bin_items, col_item, col_bd, tall_cols, seg_mask,
+        seg_cnt, lines, line_cnt, fills, dump_fills, alpha_rec, alpha_vis, masks, zbuf, fb_range, keys, vals, keys_alt,
         vals_alt, entry_rec, entry_meta, counters, scan_tmp, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen;
     uint32_t *h_counters = nullptr;  // pinned
     SceneDev *h_table = nullptr;     // pinned scene table
@@ -314,7 +314,7 @@ struct Workspace {
     }
     std::vector<DevBuf *> all_buffers() {
         return {&scene_table, &bases, &tile_delta, &tile_cnt, &tile_fill_off, &tile_alpha_idx, &tile_bd, &tile_st,
-                &path_ent, &ent_quarter, &path_tot, &bin_items, &col_item, &col_bd, &tall_cols, &curve_mask, &deep_list, &seg_cnt, &lines, &line_cnt, &fills, &dump_fills, &alpha_rec, &alpha_vis,
+                &path_ent, &ent_quarter, &path_tot, &bin_items, &col_item, &col_bd, &tall_cols, &seg_mask, &seg_cnt, &lines, &line_cnt, &fills, &dump_fills, &alpha_rec, &alpha_vis,
                 &masks, &zbuf, &fb_range, &keys, &vals, &keys_alt, &vals_alt, &entry_rec, &entry_meta, &counters, &scan_tmp,
                 &sort_tmp, &tile_clip_ai, &clip_jobs, &clip_rec, &clip_seen};
     }
@@ -1407,20 +1407,17 @@ struct Plan {
     Schedule sched;
 };
 
-// Segments per flatten wave: the schedule's choice, or enough for ~4 waves per SIMD (1024 SIMDs),
-// 64 to 1024 (a wave balances its lanes over its whole range; past 1024 too few waves share the
-// curves of a large batch).
-static uint32_t flatten_segs(const Plan &pl) {
-    if (pl.sched.flatten_segs) return pl.sched.flatten_segs;
-    const uint64_t per = (pl.S + 4096 * 64 - 1) / (4096 * 64);
-    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(64 * per, 64), 1024);
-}
-
-// Entries per deep-list region: 64 for every wave of k_flatten_lines (64 segments each) that maps
-// to the region (waves w, w + DEEP_SLOTS, ...).
-static uint32_t deep_slot_cap(uint64_t segs) {
-    const uint64_t waves = (segs + 63) / 64;
-    return (uint32_t)(64 * ((waves + DEEP_SLOTS - 1) / DEEP_SLOTS));
+// Segments a flattener wave takes: 64, one per lane, once that gives every SIMD (1024) two waves of the
+// count pass; fewer below that, whose curves' pieces still fill a wave's lanes, so that a small scene's
+// curves spread over the chip.  The emit pass, whose waves walk their points 64 at a time, takes
+// 32 up to a million segments.  Measured (count + emit, us) with 8 / 16 / 32 / 64: the 512^2
+// cubic scene (576 segments) 11 + 10 / 15 + 16 / 25 + 25 / 59 + 46, a 900^2 scene (10 k) 10 + 7 / 11 + 8 /
+// 13 + 11 / 19 + 18, the 4096^2 scene (341 k) 65 + 33 / 40 + 27 / 30 + 28 / 28 + 31, the 48-scene batch
+// (4.4 M) 714 + 358 / 396 + 244 / 235 + 188 / 165 + 162 (the count pass has since gone to 130).
+static uint32_t flatten_chunk(const Plan &pl, bool emit) {
+    uint32_t chunk = 64;
+    while (chunk > 8 && pl.S < 2048ull * chunk) chunk >>= 1;
+    return emit && chunk == 64 && pl.S < (1u << 20) ? 32 : chunk;
 }
 
 static uint32_t clamp_cap(uint64_t v) { return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(v, 64), 0xF0000000ull); }
@@ -1430,6 +1427,11 @@ static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
     w.tile_cnt.ensure(4 * pl.T + 4);
     w.tile_fill_off.ensure(4 * pl.T + 8);
     w.tile_alpha_idx.ensure(4 * pl.T + 8);
+    w.keys.ensure(4ull * pl.cap_e);
+    w.vals.ensure(4ull * pl.cap_e);
+    w.keys_alt.ensure(4ull * pl.cap_e);
+    w.vals_alt.ensure(4ull * pl.cap_e);
+    w.entry_rec.ensure(8ull * pl.cap_e);
     if (dump || pl.clips) w.tile_bd.ensure(pl.T + 4);
     if (pl.clips) {
         w.tile_clip_ai.ensure(4 * pl.T + 4);
@@ -1446,10 +1448,10 @@ static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
     w.col_bd.ensure(4 * pl.W + 4);
     w.tall_cols.ensure(4 * pl.W + 4);
     w.seg_cnt.ensure(4 * pl.S + 8);
-    w.curve_mask.ensure(8 * (pl.S / 64) + 16);
-    if (pl.sched.flatten_deep) w.deep_list.ensure(sizeof(DeepCurve) * DEEP_SLOTS * (uint64_t)deep_slot_cap(pl.S) + 16);
+    // in a fixed region the curves' bits share the tile arrays' space (curve_bits)
+    if (!w.arena.base) w.seg_mask.ensure(8 * pl.S + 8);
     w.lines.ensure(8ull * pl.cap_l);
-    w.line_cnt.ensure(4ull * pl.cap_l + 8);
+    if (dump) w.line_cnt.ensure(4ull * pl.cap_l + 8);
     w.zbuf.ensure(4 * pl.FB + 4);
     w.fb_range.ensure(8 * pl.FB + 8);
     w.counters.ensure(4 * C_COUNT);
@@ -1460,11 +1462,6 @@ static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
     w.alpha_rec.ensure(16ull * pl.cap_a);
     w.alpha_vis.ensure(4ull * (pl.clips ? std::max(pl.cap_a, pl.cap_e) : pl.cap_a));
     w.masks.ensure(256ull * pl.cap_a + 256);  // + the all-ones row
-    w.keys.ensure(4ull * pl.cap_e);
-    w.vals.ensure(4ull * pl.cap_e);
-    w.keys_alt.ensure(4ull * pl.cap_e);
-    w.vals_alt.ensure(4ull * pl.cap_e);
-    w.entry_rec.ensure(8ull * pl.cap_e);
     if (dump) w.entry_meta.ensure(8ull * pl.cap_e);
     w.sort_tmp.ensure(4 * radix_temp_elems(pl.cap_e, (uint32_t)pl.ids.size()) + 64);
 }
@@ -1478,7 +1475,8 @@ static Caps held_caps(Workspace &w, bool dump) {
     auto fit = [](size_t bytes, size_t per, size_t extra) -> uint64_t {
         return bytes > extra ? (bytes - extra) / per : 0;
     };
-    uint64_t l = std::min({fit(w.lines.bytes, 8, 0), fit(w.line_cnt.bytes, 4, 8)});
+    uint64_t l = fit(w.lines.bytes, 8, 0);
+    if (dump) l = std::min(l, fit(w.line_cnt.bytes, 4, 8));
     uint64_t f = fit(w.fills.bytes, 8, 0);
     if (dump) f = std::min(f, fit(w.dump_fills.bytes, 16, 0));
     uint64_t a = std::min({fit(w.alpha_rec.bytes, 16, 0), fit(w.alpha_vis.bytes, 4, 0), fit(w.masks.bytes, 256, 256)});
@@ -1612,6 +1610,21 @@ static void upload_tables(Workspace &w, const Plan &pl) {
                            w.stream));
 }
 
+// Where the flattener keeps its curves' bits (8 bytes a segment) between its two passes.  A fixed
+// region has no room set aside for them: they lie in the tile and entry arrays at its start, which
+// no kernel touches before the chords are out, or, with more segments than those hold (5 per tile),
+// nowhere: every curve is then flattened twice.
+static unsigned long long *curve_bits(Workspace &w, const Plan &pl) {
+    if (!w.arena.base) return w.seg_mask.as<unsigned long long>();
+    uint8_t *const at = w.tile_delta.as<uint8_t>(), *end = at;
+    for (const DevBuf *d : {&w.tile_delta, &w.tile_cnt, &w.tile_fill_off, &w.tile_alpha_idx, &w.keys, &w.vals, &w.keys_alt,
+                            &w.vals_alt, &w.entry_rec}) {
+        if (d->as<uint8_t>() != end) break;
+        end += d->bytes;
+    }
+    return (uint64_t)(end - at) >= 8 * pl.S ? reinterpret_cast<unsigned long long *>(at) : nullptr;
+}
+
 static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
     BatchDev b{};
     size_t n = pl.ids.size();
@@ -1659,12 +1672,9 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
     b.col_bd = w.col_bd.as<int32_t>();
     b.tall_cols = w.tall_cols.as<uint32_t>();
     b.seg_cnt = w.seg_cnt.as<uint32_t>();
-    b.curve_mask = w.curve_mask.as<uint64_t>();
-    b.deep_pred = pl.sched.flatten_deep;
-    b.deep_list = pl.sched.flatten_deep ? w.deep_list.as<DeepCurve>() : nullptr;
-    b.deep_slot_cap = deep_slot_cap(pl.S);
+    b.seg_mask = curve_bits(w, pl);
     b.lines = w.lines.as<float2>();
-    b.line_cnt = w.line_cnt.as<uint32_t>();
+    b.line_cnt = dump ? w.line_cnt.as<uint32_t>() : nullptr;
     b.fills = w.fills.as<uint2>();
     b.dump_fills = dump ? w.dump_fills.as<uint4>() : nullptr;
     b.alpha_rec = w.alpha_rec.as<uint4>();
@@ -1705,9 +1715,9 @@ static void stage_clear(Workspace &w, const BatchDev &b) {
 static void stage_count(Workspace &w, const BatchDev &b, const Plan &pl) {
     hipStream_t s = w.stream;
     uint32_t *tmp = w.scan_tmp.as<uint32_t>();
-    HIP_TRY(launch_flatten(b, false, flatten_segs(pl), pl.sched.flatten_take, s));
+    HIP_TRY(launch_flatten(b, false, flatten_chunk(pl, false), s));
     HIP_TRY(scan_total(b.seg_cnt, b.n_segs, b.counters, C_LINES, tmp, s));
-    HIP_TRY(launch_flatten(b, true, flatten_segs(pl), pl.sched.flatten_take, s));
+    HIP_TRY(launch_flatten(b, true, flatten_chunk(pl, true), s));
     HIP_TRY(launch_bin_items(b, s));
     HIP_TRY(launch_bin(b, false, s));
     HIP_TRY(scan_paths(b, w.scan_tmp.ptr, s));
@@ -1800,7 +1810,7 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
     hipEvent_t *ev = ctx->w->stage_ev;
     HIP_TRY(hipEventRecord(ev[0], st));
     stage_clear(*ctx->w, b);
-    HIP_TRY(launch_flatten(b, false, flatten_segs(pl), pl.sched.flatten_take, st));
+    HIP_TRY(launch_flatten(b, false, flatten_chunk(pl, false), st));
     HIP_TRY(scan_total(b.seg_cnt, b.n_segs, b.counters, C_LINES, tmp(), st));
     read_counters(ctx);  // chord count (renderer.cpp:707-724)
     uint32_t nl = ctx->w->h_counters[C_LINES];
@@ -1809,7 +1819,7 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
         ensure_sizes(*ctx->w, pl, dump);
         b = batch_dev(*ctx->w, pl, dump);
     }
-    HIP_TRY(launch_flatten(b, true, flatten_segs(pl), pl.sched.flatten_take, st));
+    HIP_TRY(launch_flatten(b, true, flatten_chunk(pl, true), st));
     HIP_TRY(hipEventRecord(ev[1], st));
     HIP_TRY(launch_bin_items(b, st));
     HIP_TRY(launch_bin(b, false, st));
@@ -1906,7 +1916,7 @@ static void batched_prepare(pfh_ctx *ctx, const int32_t *ids, int32_t n, uint32_
         upload_tables(w, pl);
         BatchDev b = batch_dev(w, pl, bl.dump);
         stage_clear(w, b);
-        HIP_TRY(launch_flatten(b, false, flatten_segs(pl), pl.sched.flatten_take, w.stream));
+        HIP_TRY(launch_flatten(b, false, flatten_chunk(pl, false), w.stream));
         HIP_TRY(scan_total(b.seg_cnt, b.n_segs, b.counters, C_LINES, w.scan_tmp.as<uint32_t>(), w.stream));
         read_counters(ctx);
         bl.plc = w.h_counters[C_LINES];
@@ -2106,7 +2116,7 @@ static uint64_t scene_launch_bytes(const pfh_ctx *ctx, const SceneHost &s) {
     }
     const double T = s.n_tiles, W = s.n_cols, S = s.n_segs, FB = (double)s.fb_w * s.fb_h;
     const double per_tile = 4 + 4 + 8 + 1 + 4 * 4 + 8;  // counts, offsets, status, sort, records
-    double b = T * per_tile + 4 * W + 16 * s.n_paths + 8 * S + 12 * FB + 12 * L + 8 * F + (16 + 4 + 256) * A;
+    double b = T * per_tile + 4 * W + 16 * s.n_paths + 12 * S + 12 * FB + 8 * L + 8 * F + (16 + 4 + 256) * A;
     return (uint64_t)b + 4096;
 }
 
@@ -2858,20 +2868,16 @@ int pfh_autotune(pfh_ctx *ctx, const int32_t *scene_ids, int32_t n, uint32_t fla
         Schedule best = ctx->sched;
         double best_ms = measure();
         if (ms_start) *ms_start = best_ms;
-        const std::vector<uint32_t> cand[8] = {{1024, 2048, 4096, 8192, 16384, 32768, 65536}, {64, 128, 256}, {64, 128, 256},
-                                              {0, 1, 2, 3}, {0, 64, 128, 256, 512, 1024, 2048}, {1, 4, 8, 16, 32},
-                                              {0, 8, 16, 32, 64}, {0, 3, 4, 5, 6}};
-        for (int param = 0; param < 8; param++) {
+        const std::vector<uint32_t> cand[5] = {{1024, 2048, 4096, 8192, 16384, 32768, 65536}, {64, 128, 256}, {64, 128, 256},
+                                              {0, 1, 2, 3}, {0, 8, 16, 32, 64}};
+        for (int param = 0; param < 5; param++) {
             for (uint32_t v : cand[param]) {
                 Schedule trial = best;
                 uint32_t *field = param == 0 ? &trial.fill_grid
                                   : param == 1 ? &trial.composite_block
                                   : param == 2 ? &trial.column_block
                                   : param == 3 ? &trial.xcd_order
-                                  : param == 4 ? &trial.flatten_segs
-                                  : param == 5 ? &trial.flatten_take
-                                  : param == 6 ? &trial.column_rows
-                                               : &trial.flatten_deep;
+                                               : &trial.column_rows;
                 if (*field == v) continue;
                 *field = v;
                 ctx->sched = trial;
