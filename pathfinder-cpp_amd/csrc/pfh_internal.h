@@ -102,6 +102,15 @@ __device__ __forceinline__ uint32_t row16_inclusive_sum(uint32_t v) {
     return v;
 }
 
+// Inclusive prefix sum across the 64-lane wave: DPP within rows, then the row totals by row
+// broadcasts (lane 15 into rows 1 and 3, then lane 31 into rows 2 and 3).
+__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
+    v = row16_inclusive_sum(v);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
+}
+
 // MI355X dispatches consecutive workgroups round-robin over its 8 XCDs (each with its own L2).
 // Logical block of hardware block b when the grid's blocks are regrouped so that each XCD
 // processes one contiguous range of logical blocks (a bijection on [0, nb)).
@@ -165,7 +174,7 @@ enum Counter {
     C_COUNT = 8 + 64 + 1 + 12
 };
 // Arrays zeroed by one launch: p[k] has end[k] - end[k - 1] words (end[-1] = 0), k < n.
-constexpr int ZERO_SPANS = 6;
+constexpr int ZERO_SPANS = 7;
 struct ZeroSpans {
     uint32_t *p[ZERO_SPANS];
     uint64_t end[ZERO_SPANS];
@@ -268,7 +277,14 @@ struct BatchDev {
     int32_t *col_bd;              // [W] above-rect backdrop, then final column sum
     uint32_t *tall_cols;          // [W] columns of the current propagate phase walked by several lanes:
                                   // the C_MID list from the front, the C_TALL list from the back
-    uint32_t *seg_cnt;            // [S + 1] chords per segment, then exclusive scan
+    uint32_t *seg_cnt;            // [S + 1] stream points per segment (flatten count), then their offsets (flatten
+                                  // emit), the total behind them
+    uint32_t *chunk_off;          // [S / seg_chunk + 2] stream points per seg_chunk segments, then exclusive scan
+    uint32_t seg_chunk;           // segments per flatten emit wave
+    // state of the device-wide scans (k_scan), cleared with the launch; null for one tile
+    unsigned long long *st_seg, *st_paths, *st_entries, *st_sort;
+    unsigned long long *scan_state;  // all of them
+    uint64_t scan_words;             // 64-bit words of it
     unsigned long long *seg_mask; // [S] a curve's leaves by their start in 64ths (0: flattened by a whole wave),
                                   // written by the flatten count pass for the emit pass; null: no room for it
     // [L] flattened chords as a point stream, in emission order: per chain of chords a NaN

@@ -389,12 +389,7 @@ __device__ uint32_t flatten_wave(const Seg4 &root, bool quad, float2 *out, uint3
         return n;
     };
     const uint32_t cnt = leaf ? (mine ? 1u : 0u) : walk(false, 0);
-    uint32_t incl = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(incl, d, 64);
-        if (lane >= (uint32_t)d) incl += o;
-    }
+    const uint32_t incl = wave_inclusive_sum(cnt);
     if (EMIT) {
         const uint32_t at = incl - cnt;
         if (!leaf) walk(true, at);
@@ -443,7 +438,6 @@ __global__ __launch_bounds__(256) void k_flatten_count(BatchDev b, uint32_t chun
             s_meta[wv][at] = lane | (quad ? 1u << 15 : 0u);
         }
         top = (uint32_t)__popcll(m);
-        if (in && !curve) b.seg_cnt[g] = f.kind == SEG_LINE ? 1u + extra : 0u;
     }
     wave_sync();
     Seg4 s{};
@@ -502,11 +496,11 @@ __global__ __launch_bounds__(256) void k_flatten_count(BatchDev b, uint32_t chun
     }
     uint64_t deep = s_deep[wv];
     deep = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(deep >> 32)) << 32) | __builtin_amdgcn_readfirstlane((uint32_t)deep);
+    uint32_t cnt = f.kind == SEG_LINE ? 1u + extra : 0u;
     if (curve) {
-        const bool dp = (deep >> lane) & 1ull;
-        const uint64_t m = s_mask[wv][lane];
-        if (b.seg_mask) b.seg_mask[g] = dp ? 0ull : m;
-        if (!dp) b.seg_cnt[g] = (uint32_t)__popcll(m) + extra;
+        const uint64_t m = (deep >> lane) & 1ull ? 0ull : s_mask[wv][lane];
+        if (b.seg_mask) b.seg_mask[g] = m;
+        cnt = (uint32_t)__popcll(m) + extra;
     }
     uint32_t guard = 0;
     while (deep) {  // wave-uniform
@@ -514,7 +508,15 @@ __global__ __launch_bounds__(256) void k_flatten_count(BatchDev b, uint32_t chun
         deep &= deep - 1;
         const FlatSeg d = load_flat_seg(b, k0, (uint32_t)w0 + i);
         const uint32_t n = flatten_wave<false>(d.s, d.kind == SEG_QUAD, nullptr, 0u, guard);
-        if (lane == 0) b.seg_cnt[(uint32_t)w0 + i] = n + (d.brk ? 2u : 0u);
+        if (lane == i) cnt += n;
+    }
+    if (in) b.seg_cnt[g] = cnt;
+    // the totals of the emit pass's chunks (this wave's segments are one of them or two)
+    const uint32_t incl = wave_inclusive_sum(cnt);
+    for (uint32_t c = 0; c < chunk; c += b.seg_chunk) {
+        const uint32_t first = (uint32_t)w0 + c, below = c ? __shfl(incl, (int)c - 1, 64) : 0u;
+        const uint32_t sum = __shfl(incl, (int)(c + b.seg_chunk - 1), 64) - below;
+        if (lane == 0 && first < b.n_segs) b.chunk_off[first / b.seg_chunk] = sum;
     }
     if (guard) atomicAdd(&b.counters[C_GUARD], guard);
 }
@@ -545,31 +547,31 @@ __device__ __forceinline__ uint32_t nth_bit(uint64_t m, uint32_t n) {
 // e splits: the node's 6 - ctz(e) - 1 ancestors halved on the way, by e's top bits.  Stores are
 // consecutive (a lane per curve scattered 8-byte stores, lines written back several times):
 // 4096^2 scene 93 -> 27 us, 48-scene batch 417 -> 159 us, passes over lines included.
-__global__ __launch_bounds__(256) void k_flatten_emit(BatchDev b, uint32_t chunk) {
+__global__ __launch_bounds__(256) void k_flatten_emit(BatchDev b) {
     __shared__ float4 s_p0c0[4][64], s_c1p1[4][64];
     __shared__ unsigned long long s_mask[4][64];
     __shared__ uint32_t s_start[4][64];  // first point in the chunk | quad << 30 | chain start << 31
     __shared__ uint8_t s_mark[4][64];    // of a window: owner + 1 where its points start
-    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, chunk = b.seg_chunk;
     const uint64_t w0 = ((uint64_t)blockIdx.x * 4 + wv) * chunk;
     if (w0 >= b.n_segs) return;  // whole wave
     const uint32_t g = (uint32_t)w0 + lane;
     const bool in = lane < chunk && g < b.n_segs;
     const int k0 = find_scene_wave(b.seg_bases, b.n_scenes, (uint32_t)w0);
-    // seg_cnt is the exclusive scan, with the total behind the last segment
-    const uint32_t base = __builtin_amdgcn_readfirstlane(b.seg_cnt[(uint32_t)w0]);
-    const uint32_t total = __builtin_amdgcn_readfirstlane(b.seg_cnt[min((uint32_t)w0 + chunk, b.n_segs)]) - base;
-    uint32_t start = 0, cnt = 0;
+    const uint32_t base = __builtin_amdgcn_readfirstlane(b.chunk_off[(uint32_t)w0 / chunk]);
+    uint32_t cnt = 0;
     uint64_t mask = 0;
     FlatSeg f{};
     if (in) {
-        start = b.seg_cnt[g] - base;
-        cnt = b.seg_cnt[g + 1] - base - start;
+        cnt = b.seg_cnt[g];
         f = load_flat_seg(b, k0, g);
         // a line is one leaf over the whole range
         // (without room for the bits every curve is flattened again by the whole wave)
         mask = f.kind > SEG_LINE ? (b.seg_mask ? b.seg_mask[g] : 0ull) : 1ull;
     }
+    const uint32_t incl = wave_inclusive_sum(cnt);
+    const uint32_t total = __builtin_amdgcn_readlane(incl, 63), start = incl - cnt;
+    if (in) b.seg_cnt[g] = base + start;  // from here on a segment's offset
     const uint64_t deep = __ballot(cnt != 0 && mask == 0);
     s_p0c0[wv][lane] = make_float4(f.s.p0.x, f.s.p0.y, f.s.c0.x, f.s.c0.y);
     s_c1p1[wv][lane] = make_float4(f.s.c1.x, f.s.c1.y, f.s.p1.x, f.s.p1.y);
@@ -628,7 +630,7 @@ __global__ __launch_bounds__(256) void k_flatten_emit(BatchDev b, uint32_t chunk
 }
 
 // ---------------------------------------------------------------------------
-// Device-wide exclusive scan (reduce / scan block sums / apply), 4096 items per block
+// Device-wide exclusive scan, 4096 items per block
 // ---------------------------------------------------------------------------
 
 constexpr int SCAN_THREADS = 256;
@@ -1041,60 +1043,81 @@ __global__ __launch_bounds__(256) void k_bin_group(BatchDev b) {
 
 
 
-// Order does not matter for the block sum: each pass reads one coalesced row of 256 items.
-template <typename T, typename Load>
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(Load ld, uint32_t n, T *block_sums) {
-    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + threadIdx.x;
-    T s = zero_of<T>();
-#pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; i++) {
-        const uint64_t j = base + (uint64_t)i * SCAN_THREADS;
-        if (j < n) s = s + ld((uint32_t)j);
-    }
-    T total;
-    block_exclusive_scan<T>(s, total);
-    if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
-}
-
-// Single block: exclusive scan of nb block sums in place; block_sums[nb] = grand total.
-// Each thread takes SCAN_ITEMS consecutive sums per round (the array is small and stays in
-// cache), so a round covers SCAN_TILE sums.
-template <typename T>
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_blocks(T *block_sums, uint32_t nb) {
-    T carry = zero_of<T>();
-    for (uint32_t start = 0; start < nb; start += SCAN_TILE) {
-        const uint32_t first = start + threadIdx.x * SCAN_ITEMS;
-        T vals[SCAN_ITEMS];
-        T s = zero_of<T>();
-#pragma unroll
-        for (int i = 0; i < SCAN_ITEMS; i++) {
-            vals[i] = first + i < nb ? block_sums[first + i] : zero_of<T>();
-            s = s + vals[i];
-        }
-        T total;
-        T run = carry + block_exclusive_scan<T>(s, total);
-#pragma unroll
-        for (int i = 0; i < SCAN_ITEMS; i++) {
-            if (first + i < nb) block_sums[first + i] = run;
-            run = run + vals[i];
-        }
-        carry = carry + total;
-    }
-    if (threadIdx.x == 0) block_sums[nb] = carry;
-}
-
 // Item s of a tile sits at LDS word s + s / 16: striped rows (lane-consecutive) and blocked
 // runs (16 per thread, threads 17 words apart) are both bank-conflict free.
 __device__ __forceinline__ uint32_t scan_pad(uint32_t s) { return s + (s >> 4); }
 
-// Loads and stores are striped (one coalesced row of 256 items at a time) and transposed
-// through LDS to the blocked order the per-thread running sum needs.
+// A tile's state word: 0 nothing yet, SCAN_SUM | its total, SCAN_PREFIX | the total up to its end.
+// Flag and value are one word, so a reader needs no ordering between two.
+constexpr unsigned long long SCAN_SUM = 1ull << 32, SCAN_PREFIX = 2ull << 32;
+template <typename T> constexpr int SCAN_WORDS = sizeof(T) / 4;  // state words per tile
+__device__ __forceinline__ uint32_t scan_part(uint32_t v, int) { return v; }
+__device__ __forceinline__ uint32_t scan_part(const U2 &v, int i) { return i ? v.y : v.x; }
+__device__ __forceinline__ void scan_set(uint32_t &v, int, uint32_t x) { v = x; }
+__device__ __forceinline__ void scan_set(U2 &v, int i, uint32_t x) { (i ? v.y : v.x) = x; }
+
+// Sum of the tiles before tile t (> 0), by one wave, which publishes its own total first and the
+// total up to its end afterwards: 64 predecessors at a time are read from the nearest back to the
+// nearest one that knows its prefix.  Tile numbers are handed out in the order workgroups start
+// (k_scan's ticket), so every predecessor has started and none waits for a later one: its words
+// arrive.  Components are looked up one after the other.
+template <typename T>
+__device__ T scan_look_back(unsigned long long *state, uint32_t t, T total) {
+    constexpr int W = SCAN_WORDS<T>;
+    const uint32_t lane = threadIdx.x & 63;
+    if (lane < (uint32_t)W)
+        __hip_atomic_store(&state[(uint64_t)t * W + lane], SCAN_SUM | scan_part(total, (int)lane), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    T before{};
+#pragma unroll
+    for (int c = 0; c < W; c++) {
+        uint32_t sum = 0;
+        for (int64_t at = (int64_t)t - 1; at >= 0; at -= 64) {  // wave-uniform
+            const int64_t i = at - (int64_t)lane;
+            unsigned long long w;
+            uint64_t known, missing;
+            do {
+                // before the first tile lies a prefix of 0
+                w = i < 0 ? SCAN_PREFIX
+                          : __hip_atomic_load(&state[(uint64_t)i * W + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                known = __ballot((w & SCAN_PREFIX) != 0);
+                missing = __ballot(w == 0);
+                if (known) missing &= (known & (0ull - known)) - 1;  // only those nearer than the first prefix matter
+            } while (missing);
+            const uint64_t use = known ? (known ^ (known - 1)) : ~0ull;  // up to and with the first prefix
+            sum += __builtin_amdgcn_readlane(wave_inclusive_sum((use >> lane) & 1ull ? (uint32_t)w : 0u), 63);
+            if (known) break;
+        }
+        scan_set(before, c, sum);
+    }
+    if (lane < (uint32_t)W)
+        __hip_atomic_store(&state[(uint64_t)t * W + lane],
+                           SCAN_PREFIX | (scan_part(before, (int)lane) + scan_part(total, (int)lane)), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    return before;
+}
+
+// Exclusive scan of n items in one launch of nb tiles of SCAN_TILE items (the store functor also gets
+// the total, as item n).  state: a ticket word and SCAN_WORDS words a tile, zeroed before; not used
+// with one tile.  Loads and stores are striped (one coalesced row of 256 items at a time) and
+// transposed through LDS to the blocked order the per-thread running sum needs.
+// Latency-bound: with three launches each (tile sums, their scan, the items) a pass's five scans took
+// 61 us on the 512^2 cubic scene, now 29; 79 on the 4096^2 scene, now 48; 89 on the 48-scene
+// batch, now 69 (its 4.4 M segments scanned per flattener chunk instead of per segment).
 template <typename T, typename Load, typename Store>
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(Load ld, Store st, uint32_t n, const T *block_sums,
-                                                             uint32_t nb) {
+__global__ __launch_bounds__(SCAN_THREADS) void k_scan(Load ld, Store st, uint32_t n, uint32_t nb,
+                                                       unsigned long long *state) {
     __shared__ T tile[SCAN_TILE + SCAN_TILE / 16];
+    __shared__ uint32_t s_ticket;
+    __shared__ T s_before;
     const uint32_t tid = threadIdx.x;
-    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
+    uint32_t t = 0;
+    if (nb > 1) {
+        if (tid == 0) s_ticket = (uint32_t)atomicAdd(state, 1ull);
+        __syncthreads();
+        t = s_ticket;
+    }
+    const uint64_t base = (uint64_t)t * SCAN_TILE;
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; i++) {
         const uint32_t si = (uint32_t)i * SCAN_THREADS + tid;
@@ -1110,7 +1133,17 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(Load ld, Store st, 
         s = s + vals[i];
     }
     T total;
-    T run = block_exclusive_scan<T>(s, total) + block_sums[blockIdx.x];  // its barriers order the reads above
+    T run = block_exclusive_scan<T>(s, total);  // its barriers order the reads above
+    T before = zero_of<T>();
+    if (nb > 1) {
+        if (tid < 64) {
+            const T bf = scan_look_back<T>(state + 1, t, total);
+            if (tid == 0) s_before = bf;
+        }
+        __syncthreads();
+        before = s_before;
+        run = run + before;
+    }
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; i++) {
         tile[scan_pad(tid * SCAN_ITEMS + (uint32_t)i)] = run;
@@ -1123,7 +1156,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(Load ld, Store st, 
         const uint64_t j = base + si;
         if (j < n) st((uint32_t)j, tile[scan_pad(si)]);
     }
-    if (blockIdx.x == nb - 1 && threadIdx.x == 0) st(n, block_sums[nb]);
+    if (t == nb - 1 && tid == 0) st(n, before + total);
 }
 
 // Scan functors --------------------------------------------------------------
@@ -1163,13 +1196,15 @@ struct LoadU32Counted {
     const uint32_t *n_ptr;
     __device__ uint32_t operator()(uint32_t i) const { return i < *n_ptr ? p[i] : 0u; }
 };
-struct StoreCounted {
-    uint32_t *p, *counters;
-    int counter;
+struct StoreChunkOff {
+    uint32_t *off, *total, *counters;
     uint32_t n;
     __device__ void operator()(uint32_t i, uint32_t v) const {
-        p[i] = v;
-        if (i == n && counter >= 0) counters[counter] = v;
+        off[i] = v;
+        if (i == n) {
+            *total = v;
+            counters[C_LINES] = v;
+        }
     }
 };
 struct StoreEntryOff {
@@ -1829,54 +1864,60 @@ hipError_t launch_zero_spans(const ZeroSpans &z, hipStream_t st) {
     return hipGetLastError();
 }
 
-size_t scan_temp_elems(uint64_t n) { return blocks_for(n, SCAN_TILE) + 1; }
+// 64-bit state words of a scan of n items of `words` 32-bit components each (none for one tile).
+uint64_t scan_state_words(uint64_t n, uint32_t words) {
+    const uint64_t nb = blocks_for(n, SCAN_TILE);
+    return nb > 1 ? 1 + words * nb : 0;
+}
 
 template <typename T, typename Load, typename Store>
-static hipError_t scan_impl(Load ld, Store st, uint32_t n, T *tmp, hipStream_t s) {
-    uint32_t nb = blocks_for(n, SCAN_TILE);
-    if (nb == 0) nb = 1;
-    hipLaunchKernelGGL((k_scan_reduce<T, Load>), dim3(nb), dim3(SCAN_THREADS), 0, s, ld, n, tmp);
-    hipLaunchKernelGGL((k_scan_blocks<T>), dim3(1), dim3(SCAN_THREADS), 0, s, tmp, nb);
-    hipLaunchKernelGGL((k_scan_apply<T, Load, Store>), dim3(nb), dim3(SCAN_THREADS), 0, s, ld, st, n, tmp, nb);
+static hipError_t scan_impl(Load ld, Store st, uint32_t n, unsigned long long *state, hipStream_t s) {
+    const uint32_t nb = std::max(1u, blocks_for(n, SCAN_TILE));
+    hipLaunchKernelGGL((k_scan<T, Load, Store>), dim3(nb), dim3(SCAN_THREADS), 0, s, ld, st, n, nb, state);
     return hipGetLastError();
 }
 
 // Exclusive scan of in[0..n) into out[0..n] (out[n] = total).  in may equal out.
-hipError_t scan_u32(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *tmp, hipStream_t s) {
-    return scan_impl<uint32_t>(LoadU32{in}, StoreU32{out}, n, tmp, s);
+hipError_t scan_u32(const uint32_t *in, uint32_t *out, uint32_t n, unsigned long long *state, hipStream_t s) {
+    return scan_impl<uint32_t>(LoadU32{in}, StoreU32{out}, n, state, s);
 }
 
-hipError_t scan_counted(uint32_t *inout, const uint32_t *n_ptr, uint32_t cap, uint32_t *counters, int counter,
-                        uint32_t *tmp, hipStream_t s) {
-    return scan_impl<uint32_t>(LoadU32Counted{inout, n_ptr}, StoreCounted{inout, counters, counter, cap}, cap, tmp, s);
+// Exclusive scan in place of the first min(*n_ptr, cap) of cap items, the others taken as 0.
+hipError_t scan_counted(uint32_t *inout, const uint32_t *n_ptr, uint32_t cap, unsigned long long *state, hipStream_t s) {
+    return scan_impl<uint32_t>(LoadU32Counted{inout, n_ptr}, StoreU32{inout}, cap, state, s);
 }
 
-// Exclusive scan in place with the total written to counters[counter].
-hipError_t scan_total(uint32_t *inout, uint32_t n, uint32_t *counters, int counter, uint32_t *tmp, hipStream_t s) {
-    return scan_impl<uint32_t>(LoadU32{inout}, StoreCounted{inout, counters, counter, n}, n, tmp, s);
+// Exclusive scan of the flattener's chunk totals in place, the batch's total to the counters and
+// behind the segments' offsets.
+hipError_t scan_chunks(const BatchDev &b, hipStream_t s) {
+    const uint32_t n = blocks_for(b.n_segs, b.seg_chunk);
+    return scan_impl<uint32_t>(LoadU32{b.chunk_off}, StoreChunkOff{b.chunk_off, b.seg_cnt + b.n_segs, b.counters, n}, n,
+                               b.st_seg, s);
 }
 
 // Exclusive scan of the per-path {entries, alpha entries} in place, totals to the counters.
-hipError_t scan_entries(uint2 *inout, uint32_t n, uint32_t *counters, void *tmp, hipStream_t s) {
-    return scan_impl<U2>(LoadPathTot{inout}, StoreEntryOff{inout, counters, n}, n, reinterpret_cast<U2 *>(tmp), s);
+hipError_t scan_entries(const BatchDev &b, hipStream_t s) {
+    return scan_impl<U2>(LoadPathTot{b.path_ent}, StoreEntryOff{b.path_ent, b.counters, b.n_paths}, b.n_paths,
+                         b.st_entries, s);
 }
 
 // Exclusive scan of the per-path {fills, alpha tiles} in place (path_tot[P] = totals), with
 // the totals also in the counters and at the end of the tile offset arrays.
-hipError_t scan_paths(const BatchDev &b, void *tmp, hipStream_t s) {
+hipError_t scan_paths(const BatchDev &b, hipStream_t s) {
     return scan_impl<U2>(LoadPathTot{b.path_tot},
                          StorePathOff{b.path_tot, b.tile_fill_off + b.n_tiles, b.tile_alpha_idx + b.n_tiles, b.counters,
                                       b.n_paths},
-                         b.n_paths, reinterpret_cast<U2 *>(tmp), s);
+                         b.n_paths, b.st_paths, s);
 }
 
-// chunk: segments a wave takes (1..64)
+// chunk: segments a count-pass wave takes (at most 64: b.seg_chunk, an emit-pass wave's, or a multiple)
 hipError_t launch_flatten(const BatchDev &b, bool emit, uint32_t chunk, hipStream_t s) {
     if (b.n_segs == 0) return hipSuccess;
-    if (chunk < 1 || chunk > 64) return hipErrorInvalidValue;
-    const dim3 grid(blocks_for(blocks_for(b.n_segs, chunk), 4));
-    if (emit) hipLaunchKernelGGL(k_flatten_emit, grid, dim3(256), 0, s, b, chunk);
-    else hipLaunchKernelGGL(k_flatten_count, grid, dim3(256), 0, s, b, chunk);
+    if (b.seg_chunk < 1 || chunk < b.seg_chunk || chunk > 64 || chunk % b.seg_chunk) return hipErrorInvalidValue;
+    if (emit)
+        hipLaunchKernelGGL(k_flatten_emit, dim3(blocks_for(blocks_for(b.n_segs, b.seg_chunk), 4)), dim3(256), 0, s, b);
+    else
+        hipLaunchKernelGGL(k_flatten_count, dim3(blocks_for(blocks_for(b.n_segs, chunk), 4)), dim3(256), 0, s, b, chunk);
     return hipGetLastError();
 }
 
@@ -1995,7 +2036,12 @@ static uint32_t rs_max_blocks(uint64_t cap, uint32_t n_scenes) { return blocks_f
 
 size_t radix_temp_elems(uint64_t cap, uint32_t n_scenes) {
     const uint64_t nh = 256ull * rs_max_blocks(cap, n_scenes);
-    return 2ull * (n_scenes + 1) + nh + 1 + scan_temp_elems(nh);
+    return 2ull * (n_scenes + 1) + nh + 1;
+}
+
+// 64-bit state words of the sort's scans (one per digit).
+uint64_t radix_state_words(uint64_t cap, uint32_t n_scenes, int bits) {
+    return (uint64_t)((bits + 7) / 8) * scan_state_words(256ull * rs_max_blocks(cap, n_scenes), 1);
 }
 
 // Sorts the batch's entry keys (b.keys[0 .. entries)), with values starting as the item
@@ -2009,7 +2055,7 @@ hipError_t radix_sort(const BatchDev &b, uint32_t *keys, uint32_t *vals, uint32_
     const uint32_t nh = 256 * nb;
     uint32_t *seg_e = tmp, *seg_b = tmp + (n_sc + 1);
     uint32_t *hist = tmp + 2 * (n_sc + 1);
-    uint32_t *scan_tmp = hist + nh + 1;
+    unsigned long long *state = b.st_sort;
     hipLaunchKernelGGL(k_rs_segments, dim3(1), dim3(RS_THREADS), 0, s, b, seg_e, seg_b);
     bool alt = false;
     for (int shift = 0; shift < bits; shift += 8) {
@@ -2019,8 +2065,9 @@ hipError_t radix_sort(const BatchDev &b, uint32_t *keys, uint32_t *vals, uint32_
         uint32_t *vo = alt ? vals : vals_alt;
         hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(RS_THREADS), 0, s, b, ki, seg_e, seg_b, shift, hist);
         // the scan covers the capacity's blocks; entries past this launch's blocks are never read
-        hipError_t e = scan_u32(hist, hist, nh, scan_tmp, s);
+        hipError_t e = scan_u32(hist, hist, nh, state, s);
         if (e != hipSuccess) return e;
+        state += scan_state_words(nh, 1);
         hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(RS_THREADS), 0, s, b, ki, vi, ko, vo, seg_e, seg_b, shift, hist);
         alt = !alt;
     }

@@ -123,15 +123,6 @@ __device__ __forceinline__ void accumulate_fill(const FillGeom &g, int col, floa
     if (n >= 1) atomicAdd(cd + r1 + 1, full - vd);  // n == 1: v1 == vd
 }
 
-// Inclusive prefix sum across the 64-lane wave: DPP within rows, then the row totals by row
-// broadcasts (lane 15 into rows 1 and 3, then lane 31 into rows 2 and 3).
-__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
-    v = row16_inclusive_sum(v);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return v;
-}
-
 // v_med3_i32: the median of three.
 __device__ __forceinline__ int32_t med3_i32(int32_t a, int32_t b, int32_t c) {
     int32_t r;

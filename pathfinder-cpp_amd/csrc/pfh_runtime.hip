@@ -23,21 +23,20 @@
 
 namespace pfh {
 hipError_t launch_zero_spans(const ZeroSpans &z, hipStream_t st);
-size_t scan_temp_elems(uint64_t n);
-hipError_t scan_u32(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *tmp, hipStream_t s);
-hipError_t scan_entries(uint2 *inout, uint32_t n, uint32_t *counters, void *tmp, hipStream_t s);
-hipError_t scan_paths(const BatchDev &b, void *tmp, hipStream_t s);
+uint64_t scan_state_words(uint64_t n, uint32_t words);
+hipError_t scan_chunks(const BatchDev &b, hipStream_t s);
+hipError_t scan_entries(const BatchDev &b, hipStream_t s);
+hipError_t scan_paths(const BatchDev &b, hipStream_t s);
+hipError_t scan_counted(uint32_t *inout, const uint32_t *n_ptr, uint32_t cap, unsigned long long *state, hipStream_t s);
 hipError_t launch_flatten(const BatchDev &b, bool emit, uint32_t chunk, hipStream_t s);
 hipError_t launch_bin(const BatchDev &b, bool emit, hipStream_t s);
-hipError_t scan_counted(uint32_t *inout, const uint32_t *n_ptr, uint32_t cap, uint32_t *counters, int counter,
-                        uint32_t *tmp, hipStream_t s);
-hipError_t scan_total(uint32_t *inout, uint32_t n, uint32_t *counters, int counter, uint32_t *tmp, hipStream_t s);
 hipError_t launch_propagate(const BatchDev &b, uint32_t block, uint32_t rows, hipStream_t s);
 hipError_t launch_entries(const BatchDev &b, bool write, hipStream_t s);
 hipError_t launch_bin_items(const BatchDev &b, hipStream_t s);
 hipError_t launch_fb_bounds(const uint32_t *sorted_keys, const uint32_t *n_ptr, uint32_t cap, uint32_t n_fb,
                             uint2 *range, hipStream_t s);
 size_t radix_temp_elems(uint64_t cap, uint32_t n_scenes);
+uint64_t radix_state_words(uint64_t cap, uint32_t n_scenes, int bits);
 hipError_t radix_sort(const BatchDev &b, uint32_t *keys, uint32_t *vals, uint32_t *keys_alt, uint32_t *vals_alt,
                       int bits, uint32_t *tmp, bool *result_alt, hipStream_t s);
 hipError_t launch_fill_masks(const BatchDev &b, uint32_t grid_alpha, uint32_t max_blocks, hipStream_t s);
@@ -239,7 +238,7 @@ struct Workspace {
     hipEvent_t kev[3] = {nullptr, nullptr, nullptr};
     DevBuf scene_table, bases, tile_delta, tile_cnt, tile_fill_off, tile_alpha_idx, tile_bd, tile_st, path_ent, ent_quarter, path_tot, bin_items, col_item, col_bd, tall_cols, seg_mask,
         seg_cnt, lines, line_cnt, fills, dump_fills, alpha_rec, alpha_vis, masks, zbuf, fb_range, keys, vals, keys_alt,
-        vals_alt, entry_rec, entry_meta, counters, scan_tmp, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen;
+        vals_alt, entry_rec, entry_meta, counters, chunk_off, scan_state, dump_state, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen;
     uint32_t *h_counters = nullptr;  // pinned
     SceneDev *h_table = nullptr;     // pinned scene table
     size_t h_table_cap = 0;
@@ -315,7 +314,7 @@ struct Workspace {
     std::vector<DevBuf *> all_buffers() {
         return {&scene_table, &bases, &tile_delta, &tile_cnt, &tile_fill_off, &tile_alpha_idx, &tile_bd, &tile_st,
                 &path_ent, &ent_quarter, &path_tot, &bin_items, &col_item, &col_bd, &tall_cols, &seg_mask, &seg_cnt, &lines, &line_cnt, &fills, &dump_fills, &alpha_rec, &alpha_vis,
-                &masks, &zbuf, &fb_range, &keys, &vals, &keys_alt, &vals_alt, &entry_rec, &entry_meta, &counters, &scan_tmp,
+                &masks, &zbuf, &fb_range, &keys, &vals, &keys_alt, &vals_alt, &entry_rec, &entry_meta, &counters, &chunk_off, &scan_state, &dump_state,
                 &sort_tmp, &tile_clip_ai, &clip_jobs, &clip_rec, &clip_seen};
     }
     size_t device_bytes() {
@@ -1420,6 +1419,20 @@ static uint32_t flatten_chunk(const Plan &pl, bool emit) {
     return emit && chunk == 64 && pl.S < (1u << 20) ? 32 : chunk;
 }
 
+// State words of a launch's scans: flattener chunks, paths' fills, paths' entries, sort digits, in order.
+struct ScanStates {
+    uint64_t paths, entries, sort, total;  // where each but the first starts
+};
+static ScanStates scan_states(const Plan &pl) {
+    const uint32_t chunk = flatten_chunk(pl, true);
+    ScanStates st;
+    st.paths = scan_state_words((pl.S + chunk - 1) / chunk, 1);
+    st.entries = st.paths + scan_state_words(pl.P, 2);
+    st.sort = st.entries + scan_state_words(pl.P, 2);
+    st.total = st.sort + radix_state_words(pl.cap_e, (uint32_t)pl.ids.size(), pl.key_bits);
+    return st;
+}
+
 static uint32_t clamp_cap(uint64_t v) { return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(v, 64), 0xF0000000ull); }
 
 static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
@@ -1455,8 +1468,9 @@ static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
     w.zbuf.ensure(4 * pl.FB + 4);
     w.fb_range.ensure(8 * pl.FB + 8);
     w.counters.ensure(4 * C_COUNT);
-    uint64_t scan_n = std::max<uint64_t>({pl.T + 1, pl.S + 1, pl.FB + 1, pl.P + 1, pl.W + 1, (uint64_t)pl.cap_l + 1, 1});
-    w.scan_tmp.ensure(16 * scan_temp_elems(scan_n) + 64);
+    w.chunk_off.ensure(4 * (pl.S / flatten_chunk(pl, true) + 2));
+    w.scan_state.ensure(8 * scan_states(pl).total + 8);
+    if (dump) w.dump_state.ensure(8 * scan_state_words(pl.cap_l, 1) + 8);
     w.fills.ensure(8ull * pl.cap_f);
     if (dump) w.dump_fills.ensure(16ull * pl.cap_f);
     w.alpha_rec.ensure(16ull * pl.cap_a);
@@ -1673,6 +1687,15 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
     b.tall_cols = w.tall_cols.as<uint32_t>();
     b.seg_cnt = w.seg_cnt.as<uint32_t>();
     b.seg_mask = curve_bits(w, pl);
+    b.chunk_off = w.chunk_off.as<uint32_t>();
+    b.seg_chunk = flatten_chunk(pl, true);
+    const ScanStates sst = scan_states(pl);
+    b.scan_state = w.scan_state.as<unsigned long long>();
+    b.scan_words = sst.total;
+    b.st_seg = b.scan_state;
+    b.st_paths = b.scan_state + sst.paths;
+    b.st_entries = b.scan_state + sst.entries;
+    b.st_sort = b.scan_state + sst.sort;
     b.lines = w.lines.as<float2>();
     b.line_cnt = dump ? w.line_cnt.as<uint32_t>() : nullptr;
     b.fills = w.fills.as<uint2>();
@@ -1707,6 +1730,7 @@ static void stage_clear(Workspace &w, const BatchDev &b) {
     z.add(reinterpret_cast<uint32_t *>(b.path_ent), 2 * (uint64_t)b.n_paths);
     z.add(reinterpret_cast<uint32_t *>(b.fb_range), 2 * (uint64_t)b.n_fb);
     z.add(b.counters, C_COUNT);
+    z.add(reinterpret_cast<uint32_t *>(b.scan_state), 2 * b.scan_words);
     if (b.clip_seen) z.add(b.clip_seen, (uint64_t)b.cap_alpha / 32 + 1);
     HIP_TRY(launch_zero_spans(z, s));
 }
@@ -1714,23 +1738,29 @@ static void stage_clear(Workspace &w, const BatchDev &b) {
 // flatten (count, scan, emit) and bin count: chords and exact fill / alpha-tile counts
 static void stage_count(Workspace &w, const BatchDev &b, const Plan &pl) {
     hipStream_t s = w.stream;
-    uint32_t *tmp = w.scan_tmp.as<uint32_t>();
     HIP_TRY(launch_flatten(b, false, flatten_chunk(pl, false), s));
-    HIP_TRY(scan_total(b.seg_cnt, b.n_segs, b.counters, C_LINES, tmp, s));
+    HIP_TRY(scan_chunks(b, s));
     HIP_TRY(launch_flatten(b, true, flatten_chunk(pl, true), s));
     HIP_TRY(launch_bin_items(b, s));
     HIP_TRY(launch_bin(b, false, s));
-    HIP_TRY(scan_paths(b, w.scan_tmp.ptr, s));
+    HIP_TRY(scan_paths(b, s));
+}
+
+// With dumps: every chord's fills' place in emission order (the first n chords).
+static void dump_offsets(Workspace &w, const BatchDev &b, uint32_t n) {
+    ZeroSpans z{};
+    z.add(w.dump_state.as<uint32_t>(), 2 * scan_state_words(n, 1));
+    HIP_TRY(launch_zero_spans(z, w.stream));
+    HIP_TRY(scan_counted(b.line_cnt, b.counters + C_LINES, n, w.dump_state.as<unsigned long long>(), w.stream));
 }
 
 static void stage_emit(Workspace &w, const BatchDev &b, const Plan &pl) {
     hipStream_t s = w.stream;
-    uint32_t *tmp = w.scan_tmp.as<uint32_t>();
-    if (b.dump) HIP_TRY(scan_counted(b.line_cnt, b.counters + C_LINES, b.cap_lines, b.counters, -1, tmp, s));
+    if (b.dump) dump_offsets(w, b, b.cap_lines);
     HIP_TRY(launch_bin(b, true, s));
     HIP_TRY(launch_propagate(b, pl.sched.column_block, pl.sched.column_rows, s));
     HIP_TRY(launch_entries(b, false, s));
-    HIP_TRY(scan_entries(b.path_ent, b.n_paths, b.counters, w.scan_tmp.ptr, s));
+    HIP_TRY(scan_entries(b, s));
 }
 
 static void stage_finish(Workspace &w, const BatchDev &b, const Plan &pl) {
@@ -1805,13 +1835,11 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
     upload_tables(*ctx->w, pl);
     BatchDev b = batch_dev(*ctx->w, pl, dump);
     hipStream_t st = ctx->w->stream;
-    // scratch is re-read at every use: ensure_sizes may reallocate it when a count grows
-    auto tmp = [ctx]() { return ctx->w->scan_tmp.as<uint32_t>(); };
     hipEvent_t *ev = ctx->w->stage_ev;
     HIP_TRY(hipEventRecord(ev[0], st));
     stage_clear(*ctx->w, b);
     HIP_TRY(launch_flatten(b, false, flatten_chunk(pl, false), st));
-    HIP_TRY(scan_total(b.seg_cnt, b.n_segs, b.counters, C_LINES, tmp(), st));
+    HIP_TRY(scan_chunks(b, st));
     read_counters(ctx);  // chord count (renderer.cpp:707-724)
     uint32_t nl = ctx->w->h_counters[C_LINES];
     if (nl > pl.cap_l) {
@@ -1823,7 +1851,7 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
     HIP_TRY(hipEventRecord(ev[1], st));
     HIP_TRY(launch_bin_items(b, st));
     HIP_TRY(launch_bin(b, false, st));
-    HIP_TRY(scan_paths(b, ctx->w->scan_tmp.ptr, st));
+    HIP_TRY(scan_paths(b, st));
     read_counters(ctx);  // fill / alpha counts (renderer.cpp:834-845)
     HIP_TRY(hipEventRecord(ev[2], st));
     uint32_t nf = ctx->w->h_counters[C_FILLS], na = ctx->w->h_counters[C_ALPHA];
@@ -1833,13 +1861,13 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
         ensure_sizes(*ctx->w, pl, dump);
         b = batch_dev(*ctx->w, pl, dump);
     }
-    if (dump) HIP_TRY(scan_counted(b.line_cnt, b.counters + C_LINES, nl, b.counters, -1, tmp(), st));
+    if (dump) dump_offsets(*ctx->w, b, nl);
     HIP_TRY(launch_bin(b, true, st));
     HIP_TRY(hipEventRecord(ev[3], st));
     HIP_TRY(launch_propagate(b, pl.sched.column_block, pl.sched.column_rows, st));
     HIP_TRY(hipEventRecord(ev[4], st));
     HIP_TRY(launch_entries(b, false, st));
-    HIP_TRY(scan_entries(b.path_ent, b.n_paths, b.counters, ctx->w->scan_tmp.ptr, st));
+    HIP_TRY(scan_entries(b, st));
     HIP_TRY(launch_entries(b, true, st));
     HIP_TRY(hipEventRecord(ev[5], st));
     bool alt = false;
@@ -1917,7 +1945,7 @@ static void batched_prepare(pfh_ctx *ctx, const int32_t *ids, int32_t n, uint32_
         BatchDev b = batch_dev(w, pl, bl.dump);
         stage_clear(w, b);
         HIP_TRY(launch_flatten(b, false, flatten_chunk(pl, false), w.stream));
-        HIP_TRY(scan_total(b.seg_cnt, b.n_segs, b.counters, C_LINES, w.scan_tmp.as<uint32_t>(), w.stream));
+        HIP_TRY(scan_chunks(b, w.stream));
         read_counters(ctx);
         bl.plc = w.h_counters[C_LINES];
         pl.cap_l = clamp_cap(std::max<uint64_t>(bl.plc, pl.cap_l));
