@@ -66,8 +66,8 @@ constexpr uint32_t RULE_CLIP_OWN = 0x2u;
 // BIN_GROUP_COLS and global atomics beyond.
 constexpr int BIN_WAVE_TILES = 512;
 constexpr int BIN_WAVE_COLS = 128;
-constexpr int BIN_WAVE_SEGS = 64;       // more segments than lanes: the group class (its walk is 4x wider)
-constexpr int BIN_GROUP_TILES = 4600;   // with the walk queues: 20 KB (emit) and 40 KB (count) of LDS
+constexpr int BIN_WAVE_SEGS = 64;       // more segments than lanes: the group class (its walk is 8x wider)
+constexpr int BIN_GROUP_TILES = 4600;   // with the walk queues: 22 KB (emit) and 33 KB (count) of LDS
 constexpr int BIN_GROUP_COLS = 512;
 constexpr int WALK_QUEUE = 128;          // per wave: chords that cross tile boundaries, waiting for a full wave
 

@@ -3,7 +3,7 @@
 // Stage map (reference GLSL compute stage -> kernel here):
 //   dice.comp                   -> k_flatten_count / k_flatten_emit: the hybrid tiler's recursive
 //                                  flatten (core/d3d9/tiler.cpp:284-315), chords in DFS order
-//   bin.comp                    -> k_bin_wave / k_bin_group <COUNT/EMIT>: the tile walk of
+//   bin.comp                    -> k_bin<COUNT/EMIT>: the tile walk of
 //                                  each chord (tiler.cpp:131-279), exact float order, per path
 //                                  with LDS counters; also writes every tile of the path's rect
 //   bound.comp                  -> (the bin count pass initialises each path's tiles)
@@ -94,61 +94,67 @@ struct Walker {
     uint2 *fills;            // EMIT: fills grouped by tile
     const uint32_t *tile_fill_off;
     uint32_t cap_fills;
-    uint32_t pend_tile, pend_n;  // COUNT: pending increments of one tile
     uint32_t count;          // fills emitted by this chord so far
     uint32_t out_base;       // first emission slot of this chord (EMIT)
     uint32_t guard;
 
-    __device__ __forceinline__ void count_add(uint32_t j, uint32_t n) {
-        if (LDS) atomicAdd(&l_cnt[j], n);
-        else atomicAdd(&tile_cnt[tbase + j], n);
+    // One coordinate of a point in a tile's 8.8 units, as the low 12 bits of the result
+    // (core/d3d9/object_builder.cpp:26-41): rint(clamp((v - origin) * 256, 0, 4095)), the origin given
+    // times 256.  The product by 256 only moves the exponent, so one fma rounds as the subtraction
+    // does; v_med3 takes a NaN to 0 as the reference's max and min do; adding 2^23 rounds to
+    // nearest even into the low mantissa bits.
+    __device__ __forceinline__ static uint32_t quant(float v, float origin256) {
+        const float t = __builtin_amdgcn_fmed3f(fmaf(v, 256.0f, -origin256), 0.0f, 4095.0f);
+        return __float_as_uint(t + 8388608.0f);
+    }
+    __device__ __forceinline__ static uint32_t pack(uint32_t x, uint32_t y) {
+        return __builtin_amdgcn_perm(y, x, 0x05040100u);  // the low halves, x below y
     }
 
-    // core/d3d9/object_builder.cpp:19-64 add_fill
-    __device__ __forceinline__ void add_fill(float2 from, float2 to, int tx, int ty) {
-        if (!(tl <= tx && tx <= tr - 1 && tt <= ty && ty <= tb - 1)) return;
-        float ox = (float)tx * 16.0f, oy = (float)ty * 16.0f;
-        float v0 = (from.x - ox) * 256.0f, v1 = (from.y - oy) * 256.0f;
-        float v2 = (to.x - ox) * 256.0f, v3 = (to.y - oy) * 256.0f;
-        uint32_t q0 = (uint32_t)rintf(sse_min(sse_max(v0, 0.0f), 4095.0f));
-        uint32_t q1 = (uint32_t)rintf(sse_min(sse_max(v1, 0.0f), 4095.0f));
-        uint32_t q2 = (uint32_t)rintf(sse_min(sse_max(v2, 0.0f), 4095.0f));
-        uint32_t q3 = (uint32_t)rintf(sse_min(sse_max(v3, 0.0f), 4095.0f));
-        if (q0 == q2) return;
-        // tile within the path's rect (rect sides are below 2^24 tiles: a 24-bit multiply-add)
-        uint32_t j = __umul24((uint32_t)(ty - tt), (uint32_t)tw) + (uint32_t)(tx - tl);
-        if (!EMIT) {
-            // consecutive fills of a chord mostly share a tile: count them locally
-            if (j != pend_tile) {
-                if (pend_n) count_add(pend_tile, pend_n);
-                pend_tile = j;
-                pend_n = 0;
-            }
-            pend_n++;
-        } else {
-            // straight into the tile's range; order inside a tile is free (coverage is
-            // accumulated in fixed point)
-            const uint32_t packed_x = q0 | (q1 << 16), packed_y = q2 | (q3 << 16);
-            uint32_t pos;
-            if (LDS) {
-                pos = atomicAdd(&l_cnt[j], 1u);
-            } else {
-                uint32_t slot = atomicSub(&tile_cnt[tbase + j], 1u) - 1u;
-                // written by this block in this launch: read from L2
-                pos = __hip_atomic_load(&tile_fill_off[tbase + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + slot;
-            }
-            if (pos < cap_fills) fills[pos] = make_uint2(packed_x, packed_y);
-            if (out) {
-                uint32_t d = out_base + count;
-                if (d < cap_fills) out[d] = make_uint4(packed_x, packed_y, tbase + j, 0u);
-            }
+    __device__ __forceinline__ void put(uint32_t pos, uint32_t a, uint32_t c, uint32_t j) {
+        if (pos < cap_fills) fills[pos] = make_uint2(a, c);
+        if (out) {
+            const uint32_t d = out_base + count;
+            if (d < cap_fills) out[d] = make_uint4(a, c, tbase + j, 0u);
         }
         count++;
     }
 
-    __device__ __forceinline__ void flush() {
-        if (!EMIT && pend_n) count_add(pend_tile, pend_n);
-        pend_n = 0;
+    // core/d3d9/object_builder.cpp:19-64 add_fill, for the fills of one step of a chord in tile
+    // (tx, ty): its piece from -> to, then, with `up`, (to, corner) or, with `down`, (corner, from),
+    // corner being the tile's origin, whose 8.8 coordinates are 0.  A fill with equal x ends is dropped.
+    // Both go to one tile: one cursor add.
+    __device__ __forceinline__ void add_fills(float2 from, float2 to, int tx, int ty, bool up, bool down) {
+        const uint32_t ox = (uint32_t)tx - (uint32_t)tl, oy = (uint32_t)ty - (uint32_t)tt;
+        if (ox >= (uint32_t)tw || oy >= (uint32_t)th) return;
+        const float ox256 = (float)tx * 4096.0f;
+        const uint32_t fx = quant(from.x, ox256), ex = quant(to.x, ox256);
+        const bool piece = fx != ex;
+        const bool aux = (up || down) && ((up ? ex : fx) & 0xffffu) != 0;
+        if (!piece && !aux) return;
+        const uint32_t n = (piece ? 1u : 0u) + (aux ? 1u : 0u);
+        // tile within the path's rect (rect sides are below 2^24 tiles: a 24-bit multiply-add)
+        const uint32_t j = __umul24(oy, (uint32_t)tw) + ox;
+        if (!EMIT) {
+            if (LDS) atomicAdd(&l_cnt[j], n);
+            else atomicAdd(&tile_cnt[tbase + j], n);
+            count += n;
+        } else {
+            // straight into the tile's range; order inside a tile is free (coverage is
+            // accumulated in fixed point)
+            uint32_t pos;
+            if (LDS) {
+                pos = atomicAdd(&l_cnt[j], n);
+            } else {
+                const uint32_t slot = atomicSub(&tile_cnt[tbase + j], n) - n;
+                // written by this block in this launch: read from L2
+                pos = __hip_atomic_load(&tile_fill_off[tbase + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + slot;
+            }
+            const float oy256 = (float)ty * 4096.0f;
+            const uint32_t a = pack(fx, quant(from.y, oy256)), c = pack(ex, quant(to.y, oy256));
+            if (piece) put(pos, a, c, j);
+            if (aux) put(pos + n - 1u, up ? c : 0u, up ? 0u : a, j);
+        }
     }
 
     // core/d3d9/object_builder.cpp:96-114 adjust_alpha_tile_backdrop
@@ -228,10 +234,11 @@ struct Walker {
         float2 cur = from;
         int cx = fx, cy = fy;
         int last = 0;  // 0 none, 1 X, 2 Y
-        int64_t dx = (int64_t)ex - fx, dy = (int64_t)ey - fy;
-        int64_t lim = (dx < 0 ? -dx : dx) + (dy < 0 ? -dy : dy) + 2;
-        for (int64_t it = 0;; it++) {
-            if (it > lim) {
+        const int64_t dx = (int64_t)ex - fx, dy = (int64_t)ey - fy;
+        // steps before the guard trips (a count of 2^31 or more, for chords of 2^31 tiles, is cut there)
+        const int64_t lim = (dx < 0 ? -dx : dx) + (dy < 0 ? -dy : dy) + 2;
+        for (uint32_t left = (uint32_t)(lim < 0x7fffffff ? lim : 0x7fffffff) + 1u;; left--) {
+            if (left == 0) {
                 guard++;
                 break;
             }
@@ -243,13 +250,9 @@ struct Walker {
             nt = (1.0f < nt) ? 1.0f : nt;  // std::min(next_t, 1.0f)
             if (cx == ex && cy == ey) next = 0;
             float2 npos = f2add(from, f2muls(vec, nt));  // LineSegmentF::sample
-            add_fill(cur, npos, cx, cy);
-            // the auxiliary fill along the tile's left edge: (npos, corner) when stepping up out of
-            // the tile, (corner, cur) when having stepped down into it; one call site for both, so
-            // lanes walking up and down do not run two copies
-            const float2 corner = make_float2((float)cx * 16.0f, (float)cy * 16.0f);
-            const bool up = sty < 0 && next == 2, down = sty > 0 && last == 2;
-            if (up || down) add_fill(up ? npos : corner, up ? corner : cur, cx, cy);
+            // with the auxiliary fill along the tile's left edge: (npos, corner) when stepping up out of
+            // the tile, (corner, cur) when having stepped down into it
+            add_fills(cur, npos, cx, cy, sty < 0 && next == 2, sty > 0 && last == 2);
             // the backdrop step when leaving to the right or having entered from the left
             if ((stx < 0 && last == 1) || (stx > 0 && next == 1)) adjust(cx, cy, stx < 0 ? 1 : -1);
             if (next == 1) {
@@ -648,10 +651,10 @@ __device__ __forceinline__ U2 shfl_up_val(U2 v, int d) { return U2{__shfl_up(v.x
 template <typename T>
 __device__ __forceinline__ T zero_of() { return T{}; }
 
-// Exclusive scan of one value per thread across a 256-thread block; returns the block total.
-template <typename T>
+// Exclusive scan of one value per thread across a block of THREADS threads; returns the block total.
+template <typename T, int THREADS = SCAN_THREADS>
 __device__ T block_exclusive_scan(T v, T &total) {
-    __shared__ T wave_tot[SCAN_THREADS / 64];
+    __shared__ T wave_tot[THREADS / 64];
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     T inc = v;
 #pragma unroll
@@ -664,7 +667,7 @@ __device__ T block_exclusive_scan(T v, T &total) {
     T base = zero_of<T>();
     T all = zero_of<T>();
 #pragma unroll
-    for (int w = 0; w < SCAN_THREADS / 64; w++) {
+    for (int w = 0; w < THREADS / 64; w++) {
         if (w < wave) base = base + wave_tot[w];
         all = all + wave_tot[w];
     }
@@ -676,7 +679,7 @@ __device__ T block_exclusive_scan(T v, T &total) {
 }
 
 // ---------------------------------------------------------------------------
-// Bin: per path, one wave (small rects) or one workgroup (large rects)
+// Bin: per path, one wave (small rects) or one workgroup (large rects or many segments)
 // ---------------------------------------------------------------------------
 //
 // The chords of a path are contiguous (flatten emits in segment order, segments are in
@@ -733,14 +736,11 @@ __device__ __forceinline__ void walk_chords(const BatchDev &b, const SceneDev &s
     w.tile_fill_off = b.tile_fill_off;
     w.cap_fills = b.cap_fills;
     auto begin = [&](uint32_t i) {
-        w.pend_tile = 0xffffffffu;
-        w.pend_n = 0;
         w.count = 0;
         w.guard = 0;
         w.out_base = (EMIT && b.dump) ? b.line_cnt[i] : 0u;
     };
     auto end = [&](uint32_t i) {
-        w.flush();
         if (!EMIT && b.dump) b.line_cnt[i] = w.count;  // fills per chord: canonical dump order only
         guard += w.guard;
     };
@@ -772,7 +772,7 @@ __device__ __forceinline__ void walk_chords(const BatchDev &b, const SceneDev &s
                 const float2 vec = f2sub(to, from);
                 // a -0 component makes a crossing time -inf: left to the full walk
                 const bool neg_zero = (vec.x == 0.0f && signbit(vec.x)) || (vec.y == 0.0f && signbit(vec.y));
-                if (fx == ex && fy == ey && !neg_zero) w.add_fill(from, f2add(from, vec), fx, fy);
+                if (fx == ex && fy == ey && !neg_zero) w.add_fills(from, f2add(from, vec), fx, fy, false, false);
                 else multi = true;
             }
             if (!multi) end(i);
@@ -853,14 +853,15 @@ __device__ __forceinline__ void wave_tile_offsets(const BatchDev &b, uint32_t tb
     }
 }
 
-// Block (256 threads) version, called by every thread of the block.
+// Block version, called by every thread of a block of THREADS.
+template <int THREADS>
 __device__ __forceinline__ void block_tile_offsets(const BatchDev &b, uint32_t tbase, uint32_t area, U2 base,
                                                    uint32_t *l_cur, uint32_t aw) {
-    for (uint32_t j0 = 0; j0 < area; j0 += 256) {
+    for (uint32_t j0 = 0; j0 < area; j0 += THREADS) {
         const uint32_t j = j0 + threadIdx.x;
         const uint32_t c = j < area ? b.tile_cnt[tbase + j] : 0u;
         U2 tot;
-        const U2 ex = block_exclusive_scan<U2>(U2{c, c > 0 ? 1u : 0u}, tot);
+        const U2 ex = block_exclusive_scan<U2, THREADS>(U2{c, c > 0 ? 1u : 0u}, tot);
         if (j < area) {
             b.tile_fill_off[tbase + j] = base.x + ex.x;
             b.tile_alpha_idx[tbase + j] = base.y + aw * ex.y;
@@ -870,28 +871,32 @@ __device__ __forceinline__ void block_tile_offsets(const BatchDev &b, uint32_t t
     }
 }
 
-// Block sum over the block's threads; `part` is 4 slots of LDS the block no longer reads.
+// Block sum over a block's THREADS threads; `part` is a slot of LDS per wave the block no longer reads.
+template <int THREADS>
 __device__ __forceinline__ U2 block_sum_u2(U2 v, U2 *part) {
     v = wave_sum_u2(v);
     __syncthreads();  // part may alias data read just before
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
-    const U2 t = part[0] + part[1] + part[2] + part[3];
+    U2 t = part[0];
+#pragma unroll
+    for (int w = 1; w < THREADS / 64; w++) t = t + part[w];
     __syncthreads();
     return t;
 }
 
-// One descriptor per binned path: thread per item, class GROUP 0 (wave) or 1 (group).
-template <int GROUP>
-__global__ __launch_bounds__(256) void k_bin_items(BatchDev b) {
-    const uint32_t n = GROUP ? b.n_bin_group : b.n_bin_wave;
-    const uint32_t *bases = GROUP ? b.bin_group_bases : b.bin_wave_bases;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// One descriptor per binned path: thread per item, the first blocks for the wave class, the others for
+// the group class.
+__global__ __launch_bounds__(256) void k_bin_items(BatchDev b, uint32_t wave_blocks) {
+    const bool grp = blockIdx.x >= wave_blocks;  // uniform over the block
+    const uint32_t n = grp ? b.n_bin_group : b.n_bin_wave;
+    const uint32_t *bases = grp ? b.bin_group_bases : b.bin_wave_bases;
+    const uint32_t i = (blockIdx.x - (grp ? wave_blocks : 0u)) * blockDim.x + threadIdx.x;
     // every lane searches (lanes past the end with the last item), then those leave
     const int k = find_scene_lanes(bases, b.n_scenes, min(i, n - 1));
     if (i >= n) return;
     const SceneDev &sc = b.scenes[k];
-    const uint32_t p = sc.bin_paths[(GROUP ? sc.n_bin_wave : 0u) + (i - bases[k])];
+    const uint32_t p = sc.bin_paths[(grp ? sc.n_bin_wave : 0u) + (i - bases[k])];
     BinItem it;
     it.rect = sc.path_rect[p];
     it.tbase = sc.tile_base + sc.path_tile_off[p];
@@ -908,21 +913,37 @@ __global__ __launch_bounds__(256) void k_bin_items(BatchDev b) {
     it.clip = cr;
     it.level = sc.path_level ? (uint32_t)sc.path_level[p] : 0u;
     it.paint = sc.path_paint ? sc.path_paint[p] : PAINT_NONE;
-    const uint32_t gi = (GROUP ? b.n_bin_wave : 0u) + i;
+    const uint32_t gi = (grp ? b.n_bin_wave : 0u) + i;
     b.bin_items[gi] = it;
     const uint32_t tw = (uint32_t)max(it.rect.z - it.rect.x, 0);
     for (uint32_t j = 0; j < tw; j++) b.col_item[it.cbase + j] = gi;
 }
 
-// Wave class: 4 paths per 256-thread block, one per wave, each with its own LDS slice.
+// LDS of a bin block: its path's arrays (group class), or a slice per wave (wave class).
+template <bool EMIT, int THREADS>
+struct BinPath {
+    uint32_t cnt[BIN_GROUP_TILES];
+    uint32_t delta[EMIT ? 1 : (BIN_GROUP_TILES + 1) / 2];  // packed, two tiles per word
+    int32_t col[EMIT ? 1 : BIN_GROUP_COLS];
+    uint32_t queue[THREADS / 64][WALK_QUEUE];
+};
 template <bool EMIT>
-__global__ __launch_bounds__(256) void k_bin_wave(BatchDev b) {
-    __shared__ uint32_t s_cnt[4][BIN_WAVE_TILES];
-    __shared__ int32_t s_delta[4][EMIT ? 1 : BIN_WAVE_TILES];
-    __shared__ int32_t s_col[4][EMIT ? 1 : BIN_WAVE_COLS];
-    __shared__ uint32_t s_queue[4][WALK_QUEUE];
+struct BinSlice {
+    uint32_t cnt[BIN_WAVE_TILES];
+    int32_t delta[EMIT ? 1 : BIN_WAVE_TILES];
+    int32_t col[EMIT ? 1 : BIN_WAVE_COLS];
+    uint32_t queue[WALK_QUEUE];
+};
+template <bool EMIT, int THREADS>
+union BinLds {
+    BinPath<EMIT, THREADS> g;
+    BinSlice<EMIT> w[THREADS / 64];
+};
+
+// Wave class: a path per wave, in its own slice.
+template <bool EMIT, int THREADS, typename Lds>
+__device__ __forceinline__ void bin_wave(const BatchDev &b, Lds &lds, uint32_t item) {
     const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const uint32_t item = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + wv);  // uniform: scalar loads below
     if (item >= b.n_bin_wave) return;  // whole wave: no block-wide barriers below
     const BinItem it = b.bin_items[item];
     const SceneDev &sc = b.scenes[it.k];
@@ -931,8 +952,8 @@ __global__ __launch_bounds__(256) void k_bin_wave(BatchDev b) {
     const uint32_t area = tw * th;
     if (area > (uint32_t)BIN_WAVE_TILES || tw > (uint32_t)BIN_WAVE_COLS) return;  // not this class (host sorts)
     const uint32_t tbase = it.tbase, cbase = it.cbase;
-    uint32_t *l_cnt = s_cnt[wv];
-    int32_t *l_delta = s_delta[wv], *l_col = s_col[wv];
+    uint32_t *l_cnt = lds[wv].cnt;
+    int32_t *l_delta = lds[wv].delta, *l_col = lds[wv].col;
     const uint32_t gp = it.gp;
     if (EMIT) {
         const uint2 base = b.path_tot[gp];
@@ -945,7 +966,7 @@ __global__ __launch_bounds__(256) void k_bin_wave(BatchDev b) {
         for (uint32_t j = lane; j < tw; j += 64) l_col[j] = 0;
     }
     wave_sync();
-    walk_chords<EMIT, true>(b, sc, rect, tbase, cbase, l_cnt, l_delta, l_col, it.c0, it.c1, lane, 64, s_queue[wv]);
+    walk_chords<EMIT, true>(b, sc, rect, tbase, cbase, l_cnt, l_delta, l_col, it.c0, it.c1, lane, 64, lds[wv].queue);
     if (!EMIT) {
         wave_sync();
         U2 tot{0, 0};
@@ -961,16 +982,10 @@ __global__ __launch_bounds__(256) void k_bin_wave(BatchDev b) {
     }
 }
 
-// Group class: one path per 256-thread block; LDS when the rect fits, else global atomics
-// on the path's own (first zeroed) tiles.
-template <bool EMIT>
-__global__ __launch_bounds__(256) void k_bin_group(BatchDev b) {
-    __shared__ uint32_t s_cnt[BIN_GROUP_TILES];
-    __shared__ uint32_t s_delta[EMIT ? 1 : (BIN_GROUP_TILES + 1) / 2];  // packed, two tiles per word
-    __shared__ int32_t s_col[EMIT ? 1 : BIN_GROUP_COLS];
-    __shared__ uint32_t s_queue[4][WALK_QUEUE];
-    const uint32_t item = blockIdx.x;
-    if (item >= b.n_bin_group) return;  // uniform over the block
+// Group class: one path per block; LDS when the rect fits, else global atomics on the path's own
+// (first zeroed) tiles.
+template <bool EMIT, int THREADS, typename Lds>
+__device__ __forceinline__ void bin_group(const BatchDev &b, Lds &lds, uint32_t item) {
     const BinItem it = b.bin_items[b.n_bin_wave + item];
     const SceneDev &sc = b.scenes[it.k];
     const int4 rect = it.rect;
@@ -979,69 +994,95 @@ __global__ __launch_bounds__(256) void k_bin_group(BatchDev b) {
     const uint32_t tbase = it.tbase, cbase = it.cbase;
     const uint32_t gp = it.gp;
     const uint32_t c0 = it.c0, c1 = it.c1;
+    uint32_t *const s_cnt = lds.cnt, *const s_delta = lds.delta;
+    int32_t *const s_col = lds.col;
+    uint32_t *const queue = lds.queue[threadIdx.x >> 6];
     // the packed LDS deltas hold sums below 2^15 in magnitude: at most one step per chord
-    const bool lds = area <= (uint32_t)BIN_GROUP_TILES && tw <= (uint32_t)BIN_GROUP_COLS &&
-                     (EMIT || c1 - c0 < (1u << 15));
-    if (lds) {
+    const bool in_lds = area <= (uint32_t)BIN_GROUP_TILES && tw <= (uint32_t)BIN_GROUP_COLS &&
+                        (EMIT || c1 - c0 < (1u << 15));
+    if (in_lds) {
         if (EMIT) {
             const uint2 base = b.path_tot[gp];
-            block_tile_offsets(b, tbase, area, U2{base.x, base.y}, s_cnt, alpha_rows(it));
+            block_tile_offsets<THREADS>(b, tbase, area, U2{base.x, base.y}, s_cnt, alpha_rows(it));
         } else {
-            for (uint32_t j = threadIdx.x; j < area; j += 256) s_cnt[j] = 0;
-            for (uint32_t j = threadIdx.x; j < (area + 1) / 2; j += 256) s_delta[j] = 0x80008000u;
-            for (uint32_t j = threadIdx.x; j < tw; j += 256) s_col[j] = 0;
+            for (uint32_t j = threadIdx.x; j < area; j += THREADS) s_cnt[j] = 0;
+            for (uint32_t j = threadIdx.x; j < (area + 1) / 2; j += THREADS) s_delta[j] = 0x80008000u;
+            for (uint32_t j = threadIdx.x; j < tw; j += THREADS) s_col[j] = 0;
         }
         __syncthreads();
         walk_chords<EMIT, true, true>(b, sc, rect, tbase, cbase, s_cnt, reinterpret_cast<int32_t *>(s_delta), s_col,
-                                      c0, c1, threadIdx.x, 256, s_queue[threadIdx.x >> 6]);
+                                      c0, c1, threadIdx.x, THREADS, queue);
         if (!EMIT) {
             __syncthreads();
             U2 tot{0, 0};
-            for (uint32_t j = threadIdx.x; j < area; j += 256) {
+            for (uint32_t j = threadIdx.x; j < area; j += THREADS) {
                 const uint32_t c = s_cnt[j];
                 b.tile_cnt[tbase + j] = c;
                 b.tile_delta[tbase + j] = (int32_t)((s_delta[j >> 1] >> (16 * (j & 1))) & 0xffffu) - 0x8000;
                 tot = tot + U2{c, c > 0 ? 1u : 0u};
             }
-            for (uint32_t j = threadIdx.x; j < tw; j += 256) b.col_bd[cbase + j] = s_col[j];
-            tot = block_sum_u2(tot, reinterpret_cast<U2 *>(s_col));
+            for (uint32_t j = threadIdx.x; j < tw; j += THREADS) b.col_bd[cbase + j] = s_col[j];
+            tot = block_sum_u2<THREADS>(tot, reinterpret_cast<U2 *>(s_col));
             if (threadIdx.x == 0) b.path_tot[gp] = make_uint2(tot.x, tot.y * alpha_rows(it));
         }
     } else {
         if (EMIT) {
             const uint2 base = b.path_tot[gp];
-            block_tile_offsets(b, tbase, area, U2{base.x, base.y}, nullptr, alpha_rows(it));
+            block_tile_offsets<THREADS>(b, tbase, area, U2{base.x, base.y}, nullptr, alpha_rows(it));
             __threadfence();  // the offsets reach L2 before any thread reads them back
             __syncthreads();
         }
         if (!EMIT) {
-            for (uint32_t j = threadIdx.x; j < area; j += 256) {
+            for (uint32_t j = threadIdx.x; j < area; j += THREADS) {
                 b.tile_cnt[tbase + j] = 0;
                 b.tile_delta[tbase + j] = 0;
             }
-            for (uint32_t j = threadIdx.x; j < tw; j += 256) b.col_bd[cbase + j] = 0;
+            for (uint32_t j = threadIdx.x; j < tw; j += THREADS) b.col_bd[cbase + j] = 0;
             __threadfence();  // the zeros reach L2 before any thread's atomics
             __syncthreads();
         }
-        walk_chords<EMIT, false>(b, sc, rect, tbase, cbase, nullptr, nullptr, nullptr, c0, c1, threadIdx.x, 256,
-                                 s_queue[threadIdx.x >> 6]);
+        walk_chords<EMIT, false>(b, sc, rect, tbase, cbase, nullptr, nullptr, nullptr, c0, c1, threadIdx.x, THREADS,
+                                 queue);
         if (!EMIT) {
             __threadfence();  // every thread's atomics are done before the counts are summed
             __syncthreads();
             U2 tot{0, 0};
-            for (uint32_t j = threadIdx.x; j < area; j += 256) {
+            for (uint32_t j = threadIdx.x; j < area; j += THREADS) {
                 const uint32_t c = __hip_atomic_load(&b.tile_cnt[tbase + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 tot = tot + U2{c, c > 0 ? 1u : 0u};
             }
-            tot = block_sum_u2(tot, reinterpret_cast<U2 *>(s_col));  // s_col is unused on this path
+            tot = block_sum_u2<THREADS>(tot, reinterpret_cast<U2 *>(s_col));  // s_col is unused on this path
             if (threadIdx.x == 0) b.path_tot[gp] = make_uint2(tot.x, tot.y * alpha_rows(it));
         }
     }
 }
 
-// ---------------------------------------------------------------------------
+// Both classes in one launch, the group class's paths first (they last longest).  512 threads: a long
+// path's walk is twice as wide as with 256, and 8 wave-class slices (40 KB in the count pass) leave the
+// wave class its 32 waves per CU.
+template <bool EMIT>
+__global__ __launch_bounds__(512) void k_bin(BatchDev b) {
+    __shared__ BinLds<EMIT, 512> lds;
+    if (blockIdx.x < b.n_bin_group) {  // uniform over the block
+        bin_group<EMIT, 512>(b, lds.g, blockIdx.x);
+    } else {
+        const uint32_t wave = (blockIdx.x - b.n_bin_group) * 8 + (threadIdx.x >> 6);
+        bin_wave<EMIT, 512>(b, lds.w, __builtin_amdgcn_readfirstlane(wave));  // uniform: scalar loads
+    }
+}
 
-
+// A class per launch, in blocks of 256: a block's LDS is held by its slowest wave, so with the chip full
+// the smaller blocks keep more waves in flight.
+template <bool EMIT>
+__global__ __launch_bounds__(256) void k_bin_wave(BatchDev b) {
+    __shared__ BinSlice<EMIT> lds[4];
+    bin_wave<EMIT, 256>(b, lds, __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)));
+}
+template <bool EMIT>
+__global__ __launch_bounds__(256) void k_bin_group(BatchDev b) {
+    __shared__ BinPath<EMIT, 256> lds;
+    bin_group<EMIT, 256>(b, lds, blockIdx.x);
+}
 
 // Item s of a tile sits at LDS word s + s / 16: striped rows (lane-consecutive) and blocked
 // runs (16 per thread, threads 17 words apart) are both bank-conflict free.
@@ -1640,31 +1681,30 @@ __device__ __forceinline__ uint2 range_entries(const BatchDev &b, const SceneDev
     return make_uint2(e, n_alpha);
 }
 
+// One launch for both binning classes, the group class's blocks first.  A block per large path: wave w
+// takes the w-th quarter of the rect's tiles (row-major, in whole 64-tile chunks), so the waves need no
+// barrier.  The count pass keeps each quarter's counts (ent_quarter) beside the path's total; the
+// write pass starts each wave after the quarters before it.  Behind them a wave per small path.
+// A clip path draws nothing: no entries.
 template <bool WRITE, bool CLIPS>
-__global__ __launch_bounds__(256) void k_entries_wave(BatchDev b) {
-    const uint32_t item = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));  // uniform
-    if (item >= b.n_bin_wave) return;  // whole wave
-    const BinItem it = b.bin_items[item];
-    const int4 r = it.rect;
-    // a clip path draws nothing: no entries
-    const uint32_t area = CLIPS && it.level != 0 ? 0u : (uint32_t)max(r.z - r.x, 0) * (uint32_t)max(r.w - r.y, 0);
-    const uint2 first = WRITE ? b.path_ent[it.gp] : make_uint2(0u, 0u);
-    const uint2 n = range_entries<WRITE, CLIPS>(b, b.scenes[it.k], it, 0, area, first);
-    if (!WRITE && (threadIdx.x & 63) == 0) b.path_ent[it.gp] = n;
-}
-
-// A block per large path: wave w takes the w-th quarter of the rect's tiles (row-major, in
-// whole 64-tile chunks), so the waves need no barrier.  The count pass keeps each quarter's
-// counts (ent_quarter) beside the path's total; the write pass starts each wave after the
-// quarters before it.
-template <bool WRITE, bool CLIPS>
-__global__ __launch_bounds__(256) void k_entries_group(BatchDev b) {
+__global__ __launch_bounds__(256) void k_entries(BatchDev b) {
+    __shared__ uint2 part[4];
+    const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (blockIdx.x >= b.n_bin_group) {  // uniform over the block
+        const uint32_t item = __builtin_amdgcn_readfirstlane((blockIdx.x - b.n_bin_group) * 4 + wv);  // uniform
+        if (item >= b.n_bin_wave) return;  // whole wave
+        const BinItem it = b.bin_items[item];
+        const int4 r = it.rect;
+        const uint32_t area = CLIPS && it.level != 0 ? 0u : (uint32_t)max(r.z - r.x, 0) * (uint32_t)max(r.w - r.y, 0);
+        const uint2 first = WRITE ? b.path_ent[it.gp] : make_uint2(0u, 0u);
+        const uint2 n = range_entries<WRITE, CLIPS>(b, b.scenes[it.k], it, 0, area, first);
+        if (!WRITE && lane == 0) b.path_ent[it.gp] = n;
+        return;
+    }
     const uint32_t item = blockIdx.x;
-    if (item >= b.n_bin_group) return;  // uniform over the block
     const BinItem it = b.bin_items[b.n_bin_wave + item];
     const int4 r = it.rect;
     const uint32_t area = CLIPS && it.level != 0 ? 0u : (uint32_t)max(r.z - r.x, 0) * (uint32_t)max(r.w - r.y, 0);
-    const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t q = (area + 255) / 256 * 64;  // tiles per quarter, whole chunks
     const uint32_t j0 = min(wv * q, area), j1 = min(j0 + q, area);
     uint2 first = make_uint2(0u, 0u);
@@ -1678,9 +1718,10 @@ __global__ __launch_bounds__(256) void k_entries_group(BatchDev b) {
     }
     const uint2 n = range_entries<WRITE, CLIPS>(b, b.scenes[it.k], it, j0, j1, first);
     if (!WRITE) {
-        if (lane == 0) b.ent_quarter[item * 4 + wv] = n;
-        __shared__ uint2 part[4];
-        if (lane == 0) part[wv] = n;
+        if (lane == 0) {
+            b.ent_quarter[item * 4 + wv] = n;
+            part[wv] = n;
+        }
         __syncthreads();
         if (threadIdx.x == 0)
             b.path_ent[it.gp] = make_uint2(part[0].x + part[1].x + part[2].x + part[3].x,
@@ -1921,24 +1962,35 @@ hipError_t launch_flatten(const BatchDev &b, bool emit, uint32_t chunk, hipStrea
     return hipGetLastError();
 }
 
-// grid_lines: chords the launch is sized for (exact in plain mode, capacity in batched mode)
+// The bin passes run as one launch of 512-thread blocks up to this many (3.5 for each the chip holds at
+// once), as a launch per class beyond: launched one after the other, each class's tail leaves most of
+// the chip idle, which counts while a launch is a few rounds of blocks.  A pass, one launch / two: 4
+// scenes of 2 587 paths 0.362 / 0.407 ms, the stress scene (2 700) 1.025 / 1.044, the 4096^2 scene (10 000 paths,
+// about 3 100 blocks) 0.593 / 0.600, 8 scenes (13 754) 0.582 / 0.589; 4 000 stars (4 000 blocks) 0.713 /
+// 0.701, the 4096^2 scene with 20 000 paths 0.968 / 0.936, 32 scenes (66 509) 1.805 / 1.716.
+constexpr uint32_t BIN_MERGED_BLOCKS = 3584;
+
 hipError_t launch_bin_items(const BatchDev &b, hipStream_t s) {
-    if (b.n_bin_wave) hipLaunchKernelGGL(k_bin_items<0>, dim3(blocks_for(b.n_bin_wave, 256)), dim3(256), 0, s, b);
-    if (b.n_bin_group) hipLaunchKernelGGL(k_bin_items<1>, dim3(blocks_for(b.n_bin_group, 256)), dim3(256), 0, s, b);
+    const uint32_t wb = blocks_for(b.n_bin_wave, 256), gb = blocks_for(b.n_bin_group, 256);
+    if (wb + gb) hipLaunchKernelGGL(k_bin_items, dim3(wb + gb), dim3(256), 0, s, b, wb);
     return hipGetLastError();
 }
 
+template <bool EMIT>
+static void launch_bin_t(const BatchDev &b, hipStream_t s) {
+    const uint32_t merged = b.n_bin_group + blocks_for(b.n_bin_wave, 8);
+    if (merged == 0) return;
+    if (merged <= BIN_MERGED_BLOCKS) {
+        hipLaunchKernelGGL(k_bin<EMIT>, dim3(merged), dim3(512), 0, s, b);
+        return;
+    }
+    if (b.n_bin_wave) hipLaunchKernelGGL(k_bin_wave<EMIT>, dim3(blocks_for(b.n_bin_wave, 4)), dim3(256), 0, s, b);
+    if (b.n_bin_group) hipLaunchKernelGGL(k_bin_group<EMIT>, dim3(b.n_bin_group), dim3(256), 0, s, b);
+}
+
 hipError_t launch_bin(const BatchDev &b, bool emit, hipStream_t s) {
-    if (b.n_bin_wave) {
-        const dim3 g(blocks_for(b.n_bin_wave, 4));
-        if (emit) hipLaunchKernelGGL(k_bin_wave<true>, g, dim3(256), 0, s, b);
-        else hipLaunchKernelGGL(k_bin_wave<false>, g, dim3(256), 0, s, b);
-    }
-    if (b.n_bin_group) {
-        const dim3 g(b.n_bin_group);
-        if (emit) hipLaunchKernelGGL(k_bin_group<true>, g, dim3(256), 0, s, b);
-        else hipLaunchKernelGGL(k_bin_group<false>, g, dim3(256), 0, s, b);
-    }
+    if (emit) launch_bin_t<true>(b, s);
+    else launch_bin_t<false>(b, s);
     return hipGetLastError();
 }
 
@@ -1970,23 +2022,16 @@ hipError_t launch_propagate(const BatchDev &b, uint32_t block, uint32_t rows, hi
     return hipGetLastError();
 }
 
-template <bool CLIPS>
-static void launch_entries_t(const BatchDev &b, bool write, hipStream_t s) {
-    if (b.n_bin_wave) {
-        const dim3 g(blocks_for(b.n_bin_wave, 4));
-        if (write) hipLaunchKernelGGL((k_entries_wave<true, CLIPS>), g, dim3(256), 0, s, b);
-        else hipLaunchKernelGGL((k_entries_wave<false, CLIPS>), g, dim3(256), 0, s, b);
-    }
-    if (b.n_bin_group) {
-        const dim3 g(b.n_bin_group);
-        if (write) hipLaunchKernelGGL((k_entries_group<true, CLIPS>), g, dim3(256), 0, s, b);
-        else hipLaunchKernelGGL((k_entries_group<false, CLIPS>), g, dim3(256), 0, s, b);
-    }
-}
-
 hipError_t launch_entries(const BatchDev &b, bool write, hipStream_t s) {
-    if (b.has_clips) launch_entries_t<true>(b, write, s);
-    else launch_entries_t<false>(b, write, s);
+    const dim3 g(b.n_bin_group + blocks_for(b.n_bin_wave, 4));
+    if (g.x == 0) return hipSuccess;
+    if (b.has_clips) {
+        if (write) hipLaunchKernelGGL((k_entries<true, true>), g, dim3(256), 0, s, b);
+        else hipLaunchKernelGGL((k_entries<false, true>), g, dim3(256), 0, s, b);
+    } else {
+        if (write) hipLaunchKernelGGL((k_entries<true, false>), g, dim3(256), 0, s, b);
+        else hipLaunchKernelGGL((k_entries<false, false>), g, dim3(256), 0, s, b);
+    }
     return hipGetLastError();
 }
 
