@@ -358,6 +358,9 @@ __device__ __forceinline__ void over_step(bool has_src, float &pr, float &pg, fl
 
 constexpr int EV_GROUP = 4;  // blend events whose mask words are loaded together
 
+// Transmittance from which on a tile is tested for being settled (see settled below).
+constexpr float SETTLED_T = 1.0f / (1 << 21);
+
 // A gradient paint's colour at pixel centre (px, py): the tile shader's colour texture coordinate
 // (shaders/d3d9/tile.vert:77, mat2(m11, m21, m12, m22) * position + (m13, m23)), for a radial
 // gradient its filter's t (shaders/d3d9/tile.frag:296-323: the larger root of the two circles'
@@ -603,6 +606,34 @@ __global__ __launch_bounds__(256) void k_composite(BatchDev b, const uint32_t *s
             return;
         }
     }
+    // Whether nothing below can change this lane's pixels' bytes: then the wave stops, once that holds
+    // for all its lanes.  What is left adds to a channel at most 255 |t| in all (t the transmittance:
+    // every weight taken from it, the loaded destination's too, times a colour of at most 255 byte
+    // units).  Each fma rounds a sum up by at most the term itself (a term below half an ulp changes
+    // nothing, a larger one exceeds the error), so the channel ends within 2 x 255 |t| above; t may
+    // pass 0 by a rounding error of an opaque layer, 2^-24 of it, and lower the channel by as much
+    // of that.  The channel's byte is settled when the one 255 |t| below and the one 4 x 255 |t| above
+    // agree, alpha's since 255 - 255 t rounds to 255.
+    // The kernel is VALU-bound, so what is left out is what it saves: the 48-scene batch (26 entries a
+    // tile, hundreds on its dense canvases) 619 -> 391 us, the 4096^2 scene (31 a tile) 71 -> 64 us.
+    auto settled = [&]() {
+        float t = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; q++) t = fmaxf(t, fabsf(tr[q]));
+        if (__ballot(t >= SETTLED_T)) return false;
+        bool same = true;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const float d = 255.0f * fabsf(tr[q]);
+            uint32_t lo = __builtin_amdgcn_cvt_pk_u8_f32(r[q] - d, 0, 0u), hi = __builtin_amdgcn_cvt_pk_u8_f32(r[q] + 4.0f * d, 0, 0u);
+            lo = __builtin_amdgcn_cvt_pk_u8_f32(g[q] - d, 1, lo);
+            hi = __builtin_amdgcn_cvt_pk_u8_f32(g[q] + 4.0f * d, 1, hi);
+            lo = __builtin_amdgcn_cvt_pk_u8_f32(bl[q] - d, 2, lo);
+            hi = __builtin_amdgcn_cvt_pk_u8_f32(bl[q] + 4.0f * d, 2, hi);
+            same = same && lo == hi;
+        }
+        return __ballot(!same) == 0;
+    };
     // chunks of 64 entries from the top one down
     for (uint32_t base = e0 + (e1 > e0 ? (e1 - e0 - 1) / 64 * 64 : 0); e1 > e0; base -= 64) {
         const uint32_t i = base + lane;
@@ -752,9 +783,10 @@ __global__ __launch_bounds__(256) void k_composite(BatchDev b, const uint32_t *s
                     blend(wcol[j], m);
                 }
             }
-            if (base == e0) break;
+            if (base == e0 || settled()) break;
             continue;
         }
+        bool done = false;
         int ja[EV_GROUP], jb[EV_GROUP];
         uint32_t ma[EV_GROUP], mb[EV_GROUP];
         take(ja, ma);
@@ -769,8 +801,10 @@ __global__ __launch_bounds__(256) void k_composite(BatchDev b, const uint32_t *s
             blend_group(jb, mb);
             __builtin_amdgcn_sched_barrier(0);
             if (ja[0] < 0) break;
+            done = settled();
+            if (done) break;
         }
-        if (base == e0) break;
+        if (base == e0 || done || settled()) break;
     }
     if (x < 0 || x >= width) return;  // a view box past the target's left or right edge
     uint8_t *const cptr = out + (int64_t)y0 * pitch + (int64_t)x * 4;  // this lane's top pixel
