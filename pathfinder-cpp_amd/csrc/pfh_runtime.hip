@@ -116,6 +116,38 @@ struct Arena {
     size_t cap = 0, top = 0;
 };
 
+// Device blocks that one use gave back and the next takes: a program that uploads a scene every frame
+// otherwise spends a millisecond on hipMalloc and hipFree (which waits for the device).  Blocks of
+// 2^k bytes up to BLOCK_BYTES, at most POOL_BYTES of them in all; the rest goes back to the runtime at once, the
+// others when the context ends.  A block is given back only when the device is done with it, and a
+// context is used by one host thread at a time.
+struct BlockPool {
+    static constexpr size_t BLOCK_BYTES = 64u << 20, POOL_BYTES = 256u << 20;
+    std::multimap<size_t, void *> blocks;
+    size_t bytes = 0;
+    void *take(size_t cap) {
+        auto it = blocks.find(cap);
+        if (it == blocks.end()) return nullptr;
+        void *p = it->second;
+        blocks.erase(it);
+        bytes -= cap;
+        return p;
+    }
+    void give(void *p, size_t cap) {
+        if (cap > BLOCK_BYTES || bytes + cap > POOL_BYTES) {
+            (void)hipFree(p);
+            return;
+        }
+        blocks.emplace(cap, p);
+        bytes += cap;
+    }
+    void clear() {
+        for (auto &b : blocks) (void)hipFree(b.second);
+        blocks.clear();
+        bytes = 0;
+    }
+};
+
 // Grow-only device buffer (the reference grows buffers to 2^k, core/d3d11/renderer.cpp:719-724).
 // With an arena the buffer is carved from it instead (no hipMalloc / hipFree): a regrowth takes
 // fresh space above the arena's top, and running past the arena's end is an error.
@@ -123,6 +155,7 @@ struct DevBuf {
     void *ptr = nullptr;
     size_t bytes = 0;
     Arena *arena = nullptr;
+    BlockPool *pool = nullptr;  // its blocks come from there and go back there
     void ensure(size_t need) {
         if (need <= bytes && ptr) return;
         if (arena) {
@@ -137,11 +170,24 @@ struct DevBuf {
         }
         size_t cap = 256;
         while (cap < need) cap <<= 1;
+        if (pool) {
+            release();
+            ptr = pool->take(cap);
+            if (ptr) {
+                bytes = cap;
+                return;
+            }
+        }
         if (ptr) HIP_TRY(hipFree(ptr));
         ptr = nullptr;
         bytes = 0;
         g_alloc_generation++;
         hipError_t e = hipMalloc(&ptr, cap);
+        if (e != hipSuccess && pool && !pool->blocks.empty()) {  // the kept blocks may be what is missing
+            (void)hipGetLastError();
+            pool->clear();
+            e = hipMalloc(&ptr, cap);
+        }
         if (e != hipSuccess) {
             (void)hipGetLastError();
             ptr = nullptr;
@@ -150,7 +196,8 @@ struct DevBuf {
         bytes = cap;
     }
     void release() {
-        if (ptr && !arena) (void)hipFree(ptr);
+        if (ptr && pool) pool->give(ptr, bytes);
+        else if (ptr && !arena) (void)hipFree(ptr);
         ptr = nullptr;
         bytes = 0;
     }
@@ -160,11 +207,88 @@ struct DevBuf {
     }
 };
 
-template <typename T>
-static void upload(DevBuf &buf, const std::vector<T> &v) {
-    buf.ensure(std::max<size_t>(v.size() * sizeof(T), 4));
-    if (!v.empty()) HIP_TRY(hipMemcpy(buf.ptr, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-}
+// Pinned host memory that copies go through, two halves in turn: a copy to or from ordinary memory
+// costs tens of microseconds on its own, and one with a pitch a transfer per row.
+struct Stage {
+    static constexpr size_t HALF = 1u << 20;
+    uint8_t *ptr = nullptr;
+    uint8_t *get() {
+        if (!ptr) HIP_TRY(hipHostMalloc((void **)&ptr, 2 * HALF));
+        return ptr;
+    }
+    void release() {
+        if (ptr) (void)hipHostFree(ptr);
+        ptr = nullptr;
+    }
+};
+
+// Bytes to the device in order, through the stage: one half is filled while the other's copy runs.
+// The stage is in use until the stream has run the last copy.
+struct StageOut {
+    uint8_t *const stage, *dev;
+    hipStream_t st;
+    hipEvent_t *ev;  // two
+    size_t fill = 0, half = 0;
+    bool pending[2] = {false, false};
+    StageOut(Stage &s, void *to, hipStream_t stream, hipEvent_t *events)
+        : stage(s.get()), dev(static_cast<uint8_t *>(to)), st(stream), ev(events) {}
+    void put(const void *src, size_t n) {  // src null: n bytes of no meaning
+        const uint8_t *from = static_cast<const uint8_t *>(src);
+        while (n) {
+            const size_t k = std::min(n, Stage::HALF - fill);
+            if (from) {
+                std::memcpy(stage + half * Stage::HALF + fill, from, k);
+                from += k;
+            }
+            fill += k;
+            n -= k;
+            if (fill == Stage::HALF) flush();
+        }
+    }
+    void flush() {
+        if (!fill) return;
+        HIP_TRY(hipMemcpyAsync(dev, stage + half * Stage::HALF, fill, hipMemcpyHostToDevice, st));
+        HIP_TRY(hipEventRecord(ev[half], st));
+        pending[half] = true;
+        dev += fill;
+        fill = 0;
+        half ^= 1;
+        if (pending[half]) HIP_TRY(hipEventSynchronize(ev[half]));
+    }
+};
+
+// Host arrays on their way to the device, laid out one after the other in one device block (their
+// buffers carved from it).
+struct Upload {
+    struct Part {
+        DevBuf *buf;
+        const void *src;
+        size_t bytes;
+    };
+    std::vector<Part> parts;
+    size_t total = 0;
+    template <typename T>
+    void add(DevBuf &buf, const std::vector<T> &v) {
+        const size_t n = v.size() * sizeof(T);
+        parts.push_back(Part{&buf, v.data(), n});
+        total += (std::max<size_t>(n, 4) + 255) & ~(size_t)255;
+    }
+    // Enqueues the copies on st.
+    void send(DevBuf &block, Arena &arena, Stage &stage, hipStream_t st, hipEvent_t *ev) {
+        block.ensure(total);
+        arena = Arena{block.as<uint8_t>(), total, 0};
+        StageOut out(stage, block.ptr, st, ev);
+        for (const Part &p : parts) {
+            p.buf->arena = &arena;
+            p.buf->ptr = nullptr;
+            p.buf->bytes = 0;
+            p.buf->ensure(std::max<size_t>(p.bytes, 4));
+            out.put(p.src, p.bytes);
+            out.put(nullptr, p.buf->bytes - p.bytes);
+        }
+        out.flush();
+    }
+};
 
 struct SceneHost {
     bool live = false;
@@ -183,6 +307,8 @@ struct SceneHost {
     std::vector<uint32_t> path_breaks;  // chord chains per path (two extra stream points each)
     uint64_t n_breaks = 0;
     std::vector<float> features;
+    DevBuf d_block;  // holds the arrays below (d_out_owned apart)
+    Arena arena;
     DevBuf d_features;
     DevBuf d_pts, d_segs, d_seg_path, d_path_rect, d_path_tile_off, d_path_col_off, d_col_path, d_path_rgba,
         d_path_rule, d_path_seg_off, d_bin_paths, d_out_owned, d_path_clip, d_path_level;
@@ -191,6 +317,10 @@ struct SceneHost {
     bool has_ops = false;  // some record composites through an op
     DevBuf d_path_paint, d_paints, d_ramps;
     uint32_t n_bin_wave = 0, n_bin_group = 0;  // paths binned by one wave / by one workgroup
+    void release() {  // once the device is done with the scene
+        d_block.release();
+        d_out_owned.release();
+    }
     uint8_t *d_out = nullptr;
     int64_t out_pitch = 0;
     // placement in the last rasterized batch (for dumps)
@@ -386,6 +516,8 @@ struct pfh_ctx {
     std::vector<float> predictor;
     float predictor_safety = 1.25f;
     DevBuf mlp_params, mlp_x, mlp_h, mlp_out;
+    BlockPool pool;  // blocks of released scenes and of the stroker's and dasher's buffers
+    Stage stage;
     pfh_stats stats{};
     Schedule sched;                  // launch schedule (pfh_set_schedule / pfh_autotune)
     std::unique_ptr<Server> server;  // request loop, when started
@@ -726,6 +858,77 @@ static void validate_style(const pfh_stroke_style &st) {
         throw PfhError{PFH_E_ARG, "invalid stroke style"};
 }
 
+// Device memory to host memory through the stage, `rows` rows of `row` bytes; returns when it is done.
+// Whole rows (with what lies between them) are copied into one half while the other's are handed out;
+// rows far apart go row by row, and adjacent ones count as one.
+static void read_rows(pfh_ctx *ctx, uint8_t *dst, size_t dst_pitch, const uint8_t *src, size_t src_pitch, size_t row,
+                      size_t rows) {
+    if (row == 0 || rows == 0) return;
+    const bool flat = rows == 1 || (src_pitch == row && dst_pitch == row);
+    if (!flat && (src_pitch > Stage::HALF || src_pitch > 2 * row)) {
+        HIP_TRY(hipMemcpy2D(dst, dst_pitch, src, src_pitch, row, rows, hipMemcpyDeviceToHost));
+        return;
+    }
+    // pieces: `per` bytes of flat memory, or `per` rows
+    const size_t all = flat ? row * rows : rows, per = flat ? Stage::HALF : Stage::HALF / src_pitch;
+    const size_t n = (all + per - 1) / per;
+    uint8_t *const stage = ctx->stage.get();
+    hipStream_t st = ctx->w->stream;
+    hipEvent_t *ev = ctx->w->stage_ev;
+    auto fetch = [&](size_t k) {
+        const size_t at = k * per, m = std::min(per, all - at);
+        HIP_TRY(hipMemcpyAsync(stage + (k & 1) * Stage::HALF, src + (flat ? at : at * src_pitch),
+                               flat ? m : (m - 1) * src_pitch + row, hipMemcpyDeviceToHost, st));
+        HIP_TRY(hipEventRecord(ev[k & 1], st));
+    };
+    struct Drain {  // nothing writes to the stage after an error
+        hipStream_t st;
+        ~Drain() { (void)hipStreamSynchronize(st); }
+    } drain{st};
+    fetch(0);
+    for (size_t k = 0; k < n; k++) {
+        if (k + 1 < n) fetch(k + 1);
+        HIP_TRY(hipEventSynchronize(ev[k & 1]));
+        const size_t at = k * per, m = std::min(per, all - at);
+        const uint8_t *from = stage + (k & 1) * Stage::HALF;
+        if (flat) {
+            std::memcpy(dst + at, from, m);
+        } else {
+            for (size_t r = 0; r < m; r++) std::memcpy(dst + (at + r) * dst_pitch, from + r * src_pitch, row);
+        }
+    }
+}
+
+// Buffers of one stroke or dash call, from the context's pool and back to it once the stream is idle.
+struct Pooled {
+    pfh_ctx *ctx;
+    std::vector<DevBuf *> bufs;
+    Pooled(pfh_ctx *c, std::vector<DevBuf *> b) : ctx(c), bufs(std::move(b)) {
+        for (DevBuf *d : bufs) d->pool = &ctx->pool;
+    }
+    ~Pooled() {
+        (void)hipStreamSynchronize(ctx->w->stream);
+        for (DevBuf *d : bufs) d->release();
+    }
+};
+
+// An array to the device and back on the current workspace's stream, through the stage; both return
+// when the copy is done.
+template <typename T>
+static void h2d(pfh_ctx *ctx, DevBuf &buf, const std::vector<T> &v) {
+    const size_t n = v.size() * sizeof(T);
+    buf.ensure(std::max<size_t>(n, 4));
+    StageOut out(ctx->stage, buf.ptr, ctx->w->stream, ctx->w->stage_ev);
+    out.put(v.data(), n);
+    out.flush();
+    HIP_TRY(hipStreamSynchronize(ctx->w->stream));
+}
+template <typename T>
+static void d2h(pfh_ctx *ctx, std::vector<T> &v, const DevBuf &buf) {
+    const size_t n = v.size() * sizeof(T);
+    read_rows(ctx, reinterpret_cast<uint8_t *>(v.data()), n, buf.as<uint8_t>(), n, n, n ? 1 : 0);
+}
+
 // Strokes every path of `in` with its style (OutlineStrokeToFill::offset + into_outline,
 // core/stroke.cpp:124-195).  The host only lays out each contour's strands of segments in the
 // reference's offsetting order (forward: SegmentsIter order with the closing line unless the
@@ -820,25 +1023,19 @@ static HostOutlines stroke_on_device(pfh_ctx *ctx, const float2 *P, const uint8_
     hipStream_t st = ctx->w->stream;
     DevBuf d_segs, d_cnt, d_off, d_leaves, d_outs, d_region_off, d_region_pts, d_region_flags, d_pcnt, d_out_off,
         d_pts, d_flags;
-    struct Release {
-        std::vector<DevBuf *> bufs;
-        ~Release() {
-            for (DevBuf *b : bufs) b->release();
-        }
-    } release{{&d_segs, &d_cnt, &d_off, &d_leaves, &d_outs, &d_region_off, &d_region_pts, &d_region_flags, &d_pcnt,
-               &d_out_off, &d_pts, &d_flags}};
-    upload(d_segs, segs);
+    Pooled pooled(ctx, {&d_segs, &d_cnt, &d_off, &d_leaves, &d_outs, &d_region_off, &d_region_pts, &d_region_flags,
+                        &d_pcnt, &d_out_off, &d_pts, &d_flags});
+    h2d(ctx, d_segs, segs);
     d_cnt.ensure(4ull * ns + 4);
     HIP_TRY(launch_offset_pieces(d_segs.as<StrokeSegment>(), ns, d_cnt.as<uint32_t>(), nullptr, nullptr, false, st));
     std::vector<uint32_t> cnt(ns);
-    if (ns) HIP_TRY(hipMemcpyAsync(cnt.data(), d_cnt.ptr, 4ull * ns, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    d2h(ctx, cnt, d_cnt);
     std::vector<uint32_t> leaf_off(ns + 1, 0);
     for (uint32_t i = 0; i < ns; i++) {
         if ((uint64_t)leaf_off[i] + cnt[i] >= 0xF0000000ull) throw PfhError{PFH_E_LIMIT, "too many stroke pieces"};
         leaf_off[i + 1] = leaf_off[i] + cnt[i];
     }
-    upload(d_off, leaf_off);
+    h2d(ctx, d_off, leaf_off);
     d_leaves.ensure(sizeof(StrokeLeaf) * ((size_t)leaf_off[ns] + 1));
     HIP_TRY(launch_offset_pieces(d_segs.as<StrokeSegment>(), ns, nullptr, d_off.as<uint32_t>(),
                                  d_leaves.as<StrokeLeaf>(), true, st));
@@ -851,8 +1048,8 @@ static HostOutlines stroke_on_device(pfh_ctx *ctx, const float2 *P, const uint8_
         if (region_off[c] + bound >= 0xF0000000ull) throw PfhError{PFH_E_LIMIT, "stroked outline too large"};
         region_off[c + 1] = region_off[c] + (uint32_t)bound;
     }
-    upload(d_outs, outs);
-    upload(d_region_off, region_off);
+    h2d(ctx, d_outs, outs);
+    h2d(ctx, d_region_off, region_off);
     d_region_pts.ensure(8ull * region_off[nc] + 8);
     d_region_flags.ensure((size_t)region_off[nc] + 4);
     d_pcnt.ensure(4ull * nc);
@@ -860,25 +1057,21 @@ static HostOutlines stroke_on_device(pfh_ctx *ctx, const float2 *P, const uint8_
                             d_segs.as<StrokeSegment>(), d_region_off.as<uint32_t>(), d_region_pts.as<float2>(),
                             d_region_flags.as<uint8_t>(), d_pcnt.as<uint32_t>(), st));
     std::vector<uint32_t> pcnt(nc);
-    HIP_TRY(hipMemcpyAsync(pcnt.data(), d_pcnt.ptr, 4ull * nc, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
+    d2h(ctx, pcnt, d_pcnt);
     std::vector<uint32_t> out_off(nc + 1, 0);
     for (uint32_t c = 0; c < nc; c++) {
         if (pcnt[c] > region_off[c + 1] - region_off[c]) throw PfhError{PFH_E_STATE, "stroke region overflow"};
         out_off[c + 1] = out_off[c] + pcnt[c];
     }
-    upload(d_out_off, out_off);
+    h2d(ctx, d_out_off, out_off);
     d_pts.ensure(8ull * out_off[nc] + 8);
     d_flags.ensure((size_t)out_off[nc] + 4);
     HIP_TRY(launch_compact(d_region_off.as<uint32_t>(), d_out_off.as<uint32_t>(), nc, d_region_pts.as<float2>(),
                            d_region_flags.as<uint8_t>(), d_pts.as<float2>(), d_flags.as<uint8_t>(), st));
     res.pts.resize(out_off[nc]);
     res.flags.resize(out_off[nc]);
-    if (out_off[nc]) {
-        HIP_TRY(hipMemcpyAsync(res.pts.data(), d_pts.ptr, 8ull * out_off[nc], hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipMemcpyAsync(res.flags.data(), d_flags.ptr, out_off[nc], hipMemcpyDeviceToHost, st));
-    }
-    HIP_TRY(hipStreamSynchronize(st));
+    d2h(ctx, res.pts, d_pts);
+    d2h(ctx, res.flags, d_flags);
     res.contour_start.assign(out_off.begin(), out_off.end());
     res.closed.assign(nc, 1);
     return res;
@@ -929,25 +1122,20 @@ static HostOutlines dash_on_device(pfh_ctx *ctx, const float2 *P, const uint8_t 
     if (n) {
         hipStream_t st = ctx->w->stream;
         DevBuf d_pts, d_flags, d_cs, d_closed, d_paths, d_dashes, d_cnt, d_off, d_opts, d_oflags, d_ocs;
-        struct Release {
-            std::vector<DevBuf *> bufs;
-            ~Release() {
-                for (DevBuf *b : bufs) b->release();
-            }
-        } release{{&d_pts, &d_flags, &d_cs, &d_closed, &d_paths, &d_dashes, &d_cnt, &d_off, &d_opts, &d_oflags, &d_ocs}};
-        upload(d_pts, std::vector<float2>(P, P + n_points));
-        upload(d_flags, std::vector<uint8_t>(F, F + n_points));
-        upload(d_cs, std::vector<int32_t>(contour_start, contour_start + n_contours + 1));
-        upload(d_closed, std::vector<uint8_t>(contour_closed, contour_closed + n_contours));
-        upload(d_paths, dp);
-        upload(d_dashes, std::vector<float>(dashes, dashes + n_dashes));
+        Pooled pooled(ctx, {&d_pts, &d_flags, &d_cs, &d_closed, &d_paths, &d_dashes, &d_cnt, &d_off, &d_opts, &d_oflags,
+                            &d_ocs});
+        h2d(ctx, d_pts, std::vector<float2>(P, P + n_points));
+        h2d(ctx, d_flags, std::vector<uint8_t>(F, F + n_points));
+        h2d(ctx, d_cs, std::vector<int32_t>(contour_start, contour_start + n_contours + 1));
+        h2d(ctx, d_closed, std::vector<uint8_t>(contour_closed, contour_closed + n_contours));
+        h2d(ctx, d_paths, dp);
+        h2d(ctx, d_dashes, std::vector<float>(dashes, dashes + n_dashes));
         d_cnt.ensure(8ull * n);
         HIP_TRY(launch_dash(d_pts.as<float2>(), d_flags.as<uint8_t>(), d_cs.as<int32_t>(), d_closed.as<uint8_t>(),
                             d_paths.as<DashPath>(), n, d_dashes.as<float>(), d_cnt.as<uint32_t>(), nullptr, nullptr,
                             nullptr, nullptr, false, st));
         std::vector<uint32_t> cnt(2 * (size_t)n);
-        HIP_TRY(hipMemcpyAsync(cnt.data(), d_cnt.ptr, 8ull * n, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
+        d2h(ctx, cnt, d_cnt);
         for (uint32_t k = 0; k < n; k++) {
             if (cnt[2 * k] == 0xFFFFFFFFu)
                 throw PfhError{PFH_E_LIMIT, "dash pattern too fine for its path (more than 2^24 dash steps)"};
@@ -956,7 +1144,7 @@ static HostOutlines dash_on_device(pfh_ctx *ctx, const float2 *P, const uint8_t 
             off[2 * k + 2] = (uint32_t)np;
             off[2 * k + 3] = (uint32_t)nc;
         }
-        upload(d_off, off);
+        h2d(ctx, d_off, off);
         d_opts.ensure(8ull * off[2 * n] + 8);
         d_oflags.ensure((size_t)off[2 * n] + 4);
         d_ocs.ensure(4ull * off[2 * n + 1] + 4);
@@ -966,12 +1154,9 @@ static HostOutlines dash_on_device(pfh_ctx *ctx, const float2 *P, const uint8_t 
         dpts.resize(off[2 * n]);
         dflags.resize(off[2 * n]);
         dcs.resize(off[2 * n + 1]);
-        if (!dpts.empty()) {
-            HIP_TRY(hipMemcpyAsync(dpts.data(), d_opts.ptr, 8 * dpts.size(), hipMemcpyDeviceToHost, st));
-            HIP_TRY(hipMemcpyAsync(dflags.data(), d_oflags.ptr, dflags.size(), hipMemcpyDeviceToHost, st));
-        }
-        if (!dcs.empty()) HIP_TRY(hipMemcpyAsync(dcs.data(), d_ocs.ptr, 4 * dcs.size(), hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
+        d2h(ctx, dpts, d_opts);
+        d2h(ctx, dflags, d_oflags);
+        d2h(ctx, dcs, d_ocs);
     }
     HostOutlines res;
     size_t k = 0;
@@ -1330,33 +1515,47 @@ static int scene_upload_desc(pfh_ctx *ctx, const pfh_scene_desc *d) {
         }
     }
     HIP_TRY(hipSetDevice(ctx->device));
-    upload(s->d_features, s->features);
-    upload(s->d_pts, pts);
-    upload(s->d_segs, segs_dev);
-    upload(s->d_seg_path, seg_path);
-    upload(s->d_path_rect, s->path_rect);
-    upload(s->d_path_tile_off, s->path_tile_off);
-    upload(s->d_path_col_off, s->path_col_off);
-    upload(s->d_col_path, col_path);
-    upload(s->d_path_rgba, s->path_rgba);
-    upload(s->d_path_rule, s->path_rule);
+    Upload up;
+    up.add(s->d_features, s->features);
+    up.add(s->d_pts, pts);
+    up.add(s->d_segs, segs_dev);
+    up.add(s->d_seg_path, seg_path);
+    up.add(s->d_path_rect, s->path_rect);
+    up.add(s->d_path_tile_off, s->path_tile_off);
+    up.add(s->d_path_col_off, s->path_col_off);
+    up.add(s->d_col_path, col_path);
+    up.add(s->d_path_rgba, s->path_rgba);
+    up.add(s->d_path_rule, s->path_rule);
     if (!s->path_paint.empty()) {
-        upload(s->d_path_paint, s->path_paint);
-        upload(s->d_paints, paints);
-        upload(s->d_ramps, ramps);
+        up.add(s->d_path_paint, s->path_paint);
+        up.add(s->d_paints, paints);
+        up.add(s->d_ramps, ramps);
     }
-    upload(s->d_path_seg_off, s->path_seg_off);
-    upload(s->d_bin_paths, bin_wave);
+    up.add(s->d_path_seg_off, s->path_seg_off);
+    up.add(s->d_bin_paths, bin_wave);
     if (s->n_clip > 0) {
-        upload(s->d_path_clip, s->path_clip);
-        upload(s->d_path_level, s->path_level);
+        up.add(s->d_path_clip, s->path_clip);
+        up.add(s->d_path_level, s->path_level);
     }
+    s->d_block.pool = s->d_out_owned.pool = &ctx->pool;
+    struct GiveBack {  // an upload that fails leaves nothing behind
+        pfh_ctx *ctx;
+        SceneHost *s;
+        ~GiveBack() {
+            if (!s) return;
+            (void)hipStreamSynchronize(ctx->w->stream);
+            s->release();
+        }
+    } give_back{ctx, s.get()};
+    up.send(s->d_block, s->arena, ctx->stage, ctx->w->stream, ctx->w->stage_ev);
     s->out_pitch = (int64_t)s->width * 4;
     s->d_out_owned.ensure((size_t)s->out_pitch * s->height);
     s->d_out = s->d_out_owned.as<uint8_t>();
     s->live = true;
     predict_scene(ctx, *s);
+    HIP_TRY(hipStreamSynchronize(ctx->w->stream));  // the copies are done: any stream may draw the scene
     ctx->scenes.push_back(std::move(s));
+    give_back.s = nullptr;
     return (int)ctx->scenes.size() - 1;
 }
 
@@ -2311,12 +2510,11 @@ void pfh_destroy(pfh_ctx *ctx) {
     ctx->fixed.destroy();
     for (auto &s : ctx->scenes) {
         if (!s) continue;
-        for (DevBuf *b : {&s->d_features, &s->d_pts, &s->d_segs, &s->d_seg_path, &s->d_path_rect, &s->d_path_tile_off,
-                          &s->d_path_col_off, &s->d_col_path, &s->d_path_rgba, &s->d_path_rule, &s->d_path_seg_off, &s->d_bin_paths, &s->d_out_owned, &s->d_path_clip,
-                          &s->d_path_level, &s->d_path_paint, &s->d_paints, &s->d_ramps})
-            b->release();
+        s->release();
     }
     for (DevBuf *b : {&ctx->mlp_params, &ctx->mlp_x, &ctx->mlp_h, &ctx->mlp_out}) b->release();
+    ctx->pool.clear();
+    ctx->stage.release();
     delete ctx;
 }
 
@@ -2396,10 +2594,7 @@ int pfh_scene_release(pfh_ctx *ctx, int32_t scene_id) {
         }
         HIP_TRY(hipStreamSynchronize(ctx->w->stream));
         drop_graphs_of_scene(ctx, scene_id);
-        for (DevBuf *b : {&s.d_features, &s.d_pts, &s.d_segs, &s.d_seg_path, &s.d_path_rect, &s.d_path_tile_off, &s.d_path_col_off,
-                          &s.d_col_path, &s.d_path_rgba, &s.d_path_rule, &s.d_path_seg_off, &s.d_bin_paths, &s.d_out_owned, &s.d_path_clip,
-                          &s.d_path_level, &s.d_path_paint, &s.d_paints, &s.d_ramps})
-            b->release();
+        s.release();
         ctx->scenes[scene_id].reset();
     });
 }
@@ -2498,8 +2693,8 @@ int pfh_readback_rgba8(pfh_ctx *ctx, int32_t scene_id, void *dst, int64_t pitch_
         SceneHost &s = get_scene(ctx, scene_id);
         if (pitch_bytes < (int64_t)s.width * 4) throw PfhError{PFH_E_ARG, "bad pitch"};
         HIP_TRY(hipStreamSynchronize(ctx->w->stream));
-        HIP_TRY(hipMemcpy2D(dst, (size_t)pitch_bytes, s.d_out, (size_t)s.out_pitch, (size_t)s.width * 4,
-                            (size_t)s.height, hipMemcpyDeviceToHost));
+        read_rows(ctx, static_cast<uint8_t *>(dst), (size_t)pitch_bytes, s.d_out, (size_t)s.out_pitch,
+                  (size_t)s.width * 4, (size_t)s.height);
     });
 }
 
