@@ -77,6 +77,7 @@ enum SegKind : uint32_t { SEG_LINE = 1, SEG_QUAD = 2, SEG_CUBIC = 3 };
 // its chord points are then preceded by a NaN separator and its start point.
 constexpr uint32_t SEG_KIND_MASK = 0xffu;
 constexpr uint32_t SEG_CHAIN_BREAK = 0x100u;
+constexpr uint32_t SEG_ORIGINAL_SHIFT = 16;  // the kind again, kept where nothing is emitted (path features)
 
 // Launch schedule (chosen by pfh_autotune; every schedule gives bit-identical results).
 struct Schedule {

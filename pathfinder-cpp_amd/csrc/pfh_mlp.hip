@@ -8,8 +8,7 @@
 //
 // Parameter layout (5187 floats): W1[12][64], b1[64], W2[64][64], b2[64], W3[64][3], b3[3]
 // (row-major, W[in][out]).  Hidden activations per sample: h1[64], h2[64].
-#include <hip/hip_runtime.h>
-#include <stdint.h>
+#include "pfh_internal.h"
 
 namespace pfh {
 
@@ -160,6 +159,124 @@ __global__ __launch_bounds__(256) void k_mlp_outer(const float *__restrict__ A, 
     }
 }
 
+
+// ---------------------------------------------------------------------------
+// Per-path features (the network's inputs), a wave per path
+// ---------------------------------------------------------------------------
+//
+// The bounding box over the canvas' longer side, log1p of the control polygon's length, of its turning
+// (the angles between its consecutive edges of non-zero length, in segment order), of the
+// line, quad and cubic counts and of the tile rect's area, log of the side, and the fill rule.
+// Lanes take consecutive segments; a segment's first edge turns from the last edge of the
+// nearest earlier segment that has one, found by ballot.  On the host this took 32 us per thousand
+// segments (an arc cosine per edge): 0.32 ms of a 900^2 scene's upload, 1.6 ms of 400 dashed
+// strokes'; 12 and 42 us here.
+__global__ __launch_bounds__(256) void k_path_features(const float2 *pts, const uint2 *segs, const uint32_t *seg_off,
+                                                       const int4 *rects, const uint8_t *rules, uint32_t n_paths,
+                                                       float side, float *out) {
+#pragma clang fp contract(off)
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t p = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (p >= n_paths) return;  // whole wave
+    const uint32_t s0 = seg_off[p], s1 = seg_off[p + 1];
+    float poly = 0.0f, turn = 0.0f, bx0 = 1e30f, by0 = 1e30f, bx1 = -1e30f, by1 = -1e30f;
+    uint32_t kinds[3] = {0, 0, 0};
+    float cx = 0.0f, cy = 0.0f;  // direction of the last edge before this round (wave-uniform)
+    bool have = false;
+    // no contraction: an arc cosine near 1 turns the last bit of its argument into 3e-4
+    auto angle = [](float ax, float ay, float bx, float by) {
+#pragma clang fp contract(off)
+        return acosf(fmaxf(-1.0f, fminf(1.0f, ax * bx + ay * by)));
+    };
+    for (uint32_t base = s0; base < s1; base += 64) {  // uniform over the wave
+        const uint32_t i = base + lane;
+        float fx = 0.0f, fy = 0.0f, lx = 0.0f, ly = 0.0f;  // this segment's first and last edge
+        bool any = false;
+        if (i < s1) {
+            const uint2 sg = segs[i];
+            const uint32_t kind = sg.y >> SEG_ORIGINAL_SHIFT;
+            kinds[0] += kind == SEG_LINE ? 1u : 0u;
+            kinds[1] += kind == SEG_QUAD ? 1u : 0u;
+            kinds[2] += kind == SEG_CUBIC ? 1u : 0u;
+            const uint32_t np = kind == SEG_LINE ? 2u : (kind == SEG_QUAD ? 3u : 4u);
+            float2 a = {};
+            for (uint32_t q = 0; q < np; q++) {
+                const float2 c = pts[sg.x + q];
+                bx0 = c.x < bx0 ? c.x : bx0;
+                by0 = c.y < by0 ? c.y : by0;
+                bx1 = bx1 < c.x ? c.x : bx1;
+                by1 = by1 < c.y ? c.y : by1;
+                if (q > 0) {
+                    const float dx = c.x - a.x, dy = c.y - a.y, len = sqrtf(dx * dx + dy * dy);
+                    poly += len;
+                    if (len > 0.0f) {
+                        const float ux = dx / len, uy = dy / len;
+                        if (any) turn += angle(ux, uy, lx, ly);
+                        else {
+                            fx = ux;
+                            fy = uy;
+                        }
+                        lx = ux;
+                        ly = uy;
+                        any = true;
+                    }
+                }
+                a = c;
+            }
+        }
+        const uint64_t m = __ballot(any);
+        const uint64_t before = m & ((1ull << lane) - 1ull);
+        const int from = before ? 63 - __clzll(before) : 0;
+        float px = __shfl(lx, from, 64), py = __shfl(ly, from, 64);
+        if (!before) {
+            px = cx;
+            py = cy;
+        }
+        if (any && (before || have)) turn += angle(fx, fy, px, py);
+        if (m) {
+            const int last = 63 - __clzll(m);
+            cx = __shfl(lx, last, 64);
+            cy = __shfl(ly, last, 64);
+            have = true;
+        }
+    }
+    for (int d = 32; d > 0; d >>= 1) {
+        poly += __shfl_xor(poly, d, 64);
+        turn += __shfl_xor(turn, d, 64);
+        const float x0 = __shfl_xor(bx0, d, 64), y0 = __shfl_xor(by0, d, 64), x1 = __shfl_xor(bx1, d, 64),
+                    y1 = __shfl_xor(by1, d, 64);
+        bx0 = x0 < bx0 ? x0 : bx0;
+        by0 = y0 < by0 ? y0 : by0;
+        bx1 = bx1 < x1 ? x1 : bx1;
+        by1 = by1 < y1 ? y1 : by1;
+        for (int k = 0; k < 3; k++) kinds[k] += __shfl_xor(kinds[k], d, 64);
+    }
+    if (bx0 > bx1) bx0 = by0 = bx1 = by1 = 0.0f;
+    if (lane == 0) {
+        const int4 r = rects[p];
+        float *f = out + (int64_t)p * NI;
+        f[0] = bx0 / side;
+        f[1] = by0 / side;
+        f[2] = bx1 / side;
+        f[3] = by1 / side;
+        f[4] = log1pf(poly);
+        f[5] = log1pf(turn);
+        f[6] = log1pf((float)kinds[0]);
+        f[7] = log1pf((float)kinds[1]);
+        f[8] = log1pf((float)kinds[2]);
+        f[9] = log1pf((float)max(0, r.z - r.x) * (float)max(0, r.w - r.y));
+        f[10] = logf(side);
+        f[11] = (float)rules[p];
+    }
+}
+
+hipError_t path_features(const float2 *pts, const uint2 *segs, const uint32_t *seg_off, const int4 *rects,
+                         const uint8_t *rules, uint32_t n_paths, float side, float *out, hipStream_t s) {
+    if (n_paths == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_path_features, dim3((n_paths + 3) / 4), dim3(256), 0, s, pts, segs, seg_off, rects, rules, n_paths,
+                       side, out);
+    return hipGetLastError();
+}
 
 // Sizing inference: per path forward pass, expm1 of the (log1p) outputs clamped at 0, summed over
 // the paths into sums[NO] (float atomics per block).  A wave per path, a lane per hidden unit with its

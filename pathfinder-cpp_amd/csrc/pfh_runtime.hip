@@ -49,6 +49,8 @@ hipError_t mlp_backward(const float *params, const float *x, int64_t n, const fl
 hipError_t mlp_adam(float *params, float *m, float *v, const float *grad, int64_t n, float lr, int step,
                     hipStream_t s);
 int64_t mlp_param_count();
+hipError_t path_features(const float2 *pts, const uint2 *segs, const uint32_t *seg_off, const int4 *rects,
+                         const uint8_t *rules, uint32_t n_paths, float side, float *out, hipStream_t s);
 hipError_t mlp_predict_sum(const float *params, const float *x, int64_t n, float *sums, hipStream_t s);
 struct StrokeSegment {
     float2 p0, c0, c1, p1;
@@ -306,8 +308,7 @@ struct SceneHost {
     uint32_t clip_levels = 0;           // deepest clip level
     std::vector<uint32_t> path_breaks;  // chord chains per path (two extra stream points each)
     uint64_t n_breaks = 0;
-    std::vector<float> features;
-    DevBuf d_block;  // holds the arrays below (d_out_owned apart)
+    DevBuf d_block;  // holds the arrays below (d_features and d_out_owned apart)
     Arena arena;
     DevBuf d_features;
     DevBuf d_pts, d_segs, d_seg_path, d_path_rect, d_path_tile_off, d_path_col_off, d_col_path, d_path_rgba,
@@ -319,6 +320,7 @@ struct SceneHost {
     uint32_t n_bin_wave = 0, n_bin_group = 0;  // paths binned by one wave / by one workgroup
     void release() {  // once the device is done with the scene
         d_block.release();
+        d_features.release();
         d_out_owned.release();
     }
     uint8_t *d_out = nullptr;
@@ -785,58 +787,6 @@ static void validate_desc(const pfh_scene_desc *d) {
 }
 
 // Features for the sizing predictor, per path (see pfh_scene_features).
-static void path_features(const SceneHost &s, const std::vector<float2> &pts, const std::vector<uint2> &segs,
-                          uint32_t p, float *f) {
-    const int4 &r = s.path_rect[p];
-    float side = (float)std::max(s.width, s.height);
-    float nl = 0, nq = 0, nc = 0, poly = 0, turn = 0;
-    float bx0 = 1e30f, by0 = 1e30f, bx1 = -1e30f, by1 = -1e30f;
-    float2 prev_dir = make_float2(0, 0);
-    bool have_prev = false;
-    for (uint32_t sg = s.path_seg_off[p]; sg < s.path_seg_off[p + 1]; sg++) {
-        uint32_t k = segs[sg].y, fp = segs[sg].x;
-        int np = k == SEG_LINE ? 2 : (k == SEG_QUAD ? 3 : 4);
-        if (k == SEG_LINE) nl += 1;
-        else if (k == SEG_QUAD) nq += 1;
-        else nc += 1;
-        for (int i = 0; i < np; i++) {
-            float2 q = pts[fp + i];
-            bx0 = std::min(bx0, q.x);
-            by0 = std::min(by0, q.y);
-            bx1 = std::max(bx1, q.x);
-            by1 = std::max(by1, q.y);
-            if (i > 0) {
-                float2 a = pts[fp + i - 1];
-                float dx = q.x - a.x, dy = q.y - a.y;
-                float len = std::sqrt(dx * dx + dy * dy);
-                poly += len;
-                if (len > 0) {
-                    float2 dir = make_float2(dx / len, dy / len);
-                    if (have_prev) {
-                        float c = std::max(-1.0f, std::min(1.0f, dir.x * prev_dir.x + dir.y * prev_dir.y));
-                        turn += std::acos(c);
-                    }
-                    prev_dir = dir;
-                    have_prev = true;
-                }
-            }
-        }
-    }
-    if (bx0 > bx1) bx0 = by0 = bx1 = by1 = 0;
-    f[0] = bx0 / side;
-    f[1] = by0 / side;
-    f[2] = bx1 / side;
-    f[3] = by1 / side;
-    f[4] = std::log1p(poly);
-    f[5] = std::log1p(turn);
-    f[6] = std::log1p(nl);
-    f[7] = std::log1p(nq);
-    f[8] = std::log1p(nc);
-    f[9] = std::log1p((float)std::max(0, r.z - r.x) * (float)std::max(0, r.w - r.y));
-    f[10] = std::log(side);
-    f[11] = (float)s.path_rule[p];
-}
-
 static void predict_scene(pfh_ctx *ctx, SceneHost &s);
 
 // ---------------------------------------------------------------------------
@@ -1478,9 +1428,6 @@ static int scene_upload_desc(pfh_ctx *ctx, const pfh_scene_desc *d) {
         }
     }
     bin_wave.insert(bin_wave.end(), bin_group.begin(), bin_group.end());
-    s->features.resize((size_t)d->n_paths * N_FEATURES);
-    for (int p = 0; p < d->n_paths; p++) path_features(*s, pts, segs, (uint32_t)p, &s->features[(size_t)p * N_FEATURES]);
-
     // On the device, segments of paths without tile columns carry kind 0: nothing can land
     // from them (add_fill culls, adjust_alpha_tile_backdrop ignores x outside [0, width)), so
     // the flattener skips them without looking up their path.  So do segments with a
@@ -1499,12 +1446,13 @@ static int scene_upload_desc(pfh_ctx *ctx, const pfh_scene_desc *d) {
         bool finite = true;
         for (uint32_t q = 0; q < np; q++) finite = finite && std::isfinite(pts[segs[i].x + q].x) && std::isfinite(pts[segs[i].x + q].y);
         if (r.z - r.x <= 0 || !finite) {
-            segs_dev[i].y = 0;
+            segs_dev[i].y = segs[i].y << SEG_ORIGINAL_SHIFT;
             continue;
         }
+        segs_dev[i].y |= segs[i].y << SEG_ORIGINAL_SHIFT;
         bool chained = false;
         for (size_t j = i; j-- > 0 && seg_path[j] == p;) {  // the previous emitting segment of the path
-            if (segs_dev[j].y == 0) break;
+            if ((segs_dev[j].y & SEG_KIND_MASK) == 0) break;
             chained = bits(pts[segs[j].x + seg_np(segs[j].y) - 1]) == bits(pts[segs[i].x]);
             break;
         }
@@ -1516,7 +1464,6 @@ static int scene_upload_desc(pfh_ctx *ctx, const pfh_scene_desc *d) {
     }
     HIP_TRY(hipSetDevice(ctx->device));
     Upload up;
-    up.add(s->d_features, s->features);
     up.add(s->d_pts, pts);
     up.add(s->d_segs, segs_dev);
     up.add(s->d_seg_path, seg_path);
@@ -1548,6 +1495,11 @@ static int scene_upload_desc(pfh_ctx *ctx, const pfh_scene_desc *d) {
         }
     } give_back{ctx, s.get()};
     up.send(s->d_block, s->arena, ctx->stage, ctx->w->stream, ctx->w->stage_ev);
+    s->d_features.pool = &ctx->pool;
+    s->d_features.ensure(4ull * N_FEATURES * s->n_paths + 4);
+    HIP_TRY(path_features(s->d_pts.as<float2>(), s->d_segs.as<uint2>(), s->d_path_seg_off.as<uint32_t>(),
+                          s->d_path_rect.as<int4>(), s->d_path_rule.as<uint8_t>(), s->n_paths,
+                          (float)std::max(s->width, s->height), s->d_features.as<float>(), ctx->w->stream));
     s->out_pitch = (int64_t)s->width * 4;
     s->d_out_owned.ensure((size_t)s->out_pitch * s->height);
     s->d_out = s->d_out_owned.as<uint8_t>();
@@ -2603,7 +2555,8 @@ int pfh_scene_features(pfh_ctx *ctx, int32_t scene_id, float *out) {
     if (!ctx || !out) return PFH_E_ARG;
     return run_guarded(ctx, [&] {
         SceneHost &s = get_scene(ctx, scene_id);
-        std::memcpy(out, s.features.data(), s.features.size() * sizeof(float));
+        const size_t n = sizeof(float) * N_FEATURES * (size_t)s.n_paths;
+        read_rows(ctx, reinterpret_cast<uint8_t *>(out), n, s.d_features.as<uint8_t>(), n, n, n ? 1 : 0);
     });
 }
 
