@@ -299,12 +299,12 @@ struct BatchDev {
     uint32_t *alpha_vis;          // [cap_vis] mask rows of the alpha entries (tiles that survive the z-cull)
     uint8_t *masks;               // [(A + 1) * 256]: row cap_alpha is all ones (written by the fill kernel)
     uint32_t *zbuf;               // [FB]
-    uint2 *fb_range;              // [FB] [start, end) of each framebuffer tile's entries in sort order
-    uint32_t *keys, *vals;        // [E] sort keys / values
-    uint32_t *keys_alt, *vals_alt;
+    uint2 *fb_range;              // [FB] [start, end) of each framebuffer tile's entries, sorted
+    uint32_t *keys, *keys_alt;    // [E] framebuffer tile (batch index) of an entry, and the sort's other buffer
     uint2 *entry_rec;             // [E] (alpha index | NO_ALPHA, rgba (alpha 0 if covers nothing)), or for a
                                   // gradient path (ENTRY_GRADIENT | mask row or ENTRY_ROW_NONE, paint index)
-    uint2 *entry_meta;            // [E] with dumps only: (local path, scene-local fb tile)
+    uint2 *rec_alt;               // [E] the sort's other buffer
+    uint2 *entry_meta, *meta_alt; // [E] with dumps only: (local path, scene-local fb tile), sorted likewise
     uint32_t *counters;           // [C_COUNT]
     int32_t dump;
     int32_t has_clips;            // some scene has clip paths: propagate in two phases, combine masks

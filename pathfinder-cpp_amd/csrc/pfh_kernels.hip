@@ -8,7 +8,7 @@
 //                                  with LDS counters; also writes every tile of the path's rect
 //   bound.comp                  -> (the bin count pass initialises each path's tiles)
 //   propagate.comp              -> k_propagate (prepare_tiles, tiler.cpp:369-439) + z-buffer
-//   sort.comp                   -> k_entries_* + stable LSD radix sort by framebuffer tile
+//   sort.comp                   -> k_entries + stable grouping by framebuffer tile
 //   fill.comp / fill.frag       -> k_fill_masks: analytic box-filtered area, fixed-point
 //   tile.comp / tile.frag       -> k_composite: premultiplied src-over in fp32, one RGBA8 store
 //
@@ -1616,7 +1616,7 @@ __device__ __forceinline__ void write_entry(const BatchDev &b, const SceneDev &s
             ry = 0u;
         }
     }
-    b.keys[e] = sc.fb_base + et.fbl;  // its value, e, is generated by the sort's first pass
+    b.keys[e] = sc.fb_base + et.fbl;
     b.entry_rec[e] = make_uint2(rx, ry);
     if (b.dump) b.entry_meta[e] = make_uint2(p, et.fbl);
 }
@@ -1730,163 +1730,325 @@ __global__ __launch_bounds__(256) void k_entries(BatchDev b) {
 }
 
 // ---------------------------------------------------------------------------
-// Stable LSD radix sort of (key, value) u32 pairs, 8 bits per pass
+// Draw entries grouped by framebuffer tile, in draw order within a tile
 // ---------------------------------------------------------------------------
+//
+// A scene's entries are contiguous, in draw order, and their keys lie in its own range of framebuffer
+// tiles, so each scene is sorted by itself, stably, by scene-local tile.  Two steps: the entries are
+// distributed over 256 buckets of consecutive tiles per scene (histogram, its scan, scatter: blocks of
+// SORT_TILE entries over the whole chip), then a block per bucket groups its entries by tile and
+// writes its tiles' ranges.  The entries' records move along, so that what reads a tile's entries
+// reads them in a row.  Where every scene is small (SORT_SMALL), the second step alone does it, a
+// block per scene.
+// Launch-bound on a single scene: as an LSD radix sort with its block table, a histogram, scan and
+// scatter per 8-bit digit and a pass for the ranges (8 launches, 5 for one digit) this took 82 us at
+// 4096x4096 with 10^4 paths and 36 us at 256x256; as 4 launches (1) 56 us and 7.
+// Bound by the stable ranking (a match per digit bit) and its LDS traffic: 48 scenes of 1024x1024,
+// 265 us before, 245 now, which also has the composite read records in a row (391 us, then 357).
+// The scatter's loads are all issued before the ranking: 16 us against 21 (48 scenes: 83, 127).
 
-constexpr int RS_THREADS = 256;
-constexpr int RS_ITEMS = 16;
-constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
+// Scenes of at most 256 framebuffer tiles and this many path tiles are sorted by one block each.
+constexpr uint64_t SORT_SMALL = 16384;
+// Buckets of this many path tiles on average (a bound of their entries) take blocks of 1024 threads while
+// there are at most SORT_WIDE_SCENES scenes.
+constexpr uint64_t SORT_WIDE = 4096;
+constexpr uint32_t SORT_WIDE_SCENES = 2;
+constexpr int SORT_THREADS = 256;
+constexpr int SORT_ITEMS = 16;
+constexpr int SORT_TILE = SORT_THREADS * SORT_ITEMS;
 
-// The sort runs per scene: a scene's entries are contiguous and its keys lie in its own range
-// of framebuffer tiles, so sorting each scene's entries by their scene-local tile index
-// (16 bits for canvases up to 4096^2) sorts the whole batch.  Sort blocks never straddle
-// scenes: scene k's entries [seg_e[k], seg_e[k + 1]) (clamped to the capacity) take blocks
-// [seg_b[k], seg_b[k + 1]) of RS_TILE items, and the digit histogram is laid out
-// [scene][digit][block of the scene], so its exclusive scan places every item inside its
-// scene's range, ordered by digit, then block, then rank.
-__global__ __launch_bounds__(RS_THREADS) void k_rs_segments(BatchDev b, uint32_t *seg_e, uint32_t *seg_b) {
+// Bits of a scene-local tile below its bucket.
+__device__ __forceinline__ uint32_t sort_shift(uint32_t n_fb) {
+    const uint32_t bits = n_fb > 1 ? 32u - (uint32_t)__clz((int)(n_fb - 1)) : 0u;
+    return bits > 8 ? bits - 8 : 0u;
+}
+
+// What is sorted: the keys (batch framebuffer tiles) and what goes with them.
+struct SortArrays {
+    uint32_t *keys;
+    uint2 *rec, *meta;  // meta: with dumps only, else null
+};
+
+// Blocks of the distribution never straddle scenes: scene k's entries [seg_e[k], seg_e[k + 1]) (clamped
+// to the capacity) take blocks [seg_b[k], seg_b[k + 1]), and the histogram is laid out
+// [scene][bucket][block of the scene], so that its exclusive scan places every entry inside its scene's
+// range, ordered by bucket, then block, then rank.  The histogram pass finds a block's scene by scanning
+// the scenes' block counts; its first block leaves them in seg_e and seg_b for the passes after it.
+struct SortBlock {
+    int k;
+    uint32_t lb, nbk, hbase, e0, e1, fb_base, shift;
+};
+__device__ __forceinline__ void sort_block(const BatchDev &b, const uint32_t *seg_e, const uint32_t *seg_b, int k,
+                                           uint32_t e, uint32_t e_next, uint32_t b0, uint32_t b1, SortBlock &sb) {
+    sb.k = k;
+    sb.lb = blockIdx.x - b0;
+    sb.nbk = b1 - b0;
+    sb.hbase = 256u * b0;
+    sb.e0 = e + sb.lb * SORT_TILE;
+    sb.e1 = min(sb.e0 + SORT_TILE, e_next);
+    sb.fb_base = b.scenes[k].fb_base;
+    sb.shift = sort_shift(b.scenes[k].n_fb);
+}
+
+__global__ __launch_bounds__(SORT_THREADS) void k_sort_hist(BatchDev b, uint32_t *seg_e, uint32_t *seg_b, uint32_t *hist) {
+    __shared__ uint32_t h[256];
+    __shared__ uint32_t s_k, s_e, s_en, s_b0, s_b1;
+    const uint32_t tid = threadIdx.x;
+    h[tid] = 0;
+    if (tid == 0) s_k = 0xffffffffu;
+    __syncthreads();
     uint32_t carry = 0;
-    for (int k0 = 0; k0 <= b.n_scenes; k0 += RS_THREADS) {
-        const int k = k0 + (int)threadIdx.x;
+    for (int k0 = 0; k0 <= b.n_scenes; k0 += SORT_THREADS) {
+        const int k = k0 + (int)tid;
         uint32_t e = 0, e_next = 0;
         if (k <= b.n_scenes) {
             const uint32_t total = min(b.counters[C_ENTRIES], b.cap_entries);
             e = k < b.n_scenes ? min(b.path_ent[b.scenes[k].path_base].x, total) : total;
             e_next = k + 1 < b.n_scenes ? min(b.path_ent[b.scenes[k + 1].path_base].x, total) : total;
-            seg_e[k] = e;
         }
-        const uint32_t nbk = k < b.n_scenes ? (e_next - e + RS_TILE - 1) / RS_TILE : 0u;
+        const uint32_t nbk = k < b.n_scenes ? (e_next - e + SORT_TILE - 1) / SORT_TILE : 0u;
         uint32_t tot;
-        const uint32_t ex = block_exclusive_scan<uint32_t>(nbk, tot);
-        if (k <= b.n_scenes) seg_b[k] = carry + ex;
+        const uint32_t at = carry + block_exclusive_scan<uint32_t>(nbk, tot);
+        if (k <= b.n_scenes && blockIdx.x == 0) {
+            seg_e[k] = e;
+            seg_b[k] = at;
+        }
+        if (blockIdx.x >= at && blockIdx.x - at < nbk) {
+            s_k = (uint32_t)k;
+            s_e = e;
+            s_en = e_next;
+            s_b0 = at;
+            s_b1 = at + nbk;
+        }
         carry += tot;
     }
-}
-
-// This block's scene and item range; false past the last block.
-struct RsBlock {
-    int k;
-    uint32_t lb, nbk, hbase, e0, e1, fb_base;
-};
-__device__ __forceinline__ bool rs_block(const BatchDev &b, const uint32_t *seg_e, const uint32_t *seg_b, RsBlock &rb) {
-    if (blockIdx.x >= seg_b[b.n_scenes]) return false;
-    rb.k = find_scene_wave(seg_b, b.n_scenes, blockIdx.x);
-    rb.lb = blockIdx.x - seg_b[rb.k];
-    rb.nbk = seg_b[rb.k + 1] - seg_b[rb.k];
-    rb.hbase = 256u * seg_b[rb.k];
-    rb.e0 = seg_e[rb.k] + rb.lb * RS_TILE;
-    rb.e1 = min(rb.e0 + RS_TILE, seg_e[rb.k + 1]);
-    rb.fb_base = b.scenes[rb.k].fb_base;
-    return true;
-}
-
-__global__ __launch_bounds__(RS_THREADS) void k_rs_hist(BatchDev b, const uint32_t *keys, const uint32_t *seg_e,
-                                                        const uint32_t *seg_b, int shift, uint32_t *hist) {
-    __shared__ uint32_t h[256];
-    RsBlock rb;
-    if (!rs_block(b, seg_e, seg_b, rb)) return;  // uniform over the block
-    h[threadIdx.x] = 0;
     __syncthreads();
+    if (s_k == 0xffffffffu) return;  // past the last block: uniform
+    SortBlock sb;
+    sort_block(b, seg_e, seg_b, (int)s_k, s_e, s_en, s_b0, s_b1, sb);
+    // neighbours mostly share a bucket: one add per run of a wave's row, by its first lane
+    const uint32_t lane = tid & 63;
 #pragma unroll 4
-    for (int i = 0; i < RS_ITEMS; i++) {
-        const uint32_t j = rb.e0 + (uint32_t)i * RS_THREADS + threadIdx.x;
-        if (j < rb.e1) atomicAdd(&h[((keys[j] - rb.fb_base) >> shift) & 255u], 1u);
+    for (int i = 0; i < SORT_ITEMS; i++) {
+        const uint32_t j = sb.e0 + (uint32_t)i * SORT_THREADS + tid;
+        const uint32_t d = j < sb.e1 ? (b.keys[j] - sb.fb_base) >> sb.shift : 256u;
+        const uint32_t left = __shfl_up(d, 1, 64);  // by every lane
+        const bool head = lane == 0 || left != d;
+        const uint64_t heads = __ballot(head), above = lane == 63 ? 0ull : heads >> (lane + 1);
+        const uint32_t run = above ? 1u + (uint32_t)__builtin_ctzll(above) : 64u - lane;
+        if (head && d < 256) atomicAdd(&h[d], run);
     }
     __syncthreads();
-    hist[rb.hbase + threadIdx.x * rb.nbk + rb.lb] = h[threadIdx.x];
+    hist[sb.hbase + tid * sb.nbk + sb.lb] = h[tid];
 }
 
-// Scatter of one 8-bit digit pass.  The block's 4096 items are first ranked stably by digit
-// into LDS, then written out in digit order: runs of equal digits land at consecutive global
-// positions, so stores coalesce instead of scattering one item per digit per row.  Each wave
-// ranks its own contiguous 1024 items (16 rows of 64) with wave-local digit counters: a ballot
-// multisplit gives an item's rank among equal digits of its row, the counter the items of
-// earlier rows; only then are the waves' counts combined per digit.  offs is the exclusive
-// scan of the [digit][block] histogram: the block's count of digit d is the difference of
-// its entry and the next one.  With no vals, an item's value is its input index.
-constexpr int RS_WAVE_ITEMS = RS_ITEMS * 64;
+// Lanes of a wave's row holding the same digit (multisplit by ballots), among `valid` ones.
+template <int BITS>
+__device__ __forceinline__ uint64_t digit_peers(uint32_t d, bool valid) {
+    uint64_t peers = __ballot(valid);
+#pragma unroll
+    for (int bit = 0; bit < BITS; bit++) {
+        const uint64_t m = __ballot((d >> bit) & 1u);
+        peers &= ((d >> bit) & 1u) ? m : ~m;
+    }
+    return peers;
+}
 
-__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(BatchDev b, const uint32_t *keys, const uint32_t *vals,
-                                                           uint32_t *keys_out, uint32_t *vals_out,
-                                                           const uint32_t *seg_e, const uint32_t *seg_b, int shift,
-                                                           const uint32_t *offs) {
-    __shared__ uint32_t skey[RS_TILE], sval[RS_TILE];
-    __shared__ uint32_t lstart[256];  // local start of each digit
-    __shared__ uint32_t goff[256];    // global start of each digit's run from this block
-    __shared__ uint32_t wcnt[RS_THREADS / 64][256];  // per wave: digit counts, then the wave's base per digit
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    RsBlock rb;
-    if (!rs_block(b, seg_e, seg_b, rb)) return;  // uniform over the block
-    const uint32_t base = rb.e0;
-    const uint32_t valid_n = rb.e1 - rb.e0;
+// Distribution over the buckets.  The block's entries are ranked stably by bucket: each wave ranks its
+// own contiguous 1024 (16 rows of 64) with wave-local counters, a ballot multisplit giving an entry's
+// rank among equal buckets of its row, the counter those of earlier rows; then the waves' counts are
+// combined.  Entries come path by path, row-major, and a bucket is a stretch of tiles: neighbouring
+// lanes mostly store to neighbouring places, so they store straight from registers (4096^2 scene 26 ->
+// 20 us against stores in bucket order through LDS; the 48-scene batch, half of whose canvases have
+// buckets of a few tiles, 119 -> 128 of 2900).  offs: the scanned histogram.
+__global__ __launch_bounds__(SORT_THREADS) void k_sort_scatter(BatchDev b, SortArrays in, SortArrays out,
+                                                               const uint32_t *seg_e, const uint32_t *seg_b,
+                                                               const uint32_t *offs) {
+    constexpr uint32_t WAVE_ITEMS = SORT_ITEMS * 64;
+    __shared__ uint32_t wcnt[SORT_THREADS / 64][256];  // per wave and bucket: counts, then where its first entry goes
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (blockIdx.x >= seg_b[b.n_scenes]) return;  // uniform
+    SortBlock sb;
     {
-        const uint32_t h = rb.hbase + threadIdx.x * rb.nbk + rb.lb;
-        const uint32_t o = offs[h];
-        goff[threadIdx.x] = o;
-        uint32_t total;
-        lstart[threadIdx.x] = block_exclusive_scan<uint32_t>(offs[h + 1] - o, total);
+        const int k = find_scene_wave(seg_b, b.n_scenes, blockIdx.x);
+        sort_block(b, seg_e, seg_b, k, seg_e[k], seg_e[k + 1], seg_b[k], seg_b[k + 1], sb);
     }
-    for (int q = threadIdx.x; q < (RS_THREADS / 64) * 256; q += RS_THREADS) (&wcnt[0][0])[q] = 0;
+    const uint32_t base = sb.e0, n = sb.e1 - sb.e0;
+    const uint32_t place = offs[sb.hbase + tid * sb.nbk + sb.lb];  // of this block's first entry of bucket tid
+    for (uint32_t q = tid; q < (SORT_THREADS / 64) * 256; q += SORT_THREADS) (&wcnt[0][0])[q] = 0;
     __syncthreads();
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     uint32_t *cnt = wcnt[wave];
-    uint32_t key[RS_ITEMS], val[RS_ITEMS], rank[RS_ITEMS];
-    const uint32_t w0 = (uint32_t)wave * RS_WAVE_ITEMS;
+    uint32_t key[SORT_ITEMS], rank[SORT_ITEMS];
+    uint2 rec[SORT_ITEMS];
+    const uint32_t w0 = wave * WAVE_ITEMS;
 #pragma unroll
-    for (int r = 0; r < RS_ITEMS; r++) {
-        const uint32_t li = w0 + (uint32_t)r * 64 + (uint32_t)lane;
-        const bool valid = li < valid_n;
-        key[r] = valid ? keys[base + li] : 0u;
-        val[r] = !valid ? 0u : (vals ? vals[base + li] : (uint32_t)(base + li));
+    for (int r = 0; r < SORT_ITEMS; r++) {
+        const uint32_t li = w0 + (uint32_t)r * 64 + lane;
+        key[r] = li < n ? in.keys[base + li] : sb.fb_base;
+        if (li < n) rec[r] = in.rec[base + li];
     }
 #pragma unroll
-    for (int r = 0; r < RS_ITEMS; r++) {
-        const uint32_t li = w0 + (uint32_t)r * 64 + (uint32_t)lane;
-        const bool valid = li < valid_n;
-        const uint32_t d = ((key[r] - rb.fb_base) >> shift) & 255u;
-        // lanes of this row holding the same digit (multisplit peer mask)
-        uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int bit = 0; bit < 8; bit++) {
-            const uint64_t m = __ballot((d >> bit) & 1u);
-            peers &= ((d >> bit) & 1u) ? m : ~m;
-        }
-        const uint32_t rk = __popcll(peers & lt_mask);
-        const uint32_t before = valid ? cnt[d] : 0u;  // items of digit d in earlier rows of this wave
+    for (int r = 0; r < SORT_ITEMS; r++) {
+        const bool valid = w0 + (uint32_t)r * 64 + lane < n;
+        const uint32_t d = (key[r] - sb.fb_base) >> sb.shift;
+        const uint64_t peers = digit_peers<8>(d, valid);
+        const uint32_t rk = (uint32_t)__popcll(peers & lt_mask);
+        const uint32_t before = valid ? cnt[d] : 0u;  // entries of bucket d in earlier rows of this wave
         rank[r] = before + rk;
-        // the last lane of each digit group advances the counter (after every lane's read: a
-        // wave's LDS operations complete in order)
+        // the last lane of each group advances the counter (after every lane's read: a wave's LDS
+        // operations complete in order)
         if (valid && rk == (uint32_t)__popcll(peers) - 1u) cnt[d] = before + rk + 1u;
     }
     __syncthreads();
-    {  // per digit: the counts of earlier waves
-        const uint32_t d = threadIdx.x;
-        uint32_t acc = 0;
+    {  // per bucket: after the entries of earlier waves
+        uint32_t acc = place;
 #pragma unroll
-        for (int w = 0; w < RS_THREADS / 64; w++) {
-            const uint32_t c = wcnt[w][d];
-            wcnt[w][d] = acc;
+        for (int w = 0; w < SORT_THREADS / 64; w++) {
+            const uint32_t c = wcnt[w][tid];
+            wcnt[w][tid] = acc;
             acc += c;
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < RS_ITEMS; r++) {
-        const uint32_t li = w0 + (uint32_t)r * 64 + (uint32_t)lane;
-        if (li < valid_n) {
-            const uint32_t d = ((key[r] - rb.fb_base) >> shift) & 255u;
-            const uint32_t pos = lstart[d] + cnt[d] + rank[r];
-            skey[pos] = key[r];
-            sval[pos] = val[r];
+    for (int r = 0; r < SORT_ITEMS; r++) {
+        const uint32_t li = w0 + (uint32_t)r * 64 + lane;
+        if (li < n) {
+            const uint32_t g = cnt[(key[r] - sb.fb_base) >> sb.shift] + rank[r];
+            out.keys[g] = key[r];
+            out.rec[g] = rec[r];
+            if (in.meta) out.meta[g] = in.meta[base + li];
         }
     }
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < valid_n; i += RS_THREADS) {
-        const uint32_t key = skey[i];
-        const uint32_t d = ((key - rb.fb_base) >> shift) & 255u;
-        const uint32_t g = goff[d] + (i - lstart[d]);
-        keys_out[g] = key;
-        vals_out[g] = sval[i];
+}
+
+// A block per bucket (SCENE: per scene, straight from the entry pass): its entries [s0, s1) of `a`
+// grouped by tile, stably, and its tiles' ranges.  A digit of 8 bits per pass from the lowest, `passes`
+// of them (the same for the whole batch), from a to c and back in turn: a histogram of the bucket
+// (where it is more than one chunk), then its entries a chunk at a time, ranked as in the
+// distribution and moved through LDS, so that a tile's entries of the chunk are stored together (an
+// entry's neighbours belong to other tiles: stored from registers each went to a line of its own).  One
+// pass covers 256 tiles, of which a bucket of a canvas up to 4096^2 holds no more: the ranges are the
+// digits'.  Above that they are marked at the runs of the sorted keys.
+template <int THREADS, bool SCENE>
+__global__ __launch_bounds__(THREADS) void k_sort_buckets(BatchDev b, SortArrays a, SortArrays c, const uint32_t *seg_b,
+                                                          const uint32_t *offs, uint32_t passes) {
+    constexpr int WAVES = THREADS / 64, ITEMS = 8;
+    constexpr uint32_t CHUNK = THREADS * ITEMS;
+    __shared__ uint32_t hist[256], next[256];   // counts; where the next entry of a digit goes
+    __shared__ uint32_t goff[256];              // chunk: that, less the digit's first place in the chunk
+    __shared__ uint32_t wcnt[WAVES][256];       // per wave and digit: counts, then places in the chunk
+    __shared__ uint2 srec[CHUNK];
+    __shared__ uint8_t sdig[CHUNK];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t k = SCENE ? blockIdx.x : blockIdx.x >> 8;
+    const SceneDev &sc = b.scenes[k];
+    const uint32_t n_fb = sc.n_fb, shift = SCENE ? 8u : sort_shift(n_fb);
+    const uint32_t bucket = SCENE ? 0u : blockIdx.x & 255u;
+    const uint64_t tile0 = (uint64_t)bucket << shift;
+    if (tile0 >= n_fb) return;  // uniform over the block
+    const uint32_t tiles = (uint32_t)min((uint64_t)n_fb - tile0, 1ull << shift);
+    const uint32_t first = sc.fb_base + (uint32_t)tile0;  // the bucket's first batch tile
+    uint32_t s0, s1;
+    if (SCENE) {
+        const uint32_t total = min(b.counters[C_ENTRIES], b.cap_entries);
+        s0 = min(b.path_ent[sc.path_base].x, total);
+        s1 = (int)k + 1 < b.n_scenes ? min(b.path_ent[b.scenes[k + 1].path_base].x, total) : total;
+    } else {
+        const uint32_t nbk = seg_b[k + 1] - seg_b[k], h = 256u * seg_b[k] + bucket * nbk;
+        s0 = offs[h];
+        s1 = offs[h + nbk];
+    }
+    if (s0 == s1) {  // uniform
+        for (uint32_t t = tid; t < tiles; t += THREADS) b.fb_range[first + t] = make_uint2(s0, s0);
+        return;
+    }
+    const bool one = s1 - s0 <= CHUNK;
+    const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    for (uint32_t p = 0; p < passes; p++) {
+        const SortArrays &in = (p & 1u) ? c : a, &out = (p & 1u) ? a : c;
+        const bool ranges = passes == 1;
+        uint32_t total;
+        if (!one) {
+            if (tid < 256) hist[tid] = 0;
+            __syncthreads();
+            for (uint32_t j = s0 + tid; j < s1; j += THREADS) atomicAdd(&hist[((in.keys[j] - first) >> (8 * p)) & 255u], 1u);
+            __syncthreads();
+            const uint32_t n = tid < 256 ? hist[tid] : 0u;
+            const uint32_t start = s0 + block_exclusive_scan<uint32_t, THREADS>(n, total);
+            if (tid < 256) next[tid] = start;
+            if (ranges && tid < tiles) b.fb_range[first + tid] = make_uint2(start, start + n);
+        }
+        for (uint32_t at = s0; at < s1; at += CHUNK) {  // uniform over the block
+            for (uint32_t q = tid; q < WAVES * 256; q += THREADS) (&wcnt[0][0])[q] = 0;
+            __syncthreads();
+            uint32_t *cnt = wcnt[wave];
+            uint32_t key[ITEMS], rank[ITEMS];
+            uint2 rec[ITEMS];
+            const uint32_t w0 = at + wave * (64 * ITEMS);
+#pragma unroll
+            for (int r = 0; r < ITEMS; r++) {
+                const uint32_t j = w0 + (uint32_t)r * 64 + lane;
+                key[r] = j < s1 ? in.keys[j] : first;
+                if (j < s1) rec[r] = in.rec[j];
+            }
+#pragma unroll
+            for (int r = 0; r < ITEMS; r++) {
+                if (w0 + (uint32_t)r * 64 >= s1) break;  // wave-uniform
+                const bool valid = w0 + (uint32_t)r * 64 + lane < s1;
+                const uint32_t d = ((key[r] - first) >> (8 * p)) & 255u;
+                const uint64_t peers = digit_peers<8>(d, valid);
+                const uint32_t rk = (uint32_t)__popcll(peers & lt_mask);
+                const uint32_t before = valid ? cnt[d] : 0u;
+                rank[r] = before + rk;
+                if (valid && rk == (uint32_t)__popcll(peers) - 1u) cnt[d] = before + rk + 1u;
+            }
+            __syncthreads();
+            uint32_t n = 0;  // the chunk's entries of digit tid
+            if (tid < 256) {
+#pragma unroll
+                for (int w = 0; w < WAVES; w++) {
+                    const uint32_t m = wcnt[w][tid];
+                    wcnt[w][tid] = n;
+                    n += m;
+                }
+            }
+            const uint32_t local = block_exclusive_scan<uint32_t, THREADS>(n, total);
+            if (tid < 256) {
+#pragma unroll
+                for (int w = 0; w < WAVES; w++) wcnt[w][tid] += local;
+                const uint32_t to = one ? s0 + local : next[tid];
+                goff[tid] = to - local;
+                next[tid] = to + n;
+                if (one && ranges && tid < tiles) b.fb_range[first + tid] = make_uint2(to, to + n);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < ITEMS; r++) {
+                const uint32_t j = w0 + (uint32_t)r * 64 + lane;
+                if (j < s1) {
+                    const uint32_t d = ((key[r] - first) >> (8 * p)) & 255u, i = cnt[d] + rank[r];
+                    srec[i] = rec[r];
+                    sdig[i] = (uint8_t)d;
+                    if (!ranges) out.keys[goff[d] + i] = key[r];
+                    if (in.meta) out.meta[goff[d] + i] = in.meta[j];
+                }
+            }
+            __syncthreads();
+            for (uint32_t i = tid; i < min(CHUNK, s1 - at); i += THREADS) out.rec[goff[sdig[i]] + i] = srec[i];
+            __syncthreads();  // the next chunk, or pass, reads and rewrites
+        }
+    }
+    if (passes > 1) {
+        const uint32_t *keys = (passes & 1u) ? c.keys : a.keys;
+        for (uint32_t t = tid; t < tiles; t += THREADS) b.fb_range[first + t] = make_uint2(s0, s0);
+        __syncthreads();
+        for (uint32_t j = s0 + tid; j < s1; j += THREADS) {
+            const uint32_t key = keys[j];
+            if (j == s0 || keys[j - 1] != key) b.fb_range[key].x = j;
+            if (j + 1 == s1 || keys[j + 1] != key) b.fb_range[key].y = j + 1;
+        }
     }
 }
 
@@ -2035,88 +2197,48 @@ hipError_t launch_entries(const BatchDev &b, bool write, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Range [start, end) of every framebuffer tile's run in the sorted keys, marked at the run
-// boundaries: item i starts its key's run when the key before differs and ends it when the
-// key after differs.  Tiles with no entries keep the cleared (0, 0).
-constexpr int FB_BOUNDS_ITEMS = 4;  // items per thread per step, all loads issued first
+// Blocks of the sort's distribution for a capacity of `cap` entries over `n_scenes` scenes (one partial
+// block each).
+static uint32_t sort_max_blocks(uint64_t cap, uint32_t n_scenes) { return blocks_for(cap, SORT_TILE) + n_scenes + 1; }
 
-__global__ __launch_bounds__(256) void k_fb_bounds(const uint32_t *keys, const uint32_t *n_ptr, uint32_t cap,
-                                                   uint32_t n_fb, uint2 *range) {
-    const uint32_t n = min(*n_ptr, cap);
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += FB_BOUNDS_ITEMS * stride) {
-        uint32_t prev[FB_BOUNDS_ITEMS], key[FB_BOUNDS_ITEMS], next[FB_BOUNDS_ITEMS];
-#pragma unroll
-        for (int j = 0; j < FB_BOUNDS_ITEMS; j++) {
-            const uint64_t i = i0 + j * stride;
-            key[j] = n_fb;  // marks nothing
-            prev[j] = next[j] = n_fb + 1;
-            if (i < n) {
-                key[j] = keys[i];
-                if (i > 0) prev[j] = keys[i - 1];
-                if (i + 1 < n) next[j] = keys[i + 1];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < FB_BOUNDS_ITEMS; j++) {
-            const uint64_t i = i0 + j * stride;
-            if (key[j] >= n_fb) continue;  // past the count (keys of the entry pass are below n_fb)
-            if (prev[j] != key[j]) range[key[j]].x = (uint32_t)i;
-            if (next[j] != key[j]) range[key[j]].y = (uint32_t)(i + 1);
-        }
-    }
+// max_fb, max_tiles: the largest scene's framebuffer tiles and path tiles (a bound of its entries).
+static bool sort_small(uint32_t max_fb, uint64_t max_tiles) { return max_fb <= 256 && max_tiles <= SORT_SMALL; }
+
+size_t sort_temp_elems(uint64_t cap, uint32_t n_scenes, uint32_t max_fb, uint64_t max_tiles) {
+    return sort_small(max_fb, max_tiles) ? 0 : 2ull * (n_scenes + 1) + 256ull * sort_max_blocks(cap, n_scenes) + 1;
 }
 
-hipError_t launch_fb_bounds(const uint32_t *sorted_keys, const uint32_t *n_ptr, uint32_t cap, uint32_t n_fb,
-                            uint2 *range, hipStream_t s) {
-    // the count is known on the device only: a grid for the capacity, strided
-    const uint32_t nb = std::min<uint32_t>(blocks_for(cap, 256 * FB_BOUNDS_ITEMS), 16384);
-    if (nb == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fb_bounds, dim3(nb), dim3(256), 0, s, sorted_keys, n_ptr, cap, n_fb, range);
-    return hipGetLastError();
+// 64-bit state words of the sort's scan.
+uint64_t sort_state_words(uint64_t cap, uint32_t n_scenes, uint32_t max_fb, uint64_t max_tiles) {
+    return sort_small(max_fb, max_tiles) ? 0 : scan_state_words(256ull * sort_max_blocks(cap, n_scenes), 1);
 }
 
-// Sort blocks for a capacity of `cap` entries over `n_scenes` scenes (one partial block each).
-static uint32_t rs_max_blocks(uint64_t cap, uint32_t n_scenes) { return blocks_for(cap, RS_TILE) + n_scenes + 1; }
-
-size_t radix_temp_elems(uint64_t cap, uint32_t n_scenes) {
-    const uint64_t nh = 256ull * rs_max_blocks(cap, n_scenes);
-    return 2ull * (n_scenes + 1) + nh + 1;
-}
-
-// 64-bit state words of the sort's scans (one per digit).
-uint64_t radix_state_words(uint64_t cap, uint32_t n_scenes, int bits) {
-    return (uint64_t)((bits + 7) / 8) * scan_state_words(256ull * rs_max_blocks(cap, n_scenes), 1);
-}
-
-// Sorts the batch's entry keys (b.keys[0 .. entries)), with values starting as the item
-// indices (vals is not read), scene by scene by the low `bits` bits of the scene-local
-// framebuffer tile, stably; returns the buffer pair holding the result via *result_alt
-// (false: keys/vals, true: keys_alt/vals_alt).
-hipError_t radix_sort(const BatchDev &b, uint32_t *keys, uint32_t *vals, uint32_t *keys_alt, uint32_t *vals_alt,
-                      int bits, uint32_t *tmp, bool *result_alt, hipStream_t s) {
+// Sorts the batch's entries; *sorted_alt: their records are in b.rec_alt (else b.entry_rec).
+hipError_t sort_entries(const BatchDev &b, uint32_t max_fb, uint64_t max_tiles, uint32_t *tmp, bool *sorted_alt,
+                        hipStream_t s) {
     const uint32_t n_sc = (uint32_t)b.n_scenes;
-    const uint32_t nb = rs_max_blocks(b.cap_entries, n_sc);
-    const uint32_t nh = 256 * nb;
-    uint32_t *seg_e = tmp, *seg_b = tmp + (n_sc + 1);
-    uint32_t *hist = tmp + 2 * (n_sc + 1);
-    unsigned long long *state = b.st_sort;
-    hipLaunchKernelGGL(k_rs_segments, dim3(1), dim3(RS_THREADS), 0, s, b, seg_e, seg_b);
-    bool alt = false;
-    for (int shift = 0; shift < bits; shift += 8) {
-        const uint32_t *ki = alt ? keys_alt : keys;
-        const uint32_t *vi = shift == 0 ? nullptr : (alt ? vals_alt : vals);  // values start as the indices
-        uint32_t *ko = alt ? keys : keys_alt;
-        uint32_t *vo = alt ? vals : vals_alt;
-        hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(RS_THREADS), 0, s, b, ki, seg_e, seg_b, shift, hist);
-        // the scan covers the capacity's blocks; entries past this launch's blocks are never read
-        hipError_t e = scan_u32(hist, hist, nh, state, s);
-        if (e != hipSuccess) return e;
-        state += scan_state_words(nh, 1);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(RS_THREADS), 0, s, b, ki, vi, ko, vo, seg_e, seg_b, shift, hist);
-        alt = !alt;
+    const SortArrays x{b.keys, b.entry_rec, b.dump ? b.entry_meta : nullptr};
+    const SortArrays y{b.keys_alt, b.rec_alt, b.dump ? b.meta_alt : nullptr};
+    if (sort_small(max_fb, max_tiles)) {
+        *sorted_alt = true;
+        hipLaunchKernelGGL((k_sort_buckets<256, true>), dim3(n_sc), dim3(256), 0, s, b, x, y, nullptr, nullptr, 1u);
+        return hipGetLastError();
     }
-    *result_alt = alt;
+    const uint32_t nb = sort_max_blocks(b.cap_entries, n_sc), nh = 256 * nb;
+    uint32_t *seg_e = tmp, *seg_b = tmp + (n_sc + 1), *hist = tmp + 2 * (n_sc + 1);
+    hipLaunchKernelGGL(k_sort_hist, dim3(nb), dim3(SORT_THREADS), 0, s, b, seg_e, seg_b, hist);
+    // the scan covers the capacity's blocks; entries past this launch's blocks are never read
+    hipError_t e = scan_u32(hist, hist, nh, b.st_sort, s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_sort_scatter, dim3(nb), dim3(SORT_THREADS), 0, s, b, x, y, seg_e, seg_b, hist);
+    uint32_t bits = 0;
+    while ((1ull << bits) < max_fb) bits++;
+    const uint32_t passes = bits > 16 ? (bits - 1) / 8 : 1;  // digits below a bucket's
+    *sorted_alt = passes % 2 == 0;
+    if (max_tiles / 256 >= SORT_WIDE && n_sc <= SORT_WIDE_SCENES)
+        hipLaunchKernelGGL((k_sort_buckets<1024, false>), dim3(256 * n_sc), dim3(1024), 0, s, b, y, x, seg_b, hist, passes);
+    else
+        hipLaunchKernelGGL((k_sort_buckets<256, false>), dim3(256 * n_sc), dim3(256), 0, s, b, y, x, seg_b, hist, passes);
     return hipGetLastError();
 }
 

@@ -487,7 +487,7 @@ __device__ float3 composite_rgb(float3 d, float3 s, uint32_t op) {
 // tile.frag's composite (:585-598): rgb = a (1 - da) src + a da B(dest, src) + (1 - a) dest,
 // alpha 1.  dest starts from the target (PFH_LOAD_DST) or transparent; premultiplied, in [0, 1].
 // Stores the lane's 4 pixels.
-__device__ void composite_back_to_front(const BatchDev &b, const SceneDev &sc, const uint32_t *sorted_vals, uint32_t e0,
+__device__ void composite_back_to_front(const BatchDev &b, const SceneDev &sc, const uint2 *recs, uint32_t e0,
                                         uint32_t e1, int x, int y0, uint32_t lane_off, uint8_t *cptr, int64_t pitch,
                                         int height, bool load_dst) {
     float dr[4], dg[4], db[4], da[4];
@@ -501,7 +501,7 @@ __device__ void composite_back_to_front(const BatchDev &b, const SceneDev &sc, c
         da[q] = (float)(px >> 24) * (1.0f / 255.0f);
     }
     for (uint32_t i = e0; i < e1; i++) {  // uniform over the wave
-        const uint2 rec = b.entry_rec[sorted_vals[i]];
+        const uint2 rec = recs[i];
         uint32_t colour = rec.y, op = 0, row = b.cap_alpha;  // row cap_alpha: full coverage
         bool empty = false;
         const PaintRec *pr = nullptr;
@@ -554,7 +554,7 @@ __device__ void composite_back_to_front(const BatchDev &b, const SceneDev &sc, c
 
 // PAINTS: some scene of the batch has paint records (the solid-only variant carries no code for them).
 template <bool PAINTS>
-__global__ __launch_bounds__(256) void k_composite(BatchDev b, const uint32_t *sorted_vals) {
+__global__ __launch_bounds__(256) void k_composite(BatchDev b, const uint2 *recs) {
     __shared__ float4 s_colour[4][64];  // per wave of the block: the chunk's premultiplied colours
     const int lane = threadIdx.x & 63;
     const uint32_t lb = (b.xcd_order & 2u) ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
@@ -594,14 +594,14 @@ __global__ __launch_bounds__(256) void k_composite(BatchDev b, const uint32_t *s
             const uint32_t i = c0 + lane;
             bool op = false;
             if (i < e1) {
-                const uint2 rec = b.entry_rec[sorted_vals[i]];
+                const uint2 rec = recs[i];
                 op = rec.x != NO_ALPHA && (rec.x & ENTRY_GRADIENT) && sc.paints[rec.y].op != 0;
             }
             ops = __ballot(op) != 0;
         }
         if (ops) {
             if (x < 0 || x >= width) return;
-            composite_back_to_front(b, sc, sorted_vals, e0, e1, x, y0, lane_off, out + (int64_t)y0 * pitch + (int64_t)x * 4,
+            composite_back_to_front(b, sc, recs, e0, e1, x, y0, lane_off, out + (int64_t)y0 * pitch + (int64_t)x * 4,
                                     pitch, height, load_dst);
             return;
         }
@@ -643,7 +643,7 @@ __global__ __launch_bounds__(256) void k_composite(BatchDev b, const uint32_t *s
         uint32_t ai = b.cap_alpha, c = 0;
         bool masked = false, grad = false;
         if (i < e1) {
-            const uint2 rec = b.entry_rec[sorted_vals[i]];
+            const uint2 rec = recs[i];
             c = rec.y;
             if (rec.x != NO_ALPHA) {
                 masked = true;  // a gradient entry never joins a solid run, with or without a mask row
@@ -998,13 +998,13 @@ hipError_t launch_fill_clipped(const BatchDev &b, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_composite(const BatchDev &b, const uint32_t *sorted_vals, uint32_t block, hipStream_t s) {
+hipError_t launch_composite(const BatchDev &b, const uint2 *recs, uint32_t block, hipStream_t s) {
     if (b.n_fb == 0) return hipSuccess;
     if (block != 64 && block != 128 && block != 256) return hipErrorInvalidValue;
     if (b.paints)
-        hipLaunchKernelGGL(k_composite<true>, dim3(blocks_for(b.n_fb, block / 64)), dim3(block), 0, s, b, sorted_vals);
+        hipLaunchKernelGGL(k_composite<true>, dim3(blocks_for(b.n_fb, block / 64)), dim3(block), 0, s, b, recs);
     else
-        hipLaunchKernelGGL(k_composite<false>, dim3(blocks_for(b.n_fb, block / 64)), dim3(block), 0, s, b, sorted_vals);
+        hipLaunchKernelGGL(k_composite<false>, dim3(blocks_for(b.n_fb, block / 64)), dim3(block), 0, s, b, recs);
     return hipGetLastError();
 }
 

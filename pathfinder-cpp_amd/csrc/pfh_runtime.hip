@@ -33,15 +33,13 @@ hipError_t launch_bin(const BatchDev &b, bool emit, hipStream_t s);
 hipError_t launch_propagate(const BatchDev &b, uint32_t block, uint32_t rows, hipStream_t s);
 hipError_t launch_entries(const BatchDev &b, bool write, hipStream_t s);
 hipError_t launch_bin_items(const BatchDev &b, hipStream_t s);
-hipError_t launch_fb_bounds(const uint32_t *sorted_keys, const uint32_t *n_ptr, uint32_t cap, uint32_t n_fb,
-                            uint2 *range, hipStream_t s);
-size_t radix_temp_elems(uint64_t cap, uint32_t n_scenes);
-uint64_t radix_state_words(uint64_t cap, uint32_t n_scenes, int bits);
-hipError_t radix_sort(const BatchDev &b, uint32_t *keys, uint32_t *vals, uint32_t *keys_alt, uint32_t *vals_alt,
-                      int bits, uint32_t *tmp, bool *result_alt, hipStream_t s);
+size_t sort_temp_elems(uint64_t cap, uint32_t n_scenes, uint32_t max_fb, uint64_t max_tiles);
+uint64_t sort_state_words(uint64_t cap, uint32_t n_scenes, uint32_t max_fb, uint64_t max_tiles);
+hipError_t sort_entries(const BatchDev &b, uint32_t max_fb, uint64_t max_tiles, uint32_t *tmp, bool *sorted_alt,
+                        hipStream_t s);
 hipError_t launch_fill_masks(const BatchDev &b, uint32_t grid_alpha, uint32_t max_blocks, hipStream_t s);
 hipError_t launch_fill_clipped(const BatchDev &b, hipStream_t s);
-hipError_t launch_composite(const BatchDev &b, const uint32_t *sorted_vals, uint32_t block, hipStream_t s);
+hipError_t launch_composite(const BatchDev &b, const uint2 *recs, uint32_t block, hipStream_t s);
 hipError_t launch_clear_outside(const BatchDev &b, uint32_t max_rows, hipStream_t s);
 hipError_t mlp_forward(const float *params, const float *x, int64_t n, float *hidden, float *out, hipStream_t s);
 hipError_t mlp_backward(const float *params, const float *x, int64_t n, const float *hidden, const float *out,
@@ -357,6 +355,7 @@ struct Server;
 // the workspace's events (Workspace::kev), which outlive every executable graph.
 struct CapturedGraph {
     hipGraphExec_t exec = nullptr;
+    bool sorted_alt = false;  // Workspace::last_sorted_alt of its launches
 };
 
 // Device working set of one launch: work buffers, stream, events and captured graphs.
@@ -369,14 +368,14 @@ struct Workspace {
     // inside captured graphs, so replays time those kernels too
     hipEvent_t kev[3] = {nullptr, nullptr, nullptr};
     DevBuf scene_table, bases, tile_delta, tile_cnt, tile_fill_off, tile_alpha_idx, tile_bd, tile_st, path_ent, ent_quarter, path_tot, bin_items, col_item, col_bd, tall_cols, seg_mask,
-        seg_cnt, lines, line_cnt, fills, dump_fills, alpha_rec, alpha_vis, masks, zbuf, fb_range, keys, vals, keys_alt,
-        vals_alt, entry_rec, entry_meta, counters, chunk_off, scan_state, dump_state, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen;
+        seg_cnt, lines, line_cnt, fills, dump_fills, alpha_rec, alpha_vis, masks, zbuf, fb_range, keys, keys_alt,
+        rec_alt, entry_rec, entry_meta, meta_alt, counters, chunk_off, scan_state, dump_state, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen;
     uint32_t *h_counters = nullptr;  // pinned
     SceneDev *h_table = nullptr;     // pinned scene table
     size_t h_table_cap = 0;
     uint32_t *h_bases = nullptr;
     size_t h_bases_cap = 0;
-    bool last_sorted_alt = false;
+    bool last_sorted_alt = false;  // the sorted entries are in rec_alt (meta_alt), not entry_rec
     std::map<GraphKey, CapturedGraph> graphs;
     uint64_t graphs_generation = 0;  // g_alloc_generation the cached graphs were captured under
     hipEvent_t stage_ev[9] = {};     // plain mode: between its stages
@@ -446,7 +445,7 @@ struct Workspace {
     std::vector<DevBuf *> all_buffers() {
         return {&scene_table, &bases, &tile_delta, &tile_cnt, &tile_fill_off, &tile_alpha_idx, &tile_bd, &tile_st,
                 &path_ent, &ent_quarter, &path_tot, &bin_items, &col_item, &col_bd, &tall_cols, &seg_mask, &seg_cnt, &lines, &line_cnt, &fills, &dump_fills, &alpha_rec, &alpha_vis,
-                &masks, &zbuf, &fb_range, &keys, &vals, &keys_alt, &vals_alt, &entry_rec, &entry_meta, &counters, &chunk_off, &scan_state, &dump_state,
+                &masks, &zbuf, &fb_range, &keys, &keys_alt, &rec_alt, &entry_rec, &entry_meta, &meta_alt, &counters, &chunk_off, &scan_state, &dump_state,
                 &sort_tmp, &tile_clip_ai, &clip_jobs, &clip_rec, &clip_seen};
     }
     size_t device_bytes() {
@@ -1553,7 +1552,8 @@ struct Plan {
     uint32_t max_rows = 0;       // tile rows of the tallest target
     uint32_t clip_levels = 0;  // deepest clip nesting level of the batch
     uint32_t cap_f = 0, cap_a = 0, cap_e = 0, cap_l = 0;
-    int key_bits = 1;
+    uint32_t max_fb = 1;         // the largest scene's framebuffer tiles and path tiles
+    uint64_t max_tiles = 0;
     Schedule sched;
 };
 
@@ -1580,7 +1580,7 @@ static ScanStates scan_states(const Plan &pl) {
     st.paths = scan_state_words((pl.S + chunk - 1) / chunk, 1);
     st.entries = st.paths + scan_state_words(pl.P, 2);
     st.sort = st.entries + scan_state_words(pl.P, 2);
-    st.total = st.sort + radix_state_words(pl.cap_e, (uint32_t)pl.ids.size(), pl.key_bits);
+    st.total = st.sort + sort_state_words(pl.cap_e, (uint32_t)pl.ids.size(), pl.max_fb, pl.max_tiles);
     return st;
 }
 
@@ -1592,10 +1592,9 @@ static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
     w.tile_fill_off.ensure(4 * pl.T + 8);
     w.tile_alpha_idx.ensure(4 * pl.T + 8);
     w.keys.ensure(4ull * pl.cap_e);
-    w.vals.ensure(4ull * pl.cap_e);
     w.keys_alt.ensure(4ull * pl.cap_e);
-    w.vals_alt.ensure(4ull * pl.cap_e);
     w.entry_rec.ensure(8ull * pl.cap_e);
+    w.rec_alt.ensure(8ull * pl.cap_e);
     if (dump || pl.clips) w.tile_bd.ensure(pl.T + 4);
     if (pl.clips) {
         w.tile_clip_ai.ensure(4 * pl.T + 4);
@@ -1627,8 +1626,11 @@ static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
     w.alpha_rec.ensure(16ull * pl.cap_a);
     w.alpha_vis.ensure(4ull * (pl.clips ? std::max(pl.cap_a, pl.cap_e) : pl.cap_a));
     w.masks.ensure(256ull * pl.cap_a + 256);  // + the all-ones row
-    if (dump) w.entry_meta.ensure(8ull * pl.cap_e);
-    w.sort_tmp.ensure(4 * radix_temp_elems(pl.cap_e, (uint32_t)pl.ids.size()) + 64);
+    if (dump) {
+        w.entry_meta.ensure(8ull * pl.cap_e);
+        w.meta_alt.ensure(8ull * pl.cap_e);
+    }
+    w.sort_tmp.ensure(4 * sort_temp_elems(pl.cap_e, (uint32_t)pl.ids.size(), pl.max_fb, pl.max_tiles) + 64);
 }
 
 // Capacities the current allocations hold, by the same per-buffer sizes ensure_sizes asks
@@ -1760,10 +1762,10 @@ static void write_tables(pfh_ctx *ctx, Plan &pl, bool load_dst) {
     pl.FB = FB;
     pl.P = P;
     // the sort runs per scene on scene-local framebuffer tiles
-    uint64_t max_fb = 1;
-    for (size_t k = 0; k < n; k++) max_fb = std::max<uint64_t>(max_fb, ctx->w->h_table[k].n_fb);
-    pl.key_bits = 1;
-    while ((1ull << pl.key_bits) < max_fb) pl.key_bits++;
+    for (size_t k = 0; k < n; k++) {
+        pl.max_fb = std::max(pl.max_fb, ctx->w->h_table[k].n_fb);
+        pl.max_tiles = std::max<uint64_t>(pl.max_tiles, ctx->w->h_table[k].n_tiles);
+    }
 }
 
 static void upload_tables(Workspace &w, const Plan &pl) {
@@ -1782,8 +1784,8 @@ static void upload_tables(Workspace &w, const Plan &pl) {
 static unsigned long long *curve_bits(Workspace &w, const Plan &pl) {
     if (!w.arena.base) return w.seg_mask.as<unsigned long long>();
     uint8_t *const at = w.tile_delta.as<uint8_t>(), *end = at;
-    for (const DevBuf *d : {&w.tile_delta, &w.tile_cnt, &w.tile_fill_off, &w.tile_alpha_idx, &w.keys, &w.vals, &w.keys_alt,
-                            &w.vals_alt, &w.entry_rec}) {
+    for (const DevBuf *d : {&w.tile_delta, &w.tile_cnt, &w.tile_fill_off, &w.tile_alpha_idx, &w.keys, &w.keys_alt, &w.entry_rec,
+                            &w.rec_alt}) {
         if (d->as<uint8_t>() != end) break;
         end += d->bytes;
     }
@@ -1857,11 +1859,11 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
     b.zbuf = w.zbuf.as<uint32_t>();
     b.fb_range = w.fb_range.as<uint2>();
     b.keys = w.keys.as<uint32_t>();
-    b.vals = w.vals.as<uint32_t>();
     b.keys_alt = w.keys_alt.as<uint32_t>();
-    b.vals_alt = w.vals_alt.as<uint32_t>();
+    b.rec_alt = w.rec_alt.as<uint2>();
     b.entry_rec = w.entry_rec.as<uint2>();
     b.entry_meta = dump ? w.entry_meta.as<uint2>() : nullptr;
+    b.meta_alt = dump ? w.meta_alt.as<uint2>() : nullptr;
     b.counters = w.counters.as<uint32_t>();
     b.dump = dump ? 1 : 0;
     b.xcd_order = pl.sched.xcd_order;
@@ -1879,7 +1881,6 @@ static void stage_clear(Workspace &w, const BatchDev &b) {
     // paths with no columns are not binned: their totals and entry counts stay zero
     z.add(reinterpret_cast<uint32_t *>(b.path_tot), 2 * (uint64_t)b.n_paths);
     z.add(reinterpret_cast<uint32_t *>(b.path_ent), 2 * (uint64_t)b.n_paths);
-    z.add(reinterpret_cast<uint32_t *>(b.fb_range), 2 * (uint64_t)b.n_fb);
     z.add(b.counters, C_COUNT);
     z.add(reinterpret_cast<uint32_t *>(b.scan_state), 2 * b.scan_words);
     if (b.clip_seen) z.add(b.clip_seen, (uint64_t)b.cap_alpha / 32 + 1);
@@ -1917,17 +1918,14 @@ static void stage_emit(Workspace &w, const BatchDev &b, const Plan &pl) {
 static void stage_finish(Workspace &w, const BatchDev &b, const Plan &pl) {
     HIP_TRY(launch_entries(b, true, w.stream));
     bool alt = false;
-    HIP_TRY(radix_sort(b, b.keys, b.vals, b.keys_alt, b.vals_alt, pl.key_bits, w.sort_tmp.as<uint32_t>(), &alt,
-                       w.stream));
+    HIP_TRY(sort_entries(b, pl.max_fb, pl.max_tiles, w.sort_tmp.as<uint32_t>(), &alt, w.stream));
     w.last_sorted_alt = alt;
-    HIP_TRY(launch_fb_bounds(alt ? b.keys_alt : b.keys, b.counters + C_ENTRIES, b.cap_entries, b.n_fb, b.fb_range,
-                             w.stream));
     HIP_TRY(hipEventRecordWithFlags(w.kev[0], w.stream, hipEventRecordExternal));
     HIP_TRY(launch_fill_masks(b, b.cap_alpha, pl.sched.fill_grid, w.stream));
     HIP_TRY(launch_fill_clipped(b, w.stream));
     HIP_TRY(hipEventRecordWithFlags(w.kev[1], w.stream, hipEventRecordExternal));
     if (pl.clear_outside) HIP_TRY(launch_clear_outside(b, pl.max_rows, w.stream));
-    HIP_TRY(launch_composite(b, alt ? b.vals_alt : b.vals, pl.sched.composite_block, w.stream));
+    HIP_TRY(launch_composite(b, alt ? b.rec_alt : b.entry_rec, pl.sched.composite_block, w.stream));
     HIP_TRY(hipEventRecordWithFlags(w.kev[2], w.stream, hipEventRecordExternal));
 }
 
@@ -2022,16 +2020,14 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
     HIP_TRY(launch_entries(b, true, st));
     HIP_TRY(hipEventRecord(ev[5], st));
     bool alt = false;
-    HIP_TRY(radix_sort(b, b.keys, b.vals, b.keys_alt, b.vals_alt, pl.key_bits, ctx->w->sort_tmp.as<uint32_t>(), &alt,
-                       st));
+    HIP_TRY(sort_entries(b, pl.max_fb, pl.max_tiles, ctx->w->sort_tmp.as<uint32_t>(), &alt, st));
     ctx->w->last_sorted_alt = alt;
-    HIP_TRY(launch_fb_bounds(alt ? b.keys_alt : b.keys, b.counters + C_ENTRIES, b.cap_entries, b.n_fb, b.fb_range, st));
     HIP_TRY(hipEventRecord(ev[6], st));
     HIP_TRY(launch_fill_masks(b, na, pl.sched.fill_grid, st));
     HIP_TRY(launch_fill_clipped(b, st));
     HIP_TRY(hipEventRecord(ev[7], st));
     if (pl.clear_outside) HIP_TRY(launch_clear_outside(b, pl.max_rows, st));
-    HIP_TRY(launch_composite(b, alt ? b.vals_alt : b.vals, pl.sched.composite_block, st));
+    HIP_TRY(launch_composite(b, alt ? b.rec_alt : b.entry_rec, pl.sched.composite_block, st));
     HIP_TRY(hipEventRecord(ev[8], st));
     read_counters(ctx);
     for (int i = 0; i < 8; i++) ctx->stats.ms_stage[i] += elapsed_ms(ctx, ev[i], ev[i + 1]);
@@ -2167,6 +2163,7 @@ static void batched_enqueue(pfh_ctx *ctx, BatchedLaunch &bl) {
                     throw;
                 }
                 HIP_TRY(hipStreamEndCapture(w.stream, &graph));
+                cg.sorted_alt = w.last_sorted_alt;
                 hipError_t ie = hipGraphInstantiate(&cg.exec, graph, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(graph);
                 HIP_TRY(ie);
@@ -2176,8 +2173,7 @@ static void batched_enqueue(pfh_ctx *ctx, BatchedLaunch &bl) {
             }
             it = w.graphs.emplace(key, cg).first;
         } else {
-            // the sort's result buffer parity depends only on the key width
-            w.last_sorted_alt = ((pl.key_bits + 7) / 8) % 2 == 1;
+            w.last_sorted_alt = it->second.sorted_alt;
         }
         HIP_TRY(hipGraphLaunch(it->second.exec, w.stream));
     } else {
@@ -2737,21 +2733,12 @@ int pfh_dump(pfh_ctx *ctx, int32_t scene_id, int32_t *path_rect, int64_t *tile_o
         d2h(&ebase, ctx->w->path_ent.as<uint2>() + s.path_base, 4);
         d2h(&eend, ctx->w->path_ent.as<uint2>() + s.path_base + s.n_paths, 4);
         uint32_t ne = eend - ebase;
-        std::vector<uint32_t> sv(ne);
-        const uint32_t *sorted = ctx->w->last_sorted_alt ? ctx->w->vals_alt.as<uint32_t>() : ctx->w->vals.as<uint32_t>();
-        d2h(sv.data(), sorted + ebase, 4 * (size_t)ne);
-        uint32_t elo = 0xffffffffu, ehi = 0;
-        for (uint32_t v : sv) {
-            elo = std::min(elo, v);
-            ehi = std::max(ehi, v + 1);
-        }
-        if (ne) {
-            std::vector<uint2> meta(ehi - elo);
-            d2h(meta.data(), ctx->w->entry_meta.as<uint2>() + elo, 8 * (size_t)(ehi - elo));
-            for (uint32_t i = 0; i < ne; i++) {
-                entry_fbtile[i] = meta[sv[i] - elo].y;
-                entry_path[i] = meta[sv[i] - elo].x;
-            }
+        const uint2 *sorted = (ctx->w->last_sorted_alt ? ctx->w->meta_alt : ctx->w->entry_meta).as<uint2>();
+        std::vector<uint2> meta(ne);
+        d2h(meta.data(), sorted + ebase, 8 * (size_t)ne);
+        for (uint32_t i = 0; i < ne; i++) {
+            entry_fbtile[i] = meta[i].y;
+            entry_path[i] = meta[i].x;
         }
         d2h(zbuf, ctx->w->zbuf.as<uint32_t>() + fbb, 4 * (size_t)nfb);
         fb_rect[0] = s.fb_x0;
