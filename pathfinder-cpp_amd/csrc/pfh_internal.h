@@ -165,14 +165,16 @@ enum Counter {
     C_ALPHA_ENTRIES = 5,  // draw entries that sample a mask
     C_LINES = 6,       // flattened chords (lines) in the batch
     C_CLIP_JOBS = 7,   // clip combine jobs (alpha tiles over clip tiles with fills)
-    C_DRAWN = 8,       // [C_DRAWN, C_DRAWN + DRAWN_SLOTS): fills the fill kernel read, spread over
-                       // slots (per block, by block index) so that no single address takes every add
-    C_CLIP_DUPS = 8 + 64,  // draw entries whose clip mask row an earlier entry already listed
-    C_TALL = 8 + 64 + 1,   // [C_TALL, C_TALL + 6): per propagate phase, columns of more than
-                           // TALL_ROWS tiles (and Schedule::column_rows) listed for a wave each
-    C_MID = 8 + 64 + 1 + 6,  // [C_MID, C_MID + 6): per phase, columns of more than
-                             // Schedule::column_rows tiles and at most TALL_ROWS (k_propagate_rows<16>)
-    C_COUNT = 8 + 64 + 1 + 12
+    C_CLIP_DUPS = 8,   // draw entries whose clip mask row an earlier entry already listed
+    C_TALL = 9,        // [C_TALL, C_TALL + 6): per propagate phase, columns of more than
+                       // TALL_ROWS tiles (and Schedule::column_rows) listed for a wave each
+    C_MID = 9 + 6,     // [C_MID, C_MID + 6): per phase, columns of more than
+                       // Schedule::column_rows tiles and at most TALL_ROWS (k_propagate_rows<16>)
+    // fills of the tiles the fill kernel read: a slot per block, by block index, each in a 128-byte
+    // line of its own.  A line takes an add every 4-5 ns: with the slots side by side the adds of
+    // 16384 blocks took 75 us by themselves (2048^2 with 2500 paths: fill 75 -> 36 us).
+    C_DRAWN = 32,
+    C_COUNT = 32 + 64 * 32
 };
 // Arrays zeroed by one launch: p[k] has end[k] - end[k - 1] words (end[-1] = 0), k < n.
 constexpr int ZERO_SPANS = 7;
@@ -188,7 +190,7 @@ struct ZeroSpans {
     }
 };
 constexpr int TALL_ROWS = 64;
-constexpr int DRAWN_SLOTS = 64;
+constexpr int DRAWN_SLOTS = 64, DRAWN_STRIDE = 32;
 
 // One scene of a batch as the kernels see it.  Scene-local arrays are resident
 // from upload; *_base fields place the scene inside the batch's work arrays.

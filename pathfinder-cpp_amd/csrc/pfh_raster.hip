@@ -313,8 +313,9 @@ __global__ __launch_bounds__(256) void k_fill_masks(BatchDev b) {
     __shared__ uint32_t sdrawn[4];
     if (lane == 0) sdrawn[wv] = drawn;
     __syncthreads();
-    if (threadIdx.x == 0)
-        atomicAdd(&b.counters[C_DRAWN + (blockIdx.x & (DRAWN_SLOTS - 1))], sdrawn[0] + sdrawn[1] + sdrawn[2] + sdrawn[3]);
+    const uint32_t all = sdrawn[0] + sdrawn[1] + sdrawn[2] + sdrawn[3];
+    if (threadIdx.x == 0 && all)
+        atomicAdd(&b.counters[C_DRAWN + DRAWN_STRIDE * (blockIdx.x & (DRAWN_SLOTS - 1))], all);
 }
 
 // ---------------------------------------------------------------------------

@@ -1944,7 +1944,7 @@ static double elapsed_ms(pfh_ctx *ctx, hipEvent_t a, hipEvent_t b) {
 static void record_counts(pfh_ctx *ctx, const Plan &pl, bool dump) {
     ctx->stats.fills = ctx->w->h_counters[C_FILLS];
     int64_t drawn = 0;
-    for (int i = 0; i < DRAWN_SLOTS; i++) drawn += ctx->w->h_counters[C_DRAWN + i];
+    for (int i = 0; i < DRAWN_SLOTS; i++) drawn += ctx->w->h_counters[C_DRAWN + DRAWN_STRIDE * i];
     ctx->stats.fills_masked = drawn;
     // the fill kernel rasterizes the alpha tiles of draw entries (every alpha tile with dumps)
     // (listed mode: one row per alpha entry, less the clip mask rows another entry listed first)
