@@ -60,7 +60,8 @@ WORKLOADS = {
 def fill_bytes(st):
     # 12 B per fill read (reference Fill layout), 8 B alpha-tile index + 4 B backdrop/ctrl
     # per alpha tile, 256 B of u8 coverage written per 16x16 alpha tile; over the alpha tiles
-    # the fill kernel rasterizes (those draw entries sample) and their fills.
+    # draw entries sample and their fills (the fill kernel leaves out those under so many
+    # translucent layers that they cannot show; they count here as well).
     return 12 * st["fills_masked"] + 8 * st["alpha_masked"] + 4 * st["alpha_masked"] + 256 * st["alpha_masked"]
 
 

@@ -29,6 +29,7 @@ namespace pfh {
 // and the coverage mask is stored column-major too: lane c writes column c's 16 bytes with
 // one 16-byte store (byte 16 c + r is pixel (c, r)).
 
+constexpr uint8_t MASK_SHOWN = 0xff;  // not a TileStatus
 constexpr int FILL_TILES_PER_BLOCK = 16;
 constexpr int FILL_COL_WORDS = 20;                          // rows 0..16 used
 constexpr int FILL_GROUP_WORDS = 16 * FILL_COL_WORDS + 8;   // pad between tiles of a wave
@@ -37,8 +38,8 @@ constexpr int FILL_GROUP_WORDS = 16 * FILL_COL_WORDS + 8;   // pad between tiles
 
 
 
-// Adds one fill's contribution to pixel column `col` of a tile's difference array
-// (FILL_COL_WORDS words per column); LDS adds, since several lanes may share a column.
+// Adds one fill's contribution to pixel column `col` of a tile, whose differences are cd[0..16] in
+// LDS; LDS adds, since several lanes may share a column.
 // Over the column's x-window [lo, hi] (width w) the fill runs linearly between heights ymin
 // and ymax.  With G(t) = ∫ max(t - y(x), 0) dx over the window (0 below ymin, w (t - ymean)
 // above ymax, w (t - ymin)^2 / (2 (ymax - ymin)) between), the covered area of pixel row r is
@@ -77,11 +78,11 @@ __device__ __forceinline__ FillGeom fill_geom(uint2 fl) {
     return g;
 }
 
-// v_max_f32 / v_min_f32 on operands that are never NaN here, without the quieting fminf and
-// fmaxf apply to values loaded from memory.
-__device__ __forceinline__ float max_f(float a, float b) {
+// max(a, |b|) and min(a, b) on operands that are never NaN here, in one instruction each: without
+// the quieting fminf and fmaxf apply to values loaded from memory.
+__device__ __forceinline__ float max_abs(float a, float b) {
     float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    asm("v_max_f32_e64 %0, %1, |%2|" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
 __device__ __forceinline__ float min_f(float a, float b) {
@@ -90,10 +91,11 @@ __device__ __forceinline__ float min_f(float a, float b) {
     return r;
 }
 
-__device__ __forceinline__ void accumulate_fill(const FillGeom &g, int col, float scale, int32_t *tile_diff) {
+__device__ __forceinline__ float uint_f(uint32_t v) { return (float)(int)v; }
+
+__device__ __forceinline__ void accumulate_fill(const FillGeom &g, uint32_t col, float scale, int32_t *cd) {
     const float xl = fabsf(g.xl_signed), xr = g.xr;
-    const float lo = max_f((float)col, xl), hi = min_f((float)(col + 1), xr);
-    if (!(hi > lo) || (uint32_t)col > 15u) return;
+    const float lo = max_abs(uint_f(col), g.xl_signed), hi = min_f(uint_f(col) + 1.0f, xr);
     const float ks = __builtin_copysignf(scale, g.xl_signed);  // sign of the fill, in fixed-point units
     const float ya = g.yl + (lo - xl) * g.slope, yb = g.yl + (hi - xl) * g.slope;
     const float ymin = fminf(ya, yb), ymax = fmaxf(ya, yb);
@@ -110,11 +112,6 @@ __device__ __forceinline__ void accumulate_fill(const FillGeom &g, int col, floa
     const float f1 = n == 1 ? fd : k2 * (2.0f * u0 + 1.0f);          // F(r0 + 1), when n >= 1
     const int32_t full = round_fix(ws), v0 = round_fix(f0), v1 = round_fix(f1), vd = round_fix(fd);
     const int32_t dm = round_fix(2.0f * k2);  // F(r) - F(r - 1) for r0 + 2 <= r <= r1 - 1
-    // 0 <= col <= 15 here: the column's word offset by a full-rate 24-bit multiply (left to
-    // itself the compiler forms it with a quarter-rate 32-bit one)
-    uint32_t col_words;
-    asm("v_mul_u32_u24 %0, %1, %2" : "=v"(col_words) : "v"((uint32_t)col), "v"((uint32_t)FILL_COL_WORDS));
-    int32_t *cd = tile_diff + col_words;
     atomicAdd(cd + r0, v0);
     atomicAdd(cd + r0 + 1, (n == 0 ? full : v1) - v0);
     for (int r = r0 + 2; r < r1; r++) atomicAdd(cd + r, dm);
@@ -164,17 +161,21 @@ __device__ __forceinline__ void resolve_column(int32_t run, const int32_t (&dv)[
     }
 }
 
-// A wave takes 4 consecutive alpha tiles (16 lanes, one pixel column each, per tile).  Their
+// A wave takes 4 alpha tiles at a time (16 lanes, one pixel column each, per tile).  Their
 // fills form one pooled list of up to 64 per chunk; the (fill, pixel column) pairs of a
 // chunk are enumerated with a wave-wide prefix sum, so every lane works on a pair that
 // contributes whatever the mix of light and heavy tiles in the wave.  The tiles are those
 // some draw entry samples, in the list the entry pass wrote: a mask hidden under an opaque
 // solid tile of a later path is never read, so it is not computed.  With dumps every alpha
-// tile is rasterized, in index order.
-__global__ __launch_bounds__(256) void k_fill_masks(BatchDev b) {
+// tile is rasterized, in index order.  `shown` (k_shown_masks): a byte each of
+// the first n_shown masks, MASK_SHOWN unless no pixel of the target can depend on it: not computed either.
+// The kernel is bound by the pairs (VALU and LDS adds), then by the prefix sums down the columns, so a
+// wave reads up to 64 list entries in a row (fewer while the list is short, so that it spreads over
+// the chip) and takes the shown ones 4 by 4.
+__global__ __launch_bounds__(256) void k_fill_masks(BatchDev b, const uint8_t *shown, uint32_t n_shown) {
     __shared__ __align__(16) int32_t diff[FILL_TILES_PER_BLOCK * FILL_GROUP_WORDS];
-    // a chunk's fills: geometry, and (first pair | tile offset in the wave's LDS << 11 | first
-    // pixel column << 27); a pair window's marks: 1 where a fill's pairs start
+    // a chunk's fills: geometry, and (first pair | first pixel column << 11 | that column's offset in
+    // the wave's LDS << 15); a pair window's marks: 1 where a fill's pairs start
     __shared__ FillGeom sgeom[4][64];
     __shared__ uint32_t smeta[4][64];
     __shared__ uint8_t smark[4][64];
@@ -185,137 +186,243 @@ __global__ __launch_bounds__(256) void k_fill_masks(BatchDev b) {
     const bool listed = !b.dump;
     const uint32_t na = min(b.counters[listed ? C_ALPHA_ENTRIES : C_ALPHA], listed ? b.cap_vis : b.cap_alpha);
     const float scale = (float)(1 << FIX_SHIFT);
-    uint32_t drawn = 0;  // fills this wave read (wave-uniform)
+    uint32_t drawn = 0;  // fills of the tiles this lane read
     // row cap_alpha of the masks is all ones: the composite's full-coverage row
     if (blockIdx.x == 0 && wv == 0)
         reinterpret_cast<uint32_t *>(b.masks)[(uint64_t)b.cap_alpha * 64 + lane] = 0xffffffffu;
-    // grid-stride over groups of 16 tiles: the grid is sized from the capacity, the count
-    // is only known on the device; the loop bound is uniform over the block
+    // the grid is sized from the capacity, the count is only known on the device: each wave takes
+    // `run` list entries, a multiple of 4, and strides on
     const uint32_t lb = (b.xcd_order & 1u) ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-    const uint32_t stride = gridDim.x * FILL_TILES_PER_BLOCK, first0 = lb * FILL_TILES_PER_BLOCK;
-    const uint32_t mine = wv * 4 + slot;  // this lane's tile within a group
-    // The tile list and the tile records are read ahead (the record one group ahead, the list
-    // entry two), so a group starts with its record in registers and waits only for its fills.
-    // ~0u: no tile.
-    auto tile_at = [&](uint32_t idx) { return idx >= na ? ~0u : (listed ? b.alpha_vis[idx] : idx); };
-    auto rec_of = [&](uint32_t a) { return a < b.cap_alpha ? b.alpha_rec[a] : make_uint4(0, 0, 0, 0); };
-    uint32_t a_next = tile_at(first0 + mine), a_after = tile_at(first0 + stride + mine);
-    uint4 rec_next = rec_of(a_next);
-    for (uint32_t first = first0; first < na; first += stride) {
-        const uint32_t a = a_next;
-        const uint4 rec = rec_next;
-        const bool valid = a < b.cap_alpha;
-        rec_next = rec_of(a_after);
-        a_next = a_after;
-        a_after = tile_at(first + 2 * stride + mine);
-#pragma unroll
-        for (int k = 0; k < FILL_COL_WORDS / 4; k++) reinterpret_cast<uint4 *>(dcol)[k] = make_uint4(0, 0, 0, 0);
+    const uint32_t waves = gridDim.x * 4;
+    const uint32_t run = min(64u, max(4u, (na / waves + 4u) & ~3u));
+    const uint64_t step = (uint64_t)waves * run;
+    for (uint64_t at = (uint64_t)(lb * 4 + wv) * run; at < na; at += step) {  // wave-uniform
+        uint32_t a_own = ~0u;  // this lane's list entry; ~0u: no tile
+        if (lane < run && at + lane < na) a_own = listed ? b.alpha_vis[at + lane] : (uint32_t)at + lane;
+        uint4 rec_own = make_uint4(0, 0, 0, 0);
+        bool take = a_own < b.cap_alpha;
+        if (take) {
+            rec_own = b.alpha_rec[a_own];
+            if (a_own < n_shown) take = shown[a_own] == MASK_SHOWN;
+        }
         // After a fill-capacity overflow a tile's range can start past the buffer: clamp both
         // ends so no count wraps (the batch is then retried).
-        const uint32_t f0 = min(rec.x, b.cap_fills);
-        const uint32_t f1 = max(f0, min(rec.y, b.cap_fills));
-        // the 4 tiles' ranges (uniform over the wave), concatenated
-        const uint32_t s0 = __builtin_amdgcn_readlane(f0, 0), n0 = __builtin_amdgcn_readlane(f1, 0) - s0;
-        const uint32_t s1 = __builtin_amdgcn_readlane(f0, 16), n1 = __builtin_amdgcn_readlane(f1, 16) - s1;
-        const uint32_t s2 = __builtin_amdgcn_readlane(f0, 32), n2 = __builtin_amdgcn_readlane(f1, 32) - s2;
-        const uint32_t s3 = __builtin_amdgcn_readlane(f0, 48), n3 = __builtin_amdgcn_readlane(f1, 48) - s3;
-        const uint32_t c1 = n0, c2 = c1 + n1, c3 = c2 + n2, ntot = c3 + n3;
-        const uint32_t o1 = s1 - c1, o2 = s2 - c2, o3 = s3 - c3;  // wrapping differences
-        drawn += ntot;
-        for (uint32_t base = 0; base < ntot; base += 64) {
-            const uint32_t k = base + lane;
-            uint32_t cnt = 0, fs = 0, c0 = 0;
-            FillGeom g{0.0f, 0.0f, 0.0f, 0.0f};
-            if (k < ntot) {
-                // fill k of the concatenated ranges: k minus its tile's first, plus that tile's start
-                const bool ge1 = k >= c1, ge2 = k >= c2, ge3 = k >= c3;
-                fs = (ge1 ? 1u : 0u) + (ge2 ? 1u : 0u) + (ge3 ? 1u : 0u);
-                uint32_t off = s0;
-                off = ge1 ? o1 : off;
-                off = ge2 ? o2 : off;
-                off = ge3 ? o3 : off;
-                const uint32_t addr = k + off;
-                g = fill_geom(b.fills[addr]);
-                const float xl = fabsf(g.xl_signed);
-                const int cl = (int)floorf(xl);
-                cnt = (uint32_t)max(0, (int)ceilf(g.xr) - cl);
-                c0 = (uint32_t)cl & 15u;  // 8.8 fills lie in [0, 16): cl <= 15
+        rec_own.x = min(rec_own.x, b.cap_fills);
+        rec_own.y = max(rec_own.x, min(rec_own.y, b.cap_fills));
+        drawn += rec_own.y - rec_own.x;
+        // The taken tiles move to the front, in order, the others (without fills) behind them; four
+        // neighbours are a group, whose fills are drawn together.
+        const uint64_t taken = __ballot(take);
+        const uint32_t n_taken = (uint32_t)__popcll(taken);
+        const uint32_t before = __builtin_amdgcn_mbcnt_hi((uint32_t)(taken >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)taken, 0u));
+        const int to = (int)(4u * (take ? before : 63u - (lane - before)));
+        const uint32_t row = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)a_own);
+        const uint32_t ctl_own = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)rec_own.z);
+        const uint32_t n_own = (uint32_t)__builtin_amdgcn_ds_permute(to, take ? (int)(rec_own.y - rec_own.x) : 0);
+        // where the tile's fills end in its group's, and its range's start less the fills before it (wrapping)
+        uint32_t end_own = n_own;
+        const uint32_t left1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)end_own, 0x90, 0xf, 0xf, false);  // quad_perm 0 0 1 2
+        end_own += (lane & 3) >= 1 ? left1 : 0u;
+        const uint32_t left2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)end_own, 0x44, 0xf, 0xf, false);  // quad_perm 0 1 0 1
+        end_own += (lane & 3) >= 2 ? left2 : 0u;
+        const uint32_t off_own = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)rec_own.x) - (end_own - n_own);
+        // fill k of the group at `g0`: its tile's slot, and the fill
+        uint32_t c0, c1, c2, c3;
+        auto group_ends = [&](uint32_t g0) {
+            c0 = __builtin_amdgcn_readlane(end_own, g0);
+            c1 = __builtin_amdgcn_readlane(end_own, g0 + 1);
+            c2 = __builtin_amdgcn_readlane(end_own, g0 + 2);
+            c3 = __builtin_amdgcn_readlane(end_own, g0 + 3);
+        };
+        auto load_fill = [&](uint32_t g0, uint32_t k, uint32_t &fs, uint2 &fl) {
+            fs = (k >= c0 ? 1u : 0u) + (k >= c1 ? 1u : 0u) + (k >= c2 ? 1u : 0u);
+            const uint32_t off = __shfl(off_own, (int)(g0 + fs), 64);
+            fl = make_uint2(0u, 0u);
+            if (k < c3) fl = b.fills[k + off];
+        };
+        // a group's first fills are loaded while the group before it is drawn
+        uint32_t fs_next;
+        uint2 fill_next;
+        group_ends(0);
+        load_fill(0, lane, fs_next, fill_next);
+        for (uint32_t g0 = 0; g0 < n_taken; g0 += 4) {
+            const uint32_t ntot = c3;
+            uint32_t fs = fs_next;
+            uint2 fill = fill_next;
+            if (ntot <= 64 && g0 + 4 < n_taken) {
+                group_ends(g0 + 4);
+                load_fill(g0 + 4, lane, fs_next, fill_next);
             }
-            const uint32_t incl = wave_inclusive_sum(cnt);
-            const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
-            const uint32_t start = incl - cnt;  // this fill's first pair (< 64 * 17)
-            sgeom[wv][lane] = g;
-            smeta[wv][lane] = start | ((fs * FILL_GROUP_WORDS) << 11) | (c0 << 27);
-            // Pairs go in windows of 64, one per lane.  The fill owning pair q is the last one
-            // starting at or before q: marks at the window's fill starts, their ballot, and the
-            // count of marks up to this lane (plus the fills that started in earlier windows)
-            // give it.  Every fill covers at least one column (the bin stage drops fills with
-            // equal x ends), so no two fills start at the same pair.
-            uint32_t carry = 0;
-            for (uint32_t q0 = 0; q0 < total; q0 += 64) {
-                smark[wv][lane] = 0;
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                if (cnt != 0 && start >= q0 && start - q0 < 64u) smark[wv][start - q0] = 1;
-                // the marks, the chunk's fills and (first chunk) the zeroed columns are visible
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                const uint64_t marks = __ballot(smark[wv][lane] != 0);
-                const uint32_t q = q0 + lane;
-                if (q < total) {
-                    const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(marks >> 32),
-                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)marks, 0u));
-                    const uint32_t j = min(carry + below + (uint32_t)((marks >> lane) & 1ull) - 1u, 63u);
-                    const FillGeom g = sgeom[wv][j];
-                    const uint32_t m = smeta[wv][j];
-                    const int col = (int)(m >> 27) + (int)(q - (m & 2047u));
-                    accumulate_fill(g, col, scale, dwave + ((m >> 11) & 2047u));
+            const bool valid = g0 + slot < n_taken;
+            const uint32_t a = __shfl(row, (int)(g0 + slot), 64), ctl = __shfl(ctl_own, (int)(g0 + slot), 64);
+#pragma unroll
+            for (int k = 0; k < FILL_COL_WORDS / 4; k++) reinterpret_cast<uint4 *>(dcol)[k] = make_uint4(0, 0, 0, 0);
+            for (uint32_t base = 0; base < ntot; base += 64) {
+                const uint32_t k = base + lane;
+                uint32_t cnt = 0, col0 = 0;
+                FillGeom g{0.0f, 0.0f, 0.0f, 0.0f};
+                if (base) load_fill(g0, k, fs, fill);
+                if (k < ntot) {
+                    g = fill_geom(fill);
+                    const float xl = fabsf(g.xl_signed);
+                    const int cl = (int)floorf(xl);
+                    col0 = (uint32_t)cl & 15u;  // 8.8 fills lie in [0, 16): cl <= 15
+                    cnt = (uint32_t)med3_i32((int)ceilf(g.xr) - cl, 0, 16 - (int)col0);
                 }
-                carry += (uint32_t)__popcll(marks);
-                // the next window rewrites the marks, the next chunk the fills
+                const uint32_t incl = wave_inclusive_sum(cnt);
+                const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
+                const uint32_t start = incl - cnt;  // this fill's first pair (< 64 * 16)
+                sgeom[wv][lane] = g;
+                smeta[wv][lane] = start | (col0 << 11) | ((fs * FILL_GROUP_WORDS + col0 * FILL_COL_WORDS) << 15);
+                // Pairs go in windows of 64, one per lane.  The fill owning pair q is the last one
+                // starting at or before q: marks at the window's fill starts, their ballot, and the
+                // count of marks up to this lane (plus the fills that started in earlier windows)
+                // give it.  Every fill covers at least one column (the bin stage drops fills with
+                // equal x ends), so no two fills start at the same pair.
+                uint32_t carry = 0;
+                for (uint32_t q0 = 0; q0 < total; q0 += 64) {
+                    smark[wv][lane] = 0;
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    if (cnt != 0 && start >= q0 && start - q0 < 64u) smark[wv][start - q0] = 1;
+                    // the marks, the chunk's fills and (first chunk) the zeroed columns are visible
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    const bool own = smark[wv][lane] != 0;
+                    const uint64_t marks = __ballot(own);
+                    const uint32_t q = q0 + lane;
+                    if (q < total) {
+                        const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(marks >> 32),
+                                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)marks, carry));
+                        const uint32_t j = below - (own ? 0u : 1u);
+                        const FillGeom g = sgeom[wv][j];
+                        const uint32_t m = smeta[wv][j];
+                        const uint32_t i = q - (m & 2047u);  // the fill's i-th column
+                        accumulate_fill(g, ((m >> 11) & 15u) + i, scale, dwave + ((m >> 15) + __umul24(i, FILL_COL_WORDS)));
+                    }
+                    carry += (uint32_t)__popcll(marks);
+                    // the next window rewrites the marks, the next chunk the fills
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                }
+            }
+            if (ntot > 64 && g0 + 4 < n_taken) {
+                group_ends(g0 + 4);
+                load_fill(g0 + 4, lane, fs_next, fill_next);
+            }
+            if (ntot == 0) {  // nothing accumulated: the zeroing still has to land first
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             }
-        }
-        if (ntot == 0) {  // nothing accumulated: the zeroing still has to land first
+            const uint32_t rule = (ctl >> 8) & 1u;
+            int32_t dv[16];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint4 v = reinterpret_cast<const uint4 *>(dcol)[k];
+                dv[4 * k] = (int32_t)v.x;
+                dv[4 * k + 1] = (int32_t)v.y;
+                dv[4 * k + 2] = (int32_t)v.z;
+                dv[4 * k + 3] = (int32_t)v.w;
+            }
+            const int32_t bd_fix = (int32_t)(int8_t)(ctl & 0xffu) * (1 << FIX_SHIFT);  // backdrop, exact
+            uint32_t packed[4];
+            // the 4 tiles of a wave nearly always belong to one path: branch on a wave-uniform rule
+            const uint64_t eo_mask = __ballot(rule != 0);
+            if (eo_mask == 0) resolve_column<0>(bd_fix, dv, rule, packed);
+            else if (eo_mask == ~0ull) resolve_column<1>(bd_fix, dv, rule, packed);
+            else resolve_column<2>(bd_fix, dv, rule, packed);
+            if (valid)
+                reinterpret_cast<uint4 *>(b.masks + (uint64_t)a * 256)[li] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+            // the next group of tiles reuses this wave's LDS
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
-        const uint32_t rule = (rec.z >> 8) & 1u;
-        int32_t dv[16];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const uint4 v = reinterpret_cast<const uint4 *>(dcol)[k];
-            dv[4 * k] = (int32_t)v.x;
-            dv[4 * k + 1] = (int32_t)v.y;
-            dv[4 * k + 2] = (int32_t)v.z;
-            dv[4 * k + 3] = (int32_t)v.w;
-        }
-        const int32_t bd_fix = (int32_t)(int8_t)(rec.z & 0xffu) * (1 << FIX_SHIFT);  // backdrop, exact
-        uint32_t packed[4];
-        // the 4 tiles of a wave nearly always belong to one path: branch on a wave-uniform rule
-        const uint64_t eo_mask = __ballot(rule != 0);
-        if (eo_mask == 0) resolve_column<0>(bd_fix, dv, rule, packed);
-        else if (eo_mask == ~0ull) resolve_column<1>(bd_fix, dv, rule, packed);
-        else resolve_column<2>(bd_fix, dv, rule, packed);
-        if (valid)
-            reinterpret_cast<uint4 *>(b.masks + (uint64_t)a * 256)[li] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-        // the next group of tiles reuses this wave's LDS
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    // one add per block, spread over slots by block index (the loop above is uniform over the block)
+    // one add per block, spread over slots by block index
     __shared__ uint32_t sdrawn[4];
-    if (lane == 0) sdrawn[wv] = drawn;
+    drawn = wave_inclusive_sum(drawn);
+    if (lane == 63) sdrawn[wv] = drawn;
     __syncthreads();
     const uint32_t all = sdrawn[0] + sdrawn[1] + sdrawn[2] + sdrawn[3];
     if (threadIdx.x == 0 && all)
         atomicAdd(&b.counters[C_DRAWN + DRAWN_STRIDE * (blockIdx.x & (DRAWN_SLOTS - 1))], all);
+}
+
+// Which masks can show: a masked entry under solid entries that let nearly nothing through changes no
+// byte of the target, whatever its mask holds, so its mask need not be computed.  shown[row] =
+// MASK_SHOWN for the rows of entries that can; shown is the tiles' status array, which the entries were
+// the last to read and every pass writes whole, with other values.
+// A solid entry of alpha a multiplies the transmittance t by 1 - a.  The composite folds a run of
+// solids in float, 1 - a as good as 2^-21, so neighbouring solids count for at most HIDE_RUN bits
+// together; t never grows.  Below 2^-34 an entry's whole contribution, at most 255 |t|, is under half an
+// ulp of every channel value from 0.25 on and is rounded away; a smaller value stays in byte 0; alpha is
+// 255 by then.  HIDE_BITS leaves two bits for the error of the bits' sum and of t (each solid's bits are
+// rounded down).  Blending through an op is not bounded like this: scenes with one show all their masks.
+// 16 lanes per framebuffer tile, from the top entry down, 16 entries at a time, until nothing below
+// can show: bound by the latency of a tile's chain (its range, its entries), so four tiles share a wave
+// (48 scenes, 532 000 tiles, 2.6 of 4.2 million masks left out: 35 us, against 95 with a wave per tile
+// reading all of its entries; the fill kernel 645 -> 294).
+constexpr uint32_t HIDE_ONE = 256;  // a bit of transmittance
+constexpr uint32_t HIDE_RUN = 18 * HIDE_ONE, HIDE_BITS = 36 * HIDE_ONE;
+
+__global__ __launch_bounds__(256) void k_shown_masks(BatchDev b, const uint2 *recs, uint8_t *shown, uint32_t n_rows) {
+    const uint32_t lane = threadIdx.x & 63, li = lane & 15, first = lane & 48;
+    const uint32_t f = blockIdx.x * 16 + (threadIdx.x >> 4);
+    uint2 range = make_uint2(0u, 0u);
+    bool bounded = true;
+    if (f < b.n_fb) {
+        range = b.fb_range[f];
+        if (b.paints) {
+            int lo = 0, hi = b.n_scenes - 1;  // the tile's scene
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) / 2;
+                if (b.fb_bases[mid] <= f) lo = mid;
+                else hi = mid - 1;
+            }
+            bounded = b.scenes[lo].has_ops == 0;
+        }
+    }
+    const uint32_t e0 = range.x;
+    uint32_t e1 = max(e0, min(range.y, b.cap_entries));  // entries left
+    uint32_t bits = 0, open = 0;  // of the entries above; of the run that goes on from there, uncapped
+    uint2 rec = make_uint2(NO_ALPHA, 0u);
+    if (e1 - e0 > li) rec = recs[e1 - 1 - li];
+    while (__ballot(e1 > e0)) {  // uniform over the wave
+        const bool in = e1 - e0 > li;
+        const uint2 cur = rec;
+        e1 = e1 - e0 > 16 ? e1 - 16 : e0;
+        rec = make_uint2(NO_ALPHA, 0u);
+        if (e1 - e0 > li) rec = recs[e1 - 1 - li];
+        const bool masked = in && cur.x != NO_ALPHA, solid = in && !masked;
+        uint32_t own = 0;
+        if (solid) {
+            const float thru = (float)(255u - (cur.y >> 24)) * (1.0f / 255.0f);
+            own = (uint32_t)(int)fminf(fmaxf(-(float)HIDE_ONE * __log2f(thru) - 1.0f, 0.0f), (float)HIDE_RUN);
+        }
+        const uint32_t solids = (uint32_t)(__ballot(solid) >> first) & 0xffffu;
+        // a run's bits, at its lowest entry here: the sum down to it less the sum above its first
+        const uint32_t sum = row16_inclusive_sum(own);
+        const uint32_t gaps = ~solids & ((1u << li) - 1u);  // not solid, above this entry
+        const uint32_t start = gaps ? 32u - (uint32_t)__builtin_clz(gaps) : 0u;
+        const uint32_t before = __shfl(sum, (int)(first + (start ? start - 1 : 0u)), 64);
+        const uint32_t run = start ? sum - before : sum + open;
+        const uint32_t counted = start ? 0u : min(open, HIDE_RUN);
+        const bool last = solid && (li == 15 || !((solids >> (li + 1)) & 1u));
+        const uint32_t credit = row16_inclusive_sum(last ? min(run, HIDE_RUN) - counted : 0u);
+        if (masked) {
+            uint32_t row = cur.x;
+            if (b.paints && (row & ENTRY_GRADIENT)) row &= ENTRY_ROW_MASK;
+            if (row < n_rows && (!bounded || bits + credit < HIDE_BITS)) shown[row] = MASK_SHOWN;
+        }
+        bits += __shfl(credit, (int)(first + 15), 64);
+        open = __shfl(solid ? run : 0u, (int)(first + 15), 64);
+        if (bounded && bits >= HIDE_BITS) e1 = e0;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -984,11 +1091,22 @@ __global__ __launch_bounds__(256) void k_fill_clipped(BatchDev b) {
 
 static inline uint32_t blocks_for(uint64_t n, uint32_t per) { return (uint32_t)((n + per - 1) / per); }
 
-hipError_t launch_fill_masks(const BatchDev &b, uint32_t grid_alpha, uint32_t max_blocks, hipStream_t s) {
+// shown: launch_shown_masks' n_shown bytes, or none.
+hipError_t launch_fill_masks(const BatchDev &b, const uint8_t *shown, uint32_t n_shown, uint32_t grid_alpha,
+                             uint32_t max_blocks, hipStream_t s) {
     // at least one workgroup (it writes the all-ones row), at most max_blocks: each loops over
     // its share of the tiles
     const uint32_t nb = std::max(1u, std::min<uint32_t>(blocks_for(grid_alpha, FILL_TILES_PER_BLOCK), max_blocks));
-    hipLaunchKernelGGL(k_fill_masks, dim3(nb), dim3(256), 0, s, b);
+    hipLaunchKernelGGL(k_fill_masks, dim3(nb), dim3(256), 0, s, b, shown, n_shown);
+    return hipGetLastError();
+}
+
+// shown[0 .. n_rows), statuses before: MASK_SHOWN for the needed ones of the masks that entries sample.  Not with clip paths (several
+// entries can sample one mask).
+hipError_t launch_shown_masks(const BatchDev &b, const uint2 *recs, uint8_t *shown, uint32_t n_rows, hipStream_t s) {
+    if (b.n_fb == 0) return hipSuccess;
+    if (b.has_clips) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_shown_masks, dim3(blocks_for(b.n_fb, 16)), dim3(256), 0, s, b, recs, shown, n_rows);
     return hipGetLastError();
 }
 
