@@ -176,15 +176,18 @@ enum Counter {
     C_DRAWN = 32,
     C_COUNT = 32 + 64 * 32
 };
-// Arrays zeroed by one launch: p[k] has end[k] - end[k - 1] words (end[-1] = 0), k < n.
-constexpr int ZERO_SPANS = 7;
+// Arrays set by one launch: p[k] has end[k] - end[k - 1] words (end[-1] = 0), k < n, copied from
+// src[k], or zeroed where that is null.
+constexpr int ZERO_SPANS = 9;
 struct ZeroSpans {
     uint32_t *p[ZERO_SPANS];
+    const uint32_t *src[ZERO_SPANS];
     uint64_t end[ZERO_SPANS];
     int n;
-    void add(uint32_t *ptr, uint64_t words) {
+    void add(uint32_t *ptr, uint64_t words, const uint32_t *from = nullptr) {
         if (!words) return;
         p[n] = ptr;
+        src[n] = from;
         end[n] = (n ? end[n - 1] : 0) + words;
         n++;
     }
@@ -308,6 +311,7 @@ struct BatchDev {
     uint2 *rec_alt;               // [E] the sort's other buffer
     uint2 *entry_meta, *meta_alt; // [E] with dumps only: (local path, scene-local fb tile), sorted likewise
     uint32_t *counters;           // [C_COUNT]
+    uint32_t *counters_out;       // [C_COUNT] pinned host memory: where the composite leaves them for the host
     int32_t dump;
     int32_t has_clips;            // some scene has clip paths: propagate in two phases, combine masks
     uint32_t xcd_order;           // Schedule::xcd_order

@@ -22,9 +22,9 @@ namespace pfh {
 // helpers
 // ---------------------------------------------------------------------------
 
-// Zeroes up to ZERO_SPANS arrays in one launch (the per-launch clears: one dispatch and one tail
-// instead of one per array): index i of their concatenation lies in the first span whose end is
-// past it.
+// Sets up to ZERO_SPANS arrays in one launch (the per-launch clears, and the tables the host wrote to
+// pinned memory: one dispatch and one tail instead of one per array and copy): index i of their
+// concatenation lies in the first span whose end is past it.
 __global__ void k_zero_spans(ZeroSpans z) {
     const uint64_t total = z.n ? z.end[z.n - 1] : 0;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -32,7 +32,7 @@ __global__ void k_zero_spans(ZeroSpans z) {
 #pragma unroll
         for (int k = 0; k < ZERO_SPANS; k++) {
             const uint64_t start = k ? z.end[k - 1] : 0;
-            if (k < z.n && i >= start && i < z.end[k]) z.p[k][i - start] = 0u;
+            if (k < z.n && i >= start && i < z.end[k]) z.p[k][i - start] = z.src[k] ? z.src[k][i - start] : 0u;
         }
     }
 }

@@ -660,12 +660,27 @@ __device__ void composite_back_to_front(const BatchDev &b, const SceneDev &sc, c
     }
 }
 
+// The counters for the host, which waits for the end of the composite anyway: a copy behind it took
+// 10 us, with the gap before it.  By one wave; of each slot of C_DRAWN only its first word counts.
+__device__ __forceinline__ void publish_counters(const BatchDev &b) {
+    static_assert(C_DRAWN <= 64 && DRAWN_SLOTS <= 64, "a lane each");
+    const uint32_t i = threadIdx.x;
+    if (i < C_DRAWN) b.counters_out[i] = b.counters[i];
+    if (i < DRAWN_SLOTS) b.counters_out[C_DRAWN + DRAWN_STRIDE * i] = b.counters[C_DRAWN + DRAWN_STRIDE * i];
+}
+
+__global__ __launch_bounds__(64) void k_publish_counters(BatchDev b) { publish_counters(b); }
+
 // PAINTS: some scene of the batch has paint records (the solid-only variant carries no code for them).
 template <bool PAINTS>
 __global__ __launch_bounds__(256) void k_composite(BatchDev b, const uint2 *recs) {
     __shared__ float4 s_colour[4][64];  // per wave of the block: the chunk's premultiplied colours
     const int lane = threadIdx.x & 63;
-    const uint32_t lb = (b.xcd_order & 2u) ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    if (blockIdx.x == gridDim.x - 1) {  // the block behind the tiles'
+        publish_counters(b);
+        return;
+    }
+    const uint32_t lb = (b.xcd_order & 2u) ? xcd_block(blockIdx.x, gridDim.x - 1) : blockIdx.x;
     // the tile and its scene are uniform over the wave: held in scalar registers, so the scene
     // record and the tile's range come through scalar loads
     const uint32_t f = __builtin_amdgcn_readfirstlane(lb * (blockDim.x >> 6) + (threadIdx.x >> 6));
@@ -1117,13 +1132,18 @@ hipError_t launch_fill_clipped(const BatchDev &b, hipStream_t s) {
     return hipGetLastError();
 }
 
+hipError_t launch_publish_counters(const BatchDev &b, hipStream_t s) {
+    hipLaunchKernelGGL(k_publish_counters, dim3(1), dim3(64), 0, s, b);
+    return hipGetLastError();
+}
+
+// Leaves the counters in b.counters_out as well.
 hipError_t launch_composite(const BatchDev &b, const uint2 *recs, uint32_t block, hipStream_t s) {
-    if (b.n_fb == 0) return hipSuccess;
     if (block != 64 && block != 128 && block != 256) return hipErrorInvalidValue;
     if (b.paints)
-        hipLaunchKernelGGL(k_composite<true>, dim3(blocks_for(b.n_fb, block / 64)), dim3(block), 0, s, b, recs);
+        hipLaunchKernelGGL(k_composite<true>, dim3(blocks_for(b.n_fb, block / 64) + 1), dim3(block), 0, s, b, recs);
     else
-        hipLaunchKernelGGL(k_composite<false>, dim3(blocks_for(b.n_fb, block / 64)), dim3(block), 0, s, b, recs);
+        hipLaunchKernelGGL(k_composite<false>, dim3(blocks_for(b.n_fb, block / 64) + 1), dim3(block), 0, s, b, recs);
     return hipGetLastError();
 }
 

@@ -42,6 +42,7 @@ hipError_t launch_fill_masks(const BatchDev &b, const uint8_t *shown, uint32_t n
                              uint32_t max_blocks, hipStream_t s);
 hipError_t launch_fill_clipped(const BatchDev &b, hipStream_t s);
 hipError_t launch_composite(const BatchDev &b, const uint2 *recs, uint32_t block, hipStream_t s);
+hipError_t launch_publish_counters(const BatchDev &b, hipStream_t s);
 hipError_t launch_clear_outside(const BatchDev &b, uint32_t max_rows, hipStream_t s);
 hipError_t mlp_forward(const float *params, const float *x, int64_t n, float *hidden, float *out, hipStream_t s);
 hipError_t mlp_backward(const float *params, const float *x, int64_t n, const float *hidden, const float *out,
@@ -372,7 +373,8 @@ struct Workspace {
     DevBuf scene_table, bases, tile_delta, tile_cnt, tile_fill_off, tile_alpha_idx, tile_bd, tile_st, path_ent, ent_quarter, path_tot, bin_items, col_item, col_bd, tall_cols, seg_mask,
         seg_cnt, lines, line_cnt, fills, dump_fills, alpha_rec, alpha_vis, masks, zbuf, fb_range, keys, keys_alt,
         rec_alt, entry_rec, entry_meta, meta_alt, counters, chunk_off, scan_state, dump_state, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen;
-    uint32_t *h_counters = nullptr;  // pinned
+    // pinned and coherent: kernels write h_counters and read the tables
+    uint32_t *h_counters = nullptr;
     SceneDev *h_table = nullptr;     // pinned scene table
     size_t h_table_cap = 0;
     uint32_t *h_bases = nullptr;
@@ -387,18 +389,19 @@ struct Workspace {
     // that a launch of at most that many scenes creates nothing.
     void create(size_t table_scenes = 0) {
         HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-        HIP_TRY(hipEventCreate(&ev0));
+        // the host waits for ev1 alone: the others only time, without a fence for it (3 us less each)
+        HIP_TRY(hipEventCreateWithFlags(&ev0, hipEventDisableSystemFence));
         HIP_TRY(hipEventCreate(&ev1));
-        for (auto &e : kev) HIP_TRY(hipEventCreate(&e));
+        for (auto &e : kev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
         // An event whose first record is an external record node inside a stream capture is
         // refused (invalid argument): record each once, eagerly, before any capture.
         for (auto &e : kev) HIP_TRY(hipEventRecord(e, stream));
-        for (auto &e : stage_ev) HIP_TRY(hipEventCreate(&e));
-        HIP_TRY(hipHostMalloc((void **)&h_counters, 4 * C_COUNT));
+        for (auto &e : stage_ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
+        HIP_TRY(hipHostMalloc((void **)&h_counters, 4 * C_COUNT, hipHostMallocCoherent));
         if (table_scenes) {
-            HIP_TRY(hipHostMalloc((void **)&h_table, sizeof(SceneDev) * table_scenes));
+            HIP_TRY(hipHostMalloc((void **)&h_table, sizeof(SceneDev) * table_scenes, hipHostMallocCoherent));
             h_table_cap = table_scenes;
-            HIP_TRY(hipHostMalloc((void **)&h_bases, sizeof(uint32_t) * 6 * (table_scenes + 1)));
+            HIP_TRY(hipHostMalloc((void **)&h_bases, sizeof(uint32_t) * 6 * (table_scenes + 1), hipHostMallocCoherent));
             h_bases_cap = 6 * (table_scenes + 1);
         }
     }
@@ -1669,12 +1672,14 @@ static void write_tables(pfh_ctx *ctx, Plan &pl, bool load_dst) {
     size_t n = pl.ids.size();
     if (ctx->w->h_table_cap < n) {
         if (ctx->w->h_table) (void)hipHostFree(ctx->w->h_table);
-        HIP_TRY(hipHostMalloc((void **)&ctx->w->h_table, sizeof(SceneDev) * n));
+        g_alloc_generation++;  // captured launches read it in place
+        HIP_TRY(hipHostMalloc((void **)&ctx->w->h_table, sizeof(SceneDev) * n, hipHostMallocCoherent));
         ctx->w->h_table_cap = n;
     }
     if (ctx->w->h_bases_cap < N_BASES * (n + 1)) {
         if (ctx->w->h_bases) (void)hipHostFree(ctx->w->h_bases);
-        HIP_TRY(hipHostMalloc((void **)&ctx->w->h_bases, sizeof(uint32_t) * N_BASES * (n + 1)));
+        g_alloc_generation++;
+        HIP_TRY(hipHostMalloc((void **)&ctx->w->h_bases, sizeof(uint32_t) * N_BASES * (n + 1), hipHostMallocCoherent));
         ctx->w->h_bases_cap = N_BASES * (n + 1);
     }
     uint64_t S = 0, T = 0, W = 0, FB = 0, BW = 0, BG = 0, P = 0;
@@ -1780,13 +1785,11 @@ static void write_tables(pfh_ctx *ctx, Plan &pl, bool load_dst) {
     }
 }
 
-static void upload_tables(Workspace &w, const Plan &pl) {
+// Room for the tables on the device, where stage_clear copies them.
+static void ensure_tables(Workspace &w, const Plan &pl) {
     size_t n = pl.ids.size();
     w.scene_table.ensure(sizeof(SceneDev) * n);
     w.bases.ensure(sizeof(uint32_t) * N_BASES * (n + 1));
-    HIP_TRY(hipMemcpyAsync(w.scene_table.ptr, w.h_table, sizeof(SceneDev) * n, hipMemcpyHostToDevice, w.stream));
-    HIP_TRY(hipMemcpyAsync(w.bases.ptr, w.h_bases, sizeof(uint32_t) * N_BASES * (n + 1), hipMemcpyHostToDevice,
-                           w.stream));
 }
 
 // Where the flattener keeps its curves' bits (8 bytes a segment) between its two passes.  A fixed
@@ -1877,6 +1880,7 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
     b.entry_meta = dump ? w.entry_meta.as<uint2>() : nullptr;
     b.meta_alt = dump ? w.meta_alt.as<uint2>() : nullptr;
     b.counters = w.counters.as<uint32_t>();
+    b.counters_out = w.h_counters;
     b.dump = dump ? 1 : 0;
     b.xcd_order = pl.sched.xcd_order;
     return b;
@@ -1887,8 +1891,12 @@ static void stage_clear(Workspace &w, const BatchDev &b) {
     hipStream_t s = w.stream;
     // tile_delta / tile_cnt / col_bd need no clearing: the bin count pass stores every
     // tile and column of every binned path (paths with no columns own none)
-    // one launch for every array (no memsets: the clears are captured into graphs)
+    // one launch for every array and the scene tables (no memsets: the clears are captured into graphs)
     ZeroSpans z{};
+    const uint64_t n = (uint64_t)b.n_scenes;
+    static_assert(sizeof(SceneDev) % 4 == 0, "copied by words");
+    z.add(w.scene_table.as<uint32_t>(), sizeof(SceneDev) / 4 * n, reinterpret_cast<const uint32_t *>(w.h_table));
+    z.add(w.bases.as<uint32_t>(), N_BASES * (n + 1), w.h_bases);
     z.add(b.zbuf, b.n_fb);
     // paths with no columns are not binned: their totals and entry counts stay zero
     z.add(reinterpret_cast<uint32_t *>(b.path_tot), 2 * (uint64_t)b.n_paths);
@@ -1954,9 +1962,9 @@ static void stage_finish(Workspace &w, const BatchDev &b, const Plan &pl) {
     HIP_TRY(hipEventRecordWithFlags(w.kev[2], w.stream, hipEventRecordExternal));
 }
 
-static void read_counters(pfh_ctx *ctx) {
+static void read_counters(pfh_ctx *ctx, const BatchDev &b) {
     ctx->stats.host_syncs++;
-    HIP_TRY(hipMemcpyAsync(ctx->w->h_counters, ctx->w->counters.ptr, 4 * C_COUNT, hipMemcpyDeviceToHost, ctx->w->stream));
+    HIP_TRY(launch_publish_counters(b, ctx->w->stream));
     HIP_TRY(hipStreamSynchronize(ctx->w->stream));
 }
 
@@ -2006,7 +2014,7 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
     pl.cap_l = held.l;
     pl.cap_e = clamp_cap(std::max<uint64_t>(pl.T, 1));
     ensure_sizes(*ctx->w, pl, dump);
-    upload_tables(*ctx->w, pl);
+    ensure_tables(*ctx->w, pl);
     BatchDev b = batch_dev(*ctx->w, pl, dump);
     hipStream_t st = ctx->w->stream;
     hipEvent_t *ev = ctx->w->stage_ev;
@@ -2014,7 +2022,7 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
     stage_clear(*ctx->w, b);
     HIP_TRY(launch_flatten(b, false, flatten_chunk(pl, false), st));
     HIP_TRY(scan_chunks(b, st));
-    read_counters(ctx);  // chord count (renderer.cpp:707-724)
+    read_counters(ctx, b);  // chord count (renderer.cpp:707-724)
     uint32_t nl = ctx->w->h_counters[C_LINES];
     if (nl > pl.cap_l) {
         pl.cap_l = clamp_cap(nl);
@@ -2026,7 +2034,7 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
     HIP_TRY(launch_bin_items(b, st));
     HIP_TRY(launch_bin(b, false, st));
     HIP_TRY(scan_paths(b, st));
-    read_counters(ctx);  // fill / alpha counts (renderer.cpp:834-845)
+    read_counters(ctx, b);  // fill / alpha counts (renderer.cpp:834-845)
     HIP_TRY(hipEventRecord(ev[2], st));
     uint32_t nf = ctx->w->h_counters[C_FILLS], na = ctx->w->h_counters[C_ALPHA];
     if (nf > pl.cap_f || na > pl.cap_a) {
@@ -2054,7 +2062,8 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
     if (pl.clear_outside) HIP_TRY(launch_clear_outside(b, pl.max_rows, st));
     HIP_TRY(launch_composite(b, alt ? b.rec_alt : b.entry_rec, pl.sched.composite_block, st));
     HIP_TRY(hipEventRecord(ev[8], st));
-    read_counters(ctx);
+    ctx->stats.host_syncs++;
+    HIP_TRY(hipStreamSynchronize(st));  // the composite left the counters
     for (int i = 0; i < 8; i++) ctx->stats.ms_stage[i] += elapsed_ms(ctx, ev[i], ev[i + 1]);
     record_counts(ctx, pl, dump);
     SceneHost &s = get_scene(ctx, id);
@@ -2113,25 +2122,25 @@ static void batched_prepare(pfh_ctx *ctx, const int32_t *ids, int32_t n, uint32_
         pl.cap_f = held.f;
         pl.cap_a = held.a;
         ensure_sizes(w, pl, bl.dump);
-        upload_tables(w, pl);
+        ensure_tables(w, pl);
         BatchDev b = batch_dev(w, pl, bl.dump);
         stage_clear(w, b);
         HIP_TRY(launch_flatten(b, false, flatten_chunk(pl, false), w.stream));
         HIP_TRY(scan_chunks(b, w.stream));
-        read_counters(ctx);
+        read_counters(ctx, b);
         bl.plc = w.h_counters[C_LINES];
         pl.cap_l = clamp_cap(std::max<uint64_t>(bl.plc, pl.cap_l));
         ensure_sizes(w, pl, bl.dump);
         b = batch_dev(w, pl, bl.dump);
         stage_clear(w, b);
         stage_count(w, b, pl);
-        read_counters(ctx);
+        read_counters(ctx, b);
         bl.pf = w.h_counters[C_FILLS];
         bl.pa = w.h_counters[C_ALPHA];
     }
 }
 
-// Enqueues one attempt on the current workspace's stream and the copy of its counters;
+// Enqueues one attempt on the current workspace's stream, which ends with its counters in h_counters;
 // returns without waiting.  ev1 marks the end of the attempt.
 static void batched_enqueue(pfh_ctx *ctx, BatchedLaunch &bl) {
     Workspace &w = *ctx->w;
@@ -2152,7 +2161,7 @@ static void batched_enqueue(pfh_ctx *ctx, BatchedLaunch &bl) {
         pl.cap_a = held.a;
         ensure_sizes(w, pl, bl.dump);
     }
-    upload_tables(w, pl);
+    ensure_tables(w, pl);
     BatchDev b = batch_dev(w, pl, bl.dump);
     HIP_TRY(hipEventRecord(w.ev0, w.stream));
     if (bl.use_graph) {
@@ -2207,7 +2216,6 @@ static void batched_enqueue(pfh_ctx *ctx, BatchedLaunch &bl) {
         stage_emit(w, b, pl);
         stage_finish(w, b, pl);
     }
-    HIP_TRY(hipMemcpyAsync(w.h_counters, w.counters.ptr, 4 * C_COUNT, hipMemcpyDeviceToHost, w.stream));
     HIP_TRY(hipEventRecord(w.ev1, w.stream));
 }
 
