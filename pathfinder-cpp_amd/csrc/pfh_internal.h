@@ -83,7 +83,7 @@ constexpr uint32_t SEG_ORIGINAL_SHIFT = 16;  // the kind again, kept where nothi
 struct Schedule {
     uint32_t fill_grid = 16384;       // max workgroups of k_fill_masks (grid-stride beyond)
     uint32_t composite_block = 256;   // threads per k_composite workgroup (a wave per fb tile)
-    uint32_t column_block = 256;      // threads per workgroup of k_propagate / k_entries
+    uint32_t column_block = 256;      // threads per workgroup of k_propagate (batches with clip paths)
     uint32_t xcd_order = 0;           // bit 0 fill, bit 1 composite: workgroups grouped per XCD
     // flatten_*: kept for callers that set them; a flattener wave takes at most one segment per lane
     // and its lanes share every curve's pieces, so there is nothing left to choose
@@ -259,9 +259,11 @@ struct BatchDev {
     uint32_t paints;              // some scene of the batch has gradient paints
     uint32_t cap_vis;             // alpha_vis capacity: cap_alpha, or with clip paths the larger of it and
                                   // cap_entries (solid tiles of several paths can take one clip mask)
-    int32_t *tile_delta;          // [T] backdrop delta (int8 arithmetic, stored widened)
+    int32_t *tile_delta;          // [T] with clip paths the backdrop delta (int8 arithmetic, stored widened), else
+                                  // the propagated backdrop of the tiles with fills
     uint32_t *tile_cnt;           // [T] fills per tile (global-atomic paths: then emit cursor)
-    uint32_t *tile_fill_off;      // [T + 1] exclusive scan of fill counts
+    uint32_t *tile_fill_off;      // [T + 1] exclusive scan of fill counts (all of it with clip paths or dumps, else
+                                  // where fills are placed through it)
     uint32_t *tile_alpha_idx;     // [T + 1] exclusive scan of alpha flags
     int8_t *tile_bd;              // [T] propagated backdrop (written with dumps or clip paths only)
     uint32_t *tile_clip_ai;       // [T] with clip paths: mask row of a TILE_CLIP_MASK tile; for a clip
@@ -280,7 +282,7 @@ struct BatchDev {
     uint2 *path_tot;              // [P + 1] {fills, alpha tiles} per batch path, then exclusive scan
     BinItem *bin_items;           // [n_bin_wave + n_bin_group] wave class, then group class
     uint32_t *col_item;           // [W] the bin item owning each column
-    int32_t *col_bd;              // [W] above-rect backdrop, then final column sum
+    int32_t *col_bd;              // [W] above-rect backdrop, then final column sum (with clip paths or dumps)
     uint32_t *tall_cols;          // [W] columns of the current propagate phase walked by several lanes:
                                   // the C_MID list from the front, the C_TALL list from the back
     uint32_t *seg_cnt;            // [S + 1] stream points per segment (flatten count), then their offsets (flatten

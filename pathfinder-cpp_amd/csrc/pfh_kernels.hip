@@ -818,9 +818,69 @@ __device__ __forceinline__ U2 wave_sum_u2(U2 v) {
     return v;
 }
 
-// Inclusive prefix sums of (count, count > 0) across the wave.
+// Mask rows per alpha tile: 2 for a clip path's tiles, whose coverage is kept under both fill rules.
 __device__ __forceinline__ uint32_t alpha_rows(const BinItem &it) { return it.level != 0 ? 2u : 1u; }
 
+// Backdrops, tile status and z-buffer (core/d3d9/tiler.cpp:369-439) of a path without clip paths in
+// its batch, at the end of its count pass, whose counts and deltas are still in LDS: a column's backdrop
+// is its running sum from the step above the rect down, which resolve_columns puts in the deltas'
+// place.  (With clip paths a tile also depends on its clip's: k_propagate, after the emit pass.)
+// As a walk of its own down the batch's columns, a thread each, this took 155 us for 48 scenes (20
+// million tiles), 30 us at 4096^2 and 25 us at 1240 x 1754, where it waited 14 times for a group of rows;
+// the count pass is longer instead: 367 -> 424 us, 65 -> 81 and 30 -> 32 (the emit pass as long as before).
+// A thread per column, 8 rows at a time: each group's reads go out before the first is used.  (Several
+// threads to a column where the rect is narrower than the block, with a sum pass before: no faster, and
+// 189 -> 209 us for the wave class of the 48 scenes.)
+template <int N, typename D>
+__device__ __forceinline__ void resolve_columns(const BatchDev &b, const BinItem &it, uint32_t tw, uint32_t th,
+                                                D *delta, int32_t bias, const int32_t *col, uint32_t t) {
+    for (uint32_t x = t; x < tw; x += N) {
+        int32_t run = col[x];
+        for (uint32_t r0 = 0; r0 < th; r0 += 8) {
+            int32_t d[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++) d[i] = r0 + i < th ? (int32_t)delta[(r0 + i) * tw + x] - bias : 0;
+#pragma unroll
+            for (uint32_t i = 0; i < 8; i++) {
+                if (r0 + i < th) delta[(r0 + i) * tw + x] = (D)((int32_t)(int8_t)run + bias);
+                run += (int8_t)d[i];
+            }
+        }
+        if (b.dump) b.col_bd[it.cbase + x] = run;
+    }
+}
+
+// Tile j of the rect (row-major, tw wide), its fills and backdrop known: its status, and for an opaque
+// solid tile the z-buffer.  An alpha tile's backdrop waits in tile_delta for its mask record, which the
+// emit pass writes once it knows the tile's place (store_tile_offset).
+__device__ __forceinline__ void resolve_tile(const BatchDev &b, const BinItem &it, const SceneDev &sc, uint32_t tw,
+                                             float inv_w, uint32_t j, uint32_t fills, int32_t bd) {
+    const uint32_t t = it.tbase + j;
+    const bool clear = (it.rule & 1u) && (bd & 1) == 0;
+    b.tile_st[t] = fills ? TILE_ALPHA : (bd == 0 ? TILE_EMPTY : (clear ? TILE_CLEAR : TILE_SOLID));
+    if (b.dump) b.tile_bd[t] = (int8_t)bd;
+    if (fills) {
+        b.tile_delta[t] = bd;
+    } else if ((it.rgba >> 24) == 255u && bd != 0 && !clear) {
+        uint32_t row = (uint32_t)((float)j * inv_w);  // off by at most one below 2^24 tiles
+        if (row * tw > j) row--;
+        else if ((row + 1) * tw <= j) row++;
+        const int x = it.rect.x - sc.fb_x0 + (int)(j - row * tw), y = it.rect.y - sc.fb_y0 + (int)row;
+        atomicMax(&b.zbuf[sc.fb_base + (uint32_t)(y * sc.fb_w + x)], it.p);
+    }
+}
+
+// Emit pass: where tile t's fills start (`fills` of them) and its mask row.  bd: its tile_delta, read
+// beside the counts (anything where it has no fills).  cursors: the fills are placed through tile_fill_off.
+__device__ __forceinline__ void store_tile_offset(const BatchDev &b, const BinItem &it, uint32_t t, uint32_t off,
+                                                  uint32_t fills, uint32_t ai, int32_t bd, bool cursors) {
+    if (b.has_clips || b.dump || cursors) b.tile_fill_off[t] = off;  // dumps read it back
+    b.tile_alpha_idx[t] = ai;  // all: whole lines (stored for alpha tiles alone, the entry pass 26 -> 34 us at 4096^2)
+    if (!b.has_clips && fills && ai < b.cap_alpha)
+        b.alpha_rec[ai] = make_uint4(off, off + fills, (uint32_t)(uint8_t)bd | ((it.rule & 1u) << 8), t);
+}
+
+// Inclusive prefix sums of (count, count > 0) across the wave.
 __device__ __forceinline__ U2 wave_inclusive_u2(uint32_t c) {
     U2 v{c, c > 0 ? 1u : 0u};
     const int lane = threadIdx.x & 63;
@@ -834,19 +894,19 @@ __device__ __forceinline__ U2 wave_inclusive_u2(uint32_t c) {
 
 // Wave: tile offsets of a rect of `area` tiles (counts in cnt_src, global) from the path's
 // scanned base; offsets go to the tile arrays and, when given, to the LDS cursors.
-// aw: mask rows per alpha tile (2 for a clip path's tiles, whose coverage is kept under both
-// fill rules; 1 otherwise).
-__device__ __forceinline__ void wave_tile_offsets(const BatchDev &b, uint32_t tbase, uint32_t area, U2 base,
-                                                  uint32_t *l_cur, uint32_t aw) {
+// Without clip paths the tiles' masks are complete here: see resolve_tile.
+__device__ __forceinline__ void wave_tile_offsets(const BatchDev &b, const BinItem &it, uint32_t area, U2 base,
+                                                  uint32_t *l_cur) {
+    const uint32_t tbase = it.tbase, aw = alpha_rows(it);
     const uint32_t lane = threadIdx.x & 63;
     for (uint32_t j0 = 0; j0 < area; j0 += 64) {
         const uint32_t j = j0 + lane;
         const uint32_t c = j < area ? b.tile_cnt[tbase + j] : 0u;
+        const int32_t bd = j < area ? b.tile_delta[tbase + j] : 0;
         const U2 inc = wave_inclusive_u2(c);
         if (j < area) {
-            const uint32_t off = base.x + inc.x - c, ai = base.y + aw * (inc.y - (c > 0 ? 1u : 0u));
-            b.tile_fill_off[tbase + j] = off;
-            b.tile_alpha_idx[tbase + j] = ai;
+            const uint32_t off = base.x + inc.x - c;
+            store_tile_offset(b, it, tbase + j, off, c, base.y + aw * (inc.y - (c > 0 ? 1u : 0u)), bd, l_cur == nullptr);
             if (l_cur) l_cur[j] = off;
         }
         base = base + U2{__shfl(inc.x, 63, 64), aw * __shfl(inc.y, 63, 64)};
@@ -855,16 +915,17 @@ __device__ __forceinline__ void wave_tile_offsets(const BatchDev &b, uint32_t tb
 
 // Block version, called by every thread of a block of THREADS.
 template <int THREADS>
-__device__ __forceinline__ void block_tile_offsets(const BatchDev &b, uint32_t tbase, uint32_t area, U2 base,
-                                                   uint32_t *l_cur, uint32_t aw) {
+__device__ __forceinline__ void block_tile_offsets(const BatchDev &b, const BinItem &it, uint32_t area, U2 base,
+                                                   uint32_t *l_cur) {
+    const uint32_t tbase = it.tbase, aw = alpha_rows(it);
     for (uint32_t j0 = 0; j0 < area; j0 += THREADS) {
         const uint32_t j = j0 + threadIdx.x;
         const uint32_t c = j < area ? b.tile_cnt[tbase + j] : 0u;
+        const int32_t bd = j < area ? b.tile_delta[tbase + j] : 0;
         U2 tot;
         const U2 ex = block_exclusive_scan<U2, THREADS>(U2{c, c > 0 ? 1u : 0u}, tot);
         if (j < area) {
-            b.tile_fill_off[tbase + j] = base.x + ex.x;
-            b.tile_alpha_idx[tbase + j] = base.y + aw * ex.y;
+            store_tile_offset(b, it, tbase + j, base.x + ex.x, c, base.y + aw * ex.y, bd, l_cur == nullptr);
             if (l_cur) l_cur[j] = base.x + ex.x;
         }
         base = base + U2{tot.x, aw * tot.y};
@@ -916,7 +977,8 @@ __global__ __launch_bounds__(256) void k_bin_items(BatchDev b, uint32_t wave_blo
     const uint32_t gi = (grp ? b.n_bin_wave : 0u) + i;
     b.bin_items[gi] = it;
     const uint32_t tw = (uint32_t)max(it.rect.z - it.rect.x, 0);
-    for (uint32_t j = 0; j < tw; j++) b.col_item[it.cbase + j] = gi;
+    if (b.has_clips)  // for k_propagate, which takes columns
+        for (uint32_t j = 0; j < tw; j++) b.col_item[it.cbase + j] = gi;
 }
 
 // LDS of a bin block: its path's arrays (group class), or a slice per wave (wave class).
@@ -957,7 +1019,7 @@ __device__ __forceinline__ void bin_wave(const BatchDev &b, Lds &lds, uint32_t i
     const uint32_t gp = it.gp;
     if (EMIT) {
         const uint2 base = b.path_tot[gp];
-        wave_tile_offsets(b, tbase, area, U2{base.x, base.y}, l_cnt, alpha_rows(it));
+        wave_tile_offsets(b, it, area, U2{base.x, base.y}, l_cnt);
     } else {
         for (uint32_t j = lane; j < area; j += 64) {
             l_cnt[j] = 0;
@@ -969,14 +1031,22 @@ __device__ __forceinline__ void bin_wave(const BatchDev &b, Lds &lds, uint32_t i
     walk_chords<EMIT, true>(b, sc, rect, tbase, cbase, l_cnt, l_delta, l_col, it.c0, it.c1, lane, 64, lds[wv].queue);
     if (!EMIT) {
         wave_sync();
+        const bool resolve = !b.has_clips;
+        if (resolve) {
+            resolve_columns<64>(b, it, tw, th, l_delta, 0, l_col, lane);
+            wave_sync();
+        }
+        const float inv_w = 1.0f / (float)(int)tw;
         U2 tot{0, 0};
         for (uint32_t j = lane; j < area; j += 64) {
             const uint32_t c = l_cnt[j];
             b.tile_cnt[tbase + j] = c;
-            b.tile_delta[tbase + j] = l_delta[j];
+            if (resolve) resolve_tile(b, it, sc, tw, inv_w, j, c, l_delta[j]);
+            else b.tile_delta[tbase + j] = l_delta[j];
             tot = tot + U2{c, c > 0 ? 1u : 0u};
         }
-        for (uint32_t j = lane; j < tw; j += 64) b.col_bd[cbase + j] = l_col[j];
+        if (!resolve)
+            for (uint32_t j = lane; j < tw; j += 64) b.col_bd[cbase + j] = l_col[j];
         tot = wave_sum_u2(tot);
         if (lane == 0) b.path_tot[gp] = make_uint2(tot.x, tot.y * alpha_rows(it));
     }
@@ -997,13 +1067,15 @@ __device__ __forceinline__ void bin_group(const BatchDev &b, Lds &lds, uint32_t 
     uint32_t *const s_cnt = lds.cnt, *const s_delta = lds.delta;
     int32_t *const s_col = lds.col;
     uint32_t *const queue = lds.queue[threadIdx.x >> 6];
+    const bool resolve = !EMIT && !b.has_clips;
+    const float inv_w = 1.0f / (float)(int)tw;
     // the packed LDS deltas hold sums below 2^15 in magnitude: at most one step per chord
     const bool in_lds = area <= (uint32_t)BIN_GROUP_TILES && tw <= (uint32_t)BIN_GROUP_COLS &&
                         (EMIT || c1 - c0 < (1u << 15));
     if (in_lds) {
         if (EMIT) {
             const uint2 base = b.path_tot[gp];
-            block_tile_offsets<THREADS>(b, tbase, area, U2{base.x, base.y}, s_cnt, alpha_rows(it));
+            block_tile_offsets<THREADS>(b, it, area, U2{base.x, base.y}, s_cnt);
         } else {
             for (uint32_t j = threadIdx.x; j < area; j += THREADS) s_cnt[j] = 0;
             for (uint32_t j = threadIdx.x; j < (area + 1) / 2; j += THREADS) s_delta[j] = 0x80008000u;
@@ -1014,21 +1086,30 @@ __device__ __forceinline__ void bin_group(const BatchDev &b, Lds &lds, uint32_t 
                                       c0, c1, threadIdx.x, THREADS, queue);
         if (!EMIT) {
             __syncthreads();
+            typedef uint16_t __attribute__((may_alias)) Half;
+            Half *const half = reinterpret_cast<Half *>(s_delta);  // tile j's delta, biased
+            if (resolve) {
+                resolve_columns<THREADS>(b, it, tw, th, half, 0x8000, s_col, threadIdx.x);
+                __syncthreads();
+            }
             U2 tot{0, 0};
             for (uint32_t j = threadIdx.x; j < area; j += THREADS) {
                 const uint32_t c = s_cnt[j];
+                const int32_t d = (int32_t)half[j] - 0x8000;
                 b.tile_cnt[tbase + j] = c;
-                b.tile_delta[tbase + j] = (int32_t)((s_delta[j >> 1] >> (16 * (j & 1))) & 0xffffu) - 0x8000;
+                if (resolve) resolve_tile(b, it, sc, tw, inv_w, j, c, d);
+                else b.tile_delta[tbase + j] = d;
                 tot = tot + U2{c, c > 0 ? 1u : 0u};
             }
-            for (uint32_t j = threadIdx.x; j < tw; j += THREADS) b.col_bd[cbase + j] = s_col[j];
+            if (!resolve)
+                for (uint32_t j = threadIdx.x; j < tw; j += THREADS) b.col_bd[cbase + j] = s_col[j];
             tot = block_sum_u2<THREADS>(tot, reinterpret_cast<U2 *>(s_col));
             if (threadIdx.x == 0) b.path_tot[gp] = make_uint2(tot.x, tot.y * alpha_rows(it));
         }
     } else {
         if (EMIT) {
             const uint2 base = b.path_tot[gp];
-            block_tile_offsets<THREADS>(b, tbase, area, U2{base.x, base.y}, nullptr, alpha_rows(it));
+            block_tile_offsets<THREADS>(b, it, area, U2{base.x, base.y}, nullptr);
             __threadfence();  // the offsets reach L2 before any thread reads them back
             __syncthreads();
         }
@@ -1047,9 +1128,33 @@ __device__ __forceinline__ void bin_group(const BatchDev &b, Lds &lds, uint32_t 
             __threadfence();  // every thread's atomics are done before the counts are summed
             __syncthreads();
             U2 tot{0, 0};
-            for (uint32_t j = threadIdx.x; j < area; j += THREADS) {
-                const uint32_t c = __hip_atomic_load(&b.tile_cnt[tbase + j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                tot = tot + U2{c, c > 0 ? 1u : 0u};
+            auto read = [](const auto *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+            if (resolve) {
+                for (uint32_t x = threadIdx.x; x < tw; x += THREADS) {  // a thread per column, 8 rows at a time
+                    int32_t run = read(&b.col_bd[cbase + x]);
+                    for (uint32_t r0 = 0; r0 < th; r0 += 8) {
+                        int32_t d[8];
+                        uint32_t c[8];
+#pragma unroll
+                        for (uint32_t i = 0; i < 8; i++) {
+                            const uint32_t t = tbase + (r0 + i) * tw + x;
+                            d[i] = r0 + i < th ? read(&b.tile_delta[t]) : 0;
+                            c[i] = r0 + i < th ? read(&b.tile_cnt[t]) : 0u;
+                        }
+#pragma unroll
+                        for (uint32_t i = 0; i < 8; i++) {
+                            if (r0 + i < th) resolve_tile(b, it, sc, tw, inv_w, (r0 + i) * tw + x, c[i], (int8_t)run);
+                            run += (int8_t)d[i];
+                            tot = tot + U2{c[i], c[i] > 0 ? 1u : 0u};
+                        }
+                    }
+                    if (b.dump) b.col_bd[cbase + x] = run;
+                }
+            } else {
+                for (uint32_t j = threadIdx.x; j < area; j += THREADS) {
+                    const uint32_t c = read(&b.tile_cnt[tbase + j]);
+                    tot = tot + U2{c, c > 0 ? 1u : 0u};
+                }
             }
             tot = block_sum_u2<THREADS>(tot, reinterpret_cast<U2 *>(s_col));  // s_col is unused on this path
             if (threadIdx.x == 0) b.path_tot[gp] = make_uint2(tot.x, tot.y * alpha_rows(it));
@@ -1059,9 +1164,9 @@ __device__ __forceinline__ void bin_group(const BatchDev &b, Lds &lds, uint32_t 
 
 // Both classes in one launch, the group class's paths first (they last longest).  512 threads: a long
 // path's walk is twice as wide as with 256, and 8 wave-class slices (40 KB in the count pass) leave the
-// wave class its 32 waves per CU.
+// wave class its 32 waves per CU (which the compiler is held to: 83 -> 80 us at 4096^2 against 7 a SIMD).
 template <bool EMIT>
-__global__ __launch_bounds__(512) void k_bin(BatchDev b) {
+__global__ __launch_bounds__(512, 8) void k_bin(BatchDev b) {
     __shared__ BinLds<EMIT, 512> lds;
     if (blockIdx.x < b.n_bin_group) {  // uniform over the block
         bin_group<EMIT, 512>(b, lds.g, blockIdx.x);
@@ -1332,11 +1437,11 @@ __device__ __forceinline__ ClipTile clip_tile_at(const BatchDev &b, const BinIte
 // tile at the same coordinates: outside its rect or over a blank tile -> culled; both with masks ->
 // a combine job (the tile's backdrop moves into it); a solid tile over a mask -> it takes that
 // mask; otherwise unchanged (a solid clip tile passes the tile through).
-// phase 0: every column (no clip paths in the batch); 1..MAX_CLIP_LEVELS: the columns of clip paths
+// Only in batches with clip paths (else the count pass does all of it: resolve_columns).
+// phase 1..MAX_CLIP_LEVELS: the columns of clip paths
 // of that level, a clip path nested in another being resolved against it like a draw path (the
 // level structure of core/d3d11/scene_builder.cpp:92-133, shaders/d3d11/propagate.comp:133-176);
 // MAX_CLIP_LEVELS + 1: the draw paths' columns.  Each phase reads only tiles of earlier phases.
-// CLIPS: the batch has clip paths (without them the kernel is the plain per-column walk).
 // What a tile of a path column reads of its clip path: the clip's tile at the same coordinates
 // and, for a clip path's tile over a clip mask, the chain record of that mask.  Both were written
 // by an earlier propagate phase, so a column loads them for a group of rows before it stores
@@ -1353,12 +1458,11 @@ __device__ __forceinline__ ClipRead clip_read(const BatchDev &b, const ColumnWal
 }
 
 // One tile of a path column, its propagated backdrop bd and its fill range [f0, f1) known (ai: its
-// mask row when it has fills), with what it reads of its clip path (CLIPS).
-template <bool CLIPS>
+// mask row when it has fills), with what it reads of its clip path.
 __device__ __forceinline__ void propagate_tile(const BatchDev &b, const ColumnWalk &cw, const ClipRead &cr, int row,
                                                int8_t bd, uint32_t f0, uint32_t f1, uint32_t ai) {
-    const bool is_clip = CLIPS && cw.level != 0;
-    const bool clipped = CLIPS && (cw.clip < CLIP_EMPTY || cw.clip == CLIP_EMPTY);
+    const bool is_clip = cw.level != 0;
+    const bool clipped = cw.clip < CLIP_EMPTY || cw.clip == CLIP_EMPTY;
     const bool opaque = (cw.rgba >> 24) == 255u;
     const uint32_t t = cw.tile(row);
     const bool alpha = f1 > f0;
@@ -1366,9 +1470,9 @@ __device__ __forceinline__ void propagate_tile(const BatchDev &b, const ColumnWa
     // Whether the tile covers without fills: backdrop != 0, except under the path's own even-odd
     // rule with an even backdrop where clip paths' own rules are taken (PFH_CLIP_RULE_OWN); the
     // reference's clip resolution tests backdrop != 0 alone (tiler.cpp:396-431).
-    const bool covers = bd != 0 && !(CLIPS && cw.own_rules && cw.rule && (bd & 1) == 0);
-    const uint32_t job_rules = CLIPS && cw.own_rules ? CLIP_JOB_OWN_RULES : 0u;
-    if (CLIPS && is_clip) {
+    const bool covers = bd != 0 && !(cw.own_rules && cw.rule && (bd & 1) == 0);
+    const uint32_t job_rules = cw.own_rules ? CLIP_JOB_OWN_RULES : 0u;
+    if (is_clip) {
         // A clip path draws nothing itself.  Its fills make two mask rows (ai, ai + 1) that
         // keep |sum + backdrop| under the nonzero and the even-odd rule (under its own rule,
         // both, where clip paths' own rules are taken), for the tiles that take them over; its
@@ -1406,7 +1510,7 @@ __device__ __forceinline__ void propagate_tile(const BatchDev &b, const ColumnWa
         b.tile_bd[t] = out_bd;
         return;
     }
-    if (CLIPS && clipped) {
+    if (clipped) {
         if (alpha && ai < b.cap_alpha)
             b.alpha_rec[ai] = make_uint4(f0, f1, (uint32_t)(uint8_t)bd | (cw.rule << 8), t);
         uint8_t st;
@@ -1448,21 +1552,20 @@ __device__ __forceinline__ void propagate_tile(const BatchDev &b, const ColumnWa
 // tile at the same coordinates: outside its rect or over a blank tile -> culled; both with masks ->
 // a combine job (the tile's backdrop moves into it); a solid tile over a mask -> it takes that
 // mask; otherwise unchanged (a solid clip tile passes the tile through).
-// phase 0: every column (no clip paths in the batch); 1..MAX_CLIP_LEVELS: the columns of clip paths
+// Only in batches with clip paths (else the count pass does all of it: resolve_columns).
+// phase 1..MAX_CLIP_LEVELS: the columns of clip paths
 // of that level, a clip path nested in another being resolved against it like a draw path (the
 // level structure of core/d3d11/scene_builder.cpp:92-133, shaders/d3d11/propagate.comp:133-176);
 // MAX_CLIP_LEVELS + 1: the draw paths' columns.  Each phase reads only tiles of earlier phases.
-// CLIPS: the batch has clip paths (without them the kernel is the plain per-column walk).
 // A thread walks its column: rows of neighbouring columns are neighbours in memory, so the
 // wave's loads coalesce.  A walk is a chain of dependent loads per group of rows, and a launch
 // lasts as long as its longest walk: a column of more than `rows` tiles (a schedule choice) is
 // listed instead for k_propagate_rows, which spreads its rows over 16 or 64 lanes (rows 0: none).
-template <bool CLIPS>
 __global__ __launch_bounds__(256) void k_propagate(BatchDev b, uint32_t phase, uint32_t rows) {
     uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= b.n_cols) return;
     const ColumnWalk cw(b, c);
-    if (CLIPS && cw.level != (phase > MAX_CLIP_LEVELS ? 0u : phase)) return;
+    if (cw.level != (phase > MAX_CLIP_LEVELS ? 0u : phase)) return;
     if (rows != 0 && (uint32_t)cw.h > rows) {
         // at most one entry per column and phase, so the two lists together hold at most n_cols
         if (cw.h > TALL_ROWS) b.tall_cols[b.n_cols - 1 - atomicAdd(&b.counters[C_TALL + phase], 1u)] = c;
@@ -1470,7 +1573,7 @@ __global__ __launch_bounds__(256) void k_propagate(BatchDev b, uint32_t phase, u
         return;
     }
     BinItem ci;
-    if (CLIPS && cw.clip < CLIP_EMPTY) ci = b.bin_items[cw.clip];
+    if (cw.clip < CLIP_EMPTY) ci = b.bin_items[cw.clip];
     int32_t running = b.col_bd[c];
     for (int row0 = 0; row0 < cw.h; row0 += COL_ROWS) {
         int32_t delta[COL_ROWS];
@@ -1494,15 +1597,15 @@ __global__ __launch_bounds__(256) void k_propagate(BatchDev b, uint32_t phase, u
             bd[i] = (int8_t)running;
             running += (int8_t)delta[i];
             ai[i] = 0;
-            // with clip paths the group's loads go out at once (the walk is latency-bound there)
-            if (row0 + i < cw.h && (CLIPS || f1[i] > f0[i])) ai[i] = b.tile_alpha_idx[cw.tile(row0 + i)];
+            // the group's loads go out at once (the walk is latency-bound)
+            if (row0 + i < cw.h) ai[i] = b.tile_alpha_idx[cw.tile(row0 + i)];
             cr[i] = ClipRead{{false, false, false, 0, 0}, make_uint4(1u, 0u, 0u, 0u)};
-            if (CLIPS && row0 + i < cw.h) cr[i] = clip_read(b, cw, ci, row0 + i);
+            if (row0 + i < cw.h) cr[i] = clip_read(b, cw, ci, row0 + i);
         }
 #pragma unroll
         for (int i = 0; i < COL_ROWS; i++) {
             if (row0 + i >= cw.h) break;
-            propagate_tile<CLIPS>(b, cw, cr[i], row0 + i, bd[i], f0[i], f1[i], ai[i]);
+            propagate_tile(b, cw, cr[i], row0 + i, bd[i], f0[i], f1[i], ai[i]);
         }
     }
     b.col_bd[c] = running;
@@ -1513,7 +1616,7 @@ __global__ __launch_bounds__(256) void k_propagate(BatchDev b, uint32_t phase, u
 // backdrop deltas across them gives each row the backdrop the serial walk reaches there (the int8
 // deltas summed in int32, as the walk does).  Every wave strides over the list (its length is
 // only known on the device), 64 / SUB columns at a time.
-template <bool CLIPS, int SUB>
+template <int SUB>
 __global__ __launch_bounds__(256) void k_propagate_rows(BatchDev b, uint32_t phase) {
     constexpr uint32_t G = 64 / SUB;  // columns per wave
     const uint32_t n = min(b.counters[(SUB == 64 ? C_TALL : C_MID) + phase], b.n_cols);
@@ -1526,7 +1629,7 @@ __global__ __launch_bounds__(256) void k_propagate_rows(BatchDev b, uint32_t pha
         const ColumnWalk cw(b, c);
         const int h = has ? cw.h : 0;
         BinItem ci;
-        if (CLIPS && has && cw.clip < CLIP_EMPTY) ci = b.bin_items[cw.clip];
+        if (has && cw.clip < CLIP_EMPTY) ci = b.bin_items[cw.clip];
         int32_t running = has ? b.col_bd[c] : 0;
         int hmax = h;
 #pragma unroll
@@ -1543,7 +1646,7 @@ __global__ __launch_bounds__(256) void k_propagate_rows(BatchDev b, uint32_t pha
                 f0 = b.tile_fill_off[t];
                 f1 = b.tile_fill_off[t + 1];
                 ai = b.tile_alpha_idx[t];
-                if (CLIPS) cr = clip_read(b, cw, ci, row);
+                cr = clip_read(b, cw, ci, row);
             }
             uint32_t incl;
             if (SUB == 16) {
@@ -1556,7 +1659,7 @@ __global__ __launch_bounds__(256) void k_propagate_rows(BatchDev b, uint32_t pha
                     if (lane >= d) incl += o;
                 }
             }
-            if (on) propagate_tile<CLIPS>(b, cw, cr, row, (int8_t)(running + (int32_t)(incl - (uint32_t)d8)), f0, f1, ai);
+            if (on) propagate_tile(b, cw, cr, row, (int8_t)(running + (int32_t)(incl - (uint32_t)d8)), f0, f1, ai);
             running += (int32_t)__shfl(incl, g * SUB + SUB - 1, 64);
         }
         if (has && li == 0) b.col_bd[c] = running;
@@ -2157,30 +2260,25 @@ hipError_t launch_bin(const BatchDev &b, bool emit, hipStream_t s) {
 }
 
 // rows: columns of more tiles are walked by several lanes each (1..64; 0: none)
-template <bool CLIPS>
 static void propagate_phase(const BatchDev &b, uint32_t block, uint32_t rows, uint32_t phase, hipStream_t s) {
-    hipLaunchKernelGGL(k_propagate<CLIPS>, dim3(blocks_for(b.n_cols, block)), dim3(block), 0, s, b, phase, rows);
+    hipLaunchKernelGGL(k_propagate, dim3(blocks_for(b.n_cols, block)), dim3(block), 0, s, b, phase, rows);
     if (rows == 0) return;
     // the listed columns' waves: enough to cover the device, striding over lists of unknown length
     if (rows < (uint32_t)TALL_ROWS)
-        hipLaunchKernelGGL((k_propagate_rows<CLIPS, 16>), dim3(std::min<uint32_t>(blocks_for(b.n_cols, 16), 2048)),
+        hipLaunchKernelGGL(k_propagate_rows<16>, dim3(std::min<uint32_t>(blocks_for(b.n_cols, 16), 2048)),
                            dim3(256), 0, s, b, phase);
-    hipLaunchKernelGGL((k_propagate_rows<CLIPS, 64>), dim3(std::min<uint32_t>(blocks_for(b.n_cols, 4), 2048)),
+    hipLaunchKernelGGL(k_propagate_rows<64>, dim3(std::min<uint32_t>(blocks_for(b.n_cols, 4), 2048)),
                        dim3(256), 0, s, b, phase);
 }
 
 hipError_t launch_propagate(const BatchDev &b, uint32_t block, uint32_t rows, hipStream_t s) {
-    if (b.n_cols == 0) return hipSuccess;
     if (block != 64 && block != 128 && block != 256) return hipErrorInvalidValue;
     if (rows > (uint32_t)TALL_ROWS) return hipErrorInvalidValue;
-    if (!b.has_clips) {
-        propagate_phase<false>(b, block, rows, 0u, s);
-    } else {
-        // clip levels from the outermost in, then the draw paths
-        for (uint32_t level = 1; level <= std::min(b.clip_levels, MAX_CLIP_LEVELS); level++)
-            propagate_phase<true>(b, block, rows, level, s);
-        propagate_phase<true>(b, block, rows, MAX_CLIP_LEVELS + 1, s);
-    }
+    if (b.n_cols == 0 || !b.has_clips) return hipSuccess;
+    // clip levels from the outermost in, then the draw paths
+    for (uint32_t level = 1; level <= std::min(b.clip_levels, MAX_CLIP_LEVELS); level++)
+        propagate_phase(b, block, rows, level, s);
+    propagate_phase(b, block, rows, MAX_CLIP_LEVELS + 1, s);
     return hipGetLastError();
 }
 

@@ -1889,8 +1889,8 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
 // Stage groups; every launch goes to ctx->w->stream so the batched sequence can be captured.
 static void stage_clear(Workspace &w, const BatchDev &b) {
     hipStream_t s = w.stream;
-    // tile_delta / tile_cnt / col_bd need no clearing: the bin count pass stores every
-    // tile and column of every binned path (paths with no columns own none)
+    // the tile and column arrays need no clearing: the bin passes store what is read of every
+    // binned path's (paths with no columns own none)
     // one launch for every array and the scene tables (no memsets: the clears are captured into graphs)
     ZeroSpans z{};
     const uint64_t n = (uint64_t)b.n_scenes;

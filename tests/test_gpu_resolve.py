@@ -1,0 +1,49 @@
+"""Backdrops, tile status and z-buffer from the count pass (batches without clip paths) and from the
+column walk (batches with one): the oracle's tiles drawn alone, and the same dump, bit for bit, drawn
+beside a scene with clip paths.  Rects one tile wide and one tile high, heights on both sides of the 8-row
+groups, more columns than a wave or a block has threads, rects beyond LDS, opaque and even-odd paths, and
+windings past int8."""
+import numpy as np
+import pytest
+
+import oracle
+import pfh
+import scenegen
+from test_gpu_parity import check_scene
+
+pytestmark = pytest.mark.gpu
+
+
+def rects(boxes, w, h, turns=1):
+    """A path per (x, y, width, height) box, its outline traced `turns` times; opaque and not, both rules."""
+    n = len(boxes)
+    pts = np.concatenate([np.tile([[x, y], [x + bw, y + 0.25], [x + bw - 0.5, y + bh], [x + 0.25, y + bh - 0.5]],
+                                  (turns, 1)) for x, y, bw, bh in boxes]).astype(np.float32)
+    a = np.array([(0xff if i % 3 else 0x80) << 24 | 0x203040 * (i + 1) & 0xffffff for i in range(n)], np.uint32)
+    return scenegen.Scene(w, h, pts, np.zeros(len(pts), np.uint8), np.arange(n + 1) * 4 * turns, np.ones(n, np.uint8),
+                          np.arange(n + 1), np.arange(n) // 2 % 2, a)
+
+
+SCENES = [
+    ("thin", rects([(3, 2, 20, 16 * k) for k in (1, 7, 8, 9, 40, 300)], 64, 5000)),
+    ("flat", rects([(1, 5, 16 * k, 20) for k in (1, 63, 64, 65, 128, 129, 600)], 9700, 48)),
+    ("wave and group", rects([(7, 9, 350, 350), (5, 5, 360, 380), (2, 3, 700, 16 * 8), (0, 0, 900, 900)], 1000, 1000)),
+    ("beyond lds", rects([(4, 4, 1100, 1120), (40, 9, 16 * 68, 16 * 67)], 1200, 1200)),
+    ("windings", rects([(8, 8, 200, 150), (60, 20, 500, 500)], 640, 640, turns=130)),
+]
+
+
+@pytest.mark.parametrize("name,sc", SCENES)
+def test_tiles_from_the_count_pass_and_the_column_walk(name, sc):
+    ctx = pfh.Context(0)
+    alone, img = check_scene(ctx, sc, name=name)
+    ids = [ctx.upload(sc), ctx.upload(scenegen.clip_scene(3, size=256, n_draw=20, n_clip=3))]
+    ctx.rasterize(ids, pfh.PFH_BATCHED | pfh.PFH_NO_GRAPH | pfh.PFH_DUMP)
+    beside = ctx.dump(ids[0])
+    for k in oracle.CANONICAL_KEYS + ("masks",):
+        np.testing.assert_array_equal(beside[k], alone[k], err_msg=k)
+    np.testing.assert_array_equal(ctx.readback(ids[0]), img)
+    for flags in (pfh.PFH_PLAIN, pfh.PFH_BATCHED | pfh.PFH_NO_GRAPH, pfh.PFH_BATCHED):
+        ctx.rasterize(ids[:1], flags)
+        np.testing.assert_array_equal(ctx.readback(ids[0]), img)
+    ctx.close()
