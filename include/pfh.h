@@ -324,16 +324,15 @@ int pfh_mlp_train(pfh_ctx *ctx, const float *x, const float *target, int64_t n, 
 typedef struct pfh_schedule {
     int32_t fill_grid;        /* max workgroups of the coverage-mask kernel (it loops beyond) */
     int32_t composite_block;  /* threads per composite workgroup: 64, 128 or 256 (a wave per 16x16 tile) */
-    int32_t column_block;     /* threads per workgroup of the per-column propagate kernel, which only
-                                 batches with clip paths run (so with column_rows) */
+    int32_t column_block;     /* 64, 128 or 256; column_rows: 0..64.  Accepted and kept, without effect:
+                                 tiles are resolved path by path */
     int32_t xcd_order;        /* bit 0 fill, bit 1 composite: workgroups regrouped so that each of the
                                  8 XCDs (own L2) works on one contiguous range of tiles */
     int32_t flatten_segs;     /* a multiple of 64 up to 65536, or 0; flatten_take: 1..64 (0: 8);
                                  flatten_deep: 0..12.  Accepted and kept, without effect: a flatten
                                  wave's lanes share the pieces of all its curves */
     int32_t flatten_take;
-    int32_t column_rows;      /* path columns of more tiles than this are propagated by 16 or 64 lanes
-                                 each instead of one (1..64; 0: every column by one lane) */
+    int32_t column_rows;
     int32_t flatten_deep;
 } pfh_schedule;
 int pfh_get_schedule(pfh_ctx *ctx, pfh_schedule *out);

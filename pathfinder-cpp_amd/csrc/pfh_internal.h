@@ -69,6 +69,7 @@ constexpr int BIN_WAVE_COLS = 128;
 constexpr int BIN_WAVE_SEGS = 64;       // more segments than lanes: the group class (its walk is 8x wider)
 constexpr int BIN_GROUP_TILES = 4600;   // with the walk queues: 22 KB (emit) and 33 KB (count) of LDS
 constexpr int BIN_GROUP_COLS = 512;
+constexpr uint32_t PROP_COLS = 32;       // columns of a propagate strip
 constexpr int WALK_QUEUE = 128;          // per wave: chords that cross tile boundaries, waiting for a full wave
 
 enum SegKind : uint32_t { SEG_LINE = 1, SEG_QUAD = 2, SEG_CUBIC = 3 };
@@ -83,14 +84,13 @@ constexpr uint32_t SEG_ORIGINAL_SHIFT = 16;  // the kind again, kept where nothi
 struct Schedule {
     uint32_t fill_grid = 16384;       // max workgroups of k_fill_masks (grid-stride beyond)
     uint32_t composite_block = 256;   // threads per k_composite workgroup (a wave per fb tile)
-    uint32_t column_block = 256;      // threads per workgroup of k_propagate (batches with clip paths)
+    uint32_t column_block = 256;      // column_*: kept for callers that set them; tiles are resolved by path
     uint32_t xcd_order = 0;           // bit 0 fill, bit 1 composite: workgroups grouped per XCD
     // flatten_*: kept for callers that set them; a flattener wave takes at most one segment per lane
     // and its lanes share every curve's pieces, so there is nothing left to choose
     uint32_t flatten_segs = 0;
     uint32_t flatten_take = 8;
-    uint32_t column_rows = 0;         // path columns of more tiles are walked by 16 or 64 lanes (1..64;
-                                      // 0: every column by one lane)
+    uint32_t column_rows = 0;
     uint32_t flatten_deep = 0;
 };
 
@@ -166,10 +166,8 @@ enum Counter {
     C_LINES = 6,       // flattened chords (lines) in the batch
     C_CLIP_JOBS = 7,   // clip combine jobs (alpha tiles over clip tiles with fills)
     C_CLIP_DUPS = 8,   // draw entries whose clip mask row an earlier entry already listed
-    C_TALL = 9,        // [C_TALL, C_TALL + 6): per propagate phase, columns of more than
-                       // TALL_ROWS tiles (and Schedule::column_rows) listed for a wave each
-    C_MID = 9 + 6,     // [C_MID, C_MID + 6): per phase, columns of more than
-                       // Schedule::column_rows tiles and at most TALL_ROWS (k_propagate_rows<16>)
+    C_CLIP_STRIPS = 9,   // strips of clip paths, of clipped draw paths (prop_strips)
+    C_DRAW_STRIPS = 10,
     // fills of the tiles the fill kernel read: a slot per block, by block index, each in a 128-byte
     // line of its own.  A line takes an add every 4-5 ns: with the slots side by side the adds of
     // 16384 blocks took 75 us by themselves (2048^2 with 2500 paths: fill 75 -> 36 us).
@@ -192,7 +190,6 @@ struct ZeroSpans {
         n++;
     }
 };
-constexpr int TALL_ROWS = 64;
 constexpr int DRAWN_SLOTS = 64, DRAWN_STRIDE = 32;
 
 // One scene of a batch as the kernels see it.  Scene-local arrays are resident
@@ -281,10 +278,9 @@ struct BatchDev {
     uint2 *ent_quarter;           // [4 n_bin_group] {draw entries, alpha entries} per quarter of a group-class rect
     uint2 *path_tot;              // [P + 1] {fills, alpha tiles} per batch path, then exclusive scan
     BinItem *bin_items;           // [n_bin_wave + n_bin_group] wave class, then group class
-    uint32_t *col_item;           // [W] the bin item owning each column
+    uint2 *prop_strips;           // [cap_strips] with clip paths: (bin item, first column) of the strips of clip
+    uint32_t cap_strips;          // paths from the front, of clipped draw paths from the back, in any order
     int32_t *col_bd;              // [W] above-rect backdrop, then final column sum (with clip paths or dumps)
-    uint32_t *tall_cols;          // [W] columns of the current propagate phase walked by several lanes:
-                                  // the C_MID list from the front, the C_TALL list from the back
     uint32_t *seg_cnt;            // [S + 1] stream points per segment (flatten count), then their offsets (flatten
                                   // emit), the total behind them
     uint32_t *chunk_off;          // [S / seg_chunk + 2] stream points per seg_chunk segments, then exclusive scan
@@ -315,7 +311,7 @@ struct BatchDev {
     uint32_t *counters;           // [C_COUNT]
     uint32_t *counters_out;       // [C_COUNT] pinned host memory: where the composite leaves them for the host
     int32_t dump;
-    int32_t has_clips;            // some scene has clip paths: propagate in two phases, combine masks
+    int32_t has_clips;            // some scene has clip paths: propagate, combine masks
     uint32_t xcd_order;           // Schedule::xcd_order
 };
 

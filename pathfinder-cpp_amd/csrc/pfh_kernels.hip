@@ -821,10 +821,13 @@ __device__ __forceinline__ U2 wave_sum_u2(U2 v) {
 // Mask rows per alpha tile: 2 for a clip path's tiles, whose coverage is kept under both fill rules.
 __device__ __forceinline__ uint32_t alpha_rows(const BinItem &it) { return it.level != 0 ? 2u : 1u; }
 
-// Backdrops, tile status and z-buffer (core/d3d9/tiler.cpp:369-439) of a path without clip paths in
-// its batch, at the end of its count pass, whose counts and deltas are still in LDS: a column's backdrop
+// Whether a path's tiles are resolved in the bin passes: not where they depend on a clip path's (k_propagate).
+__device__ __forceinline__ bool resolved_here(const BinItem &it) { return it.level == 0 && it.clip == CLIP_NONE; }
+
+// Backdrops, tile status and z-buffer (core/d3d9/tiler.cpp:369-439) of a path that no clip path
+// concerns, at the end of its count pass, whose counts and deltas are still in LDS: a column's backdrop
 // is its running sum from the step above the rect down, which resolve_columns puts in the deltas'
-// place.  (With clip paths a tile also depends on its clip's: k_propagate, after the emit pass.)
+// place.
 // As a walk of its own down the batch's columns, a thread each, this took 155 us for 48 scenes (20
 // million tiles), 30 us at 4096^2 and 25 us at 1240 x 1754, where it waited 14 times for a group of rows;
 // the count pass is longer instead: 367 -> 424 us, 65 -> 81 and 30 -> 32 (the emit pass as long as before).
@@ -876,7 +879,7 @@ __device__ __forceinline__ void store_tile_offset(const BatchDev &b, const BinIt
                                                   uint32_t fills, uint32_t ai, int32_t bd, bool cursors) {
     if (b.has_clips || b.dump || cursors) b.tile_fill_off[t] = off;  // dumps read it back
     b.tile_alpha_idx[t] = ai;  // all: whole lines (stored for alpha tiles alone, the entry pass 26 -> 34 us at 4096^2)
-    if (!b.has_clips && fills && ai < b.cap_alpha)
+    if (fills && ai < b.cap_alpha && resolved_here(it))
         b.alpha_rec[ai] = make_uint4(off, off + fills, (uint32_t)(uint8_t)bd | ((it.rule & 1u) << 8), t);
 }
 
@@ -894,7 +897,7 @@ __device__ __forceinline__ U2 wave_inclusive_u2(uint32_t c) {
 
 // Wave: tile offsets of a rect of `area` tiles (counts in cnt_src, global) from the path's
 // scanned base; offsets go to the tile arrays and, when given, to the LDS cursors.
-// Without clip paths the tiles' masks are complete here: see resolve_tile.
+// The masks of tiles resolved in the count pass are complete here: see resolve_tile.
 __device__ __forceinline__ void wave_tile_offsets(const BatchDev &b, const BinItem &it, uint32_t area, U2 base,
                                                   uint32_t *l_cur) {
     const uint32_t tbase = it.tbase, aw = alpha_rows(it);
@@ -976,9 +979,27 @@ __global__ __launch_bounds__(256) void k_bin_items(BatchDev b, uint32_t wave_blo
     it.paint = sc.path_paint ? sc.path_paint[p] : PAINT_NONE;
     const uint32_t gi = (grp ? b.n_bin_wave : 0u) + i;
     b.bin_items[gi] = it;
-    const uint32_t tw = (uint32_t)max(it.rect.z - it.rect.x, 0);
-    if (b.has_clips)  // for k_propagate, which takes columns
-        for (uint32_t j = 0; j < tw; j++) b.col_item[it.cbase + j] = gi;
+    if (!b.has_clips) return;
+    // for the propagate launches: the strips of clip paths and clipped draw paths, one add per wave and kind
+    const uint64_t here = __ballot(true);
+    const bool lead = (threadIdx.x & 63) == (uint32_t)__builtin_ctzll(here);
+    const uint32_t strips = resolved_here(it) ? 0u : ((uint32_t)max(it.rect.z - it.rect.x, 0) + PROP_COLS - 1) / PROP_COLS;
+    for (int kind = 0; kind < 2; kind++) {
+        const uint32_t left = (it.level != 0) == (kind == 0) ? strips : 0u;
+        uint32_t total = 0, before = 0;
+        // sums over the wave's active lanes, a bit of the counts at a time
+        for (uint32_t bit = 0; __ballot(left >> bit) != 0; bit++) {
+            const uint64_t m = __ballot((left >> bit) & 1u);
+            total += (uint32_t)__popcll(m) << bit;
+            before += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)) << bit;
+        }
+        if (total == 0) continue;
+        uint32_t first = 0;
+        if (lead) first = atomicAdd(&b.counters[kind == 0 ? C_CLIP_STRIPS : C_DRAW_STRIPS], total);
+        first = __builtin_amdgcn_readfirstlane(first) + before;
+        for (uint32_t q = 0; q < left; q++)
+            b.prop_strips[kind == 0 ? first + q : b.cap_strips - 1 - (first + q)] = make_uint2(gi, q * PROP_COLS);
+    }
 }
 
 // LDS of a bin block: its path's arrays (group class), or a slice per wave (wave class).
@@ -1031,7 +1052,7 @@ __device__ __forceinline__ void bin_wave(const BatchDev &b, Lds &lds, uint32_t i
     walk_chords<EMIT, true>(b, sc, rect, tbase, cbase, l_cnt, l_delta, l_col, it.c0, it.c1, lane, 64, lds[wv].queue);
     if (!EMIT) {
         wave_sync();
-        const bool resolve = !b.has_clips;
+        const bool resolve = resolved_here(it);
         if (resolve) {
             resolve_columns<64>(b, it, tw, th, l_delta, 0, l_col, lane);
             wave_sync();
@@ -1067,7 +1088,7 @@ __device__ __forceinline__ void bin_group(const BatchDev &b, Lds &lds, uint32_t 
     uint32_t *const s_cnt = lds.cnt, *const s_delta = lds.delta;
     int32_t *const s_col = lds.col;
     uint32_t *const queue = lds.queue[threadIdx.x >> 6];
-    const bool resolve = !EMIT && !b.has_clips;
+    const bool resolve = !EMIT && resolved_here(it);
     const float inv_w = 1.0f / (float)(int)tw;
     // the packed LDS deltas hold sums below 2^15 in magnitude: at most one step per chord
     const bool in_lds = area <= (uint32_t)BIN_GROUP_TILES && tw <= (uint32_t)BIN_GROUP_COLS &&
@@ -1367,15 +1388,9 @@ struct StoreEntryOff {
 };
 
 // ---------------------------------------------------------------------------
-// Backdrop propagation down each path column (tiler.cpp:369-439) + z-buffer
+// Backdrop propagation down each path column (tiler.cpp:369-439) + z-buffer, for clip paths and what they
+// clip (else the count pass does it: resolve_columns)
 // ---------------------------------------------------------------------------
-//
-// The column kernels walk a path column top to bottom, one thread per column.  Their
-// loads do not depend on earlier rows (only the running backdrop does, in registers), so
-// rows are taken COL_ROWS at a time: every load of the group is issued before the first
-// is used, and a wave waits on memory once per group instead of once per row.
-
-constexpr int COL_ROWS = 8;
 
 // Where a tile of a path column lands in its scene's framebuffer-tile grid.
 struct ColumnWalk {
@@ -1384,15 +1399,14 @@ struct ColumnWalk {
     int rx, ry;  // the path's rect origin (tiles)
     int w, h, x, fb_row0;  // fb_row0: fb tile index (scene-local) of row 0
     uint32_t fb_base, fb_w;
-    // column c of the batch, through its bin item (every column belongs to a binned path)
-    __device__ ColumnWalk(const BatchDev &b, uint32_t c) {
-        const BinItem it = b.bin_items[b.col_item[c]];
+    // column x of a binned path
+    __device__ ColumnWalk(const BatchDev &b, const BinItem &it, uint32_t column) {
         const SceneDev &sc = b.scenes[it.k];
         const int4 r = it.rect;
         p = it.p;
         w = r.z - r.x;
         h = r.w - r.y;
-        x = (int)(c - it.cbase);
+        x = (int)column;
         tbase = it.tbase;
         rgba = it.rgba;
         rule = it.rule & 1u;
@@ -1432,16 +1446,6 @@ __device__ __forceinline__ ClipTile clip_tile_at(const BatchDev &b, const BinIte
     return r;
 }
 
-// Column walk down a path's tiles (core/d3d9/tiler.cpp:369-439): backdrops, tile status, alpha
-// records, z-buffer, and clip resolution (tiler.cpp:385-431) against the clip path's resolved
-// tile at the same coordinates: outside its rect or over a blank tile -> culled; both with masks ->
-// a combine job (the tile's backdrop moves into it); a solid tile over a mask -> it takes that
-// mask; otherwise unchanged (a solid clip tile passes the tile through).
-// Only in batches with clip paths (else the count pass does all of it: resolve_columns).
-// phase 1..MAX_CLIP_LEVELS: the columns of clip paths
-// of that level, a clip path nested in another being resolved against it like a draw path (the
-// level structure of core/d3d11/scene_builder.cpp:92-133, shaders/d3d11/propagate.comp:133-176);
-// MAX_CLIP_LEVELS + 1: the draw paths' columns.  Each phase reads only tiles of earlier phases.
 // What a tile of a path column reads of its clip path: the clip's tile at the same coordinates
 // and, for a clip path's tile over a clip mask, the chain record of that mask.  Both were written
 // by an earlier propagate phase, so a column loads them for a group of rows before it stores
@@ -1450,18 +1454,20 @@ struct ClipRead {
     ClipTile ct;
     uint4 pr;
 };
+template <bool LEVELS>
 __device__ __forceinline__ ClipRead clip_read(const BatchDev &b, const ColumnWalk &cw, const BinItem &ci, int row) {
     ClipRead r{{false, false, false, 0, 0}, make_uint4(1u, 0u, 0u, 0u)};
     if (cw.clip < CLIP_EMPTY) r.ct = clip_tile_at(b, ci, cw.rx + cw.x, cw.ry + row);
-    if (cw.level != 0 && r.ct.alpha && r.ct.src < b.cap_alpha) r.pr = b.clip_rec[r.ct.src];
+    if (LEVELS && r.ct.alpha && r.ct.src < b.cap_alpha) r.pr = b.clip_rec[r.ct.src];
     return r;
 }
 
 // One tile of a path column, its propagated backdrop bd and its fill range [f0, f1) known (ai: its
-// mask row when it has fills), with what it reads of its clip path.
+// mask row when it has fills), with what it reads of its clip path.  LEVELS: the path is a clip path.
+// job: the mask combination it asks for, if any.
+template <bool LEVELS>
 __device__ __forceinline__ void propagate_tile(const BatchDev &b, const ColumnWalk &cw, const ClipRead &cr, int row,
-                                               int8_t bd, uint32_t f0, uint32_t f1, uint32_t ai) {
-    const bool is_clip = cw.level != 0;
+                                               int8_t bd, uint32_t f0, uint32_t f1, uint32_t ai, uint2 &job) {
     const bool clipped = cw.clip < CLIP_EMPTY || cw.clip == CLIP_EMPTY;
     const bool opaque = (cw.rgba >> 24) == 255u;
     const uint32_t t = cw.tile(row);
@@ -1472,7 +1478,7 @@ __device__ __forceinline__ void propagate_tile(const BatchDev &b, const ColumnWa
     // reference's clip resolution tests backdrop != 0 alone (tiler.cpp:396-431).
     const bool covers = bd != 0 && !(cw.own_rules && cw.rule && (bd & 1) == 0);
     const uint32_t job_rules = cw.own_rules ? CLIP_JOB_OWN_RULES : 0u;
-    if (is_clip) {
+    if (LEVELS) {
         // A clip path draws nothing itself.  Its fills make two mask rows (ai, ai + 1) that
         // keep |sum + backdrop| under the nonzero and the even-odd rule (under its own rule,
         // both, where clip paths' own rules are taken), for the tiles that take them over; its
@@ -1496,8 +1502,7 @@ __device__ __forceinline__ void propagate_tile(const BatchDev &b, const ColumnWa
                 out_bd = 0;
                 const uint4 pr = cr.pr;
                 rec = make_uint4(1u + min(pr.x, MAX_CLIP_LEVELS - 1u), ct.src, pr.y, pr.z);
-                const uint32_t j = atomicAdd(&b.counters[C_CLIP_JOBS], 1u);
-                if (j < b.cap_alpha) b.clip_jobs[j] = make_uint2(ai | CLIP_JOB_CLIP | job_rules, ai);
+                job = make_uint2(ai | CLIP_JOB_CLIP | job_rules, ai);
             } else if (ct.alpha && covers) {
                 st = TILE_CLIP_MASK;  // its own clip's coverage, unchanged
                 out_bd = ct.bd;
@@ -1520,8 +1525,7 @@ __device__ __forceinline__ void propagate_tile(const BatchDev &b, const ColumnWa
         } else if (ct.alpha && alpha) {
             // both masks: min(|own + backdrop|, clip coverage) replaces the mask; backdrop 0
             st = TILE_ALPHA;
-            const uint32_t j = atomicAdd(&b.counters[C_CLIP_JOBS], 1u);
-            if (j < b.cap_alpha) b.clip_jobs[j] = make_uint2(ai | job_rules, ct.src);
+            job = make_uint2(ai | job_rules, ct.src);
         } else if (ct.alpha && covers) {
             st = TILE_CLIP_MASK;  // solid over a clip mask: the clip's mask and backdrop
             out_bd = ct.bd;
@@ -1547,122 +1551,113 @@ __device__ __forceinline__ void propagate_tile(const BatchDev &b, const ColumnWa
     }
 }
 
-// Column walk down a path's tiles (core/d3d9/tiler.cpp:369-439): backdrops, tile status, alpha
+// Walk down a path's tiles (core/d3d9/tiler.cpp:369-439): backdrops, tile status, alpha
 // records, z-buffer, and clip resolution (tiler.cpp:385-431) against the clip path's resolved
 // tile at the same coordinates: outside its rect or over a blank tile -> culled; both with masks ->
 // a combine job (the tile's backdrop moves into it); a solid tile over a mask -> it takes that
 // mask; otherwise unchanged (a solid clip tile passes the tile through).
-// Only in batches with clip paths (else the count pass does all of it: resolve_columns).
-// phase 1..MAX_CLIP_LEVELS: the columns of clip paths
-// of that level, a clip path nested in another being resolved against it like a draw path (the
-// level structure of core/d3d11/scene_builder.cpp:92-133, shaders/d3d11/propagate.comp:133-176);
-// MAX_CLIP_LEVELS + 1: the draw paths' columns.  Each phase reads only tiles of earlier phases.
-// A thread walks its column: rows of neighbouring columns are neighbours in memory, so the
-// wave's loads coalesce.  A walk is a chain of dependent loads per group of rows, and a launch
-// lasts as long as its longest walk: a column of more than `rows` tiles (a schedule choice) is
-// listed instead for k_propagate_rows, which spreads its rows over 16 or 64 lanes (rows 0: none).
-__global__ __launch_bounds__(256) void k_propagate(BatchDev b, uint32_t phase, uint32_t rows) {
-    uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= b.n_cols) return;
-    const ColumnWalk cw(b, c);
-    if (cw.level != (phase > MAX_CLIP_LEVELS ? 0u : phase)) return;
-    if (rows != 0 && (uint32_t)cw.h > rows) {
-        // at most one entry per column and phase, so the two lists together hold at most n_cols
-        if (cw.h > TALL_ROWS) b.tall_cols[b.n_cols - 1 - atomicAdd(&b.counters[C_TALL + phase], 1u)] = c;
-        else b.tall_cols[atomicAdd(&b.counters[C_MID + phase], 1u)] = c;
-        return;
-    }
-    BinItem ci;
-    if (cw.clip < CLIP_EMPTY) ci = b.bin_items[cw.clip];
-    int32_t running = b.col_bd[c];
-    for (int row0 = 0; row0 < cw.h; row0 += COL_ROWS) {
-        int32_t delta[COL_ROWS];
-        uint32_t f0[COL_ROWS], f1[COL_ROWS];
-#pragma unroll
-        for (int i = 0; i < COL_ROWS; i++) {
-            delta[i] = 0;
-            f0[i] = f1[i] = 0;
-            if (row0 + i < cw.h) {
-                const uint32_t t = cw.tile(row0 + i);
-                delta[i] = b.tile_delta[t];
-                f0[i] = b.tile_fill_off[t];
-                f1[i] = b.tile_fill_off[t + 1];
-            }
-        }
-        int8_t bd[COL_ROWS];
-        uint32_t ai[COL_ROWS];
-        ClipRead cr[COL_ROWS];
-#pragma unroll
-        for (int i = 0; i < COL_ROWS; i++) {
-            bd[i] = (int8_t)running;
-            running += (int8_t)delta[i];
-            ai[i] = 0;
-            // the group's loads go out at once (the walk is latency-bound)
-            if (row0 + i < cw.h) ai[i] = b.tile_alpha_idx[cw.tile(row0 + i)];
-            cr[i] = ClipRead{{false, false, false, 0, 0}, make_uint4(1u, 0u, 0u, 0u)};
-            if (row0 + i < cw.h) cr[i] = clip_read(b, cw, ci, row0 + i);
-        }
-#pragma unroll
-        for (int i = 0; i < COL_ROWS; i++) {
-            if (row0 + i >= cw.h) break;
-            propagate_tile(b, cw, cr[i], row0 + i, bd[i], f0[i], f1[i], ai[i]);
-        }
-    }
-    b.col_bd[c] = running;
-}
+// A launch per clip level, 1..MAX_CLIP_LEVELS: the clip paths of that level, a clip path nested in
+// another being resolved against it like a draw path (the level structure of
+// core/d3d11/scene_builder.cpp:92-133, shaders/d3d11/propagate.comp:133-176); then one for the clipped
+// draw paths.  Each reads only tiles of earlier launches.
+// Columns [xa, xb) of a path, at most PROP_COLS, by a block: a thread per column and stretch of rows; each
+// sums its stretch's deltas, starts from the sums of the stretches above it and takes its rows PROP_ROWS
+// at a time, every load of a group issued before the first is used.
+// Latency-bound (dependent loads per group, a few wide clip rects per level), so the work is strips of
+// columns, listed by k_bin_items and dealt to as many blocks as the chip holds, with stretches a few
+// groups long.  The 4096^2 scene of 2 500 paths under clips nested 4 deep: with a thread per column, tall
+// columns listed for 16 or 64 lanes each in two more launches and every launch over all columns, 156 us in
+// 15 launches; with a block per path, 148 in 5; now 62 in 5.
+constexpr int PROP_ROWS = 4;
+constexpr uint32_t NO_JOB = 0xffffffffu;  // not a mask row with its flags
+constexpr int PROP_THREADS = 512;
 
-// The columns k_propagate listed for this phase (SUB 64: the C_TALL list, SUB 16: the C_MID list),
-// SUB lanes per column: a column's lanes take SUB rows at a time, and a prefix sum of the rows'
-// backdrop deltas across them gives each row the backdrop the serial walk reaches there (the int8
-// deltas summed in int32, as the walk does).  Every wave strides over the list (its length is
-// only known on the device), 64 / SUB columns at a time.
-template <int SUB>
-__global__ __launch_bounds__(256) void k_propagate_rows(BatchDev b, uint32_t phase) {
-    constexpr uint32_t G = 64 / SUB;  // columns per wave
-    const uint32_t n = min(b.counters[(SUB == 64 ? C_TALL : C_MID) + phase], b.n_cols);
-    const int lane = (int)(threadIdx.x & 63), li = lane % SUB, g = lane / SUB;
-    const uint32_t waves = gridDim.x * 4;
-    for (uint32_t j0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * G; j0 < n; j0 += waves * G) {  // wave-uniform
-        const uint32_t j = j0 + (uint32_t)g;
-        const bool has = j < n;
-        const uint32_t c = has ? b.tall_cols[SUB == 64 ? b.n_cols - 1 - j : j] : 0u;
-        const ColumnWalk cw(b, c);
-        const int h = has ? cw.h : 0;
+template <bool LEVELS>
+__device__ __forceinline__ void propagate_strip(const BatchDev &b, const BinItem &it, uint32_t xa, int32_t *part) {
+    const uint32_t t = threadIdx.x;
+    const uint32_t tw = (uint32_t)max(it.rect.z - it.rect.x, 0), cols = min(PROP_COLS, tw - xa);
+    const int th = max(it.rect.w - it.rect.y, 0);
+    const uint32_t bits = cols > 1 ? 32u - (uint32_t)__clz((int)(cols - 1)) : 0u;
+    const int parts = max(min(PROP_THREADS >> bits, th), 1);
+    const int rows = (th + parts - 1) / parts;
+    const int p = (int)(t >> bits);
+    const uint32_t x = t & ((1u << bits) - 1u);  // from xa
+    const int ra = min(p * rows, th), rb = min(ra + rows, th);
+    const int32_t start = x < cols ? b.col_bd[it.cbase + xa + x] : 0;  // before a stretch stores its column's sum
+    int32_t sum = 0;
+    if (x < cols) {
+        for (int r0 = ra; r0 < rb; r0 += 8) {
+            int32_t d[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                d[i] = r0 + i < rb ? b.tile_delta[it.tbase + (uint32_t)(r0 + i) * tw + xa + x] : 0;
+#pragma unroll
+            for (int i = 0; i < 8; i++) sum += (int8_t)d[i];
+        }
+    }
+    part[t] = sum;
+    __syncthreads();
+    if (p < parts && x < cols) {
         BinItem ci;
-        if (has && cw.clip < CLIP_EMPTY) ci = b.bin_items[cw.clip];
-        int32_t running = has ? b.col_bd[c] : 0;
-        int hmax = h;
+        if (it.clip < CLIP_EMPTY) ci = b.bin_items[it.clip];
+        const ColumnWalk cw(b, it, xa + x);
+        int32_t running = start;
+        for (int q = 0; q < p; q++) running += part[((uint32_t)q << bits) + x];
+        for (int row0 = ra; row0 < rb; row0 += PROP_ROWS) {
+            int32_t delta[PROP_ROWS];
+            uint32_t f0[PROP_ROWS], f1[PROP_ROWS], ai[PROP_ROWS];
+            ClipRead cr[PROP_ROWS];
 #pragma unroll
-        for (uint32_t k = 0; k < G; k++) hmax = max(hmax, __builtin_amdgcn_readlane(h, k * SUB));
-        for (int row0 = 0; row0 < hmax; row0 += SUB) {
-            const int row = row0 + li;
-            const bool on = row < h;
-            int32_t d8 = 0;
-            uint32_t f0 = 0, f1 = 0, ai = 0;
-            ClipRead cr{{false, false, false, 0, 0}, make_uint4(1u, 0u, 0u, 0u)};
-            if (on) {
-                const uint32_t t = cw.tile(row);
-                d8 = (int8_t)b.tile_delta[t];
-                f0 = b.tile_fill_off[t];
-                f1 = b.tile_fill_off[t + 1];
-                ai = b.tile_alpha_idx[t];
-                cr = clip_read(b, cw, ci, row);
-            }
-            uint32_t incl;
-            if (SUB == 16) {
-                incl = row16_inclusive_sum((uint32_t)d8);
-            } else {
-                incl = (uint32_t)d8;
-#pragma unroll
-                for (int d = 1; d < 64; d <<= 1) {
-                    const uint32_t o = shfl_up_val(incl, d);
-                    if (lane >= d) incl += o;
+            for (int i = 0; i < PROP_ROWS; i++) {
+                delta[i] = 0;
+                f0[i] = f1[i] = ai[i] = 0;
+                cr[i] = ClipRead{{false, false, false, 0, 0}, make_uint4(1u, 0u, 0u, 0u)};
+                if (row0 + i < rb) {
+                    const uint32_t tile = cw.tile(row0 + i);
+                    delta[i] = b.tile_delta[tile];
+                    f0[i] = b.tile_fill_off[tile];
+                    f1[i] = b.tile_fill_off[tile + 1];
+                    ai[i] = b.tile_alpha_idx[tile];
+                    cr[i] = clip_read<LEVELS>(b, cw, ci, row0 + i);
                 }
             }
-            if (on) propagate_tile(b, cw, cr, row, (int8_t)(running + (int32_t)(incl - (uint32_t)d8)), f0, f1, ai);
-            running += (int32_t)__shfl(incl, g * SUB + SUB - 1, 64);
+            uint2 job[PROP_ROWS];
+            uint32_t n_jobs = 0, at[PROP_ROWS];
+#pragma unroll
+            for (int i = 0; i < PROP_ROWS; i++) {
+                job[i] = make_uint2(NO_JOB, 0u);
+                if (row0 + i < rb) {
+                    propagate_tile<LEVELS>(b, cw, cr[i], row0 + i, (int8_t)running, f0[i], f1[i], ai[i], job[i]);
+                    running += (int8_t)delta[i];
+                }
+                const uint64_t m = __ballot(job[i].x != NO_JOB);
+                at[i] = n_jobs + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                n_jobs += (uint32_t)__popcll(m);
+            }
+            if (n_jobs == 0) continue;  // of the wave's active lanes: uniform
+            // one add for the wave's rows: the counter takes one every 4-5 ns
+            uint32_t first = 0;
+            if ((threadIdx.x & 63) == (uint32_t)__builtin_ctzll(__ballot(true)))
+                first = atomicAdd(&b.counters[C_CLIP_JOBS], n_jobs);
+            first = __builtin_amdgcn_readfirstlane(first);
+#pragma unroll
+            for (int i = 0; i < PROP_ROWS; i++)
+                if (job[i].x != NO_JOB && first + at[i] < b.cap_alpha) b.clip_jobs[first + at[i]] = job[i];
         }
-        if (has && li == 0) b.col_bd[c] = running;
+        if (b.dump && rb == th && (ra < th || th == 0)) b.col_bd[it.cbase + xa + x] = running;  // the column's last rows
+    }
+    __syncthreads();  // the next strip rewrites part
+}
+
+// LEVELS: the strips of the clip paths of a level, else those of the clipped draw paths.
+template <bool LEVELS>
+__global__ __launch_bounds__(PROP_THREADS) void k_propagate(BatchDev b, uint32_t level) {
+    __shared__ int32_t part[PROP_THREADS];
+    const uint32_t n = b.counters[LEVELS ? C_CLIP_STRIPS : C_DRAW_STRIPS];
+    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {  // uniform over the block
+        const uint2 st = b.prop_strips[LEVELS ? i : b.cap_strips - 1 - i];
+        const BinItem it = b.bin_items[st.x];
+        if (!LEVELS || it.level == level) propagate_strip<LEVELS>(b, it, st.y, part);
     }
 }
 
@@ -2259,26 +2254,13 @@ hipError_t launch_bin(const BatchDev &b, bool emit, hipStream_t s) {
     return hipGetLastError();
 }
 
-// rows: columns of more tiles are walked by several lanes each (1..64; 0: none)
-static void propagate_phase(const BatchDev &b, uint32_t block, uint32_t rows, uint32_t phase, hipStream_t s) {
-    hipLaunchKernelGGL(k_propagate, dim3(blocks_for(b.n_cols, block)), dim3(block), 0, s, b, phase, rows);
-    if (rows == 0) return;
-    // the listed columns' waves: enough to cover the device, striding over lists of unknown length
-    if (rows < (uint32_t)TALL_ROWS)
-        hipLaunchKernelGGL(k_propagate_rows<16>, dim3(std::min<uint32_t>(blocks_for(b.n_cols, 16), 2048)),
-                           dim3(256), 0, s, b, phase);
-    hipLaunchKernelGGL(k_propagate_rows<64>, dim3(std::min<uint32_t>(blocks_for(b.n_cols, 4), 2048)),
-                       dim3(256), 0, s, b, phase);
-}
-
-hipError_t launch_propagate(const BatchDev &b, uint32_t block, uint32_t rows, hipStream_t s) {
-    if (block != 64 && block != 128 && block != 256) return hipErrorInvalidValue;
-    if (rows > (uint32_t)TALL_ROWS) return hipErrorInvalidValue;
-    if (b.n_cols == 0 || !b.has_clips) return hipSuccess;
+hipError_t launch_propagate(const BatchDev &b, hipStream_t s) {
+    if (!b.has_clips || b.n_bin_wave + b.n_bin_group == 0) return hipSuccess;
+    const dim3 g(std::min<uint32_t>(b.cap_strips, 1024));
     // clip levels from the outermost in, then the draw paths
     for (uint32_t level = 1; level <= std::min(b.clip_levels, MAX_CLIP_LEVELS); level++)
-        propagate_phase(b, block, rows, level, s);
-    propagate_phase(b, block, rows, MAX_CLIP_LEVELS + 1, s);
+        hipLaunchKernelGGL(k_propagate<true>, g, dim3(PROP_THREADS), 0, s, b, level);
+    hipLaunchKernelGGL(k_propagate<false>, g, dim3(PROP_THREADS), 0, s, b, 0u);
     return hipGetLastError();
 }
 

@@ -30,7 +30,7 @@ hipError_t scan_paths(const BatchDev &b, hipStream_t s);
 hipError_t scan_counted(uint32_t *inout, const uint32_t *n_ptr, uint32_t cap, unsigned long long *state, hipStream_t s);
 hipError_t launch_flatten(const BatchDev &b, bool emit, uint32_t chunk, hipStream_t s);
 hipError_t launch_bin(const BatchDev &b, bool emit, hipStream_t s);
-hipError_t launch_propagate(const BatchDev &b, uint32_t block, uint32_t rows, hipStream_t s);
+hipError_t launch_propagate(const BatchDev &b, hipStream_t s);
 hipError_t launch_entries(const BatchDev &b, bool write, hipStream_t s);
 hipError_t launch_bin_items(const BatchDev &b, hipStream_t s);
 size_t sort_temp_elems(uint64_t cap, uint32_t n_scenes, uint32_t max_fb, uint64_t max_tiles);
@@ -370,9 +370,9 @@ struct Workspace {
     // around the fill and composite kernels of a batched launch; recorded as event nodes
     // inside captured graphs, so replays time those kernels too
     hipEvent_t kev[3] = {nullptr, nullptr, nullptr};
-    DevBuf scene_table, bases, tile_delta, tile_cnt, tile_fill_off, tile_alpha_idx, tile_bd, tile_st, path_ent, ent_quarter, path_tot, bin_items, col_item, col_bd, tall_cols, seg_mask,
+    DevBuf scene_table, bases, tile_delta, tile_cnt, tile_fill_off, tile_alpha_idx, tile_bd, tile_st, path_ent, ent_quarter, path_tot, bin_items, col_bd, seg_mask,
         seg_cnt, lines, line_cnt, fills, dump_fills, alpha_rec, alpha_vis, masks, zbuf, fb_range, keys, keys_alt,
-        rec_alt, entry_rec, entry_meta, meta_alt, counters, chunk_off, scan_state, dump_state, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen;
+        rec_alt, entry_rec, entry_meta, meta_alt, counters, chunk_off, scan_state, dump_state, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen, prop_strips;
     // pinned and coherent: kernels write h_counters and read the tables
     uint32_t *h_counters = nullptr;
     SceneDev *h_table = nullptr;     // pinned scene table
@@ -449,9 +449,9 @@ struct Workspace {
     }
     std::vector<DevBuf *> all_buffers() {
         return {&scene_table, &bases, &tile_delta, &tile_cnt, &tile_fill_off, &tile_alpha_idx, &tile_bd, &tile_st,
-                &path_ent, &ent_quarter, &path_tot, &bin_items, &col_item, &col_bd, &tall_cols, &seg_mask, &seg_cnt, &lines, &line_cnt, &fills, &dump_fills, &alpha_rec, &alpha_vis,
+                &path_ent, &ent_quarter, &path_tot, &bin_items, &col_bd, &seg_mask, &seg_cnt, &lines, &line_cnt, &fills, &dump_fills, &alpha_rec, &alpha_vis,
                 &masks, &zbuf, &fb_range, &keys, &keys_alt, &rec_alt, &entry_rec, &entry_meta, &meta_alt, &counters, &chunk_off, &scan_state, &dump_state,
-                &sort_tmp, &tile_clip_ai, &clip_jobs, &clip_rec, &clip_seen};
+                &sort_tmp, &tile_clip_ai, &clip_jobs, &clip_rec, &clip_seen, &prop_strips};
     }
     size_t device_bytes() {
         size_t n = 0;
@@ -1600,6 +1600,9 @@ static ScanStates scan_states(const Plan &pl) {
 
 static uint32_t clamp_cap(uint64_t v) { return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(v, 64), 0xF0000000ull); }
 
+// Strips of PROP_COLS columns, the last of a path's perhaps narrower.
+static uint64_t strips_cap(const Plan &pl) { return pl.W / PROP_COLS + pl.P + 1; }
+
 static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
     w.tile_delta.ensure(4 * pl.T + 4);
     w.tile_cnt.ensure(4 * pl.T + 4);
@@ -1615,15 +1618,14 @@ static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
         w.clip_jobs.ensure(8ull * pl.cap_a + 8);
         w.clip_rec.ensure(16ull * pl.cap_a + 16);
         w.clip_seen.ensure(4ull * (pl.cap_a / 32 + 1));
+        w.prop_strips.ensure(8 * strips_cap(pl));
     }
     w.tile_st.ensure(pl.T + 4);
     w.path_ent.ensure(8 * pl.P + 8);
     w.ent_quarter.ensure(32 * pl.BG + 32);
     w.path_tot.ensure(8 * pl.P + 8);
     w.bin_items.ensure(sizeof(BinItem) * (pl.BW + pl.BG) + 64);
-    w.col_item.ensure(4 * pl.W + 4);
     w.col_bd.ensure(4 * pl.W + 4);
-    w.tall_cols.ensure(4 * pl.W + 4);
     w.seg_cnt.ensure(4 * pl.S + 8);
     // in a fixed region the curves' bits share the tile arrays' space (curve_bits)
     if (!w.arena.base) w.seg_mask.ensure(8 * pl.S + 8);
@@ -1840,6 +1842,8 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
     b.tile_bd = (dump || pl.clips) ? w.tile_bd.as<int8_t>() : nullptr;
     b.tile_clip_ai = pl.clips ? w.tile_clip_ai.as<uint32_t>() : nullptr;
     b.clip_jobs = pl.clips ? w.clip_jobs.as<uint2>() : nullptr;
+    b.prop_strips = pl.clips ? w.prop_strips.as<uint2>() : nullptr;
+    b.cap_strips = pl.clips ? (uint32_t)strips_cap(pl) : 0;
     b.clip_rec = pl.clips ? w.clip_rec.as<uint4>() : nullptr;
     b.clip_seen = pl.clips ? w.clip_seen.as<uint32_t>() : nullptr;
     b.clip_levels = pl.clip_levels;
@@ -1849,10 +1853,8 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
     b.ent_quarter = w.ent_quarter.as<uint2>();
     b.path_tot = w.path_tot.as<uint2>();
     b.bin_items = w.bin_items.as<BinItem>();
-    b.col_item = w.col_item.as<uint32_t>();
     b.n_paths = (uint32_t)pl.P;
     b.col_bd = w.col_bd.as<int32_t>();
-    b.tall_cols = w.tall_cols.as<uint32_t>();
     b.seg_cnt = w.seg_cnt.as<uint32_t>();
     b.seg_mask = curve_bits(w, pl);
     b.chunk_off = w.chunk_off.as<uint32_t>();
@@ -1930,7 +1932,7 @@ static void stage_emit(Workspace &w, const BatchDev &b, const Plan &pl) {
     hipStream_t s = w.stream;
     if (b.dump) dump_offsets(w, b, b.cap_lines);
     HIP_TRY(launch_bin(b, true, s));
-    HIP_TRY(launch_propagate(b, pl.sched.column_block, pl.sched.column_rows, s));
+    HIP_TRY(launch_propagate(b, s));
     HIP_TRY(launch_entries(b, false, s));
     HIP_TRY(scan_entries(b, s));
 }
@@ -2046,7 +2048,7 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
     if (dump) dump_offsets(*ctx->w, b, nl);
     HIP_TRY(launch_bin(b, true, st));
     HIP_TRY(hipEventRecord(ev[3], st));
-    HIP_TRY(launch_propagate(b, pl.sched.column_block, pl.sched.column_rows, st));
+    HIP_TRY(launch_propagate(b, st));
     HIP_TRY(hipEventRecord(ev[4], st));
     HIP_TRY(launch_entries(b, false, st));
     HIP_TRY(scan_entries(b, st));
@@ -3064,16 +3066,13 @@ int pfh_autotune(pfh_ctx *ctx, const int32_t *scene_ids, int32_t n, uint32_t fla
         Schedule best = ctx->sched;
         double best_ms = measure();
         if (ms_start) *ms_start = best_ms;
-        const std::vector<uint32_t> cand[5] = {{1024, 2048, 4096, 8192, 16384, 32768, 65536}, {64, 128, 256}, {64, 128, 256},
-                                              {0, 1, 2, 3}, {0, 8, 16, 32, 64}};
-        for (int param = 0; param < 5; param++) {
+        const std::vector<uint32_t> cand[3] = {{1024, 2048, 4096, 8192, 16384, 32768, 65536}, {64, 128, 256}, {0, 1, 2, 3}};
+        for (int param = 0; param < 3; param++) {
             for (uint32_t v : cand[param]) {
                 Schedule trial = best;
                 uint32_t *field = param == 0 ? &trial.fill_grid
                                   : param == 1 ? &trial.composite_block
-                                  : param == 2 ? &trial.column_block
-                                  : param == 3 ? &trial.xcd_order
-                                               : &trial.column_rows;
+                                               : &trial.xcd_order;
                 if (*field == v) continue;
                 *field = v;
                 ctx->sched = trial;

@@ -47,3 +47,22 @@ def test_tiles_from_the_count_pass_and_the_column_walk(name, sc):
         ctx.rasterize(ids[:1], flags)
         np.testing.assert_array_equal(ctx.readback(ids[0]), img)
     ctx.close()
+
+
+@pytest.mark.parametrize("cols,rows", [(1, 1), (1, 513), (31, 9), (32, 16), (33, 17), (65, 130), (130, 3)])
+def test_strips_of_clips_and_clipped_paths(cols, rows):
+    """Strips of 32 columns with 16 or more threads to a column: rects, and clips nested in each other, of
+    about a strip's width and its stretches' heights."""
+    w, h = 16.0 * cols, 16.0 * rows
+    boxes = [(1 + i, 2, w - 3 - i, h - 4) for i in range(6)] + [(3, 1, w - 4, h - 2), (2.5, 2, w * 0.75, h - 3),
+                                                               (4, 3, w * 0.5, h * 0.75)]
+    sc = rects(boxes, 16 * cols + 8, 16 * rows + 8)
+    sc.n_clip_paths = 3
+    sc.path_clip = np.array([-1, 0, 1, 2, 0, 2, -1, 0, 1], np.int32)
+    ctx = pfh.Context(0)
+    _, img = check_scene(ctx, sc, name=f"{cols}x{rows} tiles")
+    sid = ctx.upload(sc)
+    for flags in (pfh.PFH_PLAIN, pfh.PFH_BATCHED | pfh.PFH_NO_GRAPH, pfh.PFH_BATCHED):
+        ctx.rasterize([sid], flags)
+        np.testing.assert_array_equal(ctx.readback(sid), img)
+    ctx.close()
