@@ -67,8 +67,18 @@ constexpr uint32_t RULE_CLIP_OWN = 0x2u;
 constexpr int BIN_WAVE_TILES = 512;
 constexpr int BIN_WAVE_COLS = 128;
 constexpr int BIN_WAVE_SEGS = 64;       // more segments than lanes: the group class (its walk is 8x wider)
-constexpr int BIN_GROUP_TILES = 4600;   // with the walk queues: 22 KB (emit) and 33 KB (count) of LDS
+// With the walk queues 27 KB (emit) and 40 KB (count) of LDS in blocks of 512, as much as the wave class's slices take
+// there.  Paths past it are slow (global atomics): the 4096^2 scene of 10^4 paths, a few of whose rects
+// have 4 600 to 5 700 tiles, 573 us with 4600, 497 with 5700.
+constexpr int BIN_GROUP_TILES = 5700;
 constexpr int BIN_GROUP_COLS = 512;
+// Group-class paths past those limits, up to these, take a block with more LDS (at most 160 KB less 1.5) where
+// their rect is the whole framebuffer: that of a destructive blend mode, whatever the path's size, so that
+// clearing and resolving tiles is most of the work.  It takes a launch of its own, which others do not
+// repay: with every rect that fits, the 4096^2 scene of 2 000 stars, whose walks are long, took 122 us to
+// count for 88.
+constexpr int BIN_BIG_TILES = 25000;
+constexpr int BIN_BIG_COLS = 1024;
 constexpr uint32_t PROP_COLS = 32;       // columns of a propagate strip
 constexpr int WALK_QUEUE = 128;          // per wave: chords that cross tile boundaries, waiting for a full wave
 
@@ -168,6 +178,7 @@ enum Counter {
     C_CLIP_DUPS = 8,   // draw entries whose clip mask row an earlier entry already listed
     C_CLIP_STRIPS = 9,   // strips of clip paths, of clipped draw paths (prop_strips)
     C_DRAW_STRIPS = 10,
+    C_BIG = 11,          // big paths (big_list)
     // fills of the tiles the fill kernel read: a slot per block, by block index, each in a 128-byte
     // line of its own.  A line takes an add every 4-5 ns: with the slots side by side the adds of
     // 16384 blocks took 75 us by themselves (2048^2 with 2500 paths: fill 75 -> 36 us).
@@ -275,9 +286,11 @@ struct BatchDev {
     uint32_t clip_levels;         // clip levels present in the batch (0: no clip paths)
     uint8_t *tile_st;             // [T] tile status (TileStatus)
     uint2 *path_ent;              // [P + 1] {draw entries, alpha entries} per batch path, then exclusive scan
-    uint2 *ent_quarter;           // [4 n_bin_group] {draw entries, alpha entries} per quarter of a group-class rect
+    uint2 *ent_part;              // [entry_waves n_bin_group] {draw entries, alpha entries} per part of a group-class rect
     uint2 *path_tot;              // [P + 1] {fills, alpha tiles} per batch path, then exclusive scan
     BinItem *bin_items;           // [n_bin_wave + n_bin_group] wave class, then group class
+    uint32_t *big_list;           // [n_big] the bin items of big paths, in any order
+    uint32_t n_big, big_tiles, big_cols;  // how many there may be, the most tiles and columns one has
     uint2 *prop_strips;           // [cap_strips] with clip paths: (bin item, first column) of the strips of clip
     uint32_t cap_strips;          // paths from the front, of clipped draw paths from the back, in any order
     int32_t *col_bd;              // [W] above-rect backdrop, then final column sum (with clip paths or dumps)

@@ -921,15 +921,29 @@ template <int THREADS>
 __device__ __forceinline__ void block_tile_offsets(const BatchDev &b, const BinItem &it, uint32_t area, U2 base,
                                                    uint32_t *l_cur) {
     const uint32_t tbase = it.tbase, aw = alpha_rows(it);
-    for (uint32_t j0 = 0; j0 < area; j0 += THREADS) {
-        const uint32_t j = j0 + threadIdx.x;
-        const uint32_t c = j < area ? b.tile_cnt[tbase + j] : 0u;
-        const int32_t bd = j < area ? b.tile_delta[tbase + j] : 0;
+    // tiles of a thread: a chunk costs a block-wide scan (50 whole-canvas rects 36 -> 24 us; no use to small rects)
+    constexpr uint32_t ITEMS = THREADS == 1024 ? 4 : 1;
+    for (uint32_t j0 = 0; j0 < area; j0 += THREADS * ITEMS) {
+        const uint32_t j = j0 + threadIdx.x * ITEMS;
+        uint32_t c[ITEMS];
+        int32_t bd[ITEMS];
+        U2 own{0, 0};
+#pragma unroll
+        for (uint32_t i = 0; i < ITEMS; i++) {
+            c[i] = j + i < area ? b.tile_cnt[tbase + j + i] : 0u;
+            bd[i] = j + i < area ? b.tile_delta[tbase + j + i] : 0;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < ITEMS; i++) own = own + U2{c[i], c[i] > 0 ? 1u : 0u};
         U2 tot;
-        const U2 ex = block_exclusive_scan<U2, THREADS>(U2{c, c > 0 ? 1u : 0u}, tot);
-        if (j < area) {
-            store_tile_offset(b, it, tbase + j, base.x + ex.x, c, base.y + aw * ex.y, bd, l_cur == nullptr);
-            if (l_cur) l_cur[j] = base.x + ex.x;
+        U2 ex = block_exclusive_scan<U2, THREADS>(own, tot);
+#pragma unroll
+        for (uint32_t i = 0; i < ITEMS; i++) {
+            if (j + i < area) {
+                store_tile_offset(b, it, tbase + j + i, base.x + ex.x, c[i], base.y + aw * ex.y, bd[i], l_cur == nullptr);
+                if (l_cur) l_cur[j + i] = base.x + ex.x;
+            }
+            ex = ex + U2{c[i], c[i] > 0 ? 1u : 0u};
         }
         base = base + U2{tot.x, aw * tot.y};
     }
@@ -947,6 +961,15 @@ __device__ __forceinline__ U2 block_sum_u2(U2 v, U2 *part) {
     for (int w = 1; w < THREADS / 64; w++) t = t + part[w];
     __syncthreads();
     return t;
+}
+
+// Group-class paths whose rect is the whole framebuffer, as destructive blend modes make it, past a bin
+// block's LDS, that fit a block with more of it (k_bin_big).
+__device__ __forceinline__ bool is_big(const BinItem &it, const SceneDev &sc) {
+    const uint32_t tw = (uint32_t)max(it.rect.z - it.rect.x, 0), th = (uint32_t)max(it.rect.w - it.rect.y, 0);
+    const uint64_t area = (uint64_t)tw * th;
+    return tw == (uint32_t)sc.fb_w && area == sc.n_fb && (area > (uint32_t)BIN_GROUP_TILES || tw > (uint32_t)BIN_GROUP_COLS) &&
+           area <= (uint32_t)BIN_BIG_TILES && tw <= (uint32_t)BIN_BIG_COLS && it.c1 - it.c0 < (1u << 15);
 }
 
 // One descriptor per binned path: thread per item, the first blocks for the wave class, the others for
@@ -979,6 +1002,7 @@ __global__ __launch_bounds__(256) void k_bin_items(BatchDev b, uint32_t wave_blo
     it.paint = sc.path_paint ? sc.path_paint[p] : PAINT_NONE;
     const uint32_t gi = (grp ? b.n_bin_wave : 0u) + i;
     b.bin_items[gi] = it;
+    if (b.n_big && is_big(it, sc)) b.big_list[atomicAdd(&b.counters[C_BIG], 1u)] = gi;
     if (!b.has_clips) return;
     // for the propagate launches: the strips of clip paths and clipped draw paths, one add per wave and kind
     const uint64_t here = __ballot(true);
@@ -1073,11 +1097,11 @@ __device__ __forceinline__ void bin_wave(const BatchDev &b, Lds &lds, uint32_t i
     }
 }
 
-// Group class: one path per block; LDS when the rect fits, else global atomics on the path's own
-// (first zeroed) tiles.
-template <bool EMIT, int THREADS, typename Lds>
-__device__ __forceinline__ void bin_group(const BatchDev &b, Lds &lds, uint32_t item) {
-    const BinItem it = b.bin_items[b.n_bin_wave + item];
+// Group class: one path per block; LDS when the rect fits (max_tiles, max_cols), else global atomics on the
+// path's own (first zeroed) tiles.
+template <bool EMIT, int THREADS>
+__device__ __forceinline__ void bin_group(const BatchDev &b, const BinItem &it, uint32_t *s_cnt, uint32_t *s_delta,
+                                          int32_t *s_col, uint32_t *queues, uint32_t max_tiles, uint32_t max_cols) {
     const SceneDev &sc = b.scenes[it.k];
     const int4 rect = it.rect;
     const uint32_t tw = (uint32_t)max(rect.z - rect.x, 0), th = (uint32_t)max(rect.w - rect.y, 0);
@@ -1085,14 +1109,11 @@ __device__ __forceinline__ void bin_group(const BatchDev &b, Lds &lds, uint32_t 
     const uint32_t tbase = it.tbase, cbase = it.cbase;
     const uint32_t gp = it.gp;
     const uint32_t c0 = it.c0, c1 = it.c1;
-    uint32_t *const s_cnt = lds.cnt, *const s_delta = lds.delta;
-    int32_t *const s_col = lds.col;
-    uint32_t *const queue = lds.queue[threadIdx.x >> 6];
+    uint32_t *const queue = queues + WALK_QUEUE * (threadIdx.x >> 6);
     const bool resolve = !EMIT && resolved_here(it);
     const float inv_w = 1.0f / (float)(int)tw;
     // the packed LDS deltas hold sums below 2^15 in magnitude: at most one step per chord
-    const bool in_lds = area <= (uint32_t)BIN_GROUP_TILES && tw <= (uint32_t)BIN_GROUP_COLS &&
-                        (EMIT || c1 - c0 < (1u << 15));
+    const bool in_lds = area <= max_tiles && tw <= max_cols && (EMIT || c1 - c0 < (1u << 15));
     if (in_lds) {
         if (EMIT) {
             const uint2 base = b.path_tot[gp];
@@ -1183,6 +1204,30 @@ __device__ __forceinline__ void bin_group(const BatchDev &b, Lds &lds, uint32_t 
     }
 }
 
+template <bool EMIT, int THREADS, typename Lds>
+__device__ __forceinline__ void bin_group_item(const BatchDev &b, Lds &lds, uint32_t item) {
+    const BinItem it = b.bin_items[b.n_bin_wave + item];
+    if (b.n_big && is_big(it, b.scenes[it.k])) return;  // uniform over the block
+    bin_group<EMIT, THREADS>(b, it, lds.cnt, lds.delta, lds.col, lds.queue[0], BIN_GROUP_TILES, BIN_GROUP_COLS);
+}
+
+// The big paths, listed by k_bin_items, a block of 1024 threads each with the LDS that the batch's largest
+// takes (max_tiles, max_cols).  Through global atomics, a 2048^2 scene of 400 paths with 50 whole-canvas rects
+// (16 384 tiles each) took 80 us to count and 50 to emit; now 22 + 18 and 24 + 20.
+template <bool EMIT>
+__global__ __launch_bounds__(1024) void k_bin_big(BatchDev b, uint32_t max_tiles, uint32_t max_cols) {
+    extern __shared__ uint32_t big_lds[];
+    uint32_t *const cnt = big_lds, *const delta = cnt + max_tiles;
+    uint32_t *const queue = delta + (EMIT ? 0u : (max_tiles + 1) / 2);
+    int32_t *const col = reinterpret_cast<int32_t *>(queue + (1024 / 64) * WALK_QUEUE);
+    const uint32_t n = b.counters[C_BIG];
+    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {  // uniform over the block
+        const BinItem it = b.bin_items[b.big_list[i]];
+        bin_group<EMIT, 1024>(b, it, cnt, delta, col, queue, max_tiles, max_cols);
+        __syncthreads();
+    }
+}
+
 // Both classes in one launch, the group class's paths first (they last longest).  512 threads: a long
 // path's walk is twice as wide as with 256, and 8 wave-class slices (40 KB in the count pass) leave the
 // wave class its 32 waves per CU (which the compiler is held to: 83 -> 80 us at 4096^2 against 7 a SIMD).
@@ -1190,7 +1235,7 @@ template <bool EMIT>
 __global__ __launch_bounds__(512, 8) void k_bin(BatchDev b) {
     __shared__ BinLds<EMIT, 512> lds;
     if (blockIdx.x < b.n_bin_group) {  // uniform over the block
-        bin_group<EMIT, 512>(b, lds.g, blockIdx.x);
+        bin_group_item<EMIT, 512>(b, lds.g, blockIdx.x);
     } else {
         const uint32_t wave = (blockIdx.x - b.n_bin_group) * 8 + (threadIdx.x >> 6);
         bin_wave<EMIT, 512>(b, lds.w, __builtin_amdgcn_readfirstlane(wave));  // uniform: scalar loads
@@ -1207,7 +1252,7 @@ __global__ __launch_bounds__(256) void k_bin_wave(BatchDev b) {
 template <bool EMIT>
 __global__ __launch_bounds__(256) void k_bin_group(BatchDev b) {
     __shared__ BinPath<EMIT, 256> lds;
-    bin_group<EMIT, 256>(b, lds, blockIdx.x);
+    bin_group_item<EMIT, 256>(b, lds, blockIdx.x);
 }
 
 // Item s of a tile sits at LDS word s + s / 16: striped rows (lane-consecutive) and blocked
@@ -1780,16 +1825,19 @@ __device__ __forceinline__ uint2 range_entries(const BatchDev &b, const SceneDev
 }
 
 // One launch for both binning classes, the group class's blocks first.  A block per large path: wave w
-// takes the w-th quarter of the rect's tiles (row-major, in whole 64-tile chunks), so the waves need no
-// barrier.  The count pass keeps each quarter's counts (ent_quarter) beside the path's total; the
-// write pass starts each wave after the quarters before it.  Behind them a wave per small path.
+// takes the w-th part of the rect's tiles (row-major, in whole 64-tile chunks), so the waves need no
+// barrier.  The count pass keeps each part's counts (ent_part) beside the path's total; the
+// write pass starts each wave after the parts before it.  Behind them a wave per small path.
 // A clip path draws nothing: no entries.
-template <bool WRITE, bool CLIPS>
-__global__ __launch_bounds__(256) void k_entries(BatchDev b) {
-    __shared__ uint2 part[4];
+// A wave takes its part's chunks one after the other, so few paths take blocks of 16 waves and many 4 (the
+// launch's choice, WAVES): 400 paths, 50 of them of 16 384 tiles, 22 + 32 us with 4 waves, 8 + 15 with 16;
+// 48 scenes with 67 000 paths 74 + 190 with 4, 90 + 251 with 8.
+template <bool WRITE, bool CLIPS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_entries(BatchDev b) {
+    __shared__ uint2 part[WAVES];
     const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (blockIdx.x >= b.n_bin_group) {  // uniform over the block
-        const uint32_t item = __builtin_amdgcn_readfirstlane((blockIdx.x - b.n_bin_group) * 4 + wv);  // uniform
+        const uint32_t item = __builtin_amdgcn_readfirstlane((blockIdx.x - b.n_bin_group) * WAVES + wv);  // uniform
         if (item >= b.n_bin_wave) return;  // whole wave
         const BinItem it = b.bin_items[item];
         const int4 r = it.rect;
@@ -1803,13 +1851,13 @@ __global__ __launch_bounds__(256) void k_entries(BatchDev b) {
     const BinItem it = b.bin_items[b.n_bin_wave + item];
     const int4 r = it.rect;
     const uint32_t area = CLIPS && it.level != 0 ? 0u : (uint32_t)max(r.z - r.x, 0) * (uint32_t)max(r.w - r.y, 0);
-    const uint32_t q = (area + 255) / 256 * 64;  // tiles per quarter, whole chunks
+    const uint32_t q = (area + 64 * WAVES - 1) / (64 * WAVES) * 64;  // tiles per part, whole chunks
     const uint32_t j0 = min(wv * q, area), j1 = min(j0 + q, area);
     uint2 first = make_uint2(0u, 0u);
     if (WRITE) {
         first = b.path_ent[it.gp];
         for (uint32_t v = 0; v < wv; v++) {
-            const uint2 c = b.ent_quarter[item * 4 + v];
+            const uint2 c = b.ent_part[item * WAVES + v];
             first.x += c.x;
             first.y += c.y;
         }
@@ -1817,13 +1865,15 @@ __global__ __launch_bounds__(256) void k_entries(BatchDev b) {
     const uint2 n = range_entries<WRITE, CLIPS>(b, b.scenes[it.k], it, j0, j1, first);
     if (!WRITE) {
         if (lane == 0) {
-            b.ent_quarter[item * 4 + wv] = n;
+            b.ent_part[item * WAVES + wv] = n;
             part[wv] = n;
         }
         __syncthreads();
-        if (threadIdx.x == 0)
-            b.path_ent[it.gp] = make_uint2(part[0].x + part[1].x + part[2].x + part[3].x,
-                                           part[0].y + part[1].y + part[2].y + part[3].y);
+        if (threadIdx.x == 0) {
+            uint2 n_all = part[0];
+            for (uint32_t v = 1; v < WAVES; v++) n_all = make_uint2(n_all.x + part[v].x, n_all.y + part[v].y);
+            b.path_ent[it.gp] = n_all;
+        }
     }
 }
 
@@ -2240,6 +2290,13 @@ template <bool EMIT>
 static void launch_bin_t(const BatchDev &b, hipStream_t s) {
     const uint32_t merged = b.n_bin_group + blocks_for(b.n_bin_wave, 8);
     if (merged == 0) return;
+    if (b.n_big) {  // first: they last longest
+        const uint32_t cols = std::max(b.big_cols, 64u);  // at least what a block's sums take
+        const size_t lds = 4 * ((size_t)b.big_tiles + (EMIT ? 0 : (b.big_tiles + 1) / 2) + (1024 / 64) * WALK_QUEUE + cols);
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bin_big<EMIT>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)lds);
+        hipLaunchKernelGGL(k_bin_big<EMIT>, dim3(std::min<uint32_t>(b.n_big, 1024)), dim3(1024), lds, s, b, b.big_tiles, cols);
+    }
     if (merged <= BIN_MERGED_BLOCKS) {
         hipLaunchKernelGGL(k_bin<EMIT>, dim3(merged), dim3(512), 0, s, b);
         return;
@@ -2264,15 +2321,30 @@ hipError_t launch_propagate(const BatchDev &b, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Waves of a group-class path in the entry passes: 16 up to this many blocks of them, 4 (the two rounds of
+// blocks that the chip then holds) beyond.
+constexpr uint32_t ENT_WIDE_BLOCKS = 1024;
+
+uint32_t entry_waves(uint32_t n_bin_group, uint32_t n_bin_wave) {
+    return n_bin_group + blocks_for(n_bin_wave, 16) <= ENT_WIDE_BLOCKS ? 16 : 4;
+}
+
+template <bool WRITE, bool CLIPS>
+static void launch_entries_t(const BatchDev &b, hipStream_t s) {
+    const uint32_t waves = entry_waves(b.n_bin_group, b.n_bin_wave);
+    const dim3 g(b.n_bin_group + blocks_for(b.n_bin_wave, waves));
+    if (g.x == 0) return;
+    if (waves == 16) hipLaunchKernelGGL((k_entries<WRITE, CLIPS, 16>), g, dim3(1024), 0, s, b);
+    else hipLaunchKernelGGL((k_entries<WRITE, CLIPS, 4>), g, dim3(256), 0, s, b);
+}
+
 hipError_t launch_entries(const BatchDev &b, bool write, hipStream_t s) {
-    const dim3 g(b.n_bin_group + blocks_for(b.n_bin_wave, 4));
-    if (g.x == 0) return hipSuccess;
     if (b.has_clips) {
-        if (write) hipLaunchKernelGGL((k_entries<true, true>), g, dim3(256), 0, s, b);
-        else hipLaunchKernelGGL((k_entries<false, true>), g, dim3(256), 0, s, b);
+        if (write) launch_entries_t<true, true>(b, s);
+        else launch_entries_t<false, true>(b, s);
     } else {
-        if (write) hipLaunchKernelGGL((k_entries<true, false>), g, dim3(256), 0, s, b);
-        else hipLaunchKernelGGL((k_entries<false, false>), g, dim3(256), 0, s, b);
+        if (write) launch_entries_t<true, false>(b, s);
+        else launch_entries_t<false, false>(b, s);
     }
     return hipGetLastError();
 }

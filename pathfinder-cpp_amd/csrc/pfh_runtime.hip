@@ -31,6 +31,7 @@ hipError_t scan_counted(uint32_t *inout, const uint32_t *n_ptr, uint32_t cap, un
 hipError_t launch_flatten(const BatchDev &b, bool emit, uint32_t chunk, hipStream_t s);
 hipError_t launch_bin(const BatchDev &b, bool emit, hipStream_t s);
 hipError_t launch_propagate(const BatchDev &b, hipStream_t s);
+uint32_t entry_waves(uint32_t n_bin_group, uint32_t n_bin_wave);
 hipError_t launch_entries(const BatchDev &b, bool write, hipStream_t s);
 hipError_t launch_bin_items(const BatchDev &b, hipStream_t s);
 size_t sort_temp_elems(uint64_t cap, uint32_t n_scenes, uint32_t max_fb, uint64_t max_tiles);
@@ -318,6 +319,7 @@ struct SceneHost {
     std::vector<uint32_t> path_paint;
     bool has_ops = false;  // some record composites through an op
     DevBuf d_path_paint, d_paints, d_ramps;
+    uint32_t n_big = 0, big_tiles = 0, big_cols = 0;  // rects past a bin block's LDS that fit a larger one's
     uint32_t n_bin_wave = 0, n_bin_group = 0;  // paths binned by one wave / by one workgroup
     void release() {  // once the device is done with the scene
         d_block.release();
@@ -370,9 +372,9 @@ struct Workspace {
     // around the fill and composite kernels of a batched launch; recorded as event nodes
     // inside captured graphs, so replays time those kernels too
     hipEvent_t kev[3] = {nullptr, nullptr, nullptr};
-    DevBuf scene_table, bases, tile_delta, tile_cnt, tile_fill_off, tile_alpha_idx, tile_bd, tile_st, path_ent, ent_quarter, path_tot, bin_items, col_bd, seg_mask,
+    DevBuf scene_table, bases, tile_delta, tile_cnt, tile_fill_off, tile_alpha_idx, tile_bd, tile_st, path_ent, ent_part, path_tot, bin_items, col_bd, seg_mask,
         seg_cnt, lines, line_cnt, fills, dump_fills, alpha_rec, alpha_vis, masks, zbuf, fb_range, keys, keys_alt,
-        rec_alt, entry_rec, entry_meta, meta_alt, counters, chunk_off, scan_state, dump_state, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen, prop_strips;
+        rec_alt, entry_rec, entry_meta, meta_alt, counters, chunk_off, scan_state, dump_state, sort_tmp, tile_clip_ai, clip_jobs, clip_rec, clip_seen, prop_strips, big_list;
     // pinned and coherent: kernels write h_counters and read the tables
     uint32_t *h_counters = nullptr;
     SceneDev *h_table = nullptr;     // pinned scene table
@@ -449,9 +451,9 @@ struct Workspace {
     }
     std::vector<DevBuf *> all_buffers() {
         return {&scene_table, &bases, &tile_delta, &tile_cnt, &tile_fill_off, &tile_alpha_idx, &tile_bd, &tile_st,
-                &path_ent, &ent_quarter, &path_tot, &bin_items, &col_bd, &seg_mask, &seg_cnt, &lines, &line_cnt, &fills, &dump_fills, &alpha_rec, &alpha_vis,
+                &path_ent, &ent_part, &path_tot, &bin_items, &col_bd, &seg_mask, &seg_cnt, &lines, &line_cnt, &fills, &dump_fills, &alpha_rec, &alpha_vis,
                 &masks, &zbuf, &fb_range, &keys, &keys_alt, &rec_alt, &entry_rec, &entry_meta, &meta_alt, &counters, &chunk_off, &scan_state, &dump_state,
-                &sort_tmp, &tile_clip_ai, &clip_jobs, &clip_rec, &clip_seen, &prop_strips};
+                &sort_tmp, &tile_clip_ai, &clip_jobs, &clip_rec, &clip_seen, &prop_strips, &big_list};
     }
     size_t device_bytes() {
         size_t n = 0;
@@ -1408,6 +1410,13 @@ static int scene_upload_desc(pfh_ctx *ctx, const pfh_scene_desc *d) {
         if (w * h <= (uint64_t)BIN_WAVE_TILES && w <= (uint64_t)BIN_WAVE_COLS && nseg <= (uint64_t)BIN_WAVE_SEGS)
             bin_wave.push_back((uint32_t)p);
         else bin_group.push_back((uint32_t)p);
+        if (w == (uint64_t)s->fb_w && h == (uint64_t)s->fb_h &&
+            (w * h > (uint64_t)BIN_GROUP_TILES || w > (uint64_t)BIN_GROUP_COLS) && w * h <= (uint64_t)BIN_BIG_TILES &&
+            w <= (uint64_t)BIN_BIG_COLS) {
+            s->n_big++;
+            s->big_tiles = std::max(s->big_tiles, (uint32_t)(w * h));
+            s->big_cols = std::max(s->big_cols, (uint32_t)w);
+        }
     }
     s->n_bin_wave = (uint32_t)bin_wave.size();
     s->n_bin_group = (uint32_t)bin_group.size();
@@ -1567,6 +1576,7 @@ struct Plan {
     uint32_t cap_f = 0, cap_a = 0, cap_e = 0, cap_l = 0;
     uint32_t max_fb = 1;         // the largest scene's framebuffer tiles and path tiles
     uint64_t max_tiles = 0;
+    uint32_t n_big = 0, big_tiles = 1, big_cols = 1;  // the batch's big rects (SceneHost::n_big)
     uint64_t deep_tiles = 0;     // path tiles of scenes covered HIDE_DEPTH deep
     Schedule sched;
 };
@@ -1622,8 +1632,9 @@ static void ensure_sizes(Workspace &w, const Plan &pl, bool dump) {
     }
     w.tile_st.ensure(pl.T + 4);
     w.path_ent.ensure(8 * pl.P + 8);
-    w.ent_quarter.ensure(32 * pl.BG + 32);
+    w.ent_part.ensure(8ull * entry_waves((uint32_t)pl.BG, (uint32_t)pl.BW) * pl.BG + 32);
     w.path_tot.ensure(8 * pl.P + 8);
+    if (pl.n_big) w.big_list.ensure(4ull * pl.n_big);
     w.bin_items.ensure(sizeof(BinItem) * (pl.BW + pl.BG) + 64);
     w.col_bd.ensure(4 * pl.W + 4);
     w.seg_cnt.ensure(4 * pl.S + 8);
@@ -1757,6 +1768,9 @@ static void write_tables(pfh_ctx *ctx, Plan &pl, bool load_dst) {
         pl.clips = pl.clips || s.n_clip > 0;
         pl.paints = pl.paints || !s.path_paint.empty();
         pl.clip_levels = std::max(pl.clip_levels, s.clip_levels);
+        pl.n_big += s.n_big;
+        pl.big_tiles = std::max(pl.big_tiles, s.big_tiles);
+        pl.big_cols = std::max(pl.big_cols, s.big_cols);
         T += s.n_tiles;
         W += s.n_cols;
         FB += d.n_fb;
@@ -1842,6 +1856,10 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
     b.tile_bd = (dump || pl.clips) ? w.tile_bd.as<int8_t>() : nullptr;
     b.tile_clip_ai = pl.clips ? w.tile_clip_ai.as<uint32_t>() : nullptr;
     b.clip_jobs = pl.clips ? w.clip_jobs.as<uint2>() : nullptr;
+    b.big_list = w.big_list.as<uint32_t>();
+    b.n_big = pl.n_big;
+    b.big_tiles = pl.big_tiles;
+    b.big_cols = pl.big_cols;
     b.prop_strips = pl.clips ? w.prop_strips.as<uint2>() : nullptr;
     b.cap_strips = pl.clips ? (uint32_t)strips_cap(pl) : 0;
     b.clip_rec = pl.clips ? w.clip_rec.as<uint4>() : nullptr;
@@ -1850,7 +1868,7 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
     b.has_clips = pl.clips ? 1 : 0;
     b.tile_st = w.tile_st.as<uint8_t>();
     b.path_ent = w.path_ent.as<uint2>();
-    b.ent_quarter = w.ent_quarter.as<uint2>();
+    b.ent_part = w.ent_part.as<uint2>();
     b.path_tot = w.path_tot.as<uint2>();
     b.bin_items = w.bin_items.as<BinItem>();
     b.n_paths = (uint32_t)pl.P;

@@ -66,3 +66,30 @@ def test_strips_of_clips_and_clipped_paths(cols, rows):
         ctx.rasterize([sid], flags)
         np.testing.assert_array_equal(ctx.readback(sid), img)
     ctx.close()
+
+
+def whole_canvas(sc, n):
+    """The first n paths in a blend mode whose rect is the view box (built_path.cpp:21)."""
+    sc.path_blend = np.full(sc.n_paths, 4, np.uint8)
+    sc.path_blend[:n] = 5  # source-in
+    return sc
+
+
+@pytest.mark.parametrize("name,sc", [
+    # rects on both sides of a bin block's LDS (5 700 tiles, 512 columns) and of the larger one's (25 000, 1 024)
+    ("square", rects([(0, 0, 16 * 75, 16 * 76), (0, 0, 16 * 76, 16 * 76), (5, 5, 2500, 2500), (0, 0, 2560, 2560)],
+                     2560, 2560)),
+    ("whole", rects([(0, 0, 16 * 158, 16 * 158), (0, 0, 16 * 60, 16 * 60)], 16 * 158, 16 * 158)),
+    ("wide", rects([(0, 3, 16 * k, 30) for k in (512, 513, 1024, 1025)], 16 * 1030, 48)),
+    ("small whole canvas", whole_canvas(scenegen.blob_scene(21, 200, 130, 40), 3)),
+    ("large whole canvas", whole_canvas(scenegen.blob_scene(22, 1500, 1100, 60), 3)),
+])
+def test_large_rects(name, sc):
+    ctx = pfh.Context(0)
+    _, img = check_scene(ctx, sc, name=name)
+    sid, other = ctx.upload(sc), ctx.upload(scenegen.blob_scene(23, 1024, 1024, 20000, r_max=300.0))  # entries by 4 waves
+    for ids in ([sid], [sid, other]):
+        for flags in (pfh.PFH_BATCHED | pfh.PFH_NO_GRAPH, pfh.PFH_BATCHED):
+            ctx.rasterize(ids, flags)
+            np.testing.assert_array_equal(ctx.readback(sid), img)
+    ctx.close()
