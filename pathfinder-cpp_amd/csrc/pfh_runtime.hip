@@ -2062,6 +2062,11 @@ static void rasterize_plain(pfh_ctx *ctx, int32_t id, uint32_t flags) {
         pl.cap_a = clamp_cap(std::max<uint64_t>(na, pl.cap_a));
         ensure_sizes(*ctx->w, pl, dump);
         b = batch_dev(*ctx->w, pl, dump);
+        if (b.clip_seen) {  // cleared at its size before, if it is the same memory at all
+            ZeroSpans z{};
+            z.add(b.clip_seen, (uint64_t)b.cap_alpha / 32 + 1);
+            HIP_TRY(launch_zero_spans(z, st));
+        }
     }
     if (dump) dump_offsets(*ctx->w, b, nl);
     HIP_TRY(launch_bin(b, true, st));

@@ -93,3 +93,22 @@ def test_large_rects(name, sc):
             ctx.rasterize(ids, flags)
             np.testing.assert_array_equal(ctx.readback(sid), img)
     ctx.close()
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_first_plain_pass_with_clips(seed):
+    """A new context's first stage-by-stage pass grows its buffers half way, in memory that earlier
+    contexts have used: the set of mask rows already listed starts empty there too."""
+    sc = scenegen.clip_scene(60 + seed, size=900, n_draw=150, n_clip=12)
+    imgs = []
+    for _ in range(3):
+        ctx = pfh.Context(0)
+        sid = ctx.upload(sc)
+        for _ in range(2):
+            ctx.rasterize([sid], pfh.PFH_PLAIN)
+            imgs.append(ctx.readback(sid))
+        ctx.rasterize([sid], pfh.PFH_BATCHED | pfh.PFH_NO_GRAPH | pfh.PFH_DUMP)
+        imgs.append(ctx.readback(sid))
+        ctx.close()
+    for img in imgs[1:]:
+        np.testing.assert_array_equal(img, imgs[0])
