@@ -1034,16 +1034,22 @@ __device__ __forceinline__ float fill_rule_f(float c, uint32_t even_odd) {
 // A draw job writes the draw path's fill rule of it to its row; a nested clip path's job writes
 // the nonzero and the even-odd rule of it to its two rows.  Where clip paths' own rules are taken
 // (CLIP_JOB_OWN_RULES) each term is its row's fill rule of fills + backdrop instead, and the min
-// of those is the coverage, written as it is.  Each lane owns 4 pixels of one column;
-// the 4 waves take every 4th fill of every term and their partial sums meet in LDS, so a long fill
-// list costs a quarter of its length in serial steps.
+// of those is the coverage, written as it is.  Each lane owns 4 pixels of one column; the 4 waves take
+// every 4th fill of a term and their partial sums meet in LDS (two buffers in turn: one barrier a term),
+// where each wave takes one of the 4 pixels.
+// A tile's fills arrive in any order, so their sum must not depend on it: each area is rounded to 2^-32
+// and added in a double, exactly (below 2^21 fills).  Summed in float, a pixel of coverage next to
+// half a byte step came out one way or the other from pass to pass (a 1278^2 scene of 1 185 paths and 94
+// clips: two images in 54 passes); 20.4 us on the 4096^2 scene with 200 clips, 19.7 so.
 constexpr int CLIP_TERMS = MAX_CLIP_LEVELS + 1;
+constexpr float CLIP_ONE = 4294967296.0f;  // the areas' unit
 
 __global__ __launch_bounds__(256) void k_fill_clipped(BatchDev b) {
-    __shared__ float part[CLIP_TERMS][4][4][64];  // term x wave x pixel row offset x lane
+    __shared__ double part[2][4][4][64];  // buffer x wave x pixel row offset x lane
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const uint32_t n = min(b.counters[C_CLIP_JOBS], b.cap_alpha);
     const float px = (float)(lane & 15u), py0 = (float)((lane >> 4) * 4u);
+    uint32_t buf = 0;
     for (uint32_t j = blockIdx.x; j < n; j += gridDim.x) {  // uniform over the block
         const uint2 job = b.clip_jobs[j];
         const bool clip_job = (job.x & CLIP_JOB_CLIP) != 0, own_rules = (job.x & CLIP_JOB_OWN_RULES) != 0;
@@ -1057,50 +1063,35 @@ __global__ __launch_bounds__(256) void k_fill_clipped(BatchDev b) {
         const uint32_t term[CLIP_TERMS] = {out, src, rec.y, rec.z, rec.w};
 #pragma unroll
         for (int k = 0; k < CLIP_TERMS; k++) ok = ok && ((uint32_t)k < first || (uint32_t)k >= nt || term[k] < b.cap_alpha);
-        int8_t bdk[CLIP_TERMS];
-        uint32_t rk[CLIP_TERMS];  // each term's fill rule (its row's)
+        if (!ok) continue;  // uniform over the block
+        uint32_t rule = 0;  // the draw path's
+        float m = INFINITY;  // the least term at this thread's pixel
 #pragma unroll
         for (int k = 0; k < CLIP_TERMS; k++) {
-            bdk[k] = 0;
-            rk[k] = 0;
-            if ((uint32_t)k < first || (uint32_t)k >= nt) continue;
-            const uint4 r = ok ? b.alpha_rec[term[k]] : make_uint4(0, 0, 0, 0);
-            bdk[k] = (int8_t)(r.z & 0xffu);
-            rk[k] = (r.z >> 8) & 1u;
-            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if ((uint32_t)k < first || (uint32_t)k >= nt) continue;  // uniform over the block
+            const uint4 r = b.alpha_rec[term[k]];
+            const uint32_t rk = (r.z >> 8) & 1u;
+            if (k == 0) rule = rk;
+            double acc[4] = {0.0, 0.0, 0.0, 0.0};
             const uint32_t f0 = min(r.x, b.cap_fills), f1 = max(f0, min(r.y, b.cap_fills));
             for (uint32_t f = f0 + wv; f < f1; f += 4) {
                 const uint2 fl = b.fills[f];
 #pragma unroll
-                for (int q = 0; q < 4; q++) acc[q] += fill_area_at(fl, px, py0 + (float)q);
+                for (int q = 0; q < 4; q++) acc[q] += (double)rintf(fill_area_at(fl, px, py0 + (float)q) * CLIP_ONE);
             }
 #pragma unroll
-            for (int q = 0; q < 4; q++) part[k][wv][q][lane] = acc[q];
+            for (int q = 0; q < 4; q++) part[buf][wv][q][lane] = acc[q];
+            __syncthreads();  // of the term after next, whose sums come here again, every thread has passed the next one
+            const double sum = part[buf][0][wv][lane] + part[buf][1][wv][lane] + part[buf][2][wv][lane] + part[buf][3][wv][lane];
+            const float v = (float)((double)(int8_t)(r.z & 0xffu) + sum * (1.0 / (double)CLIP_ONE));
+            m = fminf(m, own_rules ? fill_rule_f(v, rk) : fabsf(v));
+            buf ^= 1u;
         }
-        __syncthreads();
-        if (wv == 0 && ok) {
-            const uint32_t rule = clip_job ? 0u : (b.alpha_rec[out].z >> 8) & 1u;
-            uint32_t packed = 0, packed_eo = 0;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                float m = INFINITY;
-#pragma unroll
-                for (int k = 0; k < CLIP_TERMS; k++) {
-                    if ((uint32_t)k < first || (uint32_t)k >= nt) continue;
-                    const float v = (float)bdk[k] + part[k][0][q][lane] + part[k][1][q][lane] + part[k][2][q][lane] +
-                                    part[k][3][q][lane];
-                    m = fminf(m, own_rules ? fill_rule_f(v, rk[k]) : fabsf(v));
-                }
-                const float c = own_rules ? m : fill_rule_f(m, rule), c_eo = own_rules ? m : fill_rule_f(m, 1u);
-                packed |= (uint32_t)__float2int_rn(c * 255.0f) << (8 * q);
-                packed_eo |= (uint32_t)__float2int_rn(c_eo * 255.0f) << (8 * q);
-            }
-            // column-major mask: byte 16 x + y
-            const uint32_t off = (lane & 15u) * 16 + (lane >> 4) * 4;
-            *reinterpret_cast<uint32_t *>(b.masks + (uint64_t)out * 256 + off) = packed;
-            if (clip_job) *reinterpret_cast<uint32_t *>(b.masks + (uint64_t)(out + 1) * 256 + off) = packed_eo;
-        }
-        __syncthreads();  // the next job rewrites the partial sums
+        const float c = own_rules ? m : fill_rule_f(m, rule), c_eo = own_rules ? m : fill_rule_f(m, 1u);
+        // column-major mask: byte 16 x + y
+        const uint32_t off = (lane & 15u) * 16 + (lane >> 4) * 4 + wv;
+        b.masks[(uint64_t)out * 256 + off] = (uint8_t)__float2int_rn(c * 255.0f);
+        if (clip_job) b.masks[(uint64_t)(out + 1) * 256 + off] = (uint8_t)__float2int_rn(c_eo * 255.0f);
     }
 }
 

@@ -39,3 +39,19 @@ def test_first_plain_pass_in_used_memory(seed):
         ctx.close()
         for b in kept:
             b.free()
+
+
+def test_every_pass_draws_the_same_bytes():
+    """A tile's fills come in any order; where a clipped path's mask meets its clip's, the coverage is a sum
+    over them and has to be the same one in every pass.  This scene has a pixel next to half a byte step."""
+    sc = scenegen.stress_scene(scenegen.BASE_SEED ^ (32 * 7919 + 13), 1278, 948, 237, 94)
+    ctx = pfh.Context(0)
+    sid = ctx.upload(sc)
+    ctx.rasterize([sid], pfh.PFH_PLAIN)
+    first = ctx.readback(sid)
+    for p in range(23):
+        ctx.rasterize([sid], pfh.PFH_PLAIN if p % 2 else pfh.PFH_BATCHED | pfh.PFH_NO_GRAPH)
+        np.testing.assert_array_equal(ctx.readback(sid), first, err_msg=f"pass {p}")
+    want = np.rint(np.clip(oracle.full_model(sc, zmode=1)["image"], 0.0, 1.0) * 255.0).astype(np.int64)
+    assert np.abs(first.astype(np.int64) - want).max() <= 1
+    ctx.close()
