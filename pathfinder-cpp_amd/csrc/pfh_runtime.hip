@@ -212,17 +212,26 @@ struct DevBuf {
 };
 
 // Pinned host memory that copies go through, two halves in turn: a copy to or from ordinary memory
-// costs tens of microseconds on its own, and one with a pitch a transfer per row.
+// costs tens of microseconds on its own, and one with a pitch a transfer per row.  The host reads and
+// refills a half once the copy before it is done, which its event tells: the memory is coherent and the
+// events keep their system fence, so that what the device wrote can be seen then.
 struct Stage {
     static constexpr size_t HALF = 1u << 20;
     uint8_t *ptr = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};  // of the last copy of each half
     uint8_t *get() {
-        if (!ptr) HIP_TRY(hipHostMalloc((void **)&ptr, 2 * HALF));
+        if (!ptr) HIP_TRY(hipHostMalloc((void **)&ptr, 2 * HALF, hipHostMallocCoherent));
+        for (auto &e : ev)
+            if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         return ptr;
     }
     void release() {
         if (ptr) (void)hipHostFree(ptr);
         ptr = nullptr;
+        for (auto &e : ev) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
     }
 };
 
@@ -231,11 +240,11 @@ struct Stage {
 struct StageOut {
     uint8_t *const stage, *dev;
     hipStream_t st;
-    hipEvent_t *ev;  // two
+    hipEvent_t *ev;
     size_t fill = 0, half = 0;
     bool pending[2] = {false, false};
-    StageOut(Stage &s, void *to, hipStream_t stream, hipEvent_t *events)
-        : stage(s.get()), dev(static_cast<uint8_t *>(to)), st(stream), ev(events) {}
+    StageOut(Stage &s, void *to, hipStream_t stream)
+        : stage(s.get()), dev(static_cast<uint8_t *>(to)), st(stream), ev(s.ev) {}
     void put(const void *src, size_t n) {  // src null: n bytes of no meaning
         const uint8_t *from = static_cast<const uint8_t *>(src);
         while (n) {
@@ -246,18 +255,20 @@ struct StageOut {
             }
             fill += k;
             n -= k;
-            if (fill == Stage::HALF) flush();
+            if (fill == Stage::HALF) {
+                flush();
+                HIP_TRY(hipEventRecord(ev[half], st));
+                pending[half] = true;
+                half ^= 1;
+                if (pending[half]) HIP_TRY(hipEventSynchronize(ev[half]));
+            }
         }
     }
-    void flush() {
+    void flush() {  // at the end: what is left
         if (!fill) return;
         HIP_TRY(hipMemcpyAsync(dev, stage + half * Stage::HALF, fill, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipEventRecord(ev[half], st));
-        pending[half] = true;
         dev += fill;
         fill = 0;
-        half ^= 1;
-        if (pending[half]) HIP_TRY(hipEventSynchronize(ev[half]));
     }
 };
 
@@ -278,10 +289,10 @@ struct Upload {
         total += (std::max<size_t>(n, 4) + 255) & ~(size_t)255;
     }
     // Enqueues the copies on st.
-    void send(DevBuf &block, Arena &arena, Stage &stage, hipStream_t st, hipEvent_t *ev) {
+    void send(DevBuf &block, Arena &arena, Stage &stage, hipStream_t st) {
         block.ensure(total);
         arena = Arena{block.as<uint8_t>(), total, 0};
-        StageOut out(stage, block.ptr, st, ev);
+        StageOut out(stage, block.ptr, st);
         for (const Part &p : parts) {
             p.buf->arena = &arena;
             p.buf->ptr = nullptr;
@@ -391,7 +402,7 @@ struct Workspace {
     // that a launch of at most that many scenes creates nothing.
     void create(size_t table_scenes = 0) {
         HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-        // the host waits for ev1 alone: the others only time, without a fence for it (3 us less each)
+        // of these the host waits for ev1 alone: the others only time, without a fence for it (3 us less each)
         HIP_TRY(hipEventCreateWithFlags(&ev0, hipEventDisableSystemFence));
         HIP_TRY(hipEventCreate(&ev1));
         for (auto &e : kev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
@@ -830,21 +841,25 @@ static void read_rows(pfh_ctx *ctx, uint8_t *dst, size_t dst_pitch, const uint8_
     const size_t n = (all + per - 1) / per;
     uint8_t *const stage = ctx->stage.get();
     hipStream_t st = ctx->w->stream;
-    hipEvent_t *ev = ctx->w->stage_ev;
+    hipEvent_t *ev = ctx->stage.ev;
     auto fetch = [&](size_t k) {
         const size_t at = k * per, m = std::min(per, all - at);
         HIP_TRY(hipMemcpyAsync(stage + (k & 1) * Stage::HALF, src + (flat ? at : at * src_pitch),
                                flat ? m : (m - 1) * src_pitch + row, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipEventRecord(ev[k & 1], st));
+        if (k + 1 < n) HIP_TRY(hipEventRecord(ev[k & 1], st));
     };
     struct Drain {  // nothing writes to the stage after an error
         hipStream_t st;
-        ~Drain() { (void)hipStreamSynchronize(st); }
+        bool done = false;
+        ~Drain() {
+            if (!done) (void)hipStreamSynchronize(st);
+        }
     } drain{st};
     fetch(0);
     for (size_t k = 0; k < n; k++) {
         if (k + 1 < n) fetch(k + 1);
-        HIP_TRY(hipEventSynchronize(ev[k & 1]));
+        HIP_TRY(k + 1 < n ? hipEventSynchronize(ev[k & 1]) : hipStreamSynchronize(st));
+        drain.done = k + 1 == n;
         const size_t at = k * per, m = std::min(per, all - at);
         const uint8_t *from = stage + (k & 1) * Stage::HALF;
         if (flat) {
@@ -874,7 +889,7 @@ template <typename T>
 static void h2d(pfh_ctx *ctx, DevBuf &buf, const std::vector<T> &v) {
     const size_t n = v.size() * sizeof(T);
     buf.ensure(std::max<size_t>(n, 4));
-    StageOut out(ctx->stage, buf.ptr, ctx->w->stream, ctx->w->stage_ev);
+    StageOut out(ctx->stage, buf.ptr, ctx->w->stream);
     out.put(v.data(), n);
     out.flush();
     HIP_TRY(hipStreamSynchronize(ctx->w->stream));
@@ -1507,7 +1522,7 @@ static int scene_upload_desc(pfh_ctx *ctx, const pfh_scene_desc *d) {
             s->release();
         }
     } give_back{ctx, s.get()};
-    up.send(s->d_block, s->arena, ctx->stage, ctx->w->stream, ctx->w->stage_ev);
+    up.send(s->d_block, s->arena, ctx->stage, ctx->w->stream);
     s->d_features.pool = &ctx->pool;
     s->d_features.ensure(4ull * N_FEATURES * s->n_paths + 4);
     HIP_TRY(path_features(s->d_pts.as<float2>(), s->d_segs.as<uint2>(), s->d_path_seg_off.as<uint32_t>(),

@@ -1,0 +1,73 @@
+"""The host runtime's calls in their order, on a HIP runtime that only records them (hip_recorder.cpp; no GPU):
+what the host waits for before it reads memory that the device wrote."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+NO_FENCE = 0x20000000   # hipEventDisableSystemFence
+COHERENT = 0x40000000   # hipHostMallocCoherent
+
+
+@pytest.fixture(scope="module")
+def recorder(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip") / "hip_recorder.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", os.path.join(HERE, "hip_recorder.cpp"), "-o", so], check=True)
+    return so
+
+
+def run(recorder, scenario):
+    """A scenario of this file in a process whose HIP runtime is the recorder."""
+    code = f"import sys; sys.path.insert(0, {HERE!r}); import test_runtime_order as t; t.{scenario}(t.Hip({recorder!r}))"
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+class Hip:
+    """The recorder, loaded before the library so that the library's calls go to it."""
+
+    def __init__(self, so):
+        import conftest  # noqa: F401  (import paths)
+
+        self.lib = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)
+        self.lib.rec_log.restype = ctypes.c_char_p
+        self.lib.rec_held.restype = ctypes.c_size_t
+        self.lib.rec_limit.argtypes = [ctypes.c_size_t]
+
+    def take(self):
+        """The calls since the last time, as lists of words."""
+        calls = [line.split() for line in self.lib.rec_log().decode().splitlines()]
+        self.lib.rec_clear()
+        return calls
+
+
+def waits_scenario(hip):
+    import pfh
+    import scenegen
+
+    ctx = pfh.Context(0)
+    sid = ctx.upload(scenegen.blob_scene(1, 1024, 1024, 6000))  # several halves of the stage, both ways
+    ctx.rasterize([sid])
+    ctx.readback(sid)
+    ctx.features(sid)
+    calls = hip.take()
+    flags = {c[1]: int(c[2], 16) for c in calls if c[0] == "hipEventCreate"}
+    pinned = [(int(c[1], 16), int(c[2]), int(c[3], 16)) for c in calls if c[0] == "hipHostMalloc"]
+    waited = {c[1] for c in calls if c[0] == "hipEventSynchronize"}
+    assert len(waited) >= 2
+    for e in waited:
+        assert not flags[e] & NO_FENCE, "the host waits on an event after which device writes need not be visible"
+    read = [c for c in calls if c[0] == "hipMemcpyAsync" and c[4] == "2"]
+    assert read
+    for c in read:
+        p = [f for base, n, f in pinned if base <= int(c[1], 16) < base + n]
+        assert p and p[0] & COHERENT, "a copy for the host goes to memory whose coherence depends on the environment"
+    last = max(k for k, c in enumerate(calls) if c in read)
+    assert ["hipStreamSynchronize", calls[last][5]] in calls[last + 1:]
+
+
+def test_the_host_waits_for_what_it_reads(recorder):
+    run(recorder, "waits_scenario")
