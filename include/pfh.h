@@ -239,6 +239,7 @@ const char *pfh_last_error(const pfh_ctx *ctx);
  * core/d3d11/scene_builder.cpp:26-58).  *scene_id receives a handle.
  */
 int pfh_scene_upload(pfh_ctx *ctx, const pfh_scene_desc *desc, int32_t *scene_id);
+/* Where pfh_scene_target gave out the scene's own image, work queued on it on any stream ends first. */
 int pfh_scene_release(pfh_ctx *ctx, int32_t scene_id);
 
 /* Per-path features of an uploaded scene for the sizing predictor: [n_paths * 12] floats. */

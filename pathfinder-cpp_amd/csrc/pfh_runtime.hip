@@ -123,8 +123,9 @@ struct Arena {
 // Device blocks that one use gave back and the next takes: a program that uploads a scene every frame
 // otherwise spends a millisecond on hipMalloc and hipFree (which waits for the device).  Blocks of
 // 2^k bytes up to BLOCK_BYTES, at most POOL_BYTES of them in all; the rest goes back to the runtime at once, the
-// others when the context ends.  A block is given back only when the device is done with it, and a
-// context is used by one host thread at a time.
+// others when the context ends.  A block is given back only when the device is done with it (for an
+// image whose address a caller has, the whole device: see pfh_scene_release), and a context is used by
+// one host thread at a time.
 struct BlockPool {
     static constexpr size_t BLOCK_BYTES = 64u << 20, POOL_BYTES = 256u << 20;
     std::multimap<size_t, void *> blocks;
@@ -339,6 +340,7 @@ struct SceneHost {
     }
     uint8_t *d_out = nullptr;
     int64_t out_pitch = 0;
+    bool lent = false;  // a caller has the address of d_out_owned (pfh_scene_target)
     // placement in the last rasterized batch (for dumps)
     bool dumped = false;
     uint32_t seg_base = 0, tile_base = 0, col_base = 0, fb_base = 0, path_base = 0;
@@ -2613,7 +2615,11 @@ int pfh_scene_release(pfh_ctx *ctx, int32_t scene_id) {
             if (queued || ((size_t)scene_id < sv.scene_busy.size() && sv.scene_busy[scene_id]))
                 throw PfhError{PFH_E_STATE, "scene has requests in the request loop"};
         }
+        // The context's passes over the scene are over.  With the image's address the caller may have queued
+        // work of its own on any stream, or have pointed another scene's target there: that ends too
+        // before the block goes to the next scene, as it did before a hipFree.
         HIP_TRY(hipStreamSynchronize(ctx->w->stream));
+        if (s.lent) HIP_TRY(hipDeviceSynchronize());
         drop_graphs_of_scene(ctx, scene_id);
         s.release();
         ctx->scenes[scene_id].reset();
@@ -2704,6 +2710,7 @@ int pfh_scene_target(pfh_ctx *ctx, int32_t scene_id, void **device_rgba8, int64_
     if (!ctx || !device_rgba8 || !pitch_bytes) return PFH_E_ARG;
     return run_guarded(ctx, [&] {
         SceneHost &s = get_scene(ctx, scene_id);
+        s.lent = s.lent || s.d_out == s.d_out_owned.as<uint8_t>();
         *device_rgba8 = s.d_out;
         *pitch_bytes = s.out_pitch;
     });

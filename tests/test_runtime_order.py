@@ -1,5 +1,5 @@
 """The host runtime's calls in their order, on a HIP runtime that only records them (hip_recorder.cpp; no GPU):
-what the host waits for before it reads memory that the device wrote."""
+what the host waits for before it reads memory that the device wrote, and before memory changes hands."""
 import ctypes
 import os
 import subprocess
@@ -71,3 +71,25 @@ def waits_scenario(hip):
 
 def test_the_host_waits_for_what_it_reads(recorder):
     run(recorder, "waits_scenario")
+
+
+def release_scenario(hip):
+    import pfh
+    import scenegen
+
+    ctx = pfh.Context(0)
+    for own_target in (False, True):
+        sid = ctx.upload(scenegen.blob_scene(2, 500, 300, 20))
+        if own_target:  # and back again
+            ctx.set_target(sid, ctx.target(ctx.upload(scenegen.blob_scene(3, 500, 300, 20)))[0], 2000)
+            ctx.set_target(sid, None, 0)
+        ctx.rasterize([sid])
+        image, _ = ctx.target(sid)  # a caller's kernel on a stream of its own may read it from here on
+        hip.take()
+        ctx.release(sid)
+        calls = hip.take()
+        assert ["hipDeviceSynchronize"] in calls or ["hipFree", hex(image)] in calls
+
+
+def test_release_waits_for_work_on_a_lent_image(recorder):
+    run(recorder, "release_scenario")
