@@ -269,7 +269,8 @@ int pfh_rasterize_noalloc(pfh_ctx *ctx, const int32_t *scene_ids, int32_t n, uin
 int pfh_scene_set_target(pfh_ctx *ctx, int32_t scene_id, void *device_rgba8, int64_t pitch_bytes);
 /* Device address and pitch of a scene's RGBA8 output (premultiplied). */
 int pfh_scene_target(pfh_ctx *ctx, int32_t scene_id, void **device_rgba8, int64_t *pitch_bytes);
-/* Copies a scene's RGBA8 output to host memory (CommandEncoder::read_texture, gpu/command_encoder.h:228). */
+/* Copies a scene's RGBA8 output to host memory (CommandEncoder::read_texture, gpu/command_encoder.h:228), after
+ * what the caller has queued on the default stream where it has the output's address. */
 int pfh_readback_rgba8(pfh_ctx *ctx, int32_t scene_id, void *dst, int64_t pitch_bytes);
 
 /*

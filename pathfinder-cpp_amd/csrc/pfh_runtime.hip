@@ -220,18 +220,26 @@ struct Stage {
     static constexpr size_t HALF = 1u << 20;
     uint8_t *ptr = nullptr;
     hipEvent_t ev[2] = {nullptr, nullptr};  // of the last copy of each half
+    hipEvent_t caller = nullptr;            // follow_caller's
     uint8_t *get() {
         if (!ptr) HIP_TRY(hipHostMalloc((void **)&ptr, 2 * HALF, hipHostMallocCoherent));
-        for (auto &e : ev)
-            if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        for (hipEvent_t *e : {&ev[0], &ev[1], &caller})
+            if (!*e) HIP_TRY(hipEventCreateWithFlags(e, hipEventDisableTiming));
         return ptr;
+    }
+    // What st does from here on comes after the work that the caller has queued on the default stream, and
+    // on streams that the default stream waits for, as with a copy on the default stream itself.
+    void follow_caller(hipStream_t st) {
+        (void)get();
+        HIP_TRY(hipEventRecord(caller, nullptr));
+        HIP_TRY(hipStreamWaitEvent(st, caller, 0));
     }
     void release() {
         if (ptr) (void)hipHostFree(ptr);
         ptr = nullptr;
-        for (auto &e : ev) {
-            if (e) (void)hipEventDestroy(e);
-            e = nullptr;
+        for (hipEvent_t *e : {&ev[0], &ev[1], &caller}) {
+            if (*e) (void)hipEventDestroy(*e);
+            *e = nullptr;
         }
     }
 };
@@ -2722,6 +2730,8 @@ int pfh_readback_rgba8(pfh_ctx *ctx, int32_t scene_id, void *dst, int64_t pitch_
         SceneHost &s = get_scene(ctx, scene_id);
         if (pitch_bytes < (int64_t)s.width * 4) throw PfhError{PFH_E_ARG, "bad pitch"};
         HIP_TRY(hipStreamSynchronize(ctx->w->stream));
+        // the caller may have written to an image whose address it has
+        if (s.lent || s.d_out != s.d_out_owned.as<uint8_t>()) ctx->stage.follow_caller(ctx->w->stream);
         read_rows(ctx, static_cast<uint8_t *>(dst), (size_t)pitch_bytes, s.d_out, (size_t)s.out_pitch,
                   (size_t)s.width * 4, (size_t)s.height);
     });

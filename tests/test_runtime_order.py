@@ -93,3 +93,36 @@ def release_scenario(hip):
 
 def test_release_waits_for_work_on_a_lent_image(recorder):
     run(recorder, "release_scenario")
+
+
+def readback_scenario(hip):
+    import numpy as np
+    import pfh
+    import scenegen
+
+    ctx = pfh.Context(0)
+    sc = scenegen.blob_scene(4, 500, 300, 20)
+    mine = np.zeros(2400 * 300, np.uint8)  # device memory of the caller's
+    for lent, pitch in ((True, 2000), (False, 2000), (False, 2400)):
+        sid = ctx.upload(sc)
+        if lent:
+            ctx.target(sid)
+        else:
+            ctx.set_target(sid, mine.ctypes.data, pitch)
+        ctx.rasterize([sid])
+        hip.take()
+        ctx.readback(sid)
+        calls = hip.take()
+        behind = set()  # streams that have waited for the default stream
+        recorded = set()
+        for c in calls:
+            if c[0] == "hipEventRecord" and c[2] in ("(nil)", "0x0"):
+                recorded.add(c[1])
+            elif c[0] == "hipStreamWaitEvent" and c[2] in recorded:
+                behind.add(c[1])
+            elif c[0] == "hipMemcpyAsync":
+                assert c[5] in behind, "the copy may pass work on the default stream"
+
+
+def test_readback_follows_the_default_stream(recorder):
+    run(recorder, "readback_scenario")
