@@ -2286,16 +2286,31 @@ hipError_t launch_bin_items(const BatchDev &b, hipStream_t s) {
     return hipGetLastError();
 }
 
+// LDS of k_bin_big: counts, packed deltas, walk queues and columns.
+template <bool EMIT>
+static constexpr size_t bin_big_lds(uint32_t tiles, uint32_t cols) {
+    return 4 * ((size_t)tiles + (EMIT ? 0 : (tiles + 1) / 2) + (1024 / 64) * WALK_QUEUE + cols);
+}
+
+// Lets k_bin_big take the LDS of the largest rect it is given, on the current device.  Before any launch,
+// and always to that one size: the attribute belongs to the process, so one set to a batch's own size could
+// fall below another thread's between its call and its launch.
+hipError_t init_bin_big() {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bin_big<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)bin_big_lds<false>(BIN_BIG_TILES, BIN_BIG_COLS));
+    if (e != hipSuccess) return e;
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bin_big<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)bin_big_lds<true>(BIN_BIG_TILES, BIN_BIG_COLS));
+}
+
 template <bool EMIT>
 static void launch_bin_t(const BatchDev &b, hipStream_t s) {
     const uint32_t merged = b.n_bin_group + blocks_for(b.n_bin_wave, 8);
     if (merged == 0) return;
     if (b.n_big) {  // first: they last longest
         const uint32_t cols = std::max(b.big_cols, 64u);  // at least what a block's sums take
-        const size_t lds = 4 * ((size_t)b.big_tiles + (EMIT ? 0 : (b.big_tiles + 1) / 2) + (1024 / 64) * WALK_QUEUE + cols);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bin_big<EMIT>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)lds);
-        hipLaunchKernelGGL(k_bin_big<EMIT>, dim3(std::min<uint32_t>(b.n_big, 1024)), dim3(1024), lds, s, b, b.big_tiles, cols);
+        hipLaunchKernelGGL(k_bin_big<EMIT>, dim3(std::min<uint32_t>(b.n_big, 1024)), dim3(1024),
+                           bin_big_lds<EMIT>(b.big_tiles, cols), s, b, b.big_tiles, cols);
     }
     if (merged <= BIN_MERGED_BLOCKS) {
         hipLaunchKernelGGL(k_bin<EMIT>, dim3(merged), dim3(512), 0, s, b);

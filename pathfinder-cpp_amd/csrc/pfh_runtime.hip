@@ -29,6 +29,7 @@ hipError_t scan_entries(const BatchDev &b, hipStream_t s);
 hipError_t scan_paths(const BatchDev &b, hipStream_t s);
 hipError_t scan_counted(uint32_t *inout, const uint32_t *n_ptr, uint32_t cap, unsigned long long *state, hipStream_t s);
 hipError_t launch_flatten(const BatchDev &b, bool emit, uint32_t chunk, hipStream_t s);
+hipError_t init_bin_big();
 hipError_t launch_bin(const BatchDev &b, bool emit, hipStream_t s);
 hipError_t launch_propagate(const BatchDev &b, hipStream_t s);
 uint32_t entry_waves(uint32_t n_bin_group, uint32_t n_bin_wave);
@@ -2520,6 +2521,7 @@ int pfh_create(int device, pfh_ctx **out) {
         HIP_TRY(hipGetDeviceCount(&n));
         if (device < 0 || device >= n) throw PfhError{PFH_E_ARG, "no HIP device " + std::to_string(device)};
         HIP_TRY(hipSetDevice(device));
+        HIP_TRY(init_bin_big());
         ctx->main.create();
         ctx->fixed.create(1);  // plain mode: one scene per launch
         ctx->fixed.use_arena(scratch_on_device(device), PFH_SCRATCH_BYTES);

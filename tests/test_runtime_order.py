@@ -126,3 +126,36 @@ def readback_scenario(hip):
 
 def test_readback_follows_the_default_stream(recorder):
     run(recorder, "readback_scenario")
+
+
+def large_blocks_scenario(hip):
+    import numpy as np
+    import pfh
+    import scenegen
+
+    def whole_canvas(seed, w, h):  # a blend mode whose rect is the view box
+        sc = scenegen.blob_scene(seed, w, h, 10)
+        sc.path_blend = np.full(sc.n_paths, 2, np.uint8)  # source-in
+        return sc
+
+    a, b = pfh.Context(0), pfh.Context(0)
+    ids = [(c, c.upload(whole_canvas(k, w, h))) for k, (c, w, h) in enumerate([(a, 2500, 2400), (b, 1300, 1200), (a, 1400, 1200)])]
+    for c, sid in ids:
+        for flags in (pfh.PFH_PLAIN, pfh.PFH_BATCHED | pfh.PFH_NO_GRAPH):
+            c.rasterize([sid], flags)
+    limits, launches = {}, 0
+    for call in hip.take():
+        if call[0] == "hipFuncSetAttribute":
+            assert limits.setdefault(call[1], int(call[3])) == int(call[3]), "the limit is the process's: another thread's launch may need more"
+        elif call[0] == "hipLaunchKernel" and int(call[2]) > 0:
+            assert int(call[2]) <= limits[call[1]]
+            launches += 1
+    assert launches >= 12
+    hip.lib.rec_attr_error(1)
+    with pytest.raises(pfh.PfhError):
+        c = pfh.Context(0)
+        c.rasterize([c.upload(whole_canvas(9, 1300, 1200))])
+
+
+def test_one_limit_for_large_blocks(recorder):
+    run(recorder, "large_blocks_scenario")
