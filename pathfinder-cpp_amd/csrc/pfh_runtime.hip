@@ -124,9 +124,9 @@ struct Arena {
 // Device blocks that one use gave back and the next takes: a program that uploads a scene every frame
 // otherwise spends a millisecond on hipMalloc and hipFree (which waits for the device).  Blocks of
 // 2^k bytes up to BLOCK_BYTES, at most POOL_BYTES of them in all; the rest goes back to the runtime at once, the
-// others when the context ends.  A block is given back only when the device is done with it (for an
-// image whose address a caller has, the whole device: see pfh_scene_release), and a context is used by
-// one host thread at a time.
+// others when the context ends or any of its allocations finds no room.  A block is given back only when
+// the device is done with it (for an image whose address a caller has, the whole device: see
+// pfh_scene_release), and a context is used by one host thread at a time.
 struct BlockPool {
     static constexpr size_t BLOCK_BYTES = 64u << 20, POOL_BYTES = 256u << 20;
     std::multimap<size_t, void *> blocks;
@@ -162,6 +162,7 @@ struct DevBuf {
     size_t bytes = 0;
     Arena *arena = nullptr;
     BlockPool *pool = nullptr;  // its blocks come from there and go back there
+    BlockPool *spare = nullptr;  // without a pool of its own: the one whose blocks make room where none is left
     void ensure(size_t need) {
         if (need <= bytes && ptr) return;
         if (arena) {
@@ -189,9 +190,10 @@ struct DevBuf {
         bytes = 0;
         g_alloc_generation++;
         hipError_t e = hipMalloc(&ptr, cap);
-        if (e != hipSuccess && pool && !pool->blocks.empty()) {  // the kept blocks may be what is missing
+        BlockPool *const kept = pool ? pool : spare;
+        if (e != hipSuccess && kept && !kept->blocks.empty()) {  // the kept blocks may be what is missing
             (void)hipGetLastError();
-            pool->clear();
+            kept->clear();
             e = hipMalloc(&ptr, cap);
         }
         if (e != hipSuccess) {
@@ -410,8 +412,9 @@ struct Workspace {
     Arena arena;                     // work buffers carved from a fixed region (arena.base set)
 
     // Stream, events and pinned host buffers for `table_scenes` scenes per launch, made once so
-    // that a launch of at most that many scenes creates nothing.
-    void create(size_t table_scenes = 0) {
+    // that a launch of at most that many scenes creates nothing.  spare: the work buffers' (DevBuf::spare).
+    void create(BlockPool *spare, size_t table_scenes = 0) {
+        for (DevBuf *b : all_buffers()) b->spare = spare;
         HIP_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         // of these the host waits for ev1 alone: the others only time, without a fence for it (3 us less each)
         HIP_TRY(hipEventCreateWithFlags(&ev0, hipEventDisableSystemFence));
@@ -2522,8 +2525,9 @@ int pfh_create(int device, pfh_ctx **out) {
         if (device < 0 || device >= n) throw PfhError{PFH_E_ARG, "no HIP device " + std::to_string(device)};
         HIP_TRY(hipSetDevice(device));
         HIP_TRY(init_bin_big());
-        ctx->main.create();
-        ctx->fixed.create(1);  // plain mode: one scene per launch
+        ctx->main.create(&ctx->pool);
+        ctx->fixed.create(&ctx->pool, 1);  // plain mode: one scene per launch
+        for (DevBuf *b : {&ctx->mlp_params, &ctx->mlp_x, &ctx->mlp_h, &ctx->mlp_out}) b->spare = &ctx->pool;
         ctx->fixed.use_arena(scratch_on_device(device), PFH_SCRATCH_BYTES);
     });
     if (rc != PFH_OK) {
@@ -2940,6 +2944,9 @@ int pfh_path_counts(pfh_ctx *ctx, int32_t scene_id, int32_t *lines, int32_t *fil
 namespace {
 struct MlpDevEval {
     DevBuf params, x, h, out;
+    explicit MlpDevEval(pfh_ctx *ctx) {
+        for (DevBuf *b : {&params, &x, &h, &out}) b->spare = &ctx->pool;
+    }
 };
 }  // namespace
 
@@ -2948,7 +2955,7 @@ int pfh_mlp_eval(pfh_ctx *ctx, const float *params, const float *x, int64_t n, f
     return run_guarded(ctx, [&] {
         const int64_t np = mlp_param_count();
         if (n == 0) return;
-        MlpDevEval d;
+        MlpDevEval d(ctx);
         d.params.ensure(4 * np);
         d.x.ensure(4 * n * 12);
         d.h.ensure(4 * n * 128);
@@ -2966,6 +2973,9 @@ int pfh_mlp_eval(pfh_ctx *ctx, const float *params, const float *x, int64_t n, f
 namespace {
 struct MlpDev {
     DevBuf params, m, v, grad, loss, x, t, h, out, scratch;
+    explicit MlpDev(pfh_ctx *ctx) {
+        for (DevBuf *b : {&params, &m, &v, &grad, &loss, &x, &t, &h, &out, &scratch}) b->spare = &ctx->pool;
+    }
 };
 static void mlp_grad_dev(pfh_ctx *ctx, MlpDev &d, const float *x, const float *t, int64_t n) {
     HIP_TRY(mlp_forward(d.params.as<float>(), x, n, d.h.as<float>(), d.out.as<float>(), ctx->w->stream));
@@ -2979,7 +2989,7 @@ int pfh_mlp_grad(pfh_ctx *ctx, const float *params, const float *x, const float 
     if (!ctx || !params || !x || !target || !grad || !loss || n <= 0) return PFH_E_ARG;
     return run_guarded(ctx, [&] {
         const int64_t np = mlp_param_count();
-        MlpDev d;
+        MlpDev d(ctx);
         d.params.ensure(4 * np);
         d.grad.ensure(4 * np);
         d.loss.ensure(4);
@@ -3005,7 +3015,7 @@ int pfh_mlp_train(pfh_ctx *ctx, const float *x, const float *target, int64_t n, 
     return run_guarded(ctx, [&] {
         const int64_t np = mlp_param_count();
         const int64_t bs = std::min<int64_t>(batch, n);
-        MlpDev d;
+        MlpDev d(ctx);
         d.params.ensure(4 * np);
         d.m.ensure(4 * np);
         d.v.ensure(4 * np);
@@ -3168,7 +3178,7 @@ int pfh_server_start(pfh_ctx *ctx, int32_t slots, int64_t memory_budget_bytes, i
         sv->flags = flags & (PFH_PREDICT | PFH_NO_GRAPH);
         for (int32_t i = 0; i < slots; i++) {
             sv->slots.push_back(std::make_unique<Slot>());
-            sv->slots.back()->ws.create();
+            sv->slots.back()->ws.create(&ctx->pool);
         }
         ctx->server = std::move(sv);
     });

@@ -159,3 +159,56 @@ def large_blocks_scenario(hip):
 
 def test_one_limit_for_large_blocks(recorder):
     run(recorder, "large_blocks_scenario")
+
+
+def kept_blocks_scenario(hip):
+    import numpy as np
+    import pfh
+    import scenegen
+
+    MB = 1 << 20
+    big, other = scenegen.blob_scene(6, 3000, 3000, 50), scenegen.blob_scene(7, 900, 900, 300)
+
+    def kept(ctx):  # what two uploads leave with the context
+        before = hip.lib.rec_held()
+        for sid in [ctx.upload(big) for _ in range(2)]:
+            ctx.release(sid)
+        assert hip.lib.rec_held() - before >= 100 * MB
+
+    def work(use):  # how much `use` allocates
+        held = hip.lib.rec_held()
+        use()
+        return hip.lib.rec_held() - held
+
+    for flags in (pfh.PFH_PLAIN, pfh.PFH_BATCHED | pfh.PFH_NO_GRAPH):
+        ctx = pfh.Context(0)
+        ids = [ctx.upload(other)]
+        need = work(lambda: ctx.rasterize(ids, flags))
+        ctx.close()
+        ctx = pfh.Context(0)
+        ids = [ctx.upload(other)]
+        kept(ctx)
+        assert MB < need < 100 * MB
+        hip.lib.rec_limit(hip.lib.rec_held() + need // 2)  # enough once the kept blocks are given back
+        ctx.rasterize(ids, flags)
+        hip.lib.rec_limit(1 << 40)
+        ctx.close()
+    ctx = pfh.Context(0)  # the request loop's slots
+    ids = [ctx.upload(other)]
+    kept(ctx)
+    ctx.server_start(slots=1, memory_budget=1 << 30, max_batch=4, flags=pfh.PFH_NO_GRAPH)
+    hip.lib.rec_limit(hip.lib.rec_held() + MB)
+    ctx.submit(ids[0])
+    assert len(ctx.poll(wait_ms=5.0)) == 1
+    ctx.server_stop()
+    hip.lib.rec_limit(1 << 40)
+    kept(ctx)  # the predictor's buffers
+    x = np.zeros((40000, 12), np.float32)
+    hip.lib.rec_limit(hip.lib.rec_held() + MB)
+    ctx.mlp_eval(np.zeros(pfh.MLP_PARAMS, np.float32), x)
+    hip.lib.rec_limit(1 << 40)
+    ctx.close()
+
+
+def test_kept_blocks_make_room(recorder):
+    run(recorder, "kept_blocks_scenario")
