@@ -236,7 +236,8 @@ const char *pfh_last_error(const pfh_ctx *ctx);
  * Packs a scene (SegmentsIter order, core/data/contour.cpp:110-173; path tile rects,
  * core/data/built_path.cpp:8-34) and makes it resident on the device.  Replaces
  * SceneBuilderD3D11::build's CPU packing (core/d3d11/gpu_data.cpp:79-115,
- * core/d3d11/scene_builder.cpp:26-58).  *scene_id receives a handle.
+ * core/d3d11/scene_builder.cpp:26-58).  *scene_id receives a handle.  The scene's own image starts
+ * transparent.
  */
 int pfh_scene_upload(pfh_ctx *ctx, const pfh_scene_desc *desc, int32_t *scene_id);
 /* Where pfh_scene_target gave out the scene's own image, work queued on it on any stream ends first. */
