@@ -13,9 +13,10 @@ every scene from outlines resident in HBM to its RGBA8 framebuffer in HBM:
 
 The ``roofline`` object covers the slower of k_fill_masks and k_composite in the timed batched
 steps: HIP events recorded as nodes of the replayed graph on the library's stream bracket each
-kernel; achieved = algorithmic bytes / that time.  For the batch workload it also carries the
-kernel's HBM bytes per launch (``traffic``) and the share of the chip's VALU issue rate it uses
-(``valu_issue_share``), both from the rocprofv3 counter runs summarised in profiles/.
+kernel; achieved = the HBM bytes its counters show per launch (``traffic``) / that time, beside the
+share of the chip's VALU issue rate it uses (``valu_issue_share``), both from the rocprofv3 counter
+runs of the workload summarised in profiles/.  ``algorithmic_bytes`` counts every layer's mask and
+entry, which the kernels leave out where they cannot show.
 
 Also reported: ``single_4k`` (one 4096x4096 scene of 10 000 paths, scenegen.single_scene_4k,
 the same two modes and roofline), ``stress`` (scenegen.stress_scene: 4096x4096, 2 000 star
@@ -60,8 +61,7 @@ WORKLOADS = {
 def fill_bytes(st):
     # 12 B per fill read (reference Fill layout), 8 B alpha-tile index + 4 B backdrop/ctrl
     # per alpha tile, 256 B of u8 coverage written per 16x16 alpha tile; over the alpha tiles
-    # draw entries sample and their fills (the fill kernel leaves out those under so many
-    # translucent layers that they cannot show; they count here as well).
+    # draw entries sample and their fills.
     return 12 * st["fills_masked"] + 8 * st["alpha_masked"] + 4 * st["alpha_masked"] + 256 * st["alpha_masked"]
 
 
@@ -72,11 +72,12 @@ def composite_bytes(st, pixels, n_paths):
 
 
 PROFILES = os.path.join(ROOT, "profiles")
+PROFILED = {"batch": "batch256", "single": "single4k", "stress": "stress"}  # their files' names there
 
 
 def profiled(file, key, kernel):
-    """A per-launch figure of `kernel` on the 256-scene batch from a committed rocprofv3 summary
-    (its `key: kernel=value ...` line); None without it."""
+    """A per-launch figure of `kernel` from a committed rocprofv3 summary (its `key: kernel=value ...`
+    line); None without it."""
     try:
         for line in open(os.path.join(PROFILES, file)):
             if line.startswith(key + ":"):
@@ -87,26 +88,29 @@ def profiled(file, key, kernel):
     return None
 
 
-def roofline(st, fill_ms, comp_ms, pixels, n_paths, traffic_known=False):
-    fb, cb = fill_bytes(st), composite_bytes(st, pixels, n_paths)
-    fill_gbs = fb / (fill_ms * 1e-3) / 1e9
-    comp_gbs = cb / (comp_ms * 1e-3) / 1e9
-    if comp_ms >= fill_ms:
-        kern, nbytes, ms, gbs = "k_composite", cb, comp_ms, comp_gbs
-    else:
-        kern, nbytes, ms, gbs = "k_fill_masks", fb, fill_ms, fill_gbs
-    # HBM bytes per launch (FETCH_SIZE + WRITE_SIZE, calibrated) and the share of the chip's VALU
-    # issue rate the kernel uses, both from the batch workload's counter runs
-    traffic = profiled("batch256_hbm_traffic.md", "traffic_bytes_per_launch", kern) if traffic_known else None
-    valu = profiled("batch256_sq_counters.md", "valu_issue_share", kern) if traffic_known else None
-    return {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": int(traffic) if traffic is not None else None,
-            "valu_issue_share": valu,
-            "counters": "profiles/batch256_hbm_traffic.md, profiles/batch256_sq_counters.md" if traffic_known else None,
-            "kernel": kern,
-            "algorithmic_bytes": int(nbytes), "kernel_ms": round(ms, 4),
-            "other": {"k_fill_masks_gbs": round(fill_gbs, 1), "k_fill_masks_ms": round(fill_ms, 4),
-                      "k_composite_gbs": round(comp_gbs, 1), "k_composite_ms": round(comp_ms, 4)}}
+def roofline(st, fill_ms, comp_ms, pixels, n_paths, profile):
+    """The slower of the two pixel kernels against HBM: the bytes its counters show per launch
+    (FETCH_SIZE + WRITE_SIZE, calibrated, of the `profile` workload's counter runs) over this run's kernel
+    time.  The algorithmic bytes count every layer's mask and entry; the kernels leave out those that
+    cannot show, so what they imply over that time is no bandwidth and is not given as one."""
+    ms = {"k_fill_masks": fill_ms, "k_composite": comp_ms}
+    algorithmic = {"k_fill_masks": fill_bytes(st), "k_composite": composite_bytes(st, pixels, n_paths)}
+    traffic = {k: profiled(f"{profile}_hbm_traffic.md", "traffic_bytes_per_launch", k) for k in ms}
+    gbs = {k: traffic[k] / (ms[k] * 1e-3) / 1e9 if traffic[k] is not None else None for k in ms}
+    kern = "k_composite" if comp_ms >= fill_ms else "k_fill_masks"
+
+    def r(v, digits):
+        return None if v is None else round(v, digits)
+
+    return {"bound": "hbm", "achieved": r(gbs[kern], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": None if gbs[kern] is None else round(gbs[kern] / HBM_PEAK_GBS, 4),
+            "traffic": None if traffic[kern] is None else int(traffic[kern]),
+            # the share of the chip's VALU issue rate the kernel uses
+            "valu_issue_share": profiled(f"{profile}_sq_counters.md", "valu_issue_share", kern),
+            "counters": None if gbs[kern] is None else f"profiles/{profile}_hbm_traffic.md",
+            "kernel": kern, "kernel_ms": round(ms[kern], 4), "algorithmic_bytes": int(algorithmic[kern]),
+            "other": {f"{k}_{what}": v for k in ms for what, v in
+                      (("gbs", r(gbs[k], 1)), ("ms", round(ms[k], 4)), ("algorithmic_bytes", int(algorithmic[k])))}}
 
 
 def measure(ctx, ids, flags, steps, warmup, plain_steps, schedule=None):
@@ -341,7 +345,7 @@ def main():
         "counts": {k: st[k] for k in ("segments", "lines", "tiles", "fills", "alpha_tiles", "entries",
                                       "alpha_entries", "fills_masked", "alpha_masked", "fb_tiles", "retries",
                                       "host_syncs")},
-        "roofline": roofline(st, fill_ms, comp_ms, pixels, n_paths, traffic_known=args.config == "batch"),
+        "roofline": roofline(st, fill_ms, comp_ms, pixels, n_paths, PROFILED[args.config]),
         "autotune": tuning,
     }
 
@@ -353,7 +357,8 @@ def main():
                             "ms_per_step": round(b_s * 1e3, 4), "plain_ms_per_step": round(p_s * 1e3, 4),
                             "mpix_per_s": round(one.width * one.height / b_s / 1e6, 1),
                             "plain_stage_ms": {k: round(v, 4) for k, v in zip(names, s_ms)},
-                            "roofline": roofline(st1, f_ms, c_ms, one.width * one.height, one.n_paths),
+                            "roofline": roofline(st1, f_ms, c_ms, one.width * one.height, one.n_paths,
+                                                 PROFILED["single"]),
                             "autotune": tune1}
         ctx.release(sid)
         print(f"[bench] single_4k batched {b_s * 1e3:.3f} ms/step", flush=True)
