@@ -67,9 +67,12 @@ constexpr uint32_t RULE_CLIP_OWN = 0x2u;
 constexpr int BIN_WAVE_TILES = 512;
 constexpr int BIN_WAVE_COLS = 128;
 constexpr int BIN_WAVE_SEGS = 64;       // more segments than lanes: the group class (its walk is 8x wider)
-// With the walk queues 27 KB (emit) and 40 KB (count) of LDS in blocks of 512, as much as the wave class's slices take
-// there.  Paths past it are slow (global atomics): the 4096^2 scene of 10^4 paths, a few of whose rects
-// have 4 600 to 5 700 tiles, 573 us with 4600, 497 with 5700.
+// What the LDS of a 512-thread block holds in the count pass, packed deltas, columns and walk queues with
+// the counts, beside as much as the wave class's slices take there (40 KB, 4 blocks a CU; 27 KB to emit).
+// Paths past it go through global atomics: a 4096^2 scene of 10^4 paths, a few of whose rects have 4 600 to
+// 5 700 tiles, takes 573 us with 4 600 here and 497 so.  In batches binned by a launch per class, whose
+// blocks of 256 take as much LDS, 24 scenes of blobs up to 4096^2 take 825 and 790 us, 48 2 493 and 2 474, 24
+// up to 2048^2 1 234 and 1 243.
 constexpr int BIN_GROUP_TILES = 5700;
 constexpr int BIN_GROUP_COLS = 512;
 // Group-class paths past those limits, up to these, take a block with more LDS (at most 160 KB less 1.5) where

@@ -1854,7 +1854,8 @@ static void ensure_tables(Workspace &w, const Plan &pl) {
 // Where the flattener keeps its curves' bits (8 bytes a segment) between its two passes.  A fixed
 // region has no room set aside for them: they lie in the tile and entry arrays at its start, which
 // no kernel touches before the chords are out, or, with more segments than those hold (5 per tile),
-// nowhere: every curve is then flattened twice.
+// nowhere: every curve is then flattened twice, which is 14 us of 188 at 512^2 (132 000 segments in 8 300 tiles)
+// and 27 of 219 at 1240 x 1754 (266 000 in 15 000).
 static unsigned long long *curve_bits(Workspace &w, const Plan &pl) {
     if (!w.arena.base) return w.seg_mask.as<unsigned long long>();
     uint8_t *const at = w.tile_delta.as<uint8_t>(), *end = at;
