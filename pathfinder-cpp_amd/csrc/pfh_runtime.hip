@@ -1613,6 +1613,7 @@ struct Plan {
     bool clips = false;   // some scene has clip paths
     bool paints = false;  // some scene has gradient paints
     bool clear_outside = false;  // some scene's target reaches past its view box's tiles (and is cleared)
+    bool blank = false;          // some scene's own image is written for the first time
     uint32_t max_rows = 0;       // tile rows of the tallest target
     uint32_t clip_levels = 0;  // deepest clip nesting level of the batch
     uint32_t cap_f = 0, cap_a = 0, cap_e = 0, cap_l = 0;
@@ -1742,6 +1743,7 @@ static void write_tables(pfh_ctx *ctx, Plan &pl, bool load_dst) {
         SceneHost &s = get_scene(ctx, pl.ids[k]);
         SceneDev &d = ctx->w->h_table[k];
         if (load_dst) need_image(ctx, s);
+        pl.blank = pl.blank || (s.blank && s.draws_own());
         d.pts = s.d_pts.as<float2>();
         d.segs = s.d_segs.as<uint2>();
         d.seg_path = s.d_seg_path.as<uint32_t>();
@@ -1952,6 +1954,7 @@ static BatchDev batch_dev(Workspace &w, const Plan &pl, bool dump) {
 
 // A composite of every scene's target is enqueued, which writes it whole.
 static void image_written(pfh_ctx *ctx, const Plan &pl) {
+    if (!pl.blank) return;
     for (int32_t id : pl.ids) {
         SceneHost &s = get_scene(ctx, id);
         if (s.draws_own()) s.blank = false;
