@@ -1517,7 +1517,6 @@ static int scene_upload_desc(pfh_ctx *ctx, const pfh_scene_desc *d) {
             s->n_breaks++;
         }
     }
-    HIP_TRY(hipSetDevice(ctx->device));
     Upload up;
     up.add(s->d_pts, pts);
     up.add(s->d_segs, segs_dev);
@@ -2521,6 +2520,21 @@ static double percentile(std::vector<double> v, double q) {
     return v[k];
 }
 
+// The context's device for calls that had not changed the caller's current one, which they give back.
+struct OnDevice {
+    int before = -1;
+    explicit OnDevice(const pfh_ctx *ctx) {
+        int now = 0;
+        HIP_TRY(hipGetDevice(&now));
+        if (now == ctx->device) return;
+        HIP_TRY(hipSetDevice(ctx->device));
+        before = now;
+    }
+    ~OnDevice() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
+
 // A failed HIP call also leaves its status as the thread's last error, which the launch helpers
 // read back after each launch: clear it on the way out so that a later, unrelated call does not
 // report it again.
@@ -2587,7 +2601,10 @@ const char *pfh_last_error(const pfh_ctx *ctx) { return ctx ? ctx->err.c_str() :
 
 int pfh_scene_upload(pfh_ctx *ctx, const pfh_scene_desc *desc, int32_t *scene_id) {
     if (!ctx || !scene_id) return PFH_E_ARG;
-    return run_guarded(ctx, [&] { *scene_id = scene_upload(ctx, desc); });
+    return run_guarded(ctx, [&] {
+        HIP_TRY(hipSetDevice(ctx->device));
+        *scene_id = scene_upload(ctx, desc);
+    });
 }
 
 int pfh_gradient_compile(const pfh_gradient *g, const float *stop_offsets, const uint32_t *stop_rgba,
@@ -2650,6 +2667,7 @@ int pfh_scene_release(pfh_ctx *ctx, int32_t scene_id) {
     if (!ctx) return PFH_E_ARG;
     return run_guarded(ctx, [&] {
         SceneHost &s = get_scene(ctx, scene_id);
+        OnDevice on(ctx);
         if (ctx->server) {
             Server &sv = *ctx->server;
             bool queued = false;
@@ -2672,6 +2690,7 @@ int pfh_scene_features(pfh_ctx *ctx, int32_t scene_id, float *out) {
     if (!ctx || !out) return PFH_E_ARG;
     return run_guarded(ctx, [&] {
         SceneHost &s = get_scene(ctx, scene_id);
+        OnDevice on(ctx);
         const size_t n = sizeof(float) * N_FEATURES * (size_t)s.n_paths;
         read_rows(ctx, reinterpret_cast<uint8_t *>(out), n, s.d_features.as<uint8_t>(), n, n, n ? 1 : 0);
     });
@@ -2754,6 +2773,7 @@ int pfh_scene_target(pfh_ctx *ctx, int32_t scene_id, void **device_rgba8, int64_
         SceneHost &s = get_scene(ctx, scene_id);
         if (s.draws_own()) {
             if (s.blank) {
+                OnDevice on(ctx);
                 need_image(ctx, s);
                 HIP_TRY(hipStreamSynchronize(ctx->w->stream));
             }
@@ -2769,6 +2789,7 @@ int pfh_readback_rgba8(pfh_ctx *ctx, int32_t scene_id, void *dst, int64_t pitch_
     return run_guarded(ctx, [&] {
         SceneHost &s = get_scene(ctx, scene_id);
         if (pitch_bytes < (int64_t)s.width * 4) throw PfhError{PFH_E_ARG, "bad pitch"};
+        OnDevice on(ctx);
         HIP_TRY(hipStreamSynchronize(ctx->w->stream));
         // the caller may have written to an image whose address it has
         if (s.lent || !s.draws_own()) ctx->stage.follow_caller(ctx->w->stream);

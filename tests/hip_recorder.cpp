@@ -15,7 +15,7 @@ std::map<const void *, std::string> g_names;   // host function -> kernel
 std::map<const void *, size_t> g_vars, g_blocks;
 std::map<const void *, void *> g_var_mem;
 size_t g_held = 0, g_limit = ~(size_t)0;
-int g_attr_error = 0, g_last = 0;
+int g_attr_error = 0, g_last = 0, g_device = 0;
 uintptr_t g_handles = 0x1000;
 struct Dim3 {
     uint32_t x, y, z;
@@ -75,10 +75,18 @@ int hipFuncSetAttribute(const void *f, int attr, int value) {
     return done(g_attr_error);
 }
 int hipGetDeviceCount(int *n) {
-    *n = 1;
+    *n = 2;
     return 0;
 }
-int hipSetDevice(int) { return 0; }
+int hipSetDevice(int d) {
+    g_device = d;
+    say("hipSetDevice %d", d);
+    return 0;
+}
+int hipGetDevice(int *d) {
+    *d = g_device;
+    return 0;
+}
 const char *hipGetErrorString(int) { return "recorded error"; }
 int hipGetLastError() {
     const int e = g_last;

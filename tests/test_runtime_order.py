@@ -212,3 +212,46 @@ def kept_blocks_scenario(hip):
 
 def test_kept_blocks_make_room(recorder):
     run(recorder, "kept_blocks_scenario")
+
+
+def device_scenario(hip):
+    import pfh
+    import scenegen
+
+    ctx = pfh.Context(1)
+
+    def use(call, keeps=True):
+        """`call` while another library has device 0 current."""
+        hip.lib.hipSetDevice(0)
+        hip.take()
+        got = call()
+        device = 0
+        for c in hip.take():
+            if c[0] == "hipSetDevice":
+                device = int(c[1])
+            elif c[0] in ("hipMalloc", "hipHostMalloc", "hipEventCreate", "hipLaunchKernel", "hipDeviceSynchronize") or \
+                    c[0] == "hipEventRecord" and c[2] in ("(nil)", "0x0"):
+                assert device == 1, f"{c[0]} goes to the caller's device, not the context's"
+        assert device == 0 or not keeps, "the caller's device is another one afterwards"
+        return got
+
+    def strokes():  # the recorder's kernels leave no outlines: the stroker may refuse what it reads back
+        try:
+            ctx.upload(scenegen.dashed_stroke_scene(9, size=200, n=6))
+        except pfh.PfhError:
+            pass
+
+    use(strokes, keeps=False)
+    scene = scenegen.blob_scene(8, 500, 300, 20)
+    ids = [use(lambda: ctx.upload(scene), keeps=False) for _ in range(2)]
+    use(lambda: ctx.readback(ids[0]))
+    use(lambda: ctx.target(ids[1]))
+    use(lambda: ctx.rasterize(ids), keeps=False)
+    use(lambda: ctx.readback(ids[1]))
+    use(lambda: ctx.features(ids[0]))
+    for i in ids:
+        use(lambda: ctx.release(i))
+
+
+def test_calls_go_to_the_context_s_device(recorder):
+    run(recorder, "device_scenario")
